@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "cac_internal.h"
@@ -38,18 +39,6 @@ constexpr int kLeafMax = 128;
 // the banks instead of hitting one: with 128 int64 per row every row starts on
 // the same bank and a column access is a 64-way bank conflict.
 constexpr int kLeafStride = kLeafMax + 1;
-
-__device__ inline void wave_argmax(int64_t& key, uint32_t& idx) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    int64_t k2 = __shfl_xor(key, d, 64);
-    uint32_t i2 = __shfl_xor(idx, d, 64);
-    if (k2 > key || (k2 == key && i2 < idx)) {
-      key = k2;
-      idx = i2;
-    }
-  }
-}
 
 __device__ inline int64_t wave_sum_i64(int64_t x) { return (int64_t)wave_sum<uint64_t>((uint64_t)x); }
 
@@ -142,162 +131,118 @@ __global__ void __launch_bounds__(64) k_ks_cert(const KsLeaf* __restrict__ leave
   }
 }
 
-// Merge vertex `last` into `prev` in the LDS matrix (row and column); lanes own
-// columns lane and lane + 64.
-template <typename T>
-__device__ inline void leaf_merge(T* A, uint32_t V, uint32_t prev, uint32_t last, bool (&alive)[2]) {
-  const int lane = threadIdx.x;
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t x = lane + 64 * h;
-    if (x < V && x != prev && x != last) {
-      const T v = A[prev * kLeafStride + x] + A[last * kLeafStride + x];
-      A[prev * kLeafStride + x] = v;
-      A[x * kLeafStride + prev] = v;
-    }
-  }
-  __syncthreads();
-  if (lane == 0) {
-    A[prev * kLeafStride + last] = 0;
-    A[last * kLeafStride + prev] = 0;
-  }
-  if ((uint32_t)lane == last) alive[0] = false;
-  if ((uint32_t)lane + 64 == last) alive[1] = false;
-  __syncthreads();
-}
-
-// The base case of co_mincut_base_case.hpp:164-185 on a leaf in LDS: PR-1 pass
-// at the bound (contracting an edge of weight >= bound keeps every cut below the
-// bound, so min(bound, min cut) is unchanged), then Stoer-Wagner (J. ACM 44(4),
-// 1997): maximum adjacency order, cut of the phase, merge of the last two
-// vertices.  Result min(cut, bound).  T: the LDS entry type, uint32_t for a
-// leaf of total weight below 2^32 (66 KiB, two leaves per CU) and int64_t
-// otherwise (132 KiB, one per CU).
+// The base case of co_mincut_base_case.hpp:164-185 on a leaf in LDS: result
+// min(bound, minimum cut).  Phases of maximum adjacency orders (Stoer and
+// Wagner, J. ACM 44(4), 1997), each followed by the contractions of Nagamochi
+// and Ibaraki (SIAM J. Discrete Math. 5(1), 1992): with `best` the smallest cut
+// seen (the bound and the smallest degree to begin with), a vertex whose weight
+// to the vertices ordered before it reaches `best` is connected to its
+// predecessor by at least that much, so no cut below `best` separates the two.
+// All such pairs of a phase are contracted at once; they are runs of
+// consecutive vertices of the order.  The last vertex's weight is its degree
+// and lowers `best` if it is smaller, so every phase contracts its last pair.
+//
+// A phase is a chain of V - 1 steps (a wave maximum, two ballots, one LDS row),
+// so the phases are the cost.  Contracting only the last pair (and edges that
+// alone reach the bound) took V - 1 phases of a leaf that no such edge
+// collapses: 49 trials of a complete graph of 700 vertices, 1568 leaves of 128
+// in 64-bit entries, 21.4 ms; a phase contracts most of such a leaf at once.
+// T: the LDS entry type, uint32_t for a leaf of total weight below 2^32 (66 KiB,
+// two leaves per CU) and int64_t otherwise (132 KiB, one per CU).
 template <typename T>
 __global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf* __restrict__ leaves, const uint32_t* __restrict__ sw_list,
                                               int64_t* __restrict__ results) {
+  typedef typename std::make_unsigned<T>::type U;
   __shared__ T A[kLeafMax * kLeafStride];
   const KsLeaf lf = leaves[sw_list[blockIdx.x]];
   const uint32_t V = lf.k;
-  const int lane = threadIdx.x;
-  int64_t total = 0;  // sum of all entries: no key of the maximum adjacency order exceeds it
+  if (V < 2) return;  // no cut: the result keeps the bound
+  const uint32_t lane = threadIdx.x;
+  bool alive[2] = {lane < V, lane + 64 < V};
+  U deg[2] = {0, 0};
+#pragma unroll 8
   for (uint32_t r = 0; r < V; ++r)
-    for (uint32_t x = lane; x < V; x += 64) {
-      const int64_t a = lf.mat[(size_t)r * V + x];
-      A[r * kLeafStride + x] = (T)a;
-      total += a;
-    }
-  total = wave_sum_i64(total);
-  // keys below 2^55 pack with their vertex as (key << 8) | (255 - vertex), so the
-  // largest key, then the smallest vertex, is one unsigned wave maximum
-  const bool packed = total < (int64_t)1 << 55;
-  __syncthreads();
-  bool alive[2] = {(uint32_t)lane < V, (uint32_t)(lane + 64) < V};
-  int64_t best = INT64_MAX;
-  uint32_t nalive = V;
-  // PR-1: repeatedly contract an edge of weight >= bound (the lowest live row
-  // holding one, its lowest live column); merged-away columns hold stale values
-  // and are skipped.  col[h] is the first such column of row lane + 64 h.  A
-  // merge of last into prev (prev < last) changes only row prev and column
-  // prev among the live entries, and only upwards, so a row other than prev
-  // keeps its first column unless column prev now qualifies before it; a row
-  // whose first column was last finds prev there (it took last's weight), and
-  // row prev alone is scanned again.
-  auto first_col = [&](uint32_t u) {
-    const uint64_t live_lo = __ballot(alive[0]), live_hi = __ballot(alive[1]);
-    uint32_t c = kNoSlot;
-    for (uint32_t x = 0; x < V; ++x) {
-      const bool live_x = ((x < 64 ? live_lo : live_hi) >> (x & 63)) & 1ull;
-      if (live_x && x != u && (int64_t)A[u * kLeafStride + x] >= lf.bound) {
-        c = x;
-        break;
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t x = lane + 64 * h;
+      if (x < V) {
+        const U a = (U)lf.mat[(size_t)r * V + x];
+        A[r * kLeafStride + x] = (T)a;
+        deg[h] += a;  // symmetric: the column sum is the degree
       }
     }
-    return c;
-  };
-  uint32_t col[2] = {kNoSlot, kNoSlot};
+  __syncthreads();
+  U best = lf.bound <= 0 ? 0 : (uint64_t)lf.bound > (uint64_t)(U)~(U)0 ? (U)~(U)0 : (U)lf.bound;
+  uint32_t nalive = V;
   {
-    const uint32_t c0 = first_col((uint32_t)lane), c1 = first_col((uint32_t)lane + 64);
-    col[0] = alive[0] ? c0 : kNoSlot;
-    col[1] = alive[1] ? c1 : kNoSlot;
+    const U d0 = alive[0] ? deg[0] : (U)~(U)0, d1 = alive[1] ? deg[1] : (U)~(U)0;
+    const U dmin = wave_min<U>(d0 < d1 ? d0 : d1);
+    best = dmin < best ? dmin : best;
   }
-  while (nalive > 1) {
-    const uint64_t lo_mask = __ballot(col[0] != kNoSlot), hi_mask = __ballot(col[1] != kNoSlot);
-    if (!lo_mask && !hi_mask) break;
-    const uint32_t u = lo_mask ? (uint32_t)(__ffsll((long long)lo_mask) - 1)
-                               : 64u + (uint32_t)(__ffsll((long long)hi_mask) - 1);
-    const uint32_t x = __shfl(u < 64 ? col[0] : col[1], (int)(u & 63), 64);
-    const uint32_t prev = u < x ? u : x, last = u < x ? x : u;
-    leaf_merge(A, V, prev, last, alive);
-    --nalive;
-    // row prev again, scanned by the whole wavefront: lane l tests columns l
-    // and l + 64, and the first set bit of the ballots is the first column
-    uint32_t again;
-    {
-      const bool q0 = alive[0] && (uint32_t)lane != prev && (int64_t)A[prev * kLeafStride + lane] >= lf.bound;
-      const bool q1 =
-          alive[1] && (uint32_t)lane + 64 != prev && (int64_t)A[prev * kLeafStride + lane + 64] >= lf.bound;
-      const uint64_t b0 = __ballot(q0), b1 = __ballot(q1);
-      again = b0 ? (uint32_t)(__ffsll((long long)b0) - 1) : b1 ? 64u + (uint32_t)(__ffsll((long long)b1) - 1) : kNoSlot;
+  while (nalive > 1 && best > 0) {
+    U key[2] = {0, 0};
+    bool added[2] = {!alive[0], !alive[1]};
+    uint32_t ord0 = 0, ord1 = 0;    // lane l: the vertices at positions l and l + 64 of the order
+    uint64_t join0 = 0, join1 = 0;  // bit t: the vertex at position t (t + 64) joins its predecessor
+    uint32_t merged = 0;
+    const uint64_t live_lo = __ballot(alive[0]), live_hi = __ballot(alive[1]);
+    uint32_t v = live_lo ? (uint32_t)(__ffsll((long long)live_lo) - 1)
+                         : 64u + (uint32_t)(__ffsll((long long)live_hi) - 1);
+    for (uint32_t step = 0;; ++step) {  // v takes position `step`
+      ord0 = lane == step ? v : ord0;
+      ord1 = lane + 64 == step ? v : ord1;
+      added[0] = added[0] || lane == v;
+      added[1] = added[1] || lane + 64 == v;
+      if (step + 1 == nalive) break;
+      for (int h = 0; h < 2; ++h) key[h] += (U)A[v * kLeafStride + lane + 64 * h];
+      const U k0 = added[0] ? 0 : key[0], k1 = added[1] ? 0 : key[1];
+      const U m = wave_max<U>(k0 > k1 ? k0 : k1);
+      const uint64_t b0 = __ballot(!added[0] && key[0] == m), b1 = __ballot(!added[1] && key[1] == m);
+      v = b0 ? (uint32_t)(__ffsll((long long)b0) - 1) : 64u + (uint32_t)(__ffsll((long long)b1) - 1);
+      if (step + 2 == nalive && m < best) best = m;  // the last vertex: its degree, a cut
+      if (m >= best) {
+        if (step + 1 < 64) join0 |= 1ull << (step + 1);
+        else join1 |= 1ull << (step - 63);
+        ++merged;
+      }
+    }
+    // Rows, then columns, of every run into its first vertex; a lane owns its
+    // two columns in the first pass and its two rows in the second.
+    auto joins = [&](uint32_t t) { return ((t < 64 ? join0 >> t : join1 >> (t - 64)) & 1ull) != 0; };
+    auto at = [&](uint32_t t) { return t < 64 ? readlane_u32(ord0, (int)t) : readlane_u32(ord1, (int)(t - 64)); };
+    bool dead[2] = {false, false};
+    for (int pass = 0; pass < 2; ++pass) {
+      const uint32_t sv = pass == 0 ? kLeafStride : 1, sl = pass == 0 ? 1 : kLeafStride;
+      for (uint32_t p = 0; p + 1 < nalive;) {
+        uint32_t e = p + 1;
+        if (!joins(e)) {
+          p = e;
+          continue;
+        }
+        T* first = A + at(p) * sv + lane * sl;
+        T a0 = first[0], a1 = first[64 * sl];
+        for (; e < nalive && joins(e); ++e) {
+          const uint32_t w = at(e);
+          const T* row = A + w * sv + lane * sl;
+          a0 += row[0];
+          a1 += row[64 * sl];
+          dead[0] = dead[0] || lane == w;
+          dead[1] = dead[1] || lane + 64 == w;
+        }
+        first[0] = a0;
+        first[64 * sl] = a1;
+        p = e;
+      }
+      __syncthreads();
     }
     for (int h = 0; h < 2; ++h) {
-      const uint32_t r = lane + 64 * h;
-      if (!alive[h]) col[h] = kNoSlot;
-      else if (r == prev) col[h] = again;
-      else if (col[h] == last) col[h] = prev;
-      else if (prev < col[h] && (int64_t)A[r * kLeafStride + prev] >= lf.bound) col[h] = prev;
+      if (dead[h]) alive[h] = false;
+      if (alive[h]) A[(lane + 64 * h) * (kLeafStride + 1)] = 0;  // loops of the merged vertices
     }
+    __syncthreads();
+    nalive -= merged;
   }
-  if (lf.bound <= 0) nalive = 1;  // a non-positive bound is already the answer
-  while (nalive > 1) {
-    int64_t key[2] = {0, 0};
-    bool added[2] = {!alive[0], !alive[1]};
-    // start from the smallest live vertex
-    uint64_t live_lo = __ballot(alive[0]), live_hi = __ballot(alive[1]);
-    uint32_t start =
-        live_lo ? (uint32_t)(__ffsll((long long)live_lo) - 1) : 64u + (uint32_t)(__ffsll((long long)live_hi) - 1);
-    uint32_t prev = start, last = start;
-    if ((uint32_t)lane == start) added[0] = true;
-    if ((uint32_t)lane + 64 == start) added[1] = true;
-    for (int h = 0; h < 2; ++h) key[h] += (int64_t)A[start * kLeafStride + lane + 64 * h];
-    int64_t cut = 0;
-    for (uint32_t step = 1; step < nalive; ++step) {
-      int64_t bk = INT64_MIN;
-      uint32_t bi = 0xFFFFFFFFu;
-      if (packed) {
-        const uint64_t p0 = added[0] ? 0 : ((uint64_t)key[0] << 8) | (255u - (uint32_t)lane);
-        const uint64_t p1 = added[1] ? 0 : ((uint64_t)key[1] << 8) | (255u - (uint32_t)lane - 64u);
-        const uint64_t b = wave_max<uint64_t>(p0 > p1 ? p0 : p1);
-        if (b != 0) {
-          bk = (int64_t)(b >> 8);
-          bi = 255u - (uint32_t)(b & 255u);
-        }
-      } else {
-        for (int h = 0; h < 2; ++h) {
-          if (!added[h] && (key[h] > bk || (key[h] == bk && (uint32_t)lane + 64 * h < bi))) {
-            bk = key[h];
-            bi = lane + 64 * h;
-          }
-        }
-        wave_argmax(bk, bi);
-      }
-      if (bi >= V) break;  // no candidate: cannot happen for step < nalive
-      prev = last;
-      last = bi;
-      if ((uint32_t)lane == bi) added[0] = true;
-      if ((uint32_t)lane + 64 == bi) added[1] = true;
-      if (step + 1 == nalive) {
-        cut = bk;
-        break;
-      }
-      for (int h = 0; h < 2; ++h)
-        if (!added[h]) key[h] += (int64_t)A[bi * kLeafStride + lane + 64 * h];
-    }
-    best = cut < best ? cut : best;
-    leaf_merge(A, V, prev, last, alive);
-    --nalive;
-  }
-  best = best < lf.bound ? best : lf.bound;
-  if (lane == 0) atomicMin((long long*)&results[lf.slot], (long long)best);
+  const int64_t res = (int64_t)best < lf.bound ? (int64_t)best : lf.bound;
+  if (lane == 0) atomicMin((long long*)&results[lf.slot], (long long)res);
 }
 
 // ---- contraction -------------------------------------------------------------
