@@ -9,25 +9,25 @@
 
 namespace cac {
 
-// One trial's root: a dense n x n device matrix (row stride n) with its row
-// sums, and where its raw cut goes.  Several roots may share one matrix
-// (independent trials).  Its draws are keyed by (seed, trial, node id).
+// One trial's root: a dense n x n device matrix with its row sums, and where its
+// raw cut goes.  w32: its entries add up to less than 2^32 and the matrix and row
+// sums are uint32_t, row stride ks_stride<uint32_t>(n) (whole 16-byte pieces);
+// else int64_t, row stride n.  Several roots may share one matrix (independent
+// trials).  Its draws are keyed by (seed, trial, node id).
 struct KsRoot {
-  const int64_t* mat;
-  const int64_t* rsum;
+  const void* mat;
+  const void* rsum;
   uint32_t n, trial, slot;
   int64_t bound;     // the trial's upper bound (minimum weighted degree)
   uint32_t seed;     // Philox key word 0 of the trial
   uint32_t nid = 1;  // recursion node id of the matrix (1: the trial's root)
-  bool w32 = false;  // total weight below 2^32: every node of the recursion fits 32-bit sums
+  bool w32 = false;
 };
 
-// Row sums of a dense device matrix into d_rsum and their minimum into *d_min.
-int ks_row_sums(cac_ctx* ctx, const int64_t* d_adj, uint32_t n, int64_t* d_rsum, int64_t* d_min, hipStream_t s);
 // Upper estimate of the device bytes one root holds at once in the two level
 // buffers (even depths in one, odd depths in the other, each grown to its
-// largest level: children arrays and row pools).
-size_t ks_live_bytes_per_root(uint32_t n);
+// largest level: children arrays and row pools), by entry type.
+size_t ks_live_bytes_per_root(uint32_t n, bool w32);
 // Runs one trial per root (roots of different seeds share launches);
 // d_results[slot] (initialised to the root's bound) receives min(bound, leaves).
 int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, hipStream_t s);
@@ -64,7 +64,8 @@ int sqrt_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, 
 // Sparse Karger-Stein trials on a checked device edge list (u < v, 1 <= w < 2^40):
 // raw cut of trial_ids[i] to d_results[i], which must already hold the bound.
 int ks_sparse_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t seed,
-                  const std::vector<uint32_t>& trial_ids, int64_t bound, int64_t* d_results, hipStream_t s);
+                  const std::vector<uint32_t>& trial_ids, int64_t bound, bool w32, int64_t* d_results,
+                  hipStream_t s);
 // Sparse trials of possibly different graphs side by side: root i is trial
 // `trial` of (edges, m, n) from node 1; d_results[slot] must hold its bound.
 struct SparseRoot {
@@ -73,6 +74,7 @@ struct SparseRoot {
   uint32_t n, trial, slot;
   int64_t bound;
   uint32_t seed;
+  bool w32;  // the graph's total weight is below 2^31: the dense nodes' entries are 32-bit
 };
 int ks_sparse_roots(cac_ctx* ctx, const std::vector<SparseRoot>& roots, int64_t* d_results, hipStream_t s);
 int ks_check_matrix(cac_ctx* ctx, const int64_t* adj, uint32_t n);

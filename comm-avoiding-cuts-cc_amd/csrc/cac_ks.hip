@@ -96,9 +96,10 @@ __device__ int64_t leaf_lower_bound(const int64_t d[2], const int64_t M[2], cons
 
 // Certificate first: a leaf whose lower bound reaches the trial's bound
 // contributes the bound; the others are queued for Stoer-Wagner.
-__global__ void __launch_bounds__(64) k_ks_cert(const KsLeaf* __restrict__ leaves, int64_t* __restrict__ results,
+template <typename E>
+__global__ void __launch_bounds__(64) k_ks_cert(const KsLeaf<E>* __restrict__ leaves, int64_t* __restrict__ results,
                                                 uint32_t* __restrict__ sw_list, uint32_t* __restrict__ sw_count) {
-  const KsLeaf lf = leaves[blockIdx.x];
+  const KsLeaf<E> lf = leaves[blockIdx.x];
   const uint32_t V = lf.k;
   const int lane = threadIdx.x;
   const bool alive[2] = {(uint32_t)lane < V, (uint32_t)lane + 64 < V};
@@ -107,12 +108,12 @@ __global__ void __launch_bounds__(64) k_ks_cert(const KsLeaf* __restrict__ leave
     const uint32_t u = lane + 64 * h;
     if (!alive[h]) continue;
     if (lf.rsum && lf.rmax) {
-      d[h] = lf.rsum[u];
-      M[h] = lf.rmax[u];
+      d[h] = (int64_t)lf.rsum[u];
+      M[h] = (int64_t)lf.rmax[u];
     } else {
       int64_t sm = 0, mx = 0;
       for (uint32_t x = 0; x < V; ++x) {
-        const int64_t v = lf.mat[(size_t)u * V + x];
+        const int64_t v = (int64_t)lf.mat[(size_t)u * lf.ks + x];
         sm += v;
         mx = v > mx ? v : mx;
       }
@@ -146,15 +147,16 @@ __global__ void __launch_bounds__(64) k_ks_cert(const KsLeaf* __restrict__ leave
 // so the phases are the cost.  Contracting only the last pair (and edges that
 // alone reach the bound) took V - 1 phases of a leaf that no such edge
 // collapses: 49 trials of a complete graph of 700 vertices, 1568 leaves of 128
-// in 64-bit entries, 21.4 ms; a phase contracts most of such a leaf at once.
+// in 64-bit entries, took 21.4 of the solve's 25.3 ms; a phase contracts most of
+// such a leaf at once, and the solve takes 5.7 ms.
 // T: the LDS entry type, uint32_t for a leaf of total weight below 2^32 (66 KiB,
 // two leaves per CU) and int64_t otherwise (132 KiB, one per CU).
-template <typename T>
-__global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf* __restrict__ leaves, const uint32_t* __restrict__ sw_list,
-                                              int64_t* __restrict__ results) {
-  typedef typename std::make_unsigned<T>::type U;
+template <typename T, typename E>
+__global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf<E>* __restrict__ leaves,
+                                              const uint32_t* __restrict__ sw_list, int64_t* __restrict__ results) {
+  typedef ks_sum_t<T> U;
   __shared__ T A[kLeafMax * kLeafStride];
-  const KsLeaf lf = leaves[sw_list[blockIdx.x]];
+  const KsLeaf<E> lf = leaves[sw_list[blockIdx.x]];
   const uint32_t V = lf.k;
   if (V < 2) return;  // no cut: the result keeps the bound
   const uint32_t lane = threadIdx.x;
@@ -165,7 +167,7 @@ __global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf* __restrict__ leaves,
     for (int h = 0; h < 2; ++h) {
       const uint32_t x = lane + 64 * h;
       if (x < V) {
-        const U a = (U)lf.mat[(size_t)r * V + x];
+        const U a = (U)lf.mat[(size_t)r * lf.ks + x];
         A[r * kLeafStride + x] = (T)a;
         deg[h] += a;  // symmetric: the column sum is the degree
       }
@@ -246,53 +248,77 @@ __global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf* __restrict__ leaves,
 }
 
 // ---- contraction -------------------------------------------------------------
-// LDS layout for a child of s vertices: cap[s] i64 | cbs[nb] u64 | rep[s] u32 |
-// wslot[s] u32 | red[B/64] u64 | misc[8] u32.
+// LDS layout for a child of s vertices (U: unsigned sums of E): cap[s] U |
+// cbs[nb] U | red[(kPieces + 1) B/64] U | misc[8] u32 | rep[s] u16 | wslot[s] u16,
+// rep and cap padded to 16 bytes.  With 32-bit entries that is 8 s bytes: two
+// 1024-thread workgroups of s = 8192 share a CU.
+template <typename E>
 __host__ __device__ inline size_t contract_lds_bytes(uint32_t s, int B) {
-  const size_t nb = (s + 63) / 64;
-  return 8 * (size_t)s + 8 * nb + 8 * (size_t)s + 8 * (size_t)(kKsChunk + 1) * (B / 64) + 32;
+  const size_t e = sizeof(E), s8 = (s + 7) & ~size_t(7), nb2 = ((s + 63) / 64 + 3) & ~size_t(3);
+  return e * s8 + e * nb2 + e * (size_t)(kPieces<E> + 1) * (B / 64) + 32 + 4 * s8 + 16;
 }
 
+template <typename E>
 struct KsLds {
-  int64_t* cap;
-  uint64_t* cbs;
-  uint32_t* rep;
-  uint32_t* wslot;
-  uint64_t* red;
-  uint32_t* misc;  // [0] i  [1] k  [2] rep[k]  [5] spare pool row
+  ks_sum_t<E>* cap;
+  ks_sum_t<E>* cbs;
+  ks_sum_t<E>* red;
+  uint32_t* misc;   // [0] i  [1] k  [2] rep[k]  [5] spare pool row  [6] pool rows handed out
+  uint16_t* rep;    // padded entries past s hold 0xFFFF
+  uint16_t* wslot;  // pool row of a merged row, or kNoRow
 };
 
-__device__ inline const int64_t* ks_row(const KsChild& c, const KsPool& pool, uint32_t slot, uint32_t r) {
-  return slot == kNoSlot ? c.parent + (size_t)r * c.s : pool.base + (size_t)slot * kKsUnit;
+template <typename E>
+__device__ inline const E* ks_row(const KsChild<E>& c, uint16_t slot, uint32_t r) {
+  return slot == kNoRow ? c.parent + (size_t)r * c.ps : c.pool + (size_t)slot * ks_pool_stride(c.s);
 }
 
-// This thread's entries x = k * B + t of a row (0 past s).  The row pointer is
-// generic (it comes from a struct in memory); as a global-address-space
-// pointer the loads are global loads, which unlike flat loads do not count
-// against the LDS wait counter, so the block's LDS waits between picks do not
-// also wait for row loads in flight.
-template <int B>
-__device__ inline void load_row(const int64_t* row, uint32_t cc, uint32_t s, int64_t (&v)[kKsChunk]) {
-  typedef const __attribute__((address_space(1))) int64_t g_i64;
-  g_i64* g = (g_i64*)row;
+// This thread's pieces of a row (0 past s).  The row pointer is generic (it comes
+// from a struct in memory); as a global-address-space pointer the loads are
+// global loads, which unlike flat loads do not count against the LDS wait
+// counter, so the block's LDS waits between picks do not also wait for row loads
+// in flight.  The last piece of a row is loaded entry by entry where it is not
+// whole: what lies past s is not the row's.
+template <int B, typename E>
+__device__ inline void load_row(const E* row, uint32_t qc, uint32_t s, E (&v)[kKsChunk]) {
+  typedef typename KsPiece<E>::type piece_t;
+  typedef const __attribute__((address_space(1))) piece_t g_piece;
+  typedef const __attribute__((address_space(1))) E g_e;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
+  g_e* g = (g_e*)row;
 #pragma unroll
-  for (uint32_t k = 0; k < kKsChunk; ++k) {
-    const uint32_t x = k * B + threadIdx.x;
-    v[k] = (k < cc && x < s) ? g[x] : 0;
+  for (uint32_t q = 0; q < Q; ++q) {
+    const uint32_t x = (q * B + threadIdx.x) * V;
+    if (q < qc && x + V <= s) {
+      const piece_t p = *(g_piece*)(g + x);
+#pragma unroll
+      for (uint32_t j = 0; j < V; ++j) v[q * V + j] = p[j];
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < V; ++j) v[q * V + j] = q < qc && x + j < s ? g[x + j] : (E)0;
+    }
   }
 }
 
-template <int B>
-__device__ inline void store_row(int64_t* row, uint32_t cc, uint32_t s, const int64_t (&v)[kKsChunk]) {
+// A pool row: whole pieces, the padding past s (0 in registers) included.
+template <int B, typename E>
+__device__ inline void store_row(E* row, uint32_t qc, uint32_t s, const E (&v)[kKsChunk]) {
+  typedef typename KsPiece<E>::type piece_t;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
 #pragma unroll
-  for (uint32_t k = 0; k < kKsChunk; ++k) {
-    const uint32_t x = k * B + threadIdx.x;
-    if (k < cc && x < s) row[x] = v[k];
+  for (uint32_t q = 0; q < Q; ++q) {
+    const uint32_t x = (q * B + threadIdx.x) * V;
+    if (q < qc && x < s) {
+      piece_t p;
+#pragma unroll
+      for (uint32_t j = 0; j < V; ++j) p[j] = v[q * V + j];
+      *(piece_t*)(row + x) = p;
+    }
   }
 }
 
 // Merge row a into row b (a dies, b keeps its index).  The calling threads hold
-// their chunk of row `held` (a or b) in v, and in u the last merged row, row
+// their pieces of row `held` (a or b) in v, and in u the last merged row, row
 // `cached` (kNoSlot before the first merge), which is the other row when
 // u_has_other.  That row is written back lazily: its pool row is stale until it
 // leaves the registers.  Otherwise the other row is loaded into u here, after
@@ -306,97 +332,118 @@ __device__ inline void store_row(int64_t* row, uint32_t cc, uint32_t s, const in
 // barrier.  Each thread relabels only the representatives of the columns it
 // owns.  Returns the contracted weight (cap[a] + cap[b] - cap_new) / 2 in w;
 // false when the pool is exhausted.  Called by the whole block.
-template <int B>
-__device__ bool ks_merge(const KsChild& c, const KsPool& pool, const KsLds& L, uint32_t a, uint32_t b, uint32_t held,
-                         const int64_t (&v)[kKsChunk], int64_t (&u)[kKsChunk], uint32_t cached, bool u_has_other,
-                         uint32_t cc, int64_t& w) {
+template <int B, typename E>
+__device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uint32_t b, uint32_t held,
+                         const E (&v)[kKsChunk], E (&u)[kKsChunk], uint32_t cached, bool u_has_other, uint32_t qc,
+                         ks_sum_t<E>& w) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
+  typedef uint16_t rep_t __attribute__((ext_vector_type(V), aligned(2 * V)));
   const uint32_t s = c.s;
   const uint32_t other = held == a ? b : a;
-  const uint32_t slot_a = L.wslot[a], slot_b = L.wslot[b];
-  const bool spare = slot_b == kNoSlot && slot_a == kNoSlot;
-  const uint32_t db = slot_b != kNoSlot ? slot_b : slot_a != kNoSlot ? slot_a : L.misc[5];
+  const uint16_t slot_a = L.wslot[a], slot_b = L.wslot[b];
+  const bool spare = slot_b == kNoRow && slot_a == kNoRow;
+  const uint32_t db = slot_b != kNoRow ? slot_b : slot_a != kNoRow ? slot_a : L.misc[5];
   if (db == kNoSlot) return false;  // only a spare can be missing: the pool is exhausted
   if (!u_has_other) {
     if (cached != kNoSlot && cached != a && cached != b)  // a merged row has a pool row
-      store_row<B>(pool.base + (size_t)L.wslot[cached] * kKsUnit, cc, s, u);
-    load_row<B>(ks_row(c, pool, other == a ? slot_a : slot_b, other), cc, s, u);
+      store_row<B>(c.pool + (size_t)L.wslot[cached] * ks_pool_stride(s), qc, s, u);
+    load_row<B>(ks_row(c, other == a ? slot_a : slot_b, other), qc, s, u);
   }
-  uint64_t sum = 0;
+  U sum = 0;
 #pragma unroll
-  for (uint32_t k = 0; k < kKsChunk; ++k) {
-    const uint32_t x = k * B + threadIdx.x;
-    if (k < cc && x < s) {
-      int64_t t = v[k] + u[k];
-      const uint32_t rx = L.rep[x];
-      if (rx == a || rx == b) t = 0;  // loop of the merged vertex
-      if (rx == a) L.rep[x] = b;
-      u[k] = t;
-      sum += (uint64_t)t;
+  for (uint32_t q = 0; q < Q; ++q) {
+    const uint32_t x = (q * B + threadIdx.x) * V;
+    if (q < qc && x < s) {
+      rep_t rx = *(const rep_t*)(L.rep + x);
+      bool hit_a = false;
+#pragma unroll
+      for (uint32_t j = 0; j < V; ++j) {
+        E t = v[q * V + j] + u[q * V + j];
+        if (rx[j] == a || rx[j] == b) t = 0;  // loop of the merged vertex
+        if (rx[j] == a) {
+          rx[j] = (uint16_t)b;
+          hit_a = true;
+        }
+        u[q * V + j] = t;
+        sum += (U)t;
+      }
+      if (hit_a) *(rep_t*)(L.rep + x) = rx;
     }
   }
-  const int64_t ca = L.cap[a], cb = L.cap[b];
-  const int64_t newcap = (int64_t)block_sum_u64_open<B>(sum, L.red);
+  const U ca = L.cap[a], cb = L.cap[b];
+  const U newcap = block_sum_open<B, U>(sum, L.red);
   w = (ca + cb - newcap) / 2;
   if (B == 64) __syncthreads();  // every lane has read the slots and capacities
   if (threadIdx.x == 0) {
-    if (slot_b == kNoSlot) {
-      L.wslot[b] = db;
-      L.wslot[a] = kNoSlot;
+    if (slot_b == kNoRow) {
+      L.wslot[b] = (uint16_t)db;
+      L.wslot[a] = kNoRow;
     }
     if (spare) {
-      const unsigned long long units = (s + kKsUnit - 1) / kKsUnit;
-      const unsigned long long off = atomicAdd(pool.used_units, units);
-      L.misc[5] = off + units <= pool.cap_units ? (uint32_t)off : kNoSlot;
+      const uint32_t next = L.misc[6];
+      L.misc[5] = next < c.pool_rows ? next : kNoSlot;
+      L.misc[6] = next + 1;
     }
-    L.cbs[a / 64] -= (uint64_t)ca;
+    L.cbs[a / 64] -= ca;
     L.cap[a] = 0;
-    L.cbs[b / 64] += (uint64_t)(newcap - cb);
+    L.cbs[b / 64] += newcap - cb;
     L.cap[b] = newcap;
   }
   __syncthreads();
   return true;
 }
 
-// Below 1024 threads, at most 96 VGPRs (5 waves per SIMD): room for the two
-// rows a thread keeps (the picked row and the last merged row) without
-// spilling; at 80 VGPRs (6 waves) the kernel spills and is slower.
-template <int B>
-__global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
-    k_ks_contract(const KsChild* __restrict__ children, KsPool pool, uint32_t* __restrict__ k_out,
+// Waves per SIMD the contraction is compiled for.  32-bit entries: the two rows a
+// thread keeps (the picked row and the last merged row) take 16 registers and
+// the kernel fits 64 (8 waves: two 1024-thread workgroups per CU).  64-bit
+// entries take 32: at most 96 registers below 1024 threads (5 waves; at 80 the
+// kernel spills and is slower).
+template <int B, typename E>
+constexpr int kContractWaves = sizeof(E) == 4 ? 8 : B >= 1024 ? 1 : 5;
+
+template <int B, typename E>
+__global__ void __launch_bounds__(B, (kContractWaves<B, E>))
+    k_ks_contract(const KsChild<E>* __restrict__ children, uint32_t* __restrict__ k_out,
                   int64_t* __restrict__ results) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
   extern __shared__ __align__(16) unsigned char smem[];
-  const KsChild c = children[blockIdx.x];
+  const KsChild<E> c = children[blockIdx.x];
   const uint32_t s = c.s, nb = (s + 63) / 64;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  KsLds L;
-  L.cap = (int64_t*)smem;
-  L.cbs = (uint64_t*)(smem + 8 * (size_t)s);
-  L.rep = (uint32_t*)(smem + 8 * (size_t)s + 8 * nb);
-  L.wslot = L.rep + s;
-  L.red = (uint64_t*)(smem + 16 * (size_t)s + 8 * nb);
-  L.misc = (uint32_t*)(L.red + (kKsChunk + 1) * (B / 64));
+  const size_t s8 = (s + 7) & ~size_t(7), nb2 = (nb + 3) & ~size_t(3);
+  KsLds<E> L;
+  L.cap = (U*)smem;
+  L.cbs = L.cap + s8;
+  L.red = L.cbs + nb2;
+  L.misc = (uint32_t*)(L.red + (kPieces<E> + 1) * (B / 64));
+  L.rep = (uint16_t*)(((uintptr_t)(L.misc + 8) + 15) & ~uintptr_t(15));
+  L.wslot = L.rep + s8;
 
-  for (uint32_t x = threadIdx.x; x < s; x += B) {
-    L.cap[x] = c.prsum[x];
-    L.rep[x] = x;
-    L.wslot[x] = kNoSlot;
+  for (uint32_t x = threadIdx.x; x < s8; x += B) {
+    L.cap[x] = x < s ? (U)c.prsum[x] : 0;
+    L.rep[x] = x < s ? (uint16_t)x : (uint16_t)0xFFFF;
+    L.wslot[x] = kNoRow;
   }
   if (threadIdx.x == 0) {  // the spare pool row of the first merge of two original rows
-    const unsigned long long units = (s + kKsUnit - 1) / kKsUnit;
-    const unsigned long long off = atomicAdd(pool.used_units, units);
-    L.misc[5] = off + units <= pool.cap_units ? (uint32_t)off : kNoSlot;
+    L.misc[5] = c.pool_rows > 0 ? 0 : kNoSlot;
+    L.misc[6] = 1;
   }
   __syncthreads();
   for (uint32_t blk = wave; blk < nb; blk += B / 64) {
     const uint32_t x = blk * 64 + lane;
-    const uint64_t t = wave_sum<uint64_t>(x < s ? (uint64_t)L.cap[x] : 0);
+    const U t = wave_sum<U>(x < s ? L.cap[x] : 0);
     if (lane == 0) L.cbs[blk] = t;
   }
   __syncthreads();
   uint64_t W = 0;
   for (uint32_t blk = 0; blk < nb; ++blk) W += L.cbs[blk];
 
-  const uint32_t cc = (s + B - 1) / B;  // entries per thread, <= kKsChunk
+  // A bound that no entry of the type reaches compares like the type's maximum.
+  const U bound = c.bound > 0 && (uint64_t)c.bound > (uint64_t)(U)~(U)0 ? (U)~(U)0 : (U)c.bound;
+  const uint32_t qc = (s + B * V - 1) / (B * V);  // pieces per thread, <= Q
+  const uint32_t cc = (s + B - 1) / B;            // entries per thread in the closing pass
   const uint32_t lo = threadIdx.x * cc;
   uint32_t nv = s, pr1 = 0;
   int status = 0;  // 1 disconnected, 2 bad selection, 3 pool exhausted
@@ -404,7 +451,7 @@ __global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
   // cb (most picks touch it: the heavy super-vertex is picked or is the picked
   // row's partner, and the PR pass checks it next after merging into it), so
   // it is not loaded again
-  int64_t v[kKsChunk], u[kKsChunk];
+  E v[kKsChunk], u[kKsChunk];
   uint32_t cb = kNoSlot;
   for (uint32_t p = 0; p + c.tgt < s; ++p) {
     if (W == 0) {
@@ -413,7 +460,7 @@ __global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
     }
     const u32x4 rnd = philox4x32(c.trial, c.nid, p, 0u, c.seed, kDomKs);
     if (wave == 0) {
-      const uint32_t i = wave_select_two_level(L.cap, L.cbs, s, nb, uniform1(lo64(rnd), W));
+      const uint32_t i = wave_select_two_level<U>(L.cap, L.cbs, s, nb, (U)uniform1(lo64(rnd), W));
       if (lane == 0) L.misc[0] = i;
     }
     __syncthreads();
@@ -426,47 +473,50 @@ __global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
 #pragma unroll
       for (uint32_t q = 0; q < kKsChunk; ++q) v[q] = u[q];
     } else {
-      load_row<B>(ks_row(c, pool, L.wslot[i], i), cc, s, v);
+      load_row<B>(ks_row(c, L.wslot[i], i), qc, s, v);
     }
     const uint32_t k =
-        block_select_row<B>(v, cc, uniform1(hi64(rnd), (uint64_t)L.cap[i]), L.red, L.misc + 1, L.rep);
+        block_select_row<B, E>(v, qc, (U)uniform1(hi64(rnd), (uint64_t)L.cap[i]), L.red, L.misc + 1, L.rep);
     if (k >= s) {
       status = 2;
       break;
     }
     const uint32_t j = L.misc[2];  // rep[k], read by the selecting thread before the merge relabels
     const uint32_t a = i > j ? i : j, b = i > j ? j : i;
-    int64_t w = 0;
-    if (!ks_merge<B>(c, pool, L, a, b, i, v, u, cb, j == cb, cc, w)) {
+    U w = 0;
+    if (!ks_merge<B, E>(c, L, a, b, i, v, u, cb, j == cb, qc, w)) {
       status = 3;
       break;
     }
     cb = b;
     W -= 2 * (uint64_t)w;
     --nv;
-    if (w >= c.bound) ++pr1;
+    if (w >= bound) ++pr1;
   }
   // PR pass (indexed_adjacency_matrix::pr_pass): contract every edge of weight >= bound
   if (status == 0 && pr1 > 0 && c.bound > 0) {
     for (uint32_t i = 0; i < s && nv > 2; ++i) {
-      if (L.rep[i] != i || L.cap[i] < c.bound) continue;
+      if (L.rep[i] != i || L.cap[i] < bound) continue;
       if (i == cb) {
 #pragma unroll
         for (uint32_t q = 0; q < kKsChunk; ++q) v[q] = u[q];
       } else {
-        load_row<B>(ks_row(c, pool, L.wslot[i], i), cc, s, v);
+        load_row<B>(ks_row(c, L.wslot[i], i), qc, s, v);
       }
       uint32_t first = kNoSlot;
 #pragma unroll
-      for (uint32_t k = 0; k < kKsChunk; ++k)
-        if (first == kNoSlot && k < cc && k * B + threadIdx.x < s && v[k] >= c.bound) first = k * B + threadIdx.x;
+      for (uint32_t q = 0; q < Q; ++q) {
+#pragma unroll
+        for (uint32_t j = 0; j < V; ++j)  // an entry past s is 0, below the bound
+          if (first == kNoSlot && (U)v[q * V + j] >= bound) first = (q * B + threadIdx.x) * V + j;
+      }
       first = block_min_u32<B>(first, (uint32_t*)L.red);
       if (first == kNoSlot) continue;
       // rep[first] is not i: row i's entries of its own class are 0, below the
       // bound, so this merge's relabelling (of class i) leaves it unchanged
-      int64_t w = 0;
+      U w = 0;
       const uint32_t tgt = L.rep[first];
-      if (!ks_merge<B>(c, pool, L, i, tgt, i, v, u, cb, tgt == cb, cc, w)) {
+      if (!ks_merge<B, E>(c, L, i, tgt, i, v, u, cb, tgt == cb, qc, w)) {
         status = 3;
         break;
       }
@@ -474,7 +524,7 @@ __global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
       --nv;
     }
   }
-  if (status == 0 && cb != kNoSlot) store_row<B>(pool.base + (size_t)L.wslot[cb] * kKsUnit, cc, s, u);
+  if (status == 0 && cb != kNoSlot) store_row<B>(c.pool + (size_t)L.wslot[cb] * ks_pool_stride(s), qc, s, u);
   if (status != 0) {
     if (threadIdx.x == 0) {
       k_out[blockIdx.x] = status == 1 ? 0u : status == 2 ? kKsBad : kKsOverflow;
@@ -507,19 +557,18 @@ __global__ void __launch_bounds__(B, B >= 1024 ? 1 : 5)
     const uint32_t x = lo + k;
     if (k < cc && x < s && L.rep[x] == x) {
       rank[x] = ex;
-      const uint32_t sl = L.wslot[x];
-      c.live[ex] = sl == kNoSlot ? x : (kLiveWork | sl);
+      const uint16_t sl = L.wslot[x];
+      c.live[ex] = sl == kNoRow ? x : (kLiveWork | sl);
       ++ex;
     }
   }
   __syncthreads();
-  for (uint32_t y = threadIdx.x; y < s; y += B) c.colmap[y] = rank[L.rep[y]];
+  for (uint32_t y = threadIdx.x; y < s; y += B) c.colmap[y] = (uint16_t)rank[L.rep[y]];
   if (threadIdx.x == 0) k_out[blockIdx.x] = total;
 }
 
-// Rows per compaction workgroup for a child of t' output vertices (the LDS
-// accumulator holds rows x t' int64, at most 32 KiB unless t' alone is larger).
-constexpr uint32_t kCompactUnroll = 8;  // row elements per thread in flight in k_ks_compact
+// Row entries per thread in flight in k_ks_compact.
+constexpr uint32_t kCompactUnroll = 8;
 
 // Threads per compaction workgroup for children of tgt output vertices: the
 // context's CAC_TUNE_KS_COMPACT_BLOCK setting for tgt's class, or 512 (on
@@ -531,6 +580,8 @@ inline int compact_block(const cac_ctx* ctx, uint32_t tgt) {
   return v ? v : 512;
 }
 
+// Rows per compaction workgroup for a child of t' output vertices (the LDS
+// accumulator holds rows x t' entries, at most 4096 unless t' alone is larger).
 __host__ __device__ inline uint32_t compact_rows(uint32_t tgt) {
   const uint32_t r = 4096 / (tgt ? tgt : 1);
   return r < 1 ? 1 : (r > 64 ? 64 : r);
@@ -538,17 +589,17 @@ __host__ __device__ inline uint32_t compact_rows(uint32_t tgt) {
 
 // One workgroup per (child, group of output rows): sums every live row by column
 // class into LDS, then writes the rows with their sums and maxima.  The work
-// item's child comes from a binary search of the per-child item prefix.  CB
-// threads per workgroup: large children, whose rows go one per workgroup, take
-// more threads, so more of a row's loads are in flight per CU.  AccT: the LDS
-// accumulator, uint32_t when every node of the level weighs less than 2^32 in
-// total (no class sum can exceed it; half the LDS and one bank per atomic),
-// unsigned long long otherwise.
-template <int CB, typename AccT>
-__global__ void __launch_bounds__(CB) k_ks_compact(const KsChild* __restrict__ children,
+// item's child comes from a binary search of the per-child item prefix
+// (item_prefix).  CB threads per workgroup: large children, whose rows go one per
+// workgroup, take more threads, so more of a row's loads are in flight per CU.
+// A class sum never exceeds its node's total, so the LDS accumulator has the
+// entry type.
+template <int CB, typename E>
+__global__ void __launch_bounds__(CB) k_ks_compact(const KsChild<E>* __restrict__ children,
                                                    const uint32_t* __restrict__ k_out,
-                                                   const uint32_t* __restrict__ item_prefix, uint32_t nchild,
-                                                   KsPool pool) {
+                                                   const uint32_t* __restrict__ item_prefix, uint32_t nchild) {
+  typedef typename std::conditional<sizeof(E) == 4, uint32_t, unsigned long long>::type AccT;
+  constexpr uint32_t U = kCompactUnroll;
   extern __shared__ __align__(16) unsigned char acc_lds[];
   AccT* acc = reinterpret_cast<AccT*>(acc_lds);
   const uint32_t item = blockIdx.x;
@@ -558,31 +609,33 @@ __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild* __restrict__ c
     if (item_prefix[mid] <= item) lo = mid;
     else hi = mid;
   }
-  const KsChild c = children[lo];
+  const KsChild<E> c = children[lo];
   const uint32_t kk = k_out[lo];
   if (kk == 0 || kk > c.tgt) return;  // disconnected child, or an error code
   const uint32_t R = compact_rows(c.tgt);
   const uint32_t r0 = (item - item_prefix[lo]) * R;
   if (r0 >= kk) return;
   const uint32_t nr = min(R, kk - r0);
-  const uint32_t s = c.s;
-  for (uint32_t x = threadIdx.x; x < nr * kk; x += CB) acc[x] = 0;
+  const uint32_t s = c.s, os = ks_stride<E>(kk);
+  for (uint32_t x = threadIdx.x; x < nr * os; x += CB) acc[x] = 0;
   __syncthreads();
   // Rows and the column map are global memory (the struct's pointers are
-  // generic, which would give flat loads); kCompactUnroll elements per thread
-  // are loaded before any is added, so a wavefront keeps several 512-byte
-  // loads in flight instead of one.
-  typedef const __attribute__((address_space(1))) int64_t g_i64;
-  typedef const __attribute__((address_space(1))) uint32_t g_u32;
-  constexpr uint32_t U = kCompactUnroll;
-  g_u32* cm = (g_u32*)c.colmap;
+  // generic, which would give flat loads); kCompactUnroll entries per thread
+  // are loaded before any is added, so a wavefront keeps several loads in
+  // flight instead of one.  Neighbouring lanes take neighbouring columns: a
+  // lane's columns side by side (16-byte loads) put the lanes' LDS additions
+  // four entries apart, on a quarter of the banks.
+  typedef const __attribute__((address_space(1))) E g_e;
+  typedef const __attribute__((address_space(1))) uint16_t g_u16;
+  g_u16* cm = (g_u16*)c.colmap;
   for (uint32_t rr = 0; rr < nr; ++rr) {
     const uint32_t e = c.live[r0 + rr];
-    g_i64* src = (g_i64*)((e & kLiveWork) ? pool.base + (size_t)(e & ~kLiveWork) * kKsUnit : c.parent + (size_t)e * s);
-    AccT* a = acc + (size_t)rr * kk;
+    g_e* src = (g_e*)((e & kLiveWork) ? c.pool + (size_t)(e & ~kLiveWork) * ks_pool_stride(s)
+                                      : c.parent + (size_t)e * c.ps);
+    AccT* a = acc + (size_t)rr * os;
     uint32_t y = threadIdx.x;
     for (; y + (U - 1) * CB < s; y += U * CB) {
-      int64_t v[U];
+      E v[U];
       uint32_t m[U];
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u) {
@@ -594,7 +647,7 @@ __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild* __restrict__ c
         if (v[u]) atomicAdd(&a[m[u]], (AccT)v[u]);
     }
     for (; y < s; y += CB) {
-      const int64_t v = src[y];
+      const E v = src[y];
       if (v) atomicAdd(&a[cm[y]], (AccT)v);
     }
   }
@@ -602,35 +655,48 @@ __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild* __restrict__ c
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (uint32_t rr = wave; rr < nr; rr += CB / 64) {
     const uint32_t r = r0 + rr;
-    int64_t* dst = c.out + (size_t)r * kk;
-    int64_t sm = 0, mx = 0;
+    E* dst = c.out + (size_t)r * os;
+    ks_sum_t<E> sm = 0, mx = 0;
     for (uint32_t x = lane; x < kk; x += 64) {
-      const int64_t v = (int64_t)(uint64_t)acc[(size_t)rr * kk + x];
-      dst[x] = v;
+      const ks_sum_t<E> v = (ks_sum_t<E>)acc[(size_t)rr * os + x];
+      dst[x] = (E)v;
       sm += v;
       mx = v > mx ? v : mx;
     }
     // entries are non-negative, so the unsigned maximum is the maximum
-    sm = (int64_t)wave_sum<uint64_t>((uint64_t)sm);
-    mx = (int64_t)wave_max<uint64_t>((uint64_t)mx);
+    sm = wave_sum<ks_sum_t<E>>(sm);
+    mx = wave_max<ks_sum_t<E>>(mx);
     if (lane == 0) {
-      c.orsum[r] = sm;
-      c.ormax[r] = mx;
+      c.orsum[r] = (E)sm;
+      c.ormax[r] = (E)mx;
     }
   }
 }
 
-// Row sums of a dense matrix (one wavefront per row) and their minimum.
+// Row sums of a dense matrix (one wavefront per row) and their minimum, and on
+// the way the matrix and the sums cut to 32 bits, row stride
+// ks_stride<uint32_t>(n): exact copies when the sums add up to less than 2^32,
+// which the host decides from the 64-bit sums.
 __global__ void __launch_bounds__(256) k_row_sums(const int64_t* __restrict__ A, uint32_t n, int64_t* __restrict__ rsum,
-                                                  int64_t* out_min) {
+                                                  int64_t* out_min, uint32_t* __restrict__ A32,
+                                                  uint32_t* __restrict__ rsum32) {
   __shared__ long long wmin[4];
   long long best = INT64_MAX;
+  const uint32_t st = ks_stride<uint32_t>(n);
   for (uint32_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += gridDim.x * 4) {
     const int64_t* row = A + (size_t)r * n;
+    uint32_t* row32 = A32 + (size_t)r * st;
     uint64_t acc = 0;
-    for (uint32_t x = threadIdx.x & 63; x < n; x += 64) acc += (uint64_t)row[x];
+    for (uint32_t x = threadIdx.x & 63; x < n; x += 64) {
+      const uint64_t v = (uint64_t)row[x];
+      acc += v;
+      row32[x] = (uint32_t)v;
+    }
     acc = wave_sum<uint64_t>(acc);
-    if ((threadIdx.x & 63) == 0) rsum[r] = (int64_t)acc;
+    if ((threadIdx.x & 63) == 0) {
+      rsum[r] = (int64_t)acc;
+      rsum32[r] = (uint32_t)acc;
+    }
     best = (long long)acc < best ? (long long)acc : best;
   }
   if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = best;
@@ -697,24 +763,30 @@ int ks_reserve(cac_ctx* ctx, int which, size_t bytes, void** out) {
 }
 
 // Device bytes of the per-child arrays of one child (out, sums, maxima, map, list).
-size_t child_bytes(uint32_t s, uint32_t t) {
-  return c64((size_t)t * t * 8) + 2 * c64((size_t)t * 8) + c64((size_t)s * 4) + c64((size_t)t * 4);
+size_t child_bytes(uint32_t s, uint32_t t, size_t esize) {
+  const size_t stride = esize == 4 ? ks_stride<uint32_t>(t) : ks_stride<int64_t>(t);
+  return c64(stride * t * esize) + 2 * c64((size_t)t * esize) + c64(((size_t)s + 8) * 2) + c64((size_t)t * 4);
 }
-size_t child_pool_units(uint32_t s, uint32_t t) { return (size_t)(s - t) * ((s + kKsUnit - 1) / kKsUnit); }
+// Pool rows of a child in the first pass: one for every pick and 1/8 spare (at
+// least 8) for the PR pass.  A child that needs more comes back as kKsOverflow.
+uint32_t child_pool_rows(uint32_t s, uint32_t t) { return std::min(s, (s - t) + (s - t) / 8 + 8); }
 
-int run_leaves(cac_ctx* ctx, const std::vector<KsLeaf>& leaves, int buf, int64_t* d_results, hipStream_t s) {
+template <typename E>
+int run_leaves(cac_ctx* ctx, const std::vector<KsLeaf<E>>& leaves, int buf, int64_t* d_results, hipStream_t s) {
+  typedef KsLeaf<E> Leaf;
   const size_t n = leaves.size();
   void* base = nullptr;
-  int rc = ks_reserve(ctx, buf, c64(n * sizeof(KsLeaf)) + c64(n * 4) + 128, &base);
+  int rc = ks_reserve(ctx, buf, c64(n * sizeof(Leaf)) + c64(n * 4) + 128, &base);
   if (rc) return rc;
   Carve64 cv(base);
-  KsLeaf* d_leaves = cv.take<KsLeaf>(n);
+  Leaf* d_leaves = cv.take<Leaf>(n);
   uint32_t* d_list = cv.take<uint32_t>(n);
   uint32_t* d_count = cv.take<uint32_t>(2);  // [0] 32-bit leaves (list front), [1] the others (list back)
-  CAC_HIP(ctx, hipMemcpyAsync(d_leaves, leaves.data(), n * sizeof(KsLeaf), hipMemcpyHostToDevice, s));
+  CAC_HIP(ctx, hipMemcpyAsync(d_leaves, leaves.data(), n * sizeof(Leaf), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, (unsigned long long*)d_count, 1u);
   prof_begin(ctx, "ks_cert", s);
-  hipLaunchKernelGGL(k_ks_cert, dim3((unsigned)n), dim3(64), 0, s, (const KsLeaf*)d_leaves, d_results, d_list, d_count);
+  hipLaunchKernelGGL(k_ks_cert<E>, dim3((unsigned)n), dim3(64), 0, s, (const Leaf*)d_leaves, d_results, d_list,
+                     d_count);
   prof_end(ctx, s);
   CAC_LAUNCH_CHECK(ctx, "ks certificate");
   CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, d_count, 8, hipMemcpyDeviceToHost, s));
@@ -723,11 +795,13 @@ int run_leaves(cac_ctx* ctx, const std::vector<KsLeaf>& leaves, int buf, int64_t
   if (n32 + n64) {
     prof_begin(ctx, "ks_sw", s);
     if (n32)
-      hipLaunchKernelGGL(k_ks_sw<uint32_t>, dim3(n32), dim3(64), 0, s, (const KsLeaf*)d_leaves,
+      hipLaunchKernelGGL((k_ks_sw<uint32_t, E>), dim3(n32), dim3(64), 0, s, (const Leaf*)d_leaves,
                          (const uint32_t*)d_list, d_results);
-    if (n64)
-      hipLaunchKernelGGL(k_ks_sw<int64_t>, dim3(n64), dim3(64), 0, s, (const KsLeaf*)d_leaves,
-                         (const uint32_t*)(d_list + (n - n64)), d_results);
+    if constexpr (sizeof(E) == 8) {  // a 32-bit leaf always goes to the front
+      if (n64)
+        hipLaunchKernelGGL((k_ks_sw<int64_t, E>), dim3(n64), dim3(64), 0, s, (const Leaf*)d_leaves,
+                           (const uint32_t*)(d_list + (n - n64)), d_results);
+    }
     prof_end(ctx, s);
     CAC_LAUNCH_CHECK(ctx, "ks stoer-wagner");
   }
@@ -735,11 +809,11 @@ int run_leaves(cac_ctx* ctx, const std::vector<KsLeaf>& leaves, int buf, int64_t
   return CAC_OK;
 }
 
-template <int B>
-void launch_contract(const KsChild* d_children, uint32_t count, uint32_t smax, KsPool pool, uint32_t* d_kout,
+template <int B, typename E>
+void launch_contract(const KsChild<E>* d_children, uint32_t count, uint32_t smax, uint32_t* d_kout,
                      int64_t* d_results, hipStream_t s) {
-  hipLaunchKernelGGL(k_ks_contract<B>, dim3(count), dim3(B), contract_lds_bytes(smax, B), s, d_children, pool, d_kout,
-                     d_results);
+  hipLaunchKernelGGL((k_ks_contract<B, E>), dim3(count), dim3(B), contract_lds_bytes<E>(smax, B), s, d_children,
+                     d_kout, d_results);
 }
 
 // One level's launches for the children ch (already in d_children's order, by
@@ -747,12 +821,12 @@ void launch_contract(const KsChild* d_children, uint32_t count, uint32_t smax, K
 // then the compaction, sized by those k (a child that the PR pass collapsed
 // takes a few workgroups, not t' / rows of them), left running on the stream
 // (the next level's work follows it there).
-int contract_level(cac_ctx* ctx, const std::vector<KsChild>& ch, KsChild* d_children, uint32_t* d_prefix,
-                   uint32_t* d_kout, unsigned long long* d_used, KsPool pool, uint32_t max_tgt, int64_t* d_results,
-                   std::vector<uint32_t>& kout, bool w32, hipStream_t s) {
+template <typename E>
+int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* d_children, uint32_t* d_prefix,
+                   uint32_t* d_kout, uint32_t max_tgt, int64_t* d_results, std::vector<uint32_t>& kout,
+                   hipStream_t s) {
   const size_t nchild = ch.size();
-  CAC_HIP(ctx, hipMemcpyAsync(d_children, ch.data(), nchild * sizeof(KsChild), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, d_used, 1u);
+  CAC_HIP(ctx, hipMemcpyAsync(d_children, ch.data(), nchild * sizeof(KsChild<E>), hipMemcpyHostToDevice, s));
   prof_begin(ctx, "ks_contract", s);
   size_t c0 = 0;
   while (c0 < nchild) {
@@ -762,15 +836,18 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild>& ch, KsChild* d_chil
     while (c1 < nchild && contract_block(ctx, ch[c1].s) == B) smax = std::max(smax, ch[c1++].s);
     const uint32_t cnt = (uint32_t)(c1 - c0);
     // Fewer children than CUs (the top levels of a small solve): the device is
-    // idle but for these workgroups, and a wider block shortens each pick's
-    // row scans (ER(1000, 0.05) square_root: contraction 1.5 -> 1.33 ms per
-    // solve).  With many children the narrow block keeps occupancy up.
-    if (cnt < kFewChildren && B < 256) B = 256;
-    if (B == 1024) launch_contract<1024>(d_children + c0, cnt, smax, pool, d_kout + c0, d_results, s);
-    else if (B == 512) launch_contract<512>(d_children + c0, cnt, smax, pool, d_kout + c0, d_results, s);
-    else if (B == 256) launch_contract<256>(d_children + c0, cnt, smax, pool, d_kout + c0, d_results, s);
-    else if (B == 128) launch_contract<128>(d_children + c0, cnt, smax, pool, d_kout + c0, d_results, s);
-    else launch_contract<64>(d_children + c0, cnt, smax, pool, d_kout + c0, d_results, s);
+    // idle but for these workgroups, and with 64-bit entries a wider block
+    // shortens each pick's row scans (ER(1000, 0.05) square_root: contraction
+    // 1.5 -> 1.33 ms per solve).  With many children the narrow block keeps
+    // occupancy up, and with 32-bit entries the one wavefront of a child of
+    // s <= 512 has two pieces to scan and no barriers to wait at (the same
+    // solve: contraction 0.82 ms with 64 threads, 0.86 with 128, 0.90 with 256).
+    if (sizeof(E) == 8 && cnt < kFewChildren && B < 256) B = 256;
+    if (B == 1024) launch_contract<1024, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
+    else if (B == 512) launch_contract<512, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
+    else if (B == 256) launch_contract<256, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
+    else if (B == 128) launch_contract<128, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
+    else launch_contract<64, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
     c0 = c1;
   }
   prof_end(ctx, s);
@@ -791,23 +868,15 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild>& ch, KsChild* d_chil
   if (items == 0) return CAC_OK;
   CAC_HIP(ctx, hipMemcpyAsync(d_prefix, item_prefix.data(), (nchild + 1) * 4, hipMemcpyHostToDevice, s));
   prof_begin(ctx, "ks_compact", s);
-  const size_t acc_bytes = w32 ? 4 : 8;
-  const size_t lds = std::max<size_t>(4096, max_tgt) * acc_bytes;
+  const size_t lds = std::max<size_t>(4096 + 4 * 64, ks_stride<E>(max_tgt)) * sizeof(E);  // rows padded to whole pieces
   const int cb = compact_block(ctx, max_tgt);
-  const KsChild* dc = d_children;
+  const KsChild<E>* dc = d_children;
   const uint32_t* dk = d_kout;
   const uint32_t* dp = d_prefix;
   const uint32_t nc = (uint32_t)nchild;
-  if (w32) {
-    if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, uint32_t>), dim3(items), dim3(1024), lds, s, dc, dk, dp, nc, pool);
-    else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, uint32_t>), dim3(items), dim3(512), lds, s, dc, dk, dp, nc, pool);
-    else hipLaunchKernelGGL((k_ks_compact<256, uint32_t>), dim3(items), dim3(256), lds, s, dc, dk, dp, nc, pool);
-  } else {
-    typedef unsigned long long u64;
-    if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, u64>), dim3(items), dim3(1024), lds, s, dc, dk, dp, nc, pool);
-    else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, u64>), dim3(items), dim3(512), lds, s, dc, dk, dp, nc, pool);
-    else hipLaunchKernelGGL((k_ks_compact<256, u64>), dim3(items), dim3(256), lds, s, dc, dk, dp, nc, pool);
-  }
+  if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, E>), dim3(items), dim3(1024), lds, s, dc, dk, dp, nc);
+  else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, E>), dim3(items), dim3(512), lds, s, dc, dk, dp, nc);
+  else hipLaunchKernelGGL((k_ks_compact<256, E>), dim3(items), dim3(256), lds, s, dc, dk, dp, nc);
   prof_end(ctx, s);
   CAC_LAUNCH_CHECK(ctx, "ks compact");
   return CAC_OK;
@@ -815,71 +884,76 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild>& ch, KsChild* d_chil
 
 }  // namespace
 
-int ks_row_sums(cac_ctx* ctx, const int64_t* d_adj, uint32_t n, int64_t* d_rsum, int64_t* d_min, hipStream_t s) {
-  hipLaunchKernelGGL(k_fill_i64, dim3(1), dim3(64), 0, s, d_min, 1u, (int64_t)INT64_MAX);
-  hipLaunchKernelGGL(k_row_sums, dim3(grid_for(n, 4, 2048)), dim3(256), 0, s, d_adj, n, d_rsum, d_min);
-  CAC_LAUNCH_CHECK(ctx, "row sums");
-  return CAC_OK;
-}
-
-size_t ks_live_bytes_per_root(uint32_t n) {
-  // children of every node at one depth with their pool rows (and 1/8 spare);
-  // a depth's children go to the buffer its parents are not in, so the two
-  // buffers hold the largest even and the largest odd depth
+size_t ks_live_bytes_per_root(uint32_t n, bool w32) {
+  // children of every node at one depth with their pool rows; a depth's
+  // children go to the buffer its parents are not in, so the two buffers hold
+  // the largest even and the largest odd depth
+  const size_t esize = w32 ? 4 : 8;
   size_t best[2] = {0, 0};
   uint64_t nodes = 1;
   int depth = 0;
   for (uint32_t sz = n; sz > kKsBase; sz = ks_target(sz), nodes *= 2, ++depth) {
     const uint32_t t = ks_target(sz);
-    const size_t b =
-        2 * nodes * (child_bytes(sz, t) + sizeof(KsChild) + 16 + child_pool_units(sz, t) * kKsUnit * 8 * 9 / 8);
+    const size_t b = 2 * nodes * (child_bytes(sz, t, esize) + sizeof(KsChild<int64_t>) + 16 +
+                                  (size_t)child_pool_rows(sz, t) * ks_pool_stride(sz) * esize);
     best[depth & 1] = std::max(best[depth & 1], b);
   }
   return best[0] + best[1] + 8192;
 }
 
-// Runs one Karger-Stein trial per root.  roots[i]: device matrix (n_i x n_i)
-// with its row sums, trial id, result slot and bound; d_results[slot] must hold
-// the bound already and receives min(bound, every leaf) by atomicMin.
-int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, hipStream_t s) {
-  if (roots.empty()) return CAC_OK;
+namespace {
+
+// The contraction's dynamic LDS may exceed the default limit: raise it once.
+template <typename E>
+int contract_attr(cac_ctx* ctx) {
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute((const void*)k_ks_contract<1024, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)contract_lds_bytes<E>(kKsMaxS, 1024));
+    if (err == hipSuccess)
+      err = hipFuncSetAttribute((const void*)k_ks_contract<512, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)contract_lds_bytes<E>(512 * kKsChunk, 512));
+  });
+  CAC_HIP(ctx, err);
+  return CAC_OK;
+}
+
+// Runs one Karger-Stein trial per root of entry type E.  roots[i]: device matrix
+// (n_i x n_i, row stride ks_stride<E>(n_i)) with its row sums, trial id, result
+// slot and bound; d_results[slot] must hold the bound already and receives
+// min(bound, every leaf) by atomicMin.
+template <typename E>
+int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, hipStream_t s) {
+  typedef KsChild<E> Child;
   struct Node {
-    const int64_t* mat;
-    const int64_t* rsum;
-    const int64_t* rmax;
+    const E* mat;
+    const E* rsum;
+    const E* rmax;
     uint32_t s, trial, nid, slot;
     int64_t bound;
     uint32_t seed;
-    bool w32;  // the root's total weight is below 2^32 (a child's total never exceeds its parent's)
   };
-  static std::once_flag lds_attr;
-  hipError_t attr_err = hipSuccess;
-  std::call_once(lds_attr, [&] {
-    attr_err = hipFuncSetAttribute((const void*)k_ks_contract<1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)contract_lds_bytes(kKsMaxS, 1024));
-    if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)k_ks_contract<512>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)contract_lds_bytes(512 * kKsChunk, 512));
-  });
-  CAC_HIP(ctx, attr_err);
+  int rc = contract_attr<E>(ctx);
+  if (rc) return rc;
   // parents and children of a level live in the two level buffers
   BufPin pin0(ctx, kBufKs0), pin1(ctx, kBufKs1);
 
   std::vector<Node> level;
   for (const KsRoot& r : roots) {
     if (r.n > kKsMaxS) return fail(ctx, CAC_EINVAL, "dense Karger-Stein supports at most 8192 vertices");
-    level.push_back({r.mat, r.rsum, nullptr, r.n, r.trial, r.nid, r.slot, r.bound, r.seed, r.w32});
+    level.push_back({(const E*)r.mat, (const E*)r.rsum, nullptr, r.n, r.trial, r.nid, r.slot, r.bound, r.seed});
   }
   int buf = 0;  // level buffer for the children of this level; the parents are in the other one
   while (!level.empty()) {
-    std::vector<KsLeaf> leaves;
+    std::vector<KsLeaf<E>> leaves;
     std::vector<Node> internal;
     for (auto& nd : level) {
-      if (nd.s <= kKsBase) leaves.push_back({nd.mat, nd.rsum, nd.rmax, nd.s, nd.slot, nd.bound});
+      if (nd.s <= kKsBase) leaves.push_back({nd.mat, nd.rsum, nd.rmax, nd.s, ks_stride<E>(nd.s), nd.slot, nd.bound});
       else internal.push_back(nd);
     }
     if (!leaves.empty()) {
-      int rc = run_leaves(ctx, leaves, buf, d_results, s);
+      rc = run_leaves<E>(ctx, leaves, buf, d_results, s);
       if (rc) return rc;
     }
     if (internal.empty()) break;
@@ -888,46 +962,41 @@ int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, h
     for (uint32_t i = 0; i < internal.size(); ++i) order.push_back({-contract_block(ctx, internal[i].s), i});
     std::stable_sort(order.begin(), order.end());
     const size_t nchild = 2 * internal.size();
-    size_t arrays = 0, units = 0, max_units_child = 0;
+    size_t arrays = 0;
     uint32_t max_tgt = 0;
     for (auto& nd : internal) {
       const uint32_t t = ks_target(nd.s);
-      arrays += 2 * child_bytes(nd.s, t);
-      units += 2 * child_pool_units(nd.s, t);
-      max_units_child = std::max<size_t>(max_units_child, (nd.s + kKsUnit - 1) / kKsUnit * (size_t)nd.s);
+      arrays += 2 * (child_bytes(nd.s, t, sizeof(E)) +
+                     c64((size_t)child_pool_rows(nd.s, t) * ks_pool_stride(nd.s) * sizeof(E)));
       max_tgt = std::max(max_tgt, t);
     }
-    std::vector<KsChild> ch(nchild);
-    std::vector<uint32_t> item_prefix(nchild + 1);
+    std::vector<Child> ch(nchild);
     std::vector<uint32_t> kout(nchild);
-    // first pass: pool rows for the picks with 1/8 spare; children whose PR pass
-    // needs more come back as kKsOverflow and are redone below
-    const size_t pool_units = units + std::max<size_t>(units / 8, max_units_child);
-    if (pool_units >= kLiveWork) return fail(ctx, CAC_ENOMEM, "Karger-Stein level too large for one pass");
-    const size_t bytes = c64(nchild * sizeof(KsChild)) + c64((nchild + 1) * 4) + c64(nchild * 4) + 64 + arrays +
-                         pool_units * kKsUnit * 8 + 1024;
+    const size_t bytes = c64(nchild * sizeof(Child)) + c64((nchild + 1) * 4) + c64(nchild * 4) + arrays + 1024;
     void* base = nullptr;
-    int rc = ks_reserve(ctx, buf, bytes, &base);
+    rc = ks_reserve(ctx, buf, bytes, &base);
     if (rc) return rc;
     Carve64 cv(base);
-    KsChild* d_children = cv.take<KsChild>(nchild);
+    Child* d_children = cv.take<Child>(nchild);
     uint32_t* d_prefix = cv.take<uint32_t>(nchild + 1);
     uint32_t* d_kout = cv.take<uint32_t>(nchild);
-    unsigned long long* d_used = cv.take<unsigned long long>(1);
     size_t ci = 0;
     for (auto& o : order) {
       const Node& nd = internal[o.second];
       const uint32_t t = ks_target(nd.s);
       for (uint32_t k = 0; k < 2; ++k, ++ci) {
-        KsChild& x = ch[ci];
+        Child& x = ch[ci];
         x.parent = nd.mat;
         x.prsum = nd.rsum;
-        x.out = cv.take<int64_t>((size_t)t * t);
-        x.orsum = cv.take<int64_t>(t);
-        x.ormax = cv.take<int64_t>(t);
-        x.colmap = cv.take<uint32_t>(nd.s);
+        x.out = cv.take<E>((size_t)t * ks_stride<E>(t));
+        x.orsum = cv.take<E>(t);
+        x.ormax = cv.take<E>(t);
+        x.colmap = cv.take<uint16_t>((size_t)nd.s + 8);
         x.live = cv.take<uint32_t>(t);
+        x.pool_rows = child_pool_rows(nd.s, t);
+        x.pool = cv.take<E>((size_t)x.pool_rows * ks_pool_stride(nd.s));
         x.s = nd.s;
+        x.ps = ks_stride<E>(nd.s);
         x.tgt = t;
         x.trial = nd.trial;
         x.nid = 2 * nd.nid + k;
@@ -936,11 +1005,7 @@ int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, h
         x.bound = nd.bound;
       }
     }
-    cv.off = (cv.off + 511) & ~size_t(511);
-    KsPool pool{(int64_t*)(cv.base + cv.off), d_used, pool_units};
-    bool w32 = true;
-    for (const Node& nd : internal) w32 = w32 && nd.w32;
-    rc = contract_level(ctx, ch, d_children, d_prefix, d_kout, d_used, pool, max_tgt, d_results, kout, w32, s);
+    rc = contract_level<E>(ctx, ch, d_children, d_prefix, d_kout, max_tgt, d_results, kout, s);
     if (rc) return rc;
     // children that ran out of pool rows: again, with s pool rows each (a child
     // merges at most s - 2 times, so this cannot overflow)
@@ -948,26 +1013,26 @@ int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, h
     for (uint32_t i = 0; i < nchild; ++i)
       if (kout[i] == kKsOverflow) over.push_back(i);
     if (!over.empty()) {
-      std::vector<KsChild> rch;
-      size_t runits = 0;
+      std::vector<Child> rch;
+      size_t rpool = 0;
       for (uint32_t i : over) {
         rch.push_back(ch[i]);
-        runits += (size_t)ch[i].s * ((ch[i].s + kKsUnit - 1) / kKsUnit);
+        rpool += c64((size_t)ch[i].s * ks_pool_stride(ch[i].s) * sizeof(E));
       }
       const size_t no = rch.size();
-      if (runits >= kLiveWork) return fail(ctx, CAC_ENOMEM, "Karger-Stein level too large for one pass");
-      const size_t rbytes = c64(no * sizeof(KsChild)) + c64((no + 1) * 4) + c64(no * 4) + 64 + runits * kKsUnit * 8 + 1024;
+      const size_t rbytes = c64(no * sizeof(Child)) + c64((no + 1) * 4) + c64(no * 4) + rpool + 1024;
       rc = grow_buffer(ctx, &ctx->ks_retry_buf, &ctx->ks_retry_bytes, rbytes);
       if (rc) return rc;
       Carve64 rv(ctx->ks_retry_buf);
-      KsChild* d_rch = rv.take<KsChild>(no);
+      Child* d_rch = rv.take<Child>(no);
       uint32_t* d_rprefix = rv.take<uint32_t>(no + 1);
       uint32_t* d_rkout = rv.take<uint32_t>(no);
-      unsigned long long* d_rused = rv.take<unsigned long long>(1);
-      rv.off = (rv.off + 511) & ~size_t(511);
-      KsPool rpool{(int64_t*)(rv.base + rv.off), d_rused, runits};
+      for (Child& x : rch) {
+        x.pool_rows = x.s;
+        x.pool = rv.take<E>((size_t)x.s * ks_pool_stride(x.s));
+      }
       std::vector<uint32_t> rkout(no);
-      rc = contract_level(ctx, rch, d_rch, d_rprefix, d_rkout, d_rused, rpool, max_tgt, d_results, rkout, w32, s);
+      rc = contract_level<E>(ctx, rch, d_rch, d_rprefix, d_rkout, max_tgt, d_results, rkout, s);
       if (rc) return rc;
       for (size_t k = 0; k < no; ++k) {
         if (rkout[k] == kKsOverflow) return fail(ctx, CAC_EDEVICE, "Karger-Stein row pool overflow");
@@ -979,13 +1044,25 @@ int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, h
       if (kout[i] == kKsBad) return fail(ctx, CAC_EDEVICE, "Karger-Stein selection out of range");
       if (kout[i] == 0) continue;  // disconnected child: its 0 is already recorded
       next.push_back({ch[i].out, ch[i].orsum, ch[i].ormax, kout[i], ch[i].trial, ch[i].nid, ch[i].slot, ch[i].bound,
-                      ch[i].seed, w32});
+                      ch[i].seed});
     }
     level.swap(next);
     buf ^= 1;
   }
   CAC_HIP(ctx, hipStreamSynchronize(s));
   return CAC_OK;
+}
+
+}  // namespace
+
+// Roots of 32-bit and of 64-bit entries run one kind after the other.
+int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, hipStream_t s) {
+  std::vector<KsRoot> kind[2];
+  for (const KsRoot& r : roots) kind[r.w32 ? 1 : 0].push_back(r);
+  int rc = CAC_OK;
+  if (!kind[1].empty()) rc = ks_run_typed<uint32_t>(ctx, kind[1], d_results, s);
+  if (rc == CAC_OK && !kind[0].empty()) rc = ks_run_typed<int64_t>(ctx, kind[0], d_results, s);
+  return rc;
 }
 
 // Validates a host matrix: symmetric, zero diagonal, non-negative, no overflow.
@@ -1008,21 +1085,31 @@ int ks_dense_run(cac_ctx* ctx, const int64_t* d_adj, uint32_t n, uint32_t seed, 
                  uint32_t ntrials, int64_t* raw_cuts, int64_t* min_cut, hipStream_t s) {
   if (ntrials == 0) return fail(ctx, CAC_EINVAL, "ntrials must be >= 1");
   if (n > kKsMaxS) return fail(ctx, CAC_EINVAL, "dense Karger-Stein supports at most 8192 vertices");
-  int64_t* d_small = nullptr;  // [0] bound, [1..n] row sums, then the trial results
-  CAC_HIP(ctx, hipMalloc((void**)&d_small, 8 * ((size_t)n + ntrials + 2)));
-  int64_t* d_bound = d_small;
-  int64_t* d_rsum = d_small + 1;
-  int64_t* d_res = d_small + 1 + n;
-  int rc = ks_row_sums(ctx, d_adj, n, d_rsum, d_bound, s);
+  // the root's row sums, bound and trial results, and its 32-bit copy
+  const size_t n32 = (size_t)n * ks_stride<uint32_t>(n);
+  int rc = grow_buffer(ctx, &ctx->sp_dense_buf, &ctx->sp_dense_bytes,
+                       carve_size(8) + carve_size(8 * (size_t)n) + carve_size(8 * (size_t)ntrials) +
+                           carve_size(4 * (size_t)n) + carve_size(4 * n32));
+  if (rc) return rc;
+  BufPin pin(ctx, kBufSpDense);
+  Carver cv(ctx->sp_dense_buf);
+  int64_t* d_bound = cv.take<int64_t>(1);
+  int64_t* d_rsum = cv.take<int64_t>(n);
+  int64_t* d_res = cv.take<int64_t>(ntrials);
+  uint32_t* d_rsum32 = cv.take<uint32_t>(n);
+  uint32_t* d_adj32 = cv.take<uint32_t>(n32);
+  hipLaunchKernelGGL(k_fill_i64, dim3(1), dim3(64), 0, s, d_bound, 1u, (int64_t)INT64_MAX);
+  hipLaunchKernelGGL(k_row_sums, dim3(grid_for(n, 4, 2048)), dim3(256), 0, s, d_adj, n, d_rsum, d_bound, d_adj32,
+                     d_rsum32);
+  CAC_LAUNCH_CHECK(ctx, "row sums");
   int64_t bound = 0;
-  std::vector<int64_t> rs(n);  // the row sums: their total decides 32-bit compaction sums
-  if (rc == CAC_OK) {
-    hipError_t e = hipMemcpyAsync(&bound, d_bound, 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(rs.data(), d_rsum, 8 * (size_t)n, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = hip_fail(ctx, e, "row sums");
-  }
-  bool w32 = rc == CAC_OK;  // total weight below 2^32, checked without wrapping
+  std::vector<int64_t> rs(n);  // the row sums: their total decides the entry type
+  hipError_t e = hipMemcpyAsync(&bound, d_bound, 8, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(rs.data(), d_rsum, 8 * (size_t)n, hipMemcpyDeviceToHost, s);
+  const hipError_t e_sync = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = e_sync;
+  if (e != hipSuccess) return hip_fail(ctx, e, "row sums");
+  bool w32 = true;  // total weight below 2^32, checked without wrapping
   uint64_t total = 0;
   for (int64_t r : rs) {
     if (r < 0 || (uint64_t)r >= (1ull << 32) || (total += (uint64_t)r) >= (1ull << 32)) {
@@ -1030,31 +1117,30 @@ int ks_dense_run(cac_ctx* ctx, const int64_t* d_adj, uint32_t n, uint32_t seed, 
       break;
     }
   }
-  if (rc == CAC_OK) {
-    hipLaunchKernelGGL(k_fill_i64, dim3(grid_for(ntrials, 256, 64)), dim3(256), 0, s, d_res, ntrials, bound);
-    // trials run in batches whose two live levels fit in 3/4 of the free
-    // memory: the top levels are chains of picks with one workgroup per child,
-    // so the more trials a batch holds, the more CUs they keep busy.  Every
-    // batch but the last is as large as that allows: at n = 8192 the first of
-    // two then fills the CUs at the levels where children outnumber them (two
-    // even batches of 85 left a partial round of workgroups in each)
-    size_t avail = 0;
-    rc = device_memory_available(ctx, &avail);
-    const size_t per_trial = ks_live_bytes_per_root(n);
-    size_t batch = std::max<size_t>(1, (size_t)(0.75 * (double)avail) / per_trial);
-    batch = std::min<size_t>(batch, ntrials);
-    for (uint32_t t0 = 0; t0 < ntrials && rc == CAC_OK; t0 += (uint32_t)batch) {
-      std::vector<KsRoot> roots;
-      for (uint32_t t = t0; t < std::min<uint32_t>(ntrials, t0 + (uint32_t)batch); ++t)
-        roots.push_back({d_adj, d_rsum, n, first_trial + t, t, bound, seed, 1, w32});
-      rc = ks_run(ctx, roots, d_res, s);
-    }
+  hipLaunchKernelGGL(k_fill_i64, dim3(grid_for(ntrials, 256, 64)), dim3(256), 0, s, d_res, ntrials, bound);
+  // trials run in batches whose two live levels fit in 3/4 of the free
+  // memory: the top levels are chains of picks with one workgroup per child,
+  // so the more trials a batch holds, the more CUs they keep busy.  Every
+  // batch but the last is as large as that allows: at n = 8192 the first of
+  // two then fills the CUs at the levels where children outnumber them (two
+  // even batches of 85 left a partial round of workgroups in each)
+  size_t avail = 0;
+  rc = device_memory_available(ctx, &avail);
+  const size_t per_trial = ks_live_bytes_per_root(n, w32);
+  size_t batch = std::max<size_t>(1, (size_t)(0.75 * (double)avail) / per_trial);
+  batch = std::min<size_t>(batch, ntrials);
+  for (uint32_t t0 = 0; t0 < ntrials && rc == CAC_OK; t0 += (uint32_t)batch) {
+    std::vector<KsRoot> roots;
+    for (uint32_t t = t0; t < std::min<uint32_t>(ntrials, t0 + (uint32_t)batch); ++t)
+      roots.push_back({w32 ? (const void*)d_adj32 : (const void*)d_adj,
+                       w32 ? (const void*)d_rsum32 : (const void*)d_rsum, n, first_trial + t, t, bound, seed, 1, w32});
+    rc = ks_run(ctx, roots, d_res, s);
   }
   if (rc == CAC_OK) {
     std::vector<int64_t> res(ntrials);
-    hipError_t e = hipMemcpyAsync(res.data(), d_res, 8 * (size_t)ntrials, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = hip_fail(ctx, e, "trial results");
+    hipError_t e2 = hipMemcpyAsync(res.data(), d_res, 8 * (size_t)ntrials, hipMemcpyDeviceToHost, s);
+    if (e2 == hipSuccess) e2 = hipStreamSynchronize(s);
+    if (e2 != hipSuccess) rc = hip_fail(ctx, e2, "trial results");
     int64_t mn = INT64_MAX;
     for (uint32_t t = 0; t < ntrials && rc == CAC_OK; ++t) {
       if (raw_cuts) raw_cuts[t] = res[t];
@@ -1063,7 +1149,6 @@ int ks_dense_run(cac_ctx* ctx, const int64_t* d_adj, uint32_t n, uint32_t seed, 
     if (rc == CAC_OK && min_cut) *min_cut = mn;
   }
   (void)hipStreamSynchronize(s);
-  (void)hipFree(d_small);
   return rc;
 }
 

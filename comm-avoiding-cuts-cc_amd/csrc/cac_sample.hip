@@ -24,6 +24,7 @@
 #include <cmath>
 #include <functional>
 #include <mutex>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -46,30 +47,45 @@ constexpr int kSmpBlock = 1024;
 constexpr int kSmpWaves = kSmpBlock / 64;
 constexpr int kSmpIndex = 4096;  // LDS segment index of the weight prefix (32 KiB)
 
-// A distinct graph of a sampling launch and its flag word.
+// A distinct graph of a sampling launch, its flag word and its total weight.
 struct EdgeSpan {
   const cac_edge* edges;
   uint64_t m;
   uint32_t* mixed;
+  unsigned long long* total;
 };
 
 __global__ void k_mixed_zero(const EdgeSpan* spans, uint32_t count) {
-  for (uint32_t g = blockIdx.x * 256 + threadIdx.x; g < count; g += gridDim.x * 256)
+  for (uint32_t g = blockIdx.x * 256 + threadIdx.x; g < count; g += gridDim.x * 256) {
     __hip_atomic_store(spans[g].mixed, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(spans[g].total, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // Grid (slices, graphs): flags graph blockIdx.y when one of its edges is a loop
-// or weighs other than its first edge (or the first weighs 0).
+// or weighs other than its first edge (or the first weighs 0), and adds up its
+// weights, each cut to 2^31 (fewer than 2^32 edges cannot wrap the sum, and a
+// cut weight puts it past kTrialW32Total).
 __global__ void __launch_bounds__(256) k_mixed_weights(const EdgeSpan* spans) {
   const EdgeSpan sp = spans[blockIdx.y];
   if (sp.m == 0) return;
   const uint64_t w0 = sp.edges[0].w;
   bool bad = w0 == 0;
+  uint64_t sum = 0;
   for (uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x; e < sp.m; e += (uint64_t)gridDim.x * 256) {
     const cac_edge x = sp.edges[e];
     bad = bad || x.w != w0 || x.u == x.v;
+    sum += min((uint64_t)x.w, (uint64_t)kTrialW32Total);
   }
   if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(sp.mixed, 1u);
+  __shared__ uint64_t part[4];  // one addition per block: those to one word serialise
+  sum = wave_sum<uint64_t>(sum);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    sum = part[0] + part[1] + part[2] + part[3];
+    if (sum) atomicAdd(sp.total, (unsigned long long)sum);
+  }
 }
 
 __device__ inline uint64_t wsum64(uint64_t x) { return wave_sum<uint64_t>(x); }
@@ -363,6 +379,80 @@ __global__ void __launch_bounds__(kSmpBlock, kMinWaves)
 constexpr size_t kDensifyLds = (size_t)kKsMaxS * 8;
 constexpr int kDensifyEdges = 4;  // edges per thread in flight
 
+// The accumulation of k_densify_trials for entries of type E (row stride
+// ks_stride<E>(k)): zeroes the matrix with 16-byte stores, adds the surviving
+// edges by atomics, writes the row sums and returns the thread's part of their
+// minimum.  32-bit entries halve the zero fill, the largest write of a trial
+// (t^2 entries against m edges of 16 bytes).
+template <bool kRankLabels, typename E>
+__device__ uint64_t densify_edges(const TrialScratch& S, uint32_t k, const uint32_t* rank, unsigned char* smem) {
+  typedef typename std::conditional<sizeof(E) == 4, uint32_t, unsigned long long>::type A;
+  A* mat = (A*)S.mat;
+  A* rsum = (A*)S.rsum;
+  A* row_sum = (A*)smem;  // [k] in LDS
+  const cac_edge* __restrict__ edges = S.edges;
+  const uint64_t m = S.m;
+  const uint64_t st = ks_stride<E>(k), cells = st * k;
+  constexpr uint64_t V = 16 / sizeof(A);
+  for (uint64_t i = threadIdx.x; i < cells / V; i += kSmpBlock) ((uint4*)mat)[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (uint64_t i = cells / V * V + threadIdx.x; i < cells; i += kSmpBlock) mat[i] = 0;
+  const bool lds_rows = k <= kKsMaxS;  // else the row sums are read back from the matrix
+  for (uint32_t r = threadIdx.x; lds_rows && r < k; r += kSmpBlock) row_sum[r] = 0;
+  block_sync_global();  // ranks and zeroed rows before the accumulation
+  // kDensifyEdges edges per thread: their label and rank loads are in flight together
+  for (uint64_t base = 0; base < m; base += (uint64_t)kSmpBlock * kDensifyEdges) {
+    cac_edge x[kDensifyEdges];
+    uint32_t a[kDensifyEdges], b[kDensifyEdges];
+#pragma unroll
+    for (int j = 0; j < kDensifyEdges; ++j) {
+      const uint64_t e = base + (uint64_t)j * kSmpBlock + threadIdx.x;
+      x[j] = e < m ? edges[e] : cac_edge{0u, 0u, 0ull};  // vertex 0 stands in: same label, skipped
+    }
+#pragma unroll
+    for (int j = 0; j < kDensifyEdges; ++j) {
+      a[j] = S.lab[x[j].u];
+      b[j] = S.lab[x[j].v];
+    }
+    if constexpr (!kRankLabels) {
+#pragma unroll
+      for (int j = 0; j < kDensifyEdges; ++j) {
+        a[j] = rank[a[j]];
+        b[j] = rank[b[j]];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kDensifyEdges; ++j) {
+      if (a[j] == b[j]) continue;
+      const A w = (A)x[j].w;
+      atomicAdd(&mat[a[j] * st + b[j]], w);
+      atomicAdd(&mat[b[j] * st + a[j]], w);
+      if (lds_rows) {
+        atomicAdd(&row_sum[a[j]], w);
+        atomicAdd(&row_sum[b[j]], w);
+      }
+    }
+  }
+  block_sync_global();
+  // row sums (the Karger-Stein capacities) and bound = min row sum
+  uint64_t best = ~0ull;
+  if (lds_rows) {
+    for (uint32_t r = threadIdx.x; r < k; r += kSmpBlock) {
+      const uint64_t acc = row_sum[r];
+      if (rsum) rsum[r] = (A)acc;
+      best = acc < best ? acc : best;
+    }
+  } else {  // one wave per row
+    for (uint32_t r = threadIdx.x >> 6; r < k; r += kSmpWaves) {
+      uint64_t acc = 0;
+      for (uint32_t x = threadIdx.x & 63; x < k; x += 64) acc += (uint64_t)mat[r * st + x];
+      acc = wsum64(acc);
+      if (rsum && (threadIdx.x & 63) == 0) rsum[r] = (A)acc;
+      best = acc < best ? acc : best;
+    }
+  }
+  return best;
+}
+
 // Rank the canonical labels, accumulate the surviving edges into the k x k
 // matrix (k == t unless the sampling stopped early on a disconnected graph),
 // with its row sums in LDS, and compute the trial's bound (minimum weighted
@@ -375,10 +465,8 @@ __global__ void __launch_bounds__(kSmpBlock) k_densify_trials(const TrialScratch
                                                               int64_t* results) {
   __shared__ uint32_t wtot[kSmpWaves];
   __shared__ uint64_t lds[kSmpWaves + 2];
-  extern __shared__ unsigned long long row_sum[];  // [k]
+  extern __shared__ __align__(16) unsigned char densify_lds[];
   const TrialScratch S = scratch[blockIdx.x];
-  const cac_edge* __restrict__ edges = S.edges;
-  const uint64_t m = S.m;
   const uint32_t n = S.n, t = S.t, slot = S.slot;
   const uint32_t k = *S.nv_out;
   if (k > t) {  // disconnected: a cut of weight 0 exists
@@ -410,61 +498,8 @@ __global__ void __launch_bounds__(kSmpBlock) k_densify_trials(const TrialScratch
     block_sync_global();  // every rank written
     for (uint32_t x = threadIdx.x; x < n; x += kSmpBlock) S.lab[x] = rank[S.lab[x]];
   }
-  for (uint64_t i = threadIdx.x; i < (uint64_t)k * k; i += kSmpBlock) S.mat[i] = 0;
-  const bool lds_rows = k <= kKsMaxS;  // else the row sums are read back from the matrix
-  for (uint32_t r = threadIdx.x; lds_rows && r < k; r += kSmpBlock) row_sum[r] = 0;
-  block_sync_global();  // ranks and zeroed rows before the accumulation
-  // kDensifyEdges edges per thread: their label and rank loads are in flight together
-  for (uint64_t base = 0; base < m; base += (uint64_t)kSmpBlock * kDensifyEdges) {
-    cac_edge x[kDensifyEdges];
-    uint32_t a[kDensifyEdges], b[kDensifyEdges];
-#pragma unroll
-    for (int j = 0; j < kDensifyEdges; ++j) {
-      const uint64_t e = base + (uint64_t)j * kSmpBlock + threadIdx.x;
-      x[j] = e < m ? edges[e] : cac_edge{0u, 0u, 0ull};  // vertex 0 stands in: same label, skipped
-    }
-#pragma unroll
-    for (int j = 0; j < kDensifyEdges; ++j) {
-      a[j] = S.lab[x[j].u];
-      b[j] = S.lab[x[j].v];
-    }
-    if constexpr (!kRankLabels) {
-#pragma unroll
-      for (int j = 0; j < kDensifyEdges; ++j) {
-        a[j] = rank[a[j]];
-        b[j] = rank[b[j]];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kDensifyEdges; ++j) {
-      if (a[j] == b[j]) continue;
-      const unsigned long long w = x[j].w;
-      atomicAdd((unsigned long long*)&S.mat[(uint64_t)a[j] * k + b[j]], w);
-      atomicAdd((unsigned long long*)&S.mat[(uint64_t)b[j] * k + a[j]], w);
-      if (lds_rows) {
-        atomicAdd(&row_sum[a[j]], w);
-        atomicAdd(&row_sum[b[j]], w);
-      }
-    }
-  }
-  block_sync_global();
-  // row sums (the Karger-Stein capacities) and bound = min row sum
-  uint64_t best = ~0ull;
-  if (lds_rows) {
-    for (uint32_t r = threadIdx.x; r < k; r += kSmpBlock) {
-      const uint64_t acc = row_sum[r];
-      if (S.rsum) S.rsum[r] = (int64_t)acc;
-      best = acc < best ? acc : best;
-    }
-  } else {  // one wave per row
-    for (uint32_t r = threadIdx.x >> 6; r < k; r += kSmpWaves) {
-      uint64_t acc = 0;
-      for (uint32_t x = threadIdx.x & 63; x < k; x += 64) acc += (uint64_t)S.mat[(uint64_t)r * k + x];
-      acc = wsum64(acc);
-      if (S.rsum && (threadIdx.x & 63) == 0) S.rsum[r] = (int64_t)acc;
-      best = acc < best ? acc : best;
-    }
-  }
+  uint64_t best = trial_w32(S) ? densify_edges<kRankLabels, uint32_t>(S, k, rank, densify_lds)
+                               : densify_edges<kRankLabels, int64_t>(S, k, rank, densify_lds);
   best = wave_min<uint64_t>(best);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = best;
   __syncthreads();
@@ -553,11 +588,12 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 }
 
 
-// Points scr[i].mixed at a flag word of its graph (one per distinct edge list)
-// and launches the kernels that set the flags; spans and flags hold scr.size()
-// entries.  The flags are ready for any later launch on s.
+// Points scr[i].mixed and scr[i].total at a flag word and a total weight of its
+// graph (one per distinct edge list) and launches the kernels that set them;
+// spans, flags and totals hold scr.size() entries.  Both are ready for any later
+// launch on s.
 int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d_spans, uint32_t* d_flags,
-                       hipStream_t s) {
+                       unsigned long long* d_totals, hipStream_t s) {
   std::unordered_map<const cac_edge*, uint32_t> index;
   std::vector<EdgeSpan> spans;
   uint64_t mmax = 0;
@@ -567,12 +603,13 @@ int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d
     if (it == index.end()) {
       g = (uint32_t)spans.size();
       index.emplace(x.edges, g);
-      spans.push_back({x.edges, x.m, d_flags + g});
+      spans.push_back({x.edges, x.m, d_flags + g, d_totals + g});
       mmax = std::max(mmax, x.m);
     } else {
       g = it->second;
     }
     x.mixed = d_flags + g;
+    x.total = d_totals + g;
   }
   if (spans.empty()) return CAC_OK;
   const uint32_t count = (uint32_t)spans.size();
@@ -740,7 +777,7 @@ size_t job_sample_bytes(const SqrtJob& j, uint32_t dpr) {
 // Upper estimate of the Karger-Stein level arenas of one root of size t: each
 // level holds about t^2 entries in copy-on-write work rows plus the contracted
 // children, and two levels are alive at once.
-size_t job_ks_bytes(const SqrtJob& j) { return ks_live_bytes_per_root(j.t); }
+size_t job_ks_bytes(const SqrtJob& j) { return ks_live_bytes_per_root(j.t, false); }
 
 // Edge-count bound from which a job of the batch runs in the wide form.  One
 // workgroup scans a trial's edges in time proportional to m on one CU, while
@@ -795,7 +832,7 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
     const uint64_t m = std::max<uint64_t>(j.m, 1);
     return carve_size(sizeof(TrialScratch)) + 3 * carve_size((size_t)j.n * 4) + carve_size(m * 8) +
            carve_size((size_t)std::max(j.n, job_dpr(ctx, j.n)) * 8) + carve_size(64) + carve_size(((size_t)j.t + 2) * 8) +
-           carve_size(sizeof(EdgeSpan)) + carve_size(4) + 64 * m +  // 64 m: the shared merge buffers
+           carve_size(sizeof(EdgeSpan)) + carve_size(4) + carve_size(8) + 64 * m +  // 64 m: the shared merge buffers
            (j.m >= wmin ? wide_trial_bytes(j.m, j.n) : 0);
   };
   size_t avail = 0;
@@ -851,6 +888,7 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
     TrialScratch* d_scr = cv.take<TrialScratch>(nb);
     EdgeSpan* d_spans = cv.take<EdgeSpan>(nb);
     uint32_t* d_flags = cv.take<uint32_t>(nb);
+    unsigned long long* d_totals = cv.take<unsigned long long>(nb);
     void* wide_work = cv.take<unsigned char>(std::max<size_t>(wide_bytes, 1));
     std::vector<TrialScratch> scr(nb);
     std::vector<uint32_t*> rank(nb);
@@ -877,10 +915,9 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
       deg[i] = cv.take<unsigned long long>((size_t)j.t + 2);  // [t] degrees, [t + 1] their minimum
       offsets[i + 1] = offsets[i] + j.m;
     }
-    std::vector<TrialScratch> nar(scr.begin(), scr.begin() + w0), wid(scr.begin() + w0, scr.end());
-    rc = launch_mixed_flags(ctx, nar, d_spans, d_flags, s);
+    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, s);
     if (rc) return rc;
-    for (size_t i = 0; i < w0; ++i) scr[i] = nar[i];
+    std::vector<TrialScratch> wid(scr.begin() + w0, scr.end());
     CAC_HIP(ctx, hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s));
     CAC_HIP(ctx, hipMemcpyAsync(d_offsets, offsets.data(), (nb + 1) * 8, hipMemcpyHostToDevice, s));
     CAC_HIP(ctx, hipMemcpyAsync(d_deg, deg.data(), nb * sizeof(void*), hipMemcpyHostToDevice, s));
@@ -901,6 +938,8 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
     prof_end(ctx, s);
     CAC_LAUNCH_CHECK(ctx, "sample trials");
     std::vector<uint32_t> nv(nb);
+    std::vector<unsigned long long> totals(nb);
+    CAC_HIP(ctx, hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s));
     for (size_t i = 0; i < nb; ++i) CAC_HIP(ctx, hipMemcpyAsync(&nv[i], scr[i].nv_out, 4, hipMemcpyDeviceToHost, s));
     CAC_HIP(ctx, hipStreamSynchronize(s));
     // keys of every job (a disconnected trial's edges all become loops: its
@@ -967,7 +1006,7 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
       const uint64_t mm = firsts[i + 1] - firsts[i];
       if (nv[i] > j.t || nv[i] < 2 || mm == 0) continue;
       roots.push_back({reinterpret_cast<cac_edge*>(pairs) + firsts[i], mm, nv[i], j.trial, j.slot,
-                       (int64_t)bounds[i], j.seed});
+                       (int64_t)bounds[i], j.seed, totals[scr[i].total - d_totals] < kTrialW32Total});
     }
     rc = ks_sparse_roots(ctx, roots, d_results, s);
     if (rc) return rc;
@@ -1007,7 +1046,8 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
         wide_bytes += wide_trial_bytes(jobs[b0 + i].m, jobs[b0 + i].n);
     }
     const size_t bytes = sample_bytes + carve_size(nb * sizeof(TrialScratch)) + 2 * carve_size(nb * 8) +
-                         carve_size(nb * sizeof(EdgeSpan)) + carve_size(nb * 4) + carve_size(wide_bytes) + 1024;
+                         carve_size(nb * sizeof(EdgeSpan)) + carve_size(nb * 4) + carve_size(nb * 8) +
+                         carve_size(wide_bytes) + 1024;
     rc = grow_buffer(ctx, &ctx->smp_buf, &ctx->smp_bytes, bytes);
     if (rc) return rc;
     BufPin pin(ctx, kBufSmp);  // the sampled matrices are the dense roots
@@ -1018,6 +1058,7 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     int64_t* d_bounds = cv.take<int64_t>(nb);
     EdgeSpan* d_spans = cv.take<EdgeSpan>(nb);
     uint32_t* d_flags = cv.take<uint32_t>(nb);
+    unsigned long long* d_totals = cv.take<unsigned long long>(nb);
     void* wide_work = wide ? (void*)cv.take<unsigned char>(wide_bytes) : nullptr;
     std::vector<TrialScratch> scr(nb);
     for (size_t i = 0; i < nb; ++i) {
@@ -1035,14 +1076,12 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       x.par = cv.take<uint32_t>(j.n);
       x.pre = cv.take<uint64_t>(std::max<uint64_t>(j.m, 1));
       x.draws = cv.take<uint2>(std::max(j.n, x.dpr));
-      x.mat = cv.take<int64_t>((size_t)j.t * j.t);
+      x.mat = cv.take<int64_t>((size_t)j.t * j.t);  // room for either entry type
       x.rsum = cv.take<int64_t>(j.t);
       x.nv_out = d_nv + i;
     }
-    if (!wide) {
-      rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, s);
-      if (rc) return rc;
-    }
+    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, s);
+    if (rc) return rc;
     e = hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "job descriptors");
     if (rc == CAC_OK && wide) {
@@ -1072,9 +1111,11 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     }
     std::vector<uint32_t> nvs(nb);
     std::vector<int64_t> hb(nb);
+    std::vector<unsigned long long> totals(nb);
     if (rc == CAC_OK) {
       (void)hipMemcpyAsync(nvs.data(), d_nv, nb * 4, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(hb.data(), d_bounds, nb * 8, hipMemcpyDeviceToHost, s);
+      (void)hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s);
       e = hipStreamSynchronize(s);
       if (e != hipSuccess) rc = hip_fail(ctx, e, "sampling kernels");
     }
@@ -1082,7 +1123,8 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       std::vector<KsRoot> roots;
       for (size_t i = 0; i < nb; ++i)
         if (nvs[i] >= 2 && nvs[i] <= scr[i].t)
-          roots.push_back({scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed});
+          roots.push_back({scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed, 1,
+                           totals[scr[i].total - d_totals] < kTrialW32Total});
       rc = ks_run(ctx, roots, d_results, s);
     }
     (void)hipStreamSynchronize(s);
@@ -1152,7 +1194,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   const uint32_t dpr = job_dpr(ctx, n);
   const size_t bytes = carve_size((size_t)n * 4) * 2 + carve_size(std::max<uint64_t>(m, 1) * 8) +
                        carve_size((size_t)std::max(n, dpr) * 8) + 4 * carve_size(64) + carve_size(sizeof(TrialScratch)) +
-                       carve_size(sizeof(EdgeSpan)) + carve_size(4);
+                       carve_size(sizeof(EdgeSpan)) + carve_size(4) + carve_size(8);
   CAC_HIP(ctx, hipMalloc(&out->arena, bytes));
   Carver cv(out->arena);
   TrialScratch h{};
@@ -1173,12 +1215,14 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   int64_t* d_misc = cv.take<int64_t>(2);
   EdgeSpan* d_span = cv.take<EdgeSpan>(1);
   uint32_t* d_flag = cv.take<uint32_t>(1);
+  unsigned long long* d_total = cv.take<unsigned long long>(1);
   h.mat = nullptr;
   h.rsum = nullptr;
   std::vector<TrialScratch> one{h};
-  int rc = launch_mixed_flags(ctx, one, d_span, d_flag, s);
+  int rc = launch_mixed_flags(ctx, one, d_span, d_flag, d_total, s);
   if (rc) return rc;
   h = one[0];
+  h.total = nullptr;  // the merged matrix is read as int64
   CAC_HIP(ctx, hipMemcpyAsync(d_scr, &h, sizeof h, hipMemcpyHostToDevice, s));
   rc = launch_sampling(ctx, 1, m, n, d_scr, s);
   if (rc) return rc;
@@ -1186,7 +1230,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   uint32_t k = 0;
   CAC_HIP(ctx, hipMemcpyAsync(&k, h.nv_out, 4, hipMemcpyDeviceToHost, s));
   CAC_HIP(ctx, hipStreamSynchronize(s));
-  CAC_HIP(ctx, hipMalloc((void**)&h.mat, std::max<size_t>((size_t)k * k, 1) * 8));
+  CAC_HIP(ctx, hipMalloc(&h.mat, std::max<size_t>((size_t)k * k, 1) * 8));
   h.t = k;
   CAC_HIP(ctx, hipMemcpyAsync(d_scr, &h, sizeof h, hipMemcpyHostToDevice, s));
   rc = densify_attr(ctx);
@@ -1196,7 +1240,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   CAC_LAUNCH_CHECK(ctx, "densify trial");
   CAC_HIP(ctx, hipStreamSynchronize(s));
   out->lab = h.lab;
-  out->mat = h.mat;
+  out->mat = (int64_t*)h.mat;
   out->k = k;
   return CAC_OK;
 }

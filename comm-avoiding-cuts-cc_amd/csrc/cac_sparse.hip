@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <string>
 #include <vector>
 
@@ -535,23 +536,27 @@ void launch_sparse_contract(const SpChild* d_children, uint32_t nchild, uint64_t
 // workgroup sums each band's entries in LDS and writes the band's rows, zeros
 // included, and their row sums, once.  Every matrix entry is written once and
 // never read back; the only atomics are on LDS and on per-tile band cursors.
-constexpr uint32_t kSpBandEntries = 8192;                       // int64 entries of a band (64 KiB of LDS)
+constexpr uint32_t kSpBandEntries = 8192;                       // entries of a band (32 or 64 KiB of LDS)
 constexpr int kSpBucketBlock = 1024;                            // bucketing: edges per thread x block = a tile
 constexpr int kSpBucketEdges = 8;
 constexpr uint64_t kSpBucketTile = (uint64_t)kSpBucketBlock * kSpBucketEdges;
 constexpr int kSpBuildBlock = 512;
 constexpr size_t kSpBucketLdsMax = (size_t)kKsMaxS * 12;        // bands <= n <= kKsMaxS: u64 base + u32 count
 
+// E: the matrix's entry type (uint32_t when the trial's graph weighs less than
+// 2^31 in total, int64_t otherwise); A: its unsigned accumulator.
+template <typename E>
 struct SpDense {
+  typedef typename std::conditional<sizeof(E) == 4, uint32_t, unsigned long long>::type A;
   const cac_edge* edges;
   uint64_t m;
   uint32_t n, rows;              // rows per band
   uint32_t bands, pad;           // ceil(n / rows)
-  int64_t* mat;                  // n x n
-  int64_t* rsum;                 // [n]
+  E* mat;                        // n x n, row stride ks_stride<E>(n)
+  E* rsum;                       // [n]
   unsigned long long* boff;      // [bands + 1]: entry counts, then their exclusive prefix (zeroed first)
   unsigned long long* bcur;      // [bands]: placement cursors
-  unsigned long long* ew;        // [2m] entry weights, grouped by band
+  A* ew;                         // [2m] entry weights, grouped by band
   uint16_t* eli;                 // [2m] entry index inside its band: (row - band * rows) * n + column
 };
 
@@ -562,10 +567,11 @@ inline uint32_t band_rows(uint32_t n) { return n ? std::max(1u, std::min(n, kSpB
 // band v / rows.  Placing reserves each band's range of the tile with one
 // atomic on the band's cursor; the order inside a range is arbitrary, which
 // the integer sums do not see.  Dynamic LDS: bands x (8 + 4) bytes.
-template <bool kPlace>
-__global__ void __launch_bounds__(kSpBucketBlock) k_sp_band_bucket(const SpDense* __restrict__ nodes) {
+template <bool kPlace, typename E>
+__global__ void __launch_bounds__(kSpBucketBlock) k_sp_band_bucket(const SpDense<E>* __restrict__ nodes) {
+  typedef typename SpDense<E>::A A;
   extern __shared__ unsigned long long band_lds[];
-  const SpDense d = nodes[blockIdx.y];
+  const SpDense<E> d = nodes[blockIdx.y];
   const uint64_t e0 = (uint64_t)blockIdx.x * kSpBucketTile;
   if (e0 >= d.m) return;  // the same for the whole block
   unsigned long long* base = band_lds;                            // [bands] (place)
@@ -603,10 +609,10 @@ __global__ void __launch_bounds__(kSpBucketBlock) k_sp_band_bucket(const SpDense
     for (int j = 0; j < kSpBucketEdges; ++j) {
       if (e0 + (uint64_t)j * kSpBucketBlock + threadIdx.x >= d.m) continue;
       const uint64_t pu = base[bu[j]] + atomicAdd(&cnt[bu[j]], 1u);
-      d.ew[pu] = x[j].w;
+      d.ew[pu] = (A)x[j].w;
       d.eli[pu] = (uint16_t)((x[j].u - bu[j] * R) * d.n + x[j].v);
       const uint64_t pv = base[bv[j]] + atomicAdd(&cnt[bv[j]], 1u);
-      d.ew[pv] = x[j].w;
+      d.ew[pv] = (A)x[j].w;
       d.eli[pv] = (uint16_t)((x[j].v - bv[j] * R) * d.n + x[j].u);
     }
   }
@@ -614,9 +620,10 @@ __global__ void __launch_bounds__(kSpBucketBlock) k_sp_band_bucket(const SpDense
 
 // Exclusive prefix of the band counts, one workgroup per node: boff[b] becomes
 // the band's first entry, boff[bands] the total, and the cursors start there.
-__global__ void __launch_bounds__(1024) k_sp_band_scan(const SpDense* __restrict__ nodes) {
+template <typename E>
+__global__ void __launch_bounds__(1024) k_sp_band_scan(const SpDense<E>* __restrict__ nodes) {
   __shared__ unsigned long long wtot[16];
-  const SpDense d = nodes[blockIdx.x];
+  const SpDense<E> d = nodes[blockIdx.x];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned long long carry = 0;
   for (uint32_t b0 = 0; b0 < d.bands; b0 += 1024) {
@@ -643,10 +650,13 @@ __global__ void __launch_bounds__(1024) k_sp_band_scan(const SpDense* __restrict
 
 // Sums each band's entries in LDS, then writes the band's row sums and its
 // rows (every entry, zeros included) and clears the LDS it read.  Workgroups
-// stride over a node's bands.  Dynamic LDS: kSpBandEntries u64.
-__global__ void __launch_bounds__(kSpBuildBlock) k_sp_band_build(const SpDense* __restrict__ nodes) {
-  extern __shared__ unsigned long long band_acc[];
-  const SpDense d = nodes[blockIdx.y];
+// stride over a node's bands.  Dynamic LDS: kSpBandEntries entries.
+template <typename E>
+__global__ void __launch_bounds__(kSpBuildBlock) k_sp_band_build(const SpDense<E>* __restrict__ nodes) {
+  typedef typename SpDense<E>::A A;
+  extern __shared__ __align__(16) unsigned char band_build_lds[];
+  A* band_acc = (A*)band_build_lds;
+  const SpDense<E> d = nodes[blockIdx.y];
   const uint32_t n = d.n, R = d.rows;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (uint32_t i = threadIdx.x; i < R * n; i += kSpBuildBlock) band_acc[i] = 0;
@@ -655,18 +665,19 @@ __global__ void __launch_bounds__(kSpBuildBlock) k_sp_band_build(const SpDense* 
     const uint64_t i1 = d.boff[b + 1];
     for (uint64_t i = d.boff[b] + threadIdx.x; i < i1; i += kSpBuildBlock) atomicAdd(&band_acc[d.eli[i]], d.ew[i]);
     __syncthreads();
+    // one wave per row: its sum, the row itself, and the LDS cleared
     const uint32_t r0 = b * R, nr = min(R, n - r0);
     for (uint32_t r = wave; r < nr; r += kSpBuildBlock / 64) {
-      uint64_t acc = 0;
-      for (uint32_t c = lane; c < n; c += 64) acc += band_acc[r * n + c];
-      acc = wave_sum<uint64_t>(acc);
-      if (lane == 0) d.rsum[r0 + r] = (int64_t)acc;
-    }
-    __syncthreads();
-    int64_t* out = d.mat + (uint64_t)r0 * n;
-    for (uint32_t j = threadIdx.x; j < nr * n; j += kSpBuildBlock) {
-      out[j] = (int64_t)band_acc[j];
-      band_acc[j] = 0;
+      E* out = d.mat + (uint64_t)(r0 + r) * ks_stride<E>(n);
+      A acc = 0;
+      for (uint32_t c = lane; c < n; c += 64) {
+        const A v = band_acc[r * n + c];
+        band_acc[r * n + c] = 0;
+        out[c] = (E)v;
+        acc += v;
+      }
+      acc = (A)wave_sum<ks_sum_t<E>>((ks_sum_t<E>)acc);
+      if (lane == 0) d.rsum[r0 + r] = (E)acc;
     }
   }
 }
@@ -731,6 +742,7 @@ struct SpNode {
   uint32_t n, trial, nid, slot;
   int64_t bound;  // the trial's bound (minimum weighted degree of its root)
   uint32_t seed;  // Philox key word 0 of the trial
+  bool w32;       // dense nodes have 32-bit entries
 };
 
 // Device bytes of one child: what stays alive for the next depth (its edge
@@ -742,24 +754,27 @@ size_t child_tmp_bytes(const SpNode& nd) {
 }
 size_t dense_bytes(const SpNode& nd) {
   const uint32_t bands = (nd.n + band_rows(nd.n) - 1) / band_rows(nd.n);
-  return carve_size((size_t)nd.n * nd.n * 8) + carve_size((size_t)nd.n * 8) + sizeof(SpDense) +
-         ((size_t)bands + 1) * 8 + 256 + carve_size((size_t)bands * 8) + carve_size(nd.m * 16) + carve_size(nd.m * 4);
+  const size_t es = nd.w32 ? 4 : 8, st = nd.w32 ? ks_stride<uint32_t>(nd.n) : nd.n;
+  return carve_size((size_t)nd.n * st * es) + carve_size((size_t)nd.n * es) + sizeof(SpDense<int64_t>) +
+         ((size_t)bands + 1) * 8 + 256 + carve_size((size_t)bands * 8) + carve_size(nd.m * 2 * es) +
+         carve_size(nd.m * 4);
 }
 
 // The bucketing and band kernels' dynamic LDS may exceed the default limit:
 // raise it once.
+template <typename E>
 int band_attr(cac_ctx* ctx) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-    err = hipFuncSetAttribute((const void*)k_sp_band_bucket<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    err = hipFuncSetAttribute((const void*)k_sp_band_bucket<true, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kSpBucketLdsMax);
     if (err == hipSuccess)
-      err = hipFuncSetAttribute((const void*)k_sp_band_bucket<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      err = hipFuncSetAttribute((const void*)k_sp_band_bucket<false, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)kSpBucketLdsMax);
     if (err == hipSuccess)
-      err = hipFuncSetAttribute((const void*)k_sp_band_build, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(kSpBandEntries * 8));
+      err = hipFuncSetAttribute((const void*)k_sp_band_build<E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)(kSpBandEntries * sizeof(E)));
   });
   CAC_HIP(ctx, err);
   return CAC_OK;
@@ -775,6 +790,15 @@ struct SpRun {
   // Densifies nodes in batches that fit the free memory (matrices plus the
   // dense engine's level buffers) and runs the dense engine on them.
   int dense(const std::vector<SpNode>& nodes) {
+    std::vector<SpNode> kind[2];
+    for (const SpNode& nd : nodes) kind[nd.w32 ? 1 : 0].push_back(nd);
+    int rc = dense_typed<uint32_t>(kind[1]);
+    return rc ? rc : dense_typed<int64_t>(kind[0]);
+  }
+
+  template <typename E>
+  int dense_typed(const std::vector<SpNode>& nodes) {
+    typedef SpDense<E> Dense;
     size_t i0 = 0;
     while (i0 < nodes.size()) {
       size_t avail = 0;
@@ -785,7 +809,7 @@ struct SpRun {
       size_t i1 = i0, bytes = 256, mats = 256;
       uint32_t nmax = 0;
       while (i1 < nodes.size() && i1 - i0 < 4096) {
-        const size_t b = dense_bytes(nodes[i1]) + ks_live_bytes_per_root(nodes[i1].n);
+        const size_t b = dense_bytes(nodes[i1]) + ks_live_bytes_per_root(nodes[i1].n, sizeof(E) == 4);
         if (i1 > i0 && bytes + b > budget) break;
         bytes += b;
         mats += dense_bytes(nodes[i1]);
@@ -795,11 +819,11 @@ struct SpRun {
       const size_t count = i1 - i0;
       rc = grow_buffer(ctx, &ctx->sp_dense_buf, &ctx->sp_dense_bytes, mats);
       if (rc) return rc;
-      rc = band_attr(ctx);
+      rc = band_attr<E>(ctx);
       if (rc) return rc;
       BufPin pin(ctx, kBufSpDense);
       Carver cv(ctx->sp_dense_buf);
-      SpDense* d_nodes = cv.take<SpDense>(count);
+      Dense* d_nodes = cv.take<Dense>(count);
       uint64_t nboff = 0;
       uint32_t bmax = 0;
       for (size_t i = 0; i < count; ++i) {
@@ -810,43 +834,45 @@ struct SpRun {
         bmax = std::max(bmax, bands);
       }
       unsigned long long* d_boff = cv.take<unsigned long long>(nboff);
-      std::vector<SpDense> hd(count);
+      std::vector<Dense> hd(count);
       std::vector<KsRoot> roots;
       uint64_t mmax = 0, boff_at = 0;
       for (size_t i = 0; i < count; ++i) {
         const SpNode& nd = nodes[i0 + i];
         const uint32_t R = band_rows(nd.n), bands = (nd.n + R - 1) / R;
-        SpDense& d = hd[i];
+        Dense& d = hd[i];
         d.edges = nd.edges;
         d.m = nd.m;
         d.n = nd.n;
         d.rows = R;
         d.bands = bands;
         d.pad = 0;
-        d.mat = cv.take<int64_t>((size_t)nd.n * nd.n);
-        d.rsum = cv.take<int64_t>(nd.n);
+        d.mat = cv.take<E>((size_t)nd.n * ks_stride<E>(nd.n));
+        d.rsum = cv.take<E>(nd.n);
         d.boff = d_boff + boff_at;
         boff_at += bands + 1;
         d.bcur = cv.take<unsigned long long>(bands);
-        d.ew = cv.take<unsigned long long>(2 * nd.m);
+        d.ew = cv.take<typename Dense::A>(2 * nd.m);
         d.eli = cv.take<uint16_t>(2 * nd.m);
         KsRoot r{d.mat, d.rsum, nd.n, nd.trial, nd.slot, nd.bound, nd.seed};
         r.nid = nd.nid;
+        r.w32 = sizeof(E) == 4;
         roots.push_back(r);
         mmax = std::max(mmax, nd.m);
       }
-      CAC_HIP(ctx, hipMemcpyAsync(d_nodes, hd.data(), count * sizeof(SpDense), hipMemcpyHostToDevice, s));
+      CAC_HIP(ctx, hipMemcpyAsync(d_nodes, hd.data(), count * sizeof(Dense), hipMemcpyHostToDevice, s));
       const unsigned tiles = (unsigned)std::max<uint64_t>(1, (mmax + kSpBucketTile - 1) / kSpBucketTile);
       const unsigned gb = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(bmax, (2048 + count - 1) / count));
       prof_begin(ctx, "sparse_densify", s);
       hipLaunchKernelGGL(k_sp_fill, dim3(grid_for(nboff, 256, 1024)), dim3(256), 0, s, d_boff, nboff, 0ull);
-      hipLaunchKernelGGL(k_sp_band_bucket<false>, dim3(tiles, (unsigned)count), dim3(kSpBucketBlock),
-                         (size_t)bmax * 4, s, (const SpDense*)d_nodes);
-      hipLaunchKernelGGL(k_sp_band_scan, dim3((unsigned)count), dim3(1024), 0, s, (const SpDense*)d_nodes);
-      hipLaunchKernelGGL(k_sp_band_bucket<true>, dim3(tiles, (unsigned)count), dim3(kSpBucketBlock),
-                         (size_t)bmax * 12, s, (const SpDense*)d_nodes);
-      hipLaunchKernelGGL(k_sp_band_build, dim3(gb, (unsigned)count), dim3(kSpBuildBlock), (size_t)kSpBandEntries * 8,
-                         s, (const SpDense*)d_nodes);
+      const Dense* dn = d_nodes;
+      hipLaunchKernelGGL((k_sp_band_bucket<false, E>), dim3(tiles, (unsigned)count), dim3(kSpBucketBlock),
+                         (size_t)bmax * 4, s, dn);
+      hipLaunchKernelGGL(k_sp_band_scan<E>, dim3((unsigned)count), dim3(1024), 0, s, dn);
+      hipLaunchKernelGGL((k_sp_band_bucket<true, E>), dim3(tiles, (unsigned)count), dim3(kSpBucketBlock),
+                         (size_t)bmax * 12, s, dn);
+      hipLaunchKernelGGL(k_sp_band_build<E>, dim3(gb, (unsigned)count), dim3(kSpBuildBlock),
+                         (size_t)kSpBandEntries * sizeof(E), s, dn);
       prof_end(ctx, s);
       CAC_LAUNCH_CHECK(ctx, "sparse densify");
       rc = ks_run(ctx, roots, d_results, s);
@@ -930,7 +956,8 @@ struct SpRun {
       for (size_t i = 0; i < nchild; ++i) {
         if (mout[i] == kSpDisconnected) continue;  // its cut of 0 is already recorded
         next.push_back(
-            {ch[i].out, mout[i], ch[i].tgt, ch[i].trial, ch[i].nid, ch[i].slot, sp[i0 + i / 2].bound, ch[i].seed});
+            {ch[i].out, mout[i], ch[i].tgt, ch[i].trial, ch[i].nid, ch[i].slot, sp[i0 + i / 2].bound, ch[i].seed,
+             sp[i0 + i / 2].w32});
       }
       rc = level(next, depth + 1);
       if (rc) return rc;
@@ -961,7 +988,7 @@ int ks_sparse_roots(cac_ctx* ctx, const std::vector<SparseRoot>& roots, int64_t*
   const size_t depth = sparse_depth(nmax);
   SpRun run{ctx, d_results, s, (size_t)(0.4 * (double)avail) / (depth + 1), (size_t)(0.15 * (double)avail)};
   std::vector<SpNode> level;
-  for (const SparseRoot& r : roots) level.push_back({r.edges, r.m, r.n, r.trial, 1u, r.slot, r.bound, r.seed});
+  for (const SparseRoot& r : roots) level.push_back({r.edges, r.m, r.n, r.trial, 1u, r.slot, r.bound, r.seed, r.w32});
   rc = run.level(level, 0);
   if (rc) return rc;
   CAC_HIP(ctx, hipStreamSynchronize(s));
@@ -969,10 +996,11 @@ int ks_sparse_roots(cac_ctx* ctx, const std::vector<SparseRoot>& roots, int64_t*
 }
 
 int ks_sparse_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t seed,
-                  const std::vector<uint32_t>& trial_ids, int64_t bound, int64_t* d_results, hipStream_t s) {
+                  const std::vector<uint32_t>& trial_ids, int64_t bound, bool w32, int64_t* d_results,
+                  hipStream_t s) {
   std::vector<SparseRoot> roots;
   for (size_t i = 0; i < trial_ids.size(); ++i)
-    roots.push_back({d_edges, m, n, trial_ids[i], (uint32_t)i, bound, seed});
+    roots.push_back({d_edges, m, n, trial_ids[i], (uint32_t)i, bound, seed, w32});
   return ks_sparse_roots(ctx, roots, d_results, s);
 }
 
@@ -1027,7 +1055,8 @@ int cac_ks_sparse(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, u
                        (unsigned long long*)d_res, (uint64_t)ntrials, bound);
     std::vector<uint32_t> ids(ntrials);
     for (uint32_t i = 0; i < ntrials; ++i) ids[i] = first_trial + i;
-    rc = cac::ks_sparse_run(ctx, d_e, m, n, seed, ids, (int64_t)bound, d_res, s);
+    const bool w32 = ((unsigned __int128)wsum[0] << 20) + wsum[1] < ((unsigned __int128)1 << 31);
+    rc = cac::ks_sparse_run(ctx, d_e, m, n, seed, ids, (int64_t)bound, w32, d_res, s);
   }
   if (rc == CAC_OK) {
     std::vector<int64_t> res(ntrials);

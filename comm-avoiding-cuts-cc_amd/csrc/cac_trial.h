@@ -25,13 +25,20 @@ struct TrialScratch {
   uint32_t* par;          // [n]
   uint64_t* pre;          // [m]
   uint2* draws;           // [n]
-  int64_t* mat;           // [t x t]
-  int64_t* rsum;          // [t] row sums of mat (may be null)
+  void* mat;              // [t x t] entries of trial_w32's type, row stride ks_stride
+  void* rsum;             // [t] row sums of mat, same type (may be null)
   uint32_t* nv_out;       // [1]
   // [1] of the job's graph, nonzero when an edge is a loop or two weights
   // differ (may be null: then every round builds the prefix)
   const uint32_t* mixed;
+  // [1] total edge weight of the job's graph, saturating (null: entries are 64-bit)
+  const unsigned long long* total;
 };
+
+// The contracted matrix's entries add up to at most twice the graph's total
+// weight: below 2^32 the matrix and its row sums are uint32_t, else int64_t.
+constexpr unsigned long long kTrialW32Total = 1ull << 31;
+__device__ inline bool trial_w32(const TrialScratch& S) { return S.total && *S.total < kTrialW32Total; }
 
 // Device bytes of the per-trial state of the wide form beside TrialScratch's
 // buffers (tile totals and the round's control words).

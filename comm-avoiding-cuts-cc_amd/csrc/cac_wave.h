@@ -70,6 +70,15 @@ __device__ inline T wave_incl_scan(T x) {
   x += dpp_move<kDppBcast31, 0xc>(x, (T)0);
   return x;
 }
+// Inclusive prefix sum inside each row of 16 lanes.
+template <class T>
+__device__ inline T row_incl_scan(T x) {
+  x += dpp_move<kDppRowShr1, 0xf>(x, (T)0);
+  x += dpp_move<kDppRowShr2, 0xf>(x, (T)0);
+  x += dpp_move<kDppRowShr4, 0xf>(x, (T)0);
+  x += dpp_move<kDppRowShr8, 0xf>(x, (T)0);
+  return x;
+}
 // Wave total, returned to every lane.
 template <class T>
 __device__ inline T wave_sum(T x) {

@@ -42,6 +42,7 @@
 #include "cac_common.h"
 #include "cac_internal.h"
 #include "cac_ks.h"
+#include "cac_ks_kernels.h"
 #include "cac_wave.h"
 #include "cac_trial.h"
 
@@ -638,8 +639,10 @@ __global__ void __launch_bounds__(kWB) k_w_zero(const TrialScratch* __restrict__
   const TrialScratch& S = scr[blockIdx.y];
   const uint32_t k = st[blockIdx.y].nv;
   if (k > S.t) return;
-  const uint64_t cells = (uint64_t)k * k;
-  for (uint64_t i = (uint64_t)blockIdx.x * kWB + threadIdx.x; i < cells; i += (uint64_t)gridDim.x * kWB) S.mat[i] = 0;
+  // in 8-byte words, whichever entry type the trial has
+  const uint64_t words = trial_w32(S) ? (uint64_t)k * ks_stride<uint32_t>(k) / 2 : (uint64_t)k * k;
+  uint64_t* mat = (uint64_t*)S.mat;
+  for (uint64_t i = (uint64_t)blockIdx.x * kWB + threadIdx.x; i < words; i += (uint64_t)gridDim.x * kWB) mat[i] = 0;
 }
 
 // Grid (input tiles, trials): accumulate the surviving edges into the matrix.
@@ -652,6 +655,8 @@ __global__ void __launch_bounds__(kWB) k_w_accum(const TrialScratch* __restrict_
   const uint64_t count = w.scanned ? w.len : S.m;
   const uint64_t base = (uint64_t)blockIdx.x * kWTile;
   if (base >= count) return;
+  const bool w32 = trial_w32(S);
+  const uint64_t stride = w32 ? ks_stride<uint32_t>(k) : ks_stride<int64_t>(k);
 #pragma unroll 4
   for (int j = 0; j < kWItems; ++j) {
     const uint64_t i = base + (uint64_t)j * kWB + threadIdx.x;
@@ -660,8 +665,13 @@ __global__ void __launch_bounds__(kWB) k_w_accum(const TrialScratch* __restrict_
     const uint32_t la = S.lab[x.u], lb = S.lab[x.v];
     if (la == lb) continue;
     const uint32_t a = S.par[la], b = S.par[lb];
-    atomicAdd((unsigned long long*)&S.mat[(uint64_t)a * k + b], (unsigned long long)x.w);
-    atomicAdd((unsigned long long*)&S.mat[(uint64_t)b * k + a], (unsigned long long)x.w);
+    if (w32) {
+      atomicAdd((uint32_t*)S.mat + a * stride + b, (uint32_t)x.w);
+      atomicAdd((uint32_t*)S.mat + b * stride + a, (uint32_t)x.w);
+    } else {
+      atomicAdd((unsigned long long*)S.mat + a * stride + b, (unsigned long long)x.w);
+      atomicAdd((unsigned long long*)S.mat + b * stride + a, (unsigned long long)x.w);
+    }
   }
 }
 
@@ -673,11 +683,19 @@ __global__ void __launch_bounds__(kWB) k_w_rowsum(const TrialScratch* __restrict
   if (k > S.t) return;
   const uint32_t r = blockIdx.x * kWWaves + (threadIdx.x >> 6);
   if (r >= k) return;
+  const bool w32 = trial_w32(S);
   uint64_t acc = 0;
-  for (uint32_t x = threadIdx.x & 63; x < k; x += 64) acc += (uint64_t)S.mat[(uint64_t)r * k + x];
+  if (w32) {
+    const uint32_t* row = (const uint32_t*)S.mat + (uint64_t)r * ks_stride<uint32_t>(k);
+    for (uint32_t x = threadIdx.x & 63; x < k; x += 64) acc += row[x];
+  } else {
+    const uint64_t* row = (const uint64_t*)S.mat + (uint64_t)r * ks_stride<int64_t>(k);
+    for (uint32_t x = threadIdx.x & 63; x < k; x += 64) acc += row[x];
+  }
   acc = wave_sum64(acc);
   if ((threadIdx.x & 63) == 0) {
-    if (S.rsum) S.rsum[r] = (int64_t)acc;
+    if (S.rsum && w32) ((uint32_t*)S.rsum)[r] = (uint32_t)acc;
+    else if (S.rsum) ((int64_t*)S.rsum)[r] = (int64_t)acc;
     atomicMin((unsigned long long*)&w.bmin, (unsigned long long)acc);
   }
 }

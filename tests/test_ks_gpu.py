@@ -174,3 +174,23 @@ def test_ks_compaction_tune_rejects_bad_values():
         assert c.tune_get(cac.TUNE_KS_COMPACT_BLOCK, 8192) == 1024
         c.tune_set(cac.TUNE_KS_COMPACT_BLOCK, 8192, 0)
         assert c.tune_get(cac.TUNE_KS_COMPACT_BLOCK, 8192) == 0
+
+
+@pytest.mark.parametrize("total", [2**32 - 2, 2**32, 2**32 + 2])
+@pytest.mark.parametrize("n,k,deg_in", [(131, 33, 2.0), (515, 129, 2.0), (1501, 375, 2.0)])
+def test_ks_entry_width_boundary(ctx, orc, n, k, deg_in, total):
+    """Matrices whose entries sum to just below and to 2^32: the first runs with
+    32-bit entries, the others with 64-bit ones; the raw cuts are the oracle's
+    (exact integers: no tolerance).  Odd sizes leave partial 16-byte pieces."""
+    rng = np.random.default_rng(n)
+    A = dense(n, necklace(rng, n, k, 3 * 10**6, deg_in))
+    A = A * (2**32 - 2**20) // int(A.sum())
+    i, j = np.unravel_index(int(np.argmax(A)), A.shape)
+    A[i, j] += (total - int(A.sum())) // 2
+    A[j, i] = A[i, j]
+    assert int(A.sum()) == total and A[i, j] > 0
+    T = 6
+    _say(f"ks entry width n {n} total {total}")
+    want = [orc.ks_trial(A, 9, t) for t in range(T)]
+    raw, mn = ctx.ks_dense(A, 9, 0, T)
+    assert raw.tolist() == want and mn == min(want)
