@@ -11,9 +11,9 @@
 // Per level of the recursion tree:
 //   1. k_ks_contract<B>: one workgroup per child (B = 64, 256 or 1024 threads by
 //      size) draws s - t' picks, merges rows into pool rows, runs the PR pass and
-//      writes the column map and the live-row list;
-//   2. k_ks_compact: workgroups of a few output rows each sum live rows by column
-//      class into the child's t' x t' matrix, with row sums and row maxima;
+//      writes the lists of live rows, live columns and merged-away columns;
+//   2. k_ks_compact: teams of threads each fold a live row's merged-away columns
+//      into their representatives in LDS and write the child's row;
 //   3. children of at most 128 vertices are leaves: k_ks_cert settles most of them
 //      from row sums and maxima; k_ks_sw runs Stoer-Wagner on the rest.
 // Device memory for a level comes from two grow-only buffers of the context used
@@ -532,9 +532,9 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
     }
     return;
   }
-  // ranks of the live rows (natural order), live-row list, column map
+  // live rows and columns in natural order with the rows' sums (their
+  // capacities), and the merged-away columns with their representatives
   __syncthreads();
-  uint32_t* rank = (uint32_t*)L.cap;  // capacities are no longer needed
   uint32_t cnt = 0;
 #pragma unroll
   for (uint32_t k = 0; k < kKsChunk; ++k)
@@ -555,53 +555,71 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
 #pragma unroll
   for (uint32_t k = 0; k < kKsChunk; ++k) {
     const uint32_t x = lo + k;
-    if (k < cc && x < s && L.rep[x] == x) {
-      rank[x] = ex;
+    if (k >= cc || x >= s) break;
+    const uint32_t rx = L.rep[x];
+    if (rx == x) {
       const uint16_t sl = L.wslot[x];
       c.live[ex] = sl == kNoRow ? x : (kLiveWork | sl);
+      c.repcol[ex] = (uint16_t)x;
+      c.orsum[ex] = (E)L.cap[x];
       ++ex;
+    } else {
+      c.dead[x - ex] = x | (rx << 16);
     }
   }
-  __syncthreads();
-  for (uint32_t y = threadIdx.x; y < s; y += B) c.colmap[y] = (uint16_t)rank[L.rep[y]];
   if (threadIdx.x == 0) k_out[blockIdx.x] = total;
 }
 
-// Row entries per thread in flight in k_ks_compact.
-constexpr uint32_t kCompactUnroll = 8;
-
-// Threads per compaction workgroup for children of tgt output vertices: the
-// context's CAC_TUNE_KS_COMPACT_BLOCK setting for tgt's class, or 512 (on
-// MI355X 17% less compaction time than 256 on the n = 8192 complete graph,
-// and 1024 was slower than either).
-inline int compact_block(const cac_ctx* ctx, uint32_t tgt) {
+// Threads per compaction workgroup of a class of children whose longest parent
+// row takes row_bytes: the context's CAC_TUNE_KS_COMPACT_BLOCK setting for tgt's
+// class, or 256, and 512 for rows above 16 KiB.
+inline int compact_block(const cac_ctx* ctx, uint32_t tgt, size_t row_bytes) {
   const int cls = tgt <= 512 ? 0 : tgt <= 1024 ? 1 : tgt <= 2048 ? 2 : tgt <= 4096 ? 3 : 4;
   const int v = ctx->ks_compact_block[cls];
-  return v ? v : 512;
+  return v ? v : row_bytes <= 16384 ? 256 : 512;
 }
+// A wavefront takes a row of its own up to this size, the whole workgroup above.
+constexpr size_t kCompactWaveRow = 8192;
 
-// Rows per compaction workgroup for a child of t' output vertices (the LDS
-// accumulator holds rows x t' entries, at most 4096 unless t' alone is larger).
+// Output rows per compaction workgroup.
 __host__ __device__ inline uint32_t compact_rows(uint32_t tgt) {
-  const uint32_t r = 4096 / (tgt ? tgt : 1);
-  return r < 1 ? 1 : (r > 64 ? 64 : r);
+  const uint32_t r = 8192 / (tgt ? tgt : 1);
+  return r < 4 ? 4 : (r > 64 ? 64 : r);
 }
 
-// One workgroup per (child, group of output rows): sums every live row by column
-// class into LDS, then writes the rows with their sums and maxima.  The work
+// Team barrier: a team of one wavefront runs its LDS accesses in order, so only
+// the compiler has to keep them in order.
+template <int TEAM>
+__device__ inline void team_sync() {
+  if constexpr (TEAM == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// One workgroup per (child, group of output rows), its rows dealt to teams of
+// TEAM threads.  A team copies a live row to LDS with 16-byte loads, adds the
+// entries of the merged-away columns to their representatives' (the only
+// atomics), and writes the representatives' entries in column order.  The work
 // item's child comes from a binary search of the per-child item prefix
-// (item_prefix).  CB threads per workgroup: large children, whose rows go one per
-// workgroup, take more threads, so more of a row's loads are in flight per CU.
-// A class sum never exceeds its node's total, so the LDS accumulator has the
-// entry type.
-template <int CB, typename E>
+// (item_prefix).  The bound is the rows' HBM traffic plus the LDS passes; adding
+// every column into an accumulator by its class took s atomics per row instead
+// of s - k.  Row maxima are written for leaves only, which alone read them.
+template <int CB, int TEAM, typename E>
 __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild<E>* __restrict__ children,
                                                    const uint32_t* __restrict__ k_out,
-                                                   const uint32_t* __restrict__ item_prefix, uint32_t nchild) {
+                                                   const uint32_t* __restrict__ item_prefix, uint32_t nchild,
+                                                   uint32_t row_stride) {
   typedef typename std::conditional<sizeof(E) == 4, uint32_t, unsigned long long>::type AccT;
-  constexpr uint32_t U = kCompactUnroll;
-  extern __shared__ __align__(16) unsigned char acc_lds[];
-  AccT* acc = reinterpret_cast<AccT*>(acc_lds);
+  typedef typename KsPiece<E>::type piece_t;
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>;
+  extern __shared__ __align__(16) unsigned char row_lds[];
+  __shared__ U wave_top[CB / 64];
+  const uint32_t team = threadIdx.x / TEAM, t = threadIdx.x % TEAM;
+  AccT* row = reinterpret_cast<AccT*>(row_lds) + (size_t)team * row_stride;
   const uint32_t item = blockIdx.x;
   uint32_t lo = 0, hi = nchild;  // last child with item_prefix[child] <= item
   while (hi - lo > 1) {
@@ -615,61 +633,53 @@ __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild<E>* __restrict_
   const uint32_t R = compact_rows(c.tgt);
   const uint32_t r0 = (item - item_prefix[lo]) * R;
   if (r0 >= kk) return;
-  const uint32_t nr = min(R, kk - r0);
-  const uint32_t s = c.s, os = ks_stride<E>(kk);
-  for (uint32_t x = threadIdx.x; x < nr * os; x += CB) acc[x] = 0;
-  __syncthreads();
-  // Rows and the column map are global memory (the struct's pointers are
-  // generic, which would give flat loads); kCompactUnroll entries per thread
-  // are loaded before any is added, so a wavefront keeps several loads in
-  // flight instead of one.  Neighbouring lanes take neighbouring columns: a
-  // lane's columns side by side (16-byte loads) put the lanes' LDS additions
-  // four entries apart, on a quarter of the banks.
+  const uint32_t r1 = min(r0 + R, kk);
+  const uint32_t s = c.s, os = ks_stride<E>(kk), nd = s - kk;
+  // Rows and lists are global memory (the struct's pointers are generic, which
+  // would give flat loads).
+  typedef const __attribute__((address_space(1))) piece_t g_piece;
   typedef const __attribute__((address_space(1))) E g_e;
   typedef const __attribute__((address_space(1))) uint16_t g_u16;
-  g_u16* cm = (g_u16*)c.colmap;
-  for (uint32_t rr = 0; rr < nr; ++rr) {
-    const uint32_t e = c.live[r0 + rr];
+  typedef const __attribute__((address_space(1))) uint32_t g_u32;
+  g_u16* repcol = (g_u16*)c.repcol;
+  g_u32* dead = (g_u32*)c.dead;
+  for (uint32_t r = r0 + team; r < r1; r += CB / TEAM) {
+    const uint32_t e = c.live[r];
     g_e* src = (g_e*)((e & kLiveWork) ? c.pool + (size_t)(e & ~kLiveWork) * ks_pool_stride(s)
                                       : c.parent + (size_t)e * c.ps);
-    AccT* a = acc + (size_t)rr * os;
-    uint32_t y = threadIdx.x;
-    for (; y + (U - 1) * CB < s; y += U * CB) {
-      E v[U];
-      uint32_t m[U];
-#pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        v[u] = src[y + u * CB];
-        m[u] = cm[y + u * CB];
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < U; ++u)
-        if (v[u]) atomicAdd(&a[m[u]], (AccT)v[u]);
+#pragma unroll 4
+    for (uint32_t x = t * V; x + V <= s; x += TEAM * V) *(piece_t*)(row + x) = *(g_piece*)(src + x);
+    for (uint32_t x = s / V * V + t; x < s; x += TEAM) row[x] = (AccT)src[x];
+    team_sync<TEAM>();
+#pragma unroll 4
+    for (uint32_t i = t; i < nd; i += TEAM) {
+      const uint32_t d = dead[i];
+      const AccT v = row[d & 0xFFFFu];
+      if (v) atomicAdd(&row[d >> 16], v);
     }
-    for (; y < s; y += CB) {
-      const E v = src[y];
-      if (v) atomicAdd(&a[cm[y]], (AccT)v);
-    }
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (uint32_t rr = wave; rr < nr; rr += CB / 64) {
-    const uint32_t r = r0 + rr;
+    team_sync<TEAM>();
     E* dst = c.out + (size_t)r * os;
-    ks_sum_t<E> sm = 0, mx = 0;
-    for (uint32_t x = lane; x < kk; x += 64) {
-      const ks_sum_t<E> v = (ks_sum_t<E>)acc[(size_t)rr * os + x];
+    U mx = 0;
+#pragma unroll 4
+    for (uint32_t x = t; x < kk; x += TEAM) {
+      const U v = (U)row[repcol[x]];
       dst[x] = (E)v;
-      sm += v;
       mx = v > mx ? v : mx;
     }
-    // entries are non-negative, so the unsigned maximum is the maximum
-    sm = wave_sum<ks_sum_t<E>>(sm);
-    mx = wave_max<ks_sum_t<E>>(mx);
-    if (lane == 0) {
-      c.orsum[r] = (E)sm;
-      c.ormax[r] = (E)mx;
+    if (kk <= kKsBase) {  // entries are non-negative, so the unsigned maximum is the maximum
+      mx = wave_max<U>(mx);
+      if (TEAM == 64) {
+        if (t == 0) c.ormax[r] = (E)mx;
+      } else {
+        if ((t & 63) == 0) wave_top[t >> 6] = mx;
+        __syncthreads();
+        if (t == 0) {
+          for (int w = 1; w < TEAM / 64; ++w) mx = wave_top[w] > mx ? wave_top[w] : mx;
+          c.ormax[r] = (E)mx;
+        }
+      }
     }
+    team_sync<TEAM>();
   }
 }
 
@@ -762,10 +772,11 @@ int ks_reserve(cac_ctx* ctx, int which, size_t bytes, void** out) {
   return rc;
 }
 
-// Device bytes of the per-child arrays of one child (out, sums, maxima, map, list).
+// Device bytes of the per-child arrays of one child (out, sums, maxima, lists).
 size_t child_bytes(uint32_t s, uint32_t t, size_t esize) {
   const size_t stride = esize == 4 ? ks_stride<uint32_t>(t) : ks_stride<int64_t>(t);
-  return c64(stride * t * esize) + 2 * c64((size_t)t * esize) + c64(((size_t)s + 8) * 2) + c64((size_t)t * 4);
+  return c64(stride * t * esize) + 2 * c64((size_t)t * esize) + c64((size_t)t * 4) + c64((size_t)t * 2) +
+         c64((size_t)s * 4);
 }
 // Pool rows of a child in the first pass: one for every pick and 1/8 spare (at
 // least 8) for the PR pass.  A child that needs more comes back as kKsOverflow.
@@ -823,11 +834,11 @@ void launch_contract(const KsChild<E>* d_children, uint32_t count, uint32_t smax
 // (the next level's work follows it there).
 template <typename E>
 int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* d_children, uint32_t* d_prefix,
-                   uint32_t* d_kout, uint32_t max_tgt, int64_t* d_results, std::vector<uint32_t>& kout,
-                   hipStream_t s) {
+                   uint32_t* d_kout, int64_t* d_results, std::vector<uint32_t>& kout, hipStream_t s) {
   const size_t nchild = ch.size();
   CAC_HIP(ctx, hipMemcpyAsync(d_children, ch.data(), nchild * sizeof(KsChild<E>), hipMemcpyHostToDevice, s));
   prof_begin(ctx, "ks_contract", s);
+  std::vector<size_t> group;  // first child of each block-size class, then nchild
   size_t c0 = 0;
   while (c0 < nchild) {
     int B = contract_block(ctx, ch[c0].s);
@@ -835,6 +846,7 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
     uint32_t smax = 0;
     while (c1 < nchild && contract_block(ctx, ch[c1].s) == B) smax = std::max(smax, ch[c1++].s);
     const uint32_t cnt = (uint32_t)(c1 - c0);
+    group.push_back(c0);
     // Fewer children than CUs (the top levels of a small solve): the device is
     // idle but for these workgroups, and with 64-bit entries a wider block
     // shortens each pick's row scans (ER(1000, 0.05) square_root: contraction
@@ -850,33 +862,55 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
     else launch_contract<64, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
     c0 = c1;
   }
+  group.push_back(nchild);
   prof_end(ctx, s);
   CAC_LAUNCH_CHECK(ctx, "ks contract");
   CAC_HIP(ctx, hipMemcpyAsync(kout.data(), d_kout, nchild * 4, hipMemcpyDeviceToHost, s));
   CAC_HIP(ctx, hipStreamSynchronize(s));
   // compaction work items: ceil(k / rows) per child of 1 <= k <= t' (0 for a
-  // disconnected child and for the error codes)
+  // disconnected child and for the error codes); one launch per block-size
+  // class, so that a class of small children does not take the large ones' LDS
   std::vector<uint32_t>& item_prefix = ctx->ks_items;  // rewritten only after the next synchronisation
-  item_prefix.assign(nchild + 1, 0u);
-  uint32_t items = 0;
-  for (size_t i = 0; i < nchild; ++i) {
-    item_prefix[i] = items;
-    const uint32_t k = kout[i];
-    if (k >= 1 && k <= ch[i].tgt) items += (k + compact_rows(ch[i].tgt) - 1) / compact_rows(ch[i].tgt);
+  item_prefix.clear();
+  std::vector<uint32_t> items(group.size() - 1);
+  for (size_t g = 0; g + 1 < group.size(); ++g) {
+    uint32_t n = 0;
+    for (size_t i = group[g]; i < group[g + 1]; ++i) {
+      item_prefix.push_back(n);
+      const uint32_t k = kout[i];
+      if (k >= 1 && k <= ch[i].tgt) n += (k + compact_rows(ch[i].tgt) - 1) / compact_rows(ch[i].tgt);
+    }
+    items[g] = n;
   }
-  item_prefix[nchild] = items;
-  if (items == 0) return CAC_OK;
-  CAC_HIP(ctx, hipMemcpyAsync(d_prefix, item_prefix.data(), (nchild + 1) * 4, hipMemcpyHostToDevice, s));
+  CAC_HIP(ctx, hipMemcpyAsync(d_prefix, item_prefix.data(), nchild * 4, hipMemcpyHostToDevice, s));
   prof_begin(ctx, "ks_compact", s);
-  const size_t lds = std::max<size_t>(4096 + 4 * 64, ks_stride<E>(max_tgt)) * sizeof(E);  // rows padded to whole pieces
-  const int cb = compact_block(ctx, max_tgt);
-  const KsChild<E>* dc = d_children;
-  const uint32_t* dk = d_kout;
-  const uint32_t* dp = d_prefix;
-  const uint32_t nc = (uint32_t)nchild;
-  if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, E>), dim3(items), dim3(1024), lds, s, dc, dk, dp, nc);
-  else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, E>), dim3(items), dim3(512), lds, s, dc, dk, dp, nc);
-  else hipLaunchKernelGGL((k_ks_compact<256, E>), dim3(items), dim3(256), lds, s, dc, dk, dp, nc);
+  for (size_t g = 0; g + 1 < group.size(); ++g) {
+    if (items[g] == 0) continue;
+    uint32_t smax = 0, tmax = 0;
+    for (size_t i = group[g]; i < group[g + 1]; ++i) {
+      smax = std::max(smax, ch[i].s);
+      tmax = std::max(tmax, ch[i].tgt);
+    }
+    const uint32_t stride = (smax + 15) & ~15u;
+    const size_t row_bytes = stride * sizeof(E);
+    const bool waves = row_bytes <= kCompactWaveRow;
+    const int cb = compact_block(ctx, tmax, row_bytes);
+    const size_t lds = (waves ? cb / 64 : 1) * row_bytes;
+    const KsChild<E>* dc = d_children + group[g];
+    const uint32_t* dk = d_kout + group[g];
+    const uint32_t* dp = d_prefix + group[g];
+    const uint32_t nc = (uint32_t)(group[g + 1] - group[g]);
+    const dim3 grid(items[g]), block((unsigned)cb);
+    if (waves) {
+      if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+      else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+      else hipLaunchKernelGGL((k_ks_compact<256, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+    } else {
+      if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, 1024, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+      else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, 512, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+      else hipLaunchKernelGGL((k_ks_compact<256, 256, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
+    }
+  }
   prof_end(ctx, s);
   CAC_LAUNCH_CHECK(ctx, "ks compact");
   return CAC_OK;
@@ -903,7 +937,8 @@ size_t ks_live_bytes_per_root(uint32_t n, bool w32) {
 
 namespace {
 
-// The contraction's dynamic LDS may exceed the default limit: raise it once.
+// The contraction's and the compaction's dynamic LDS may exceed the default
+// limit: raise it once.
 template <typename E>
 int contract_attr(cac_ctx* ctx) {
   static std::once_flag once;
@@ -914,6 +949,12 @@ int contract_attr(cac_ctx* ctx) {
     if (err == hipSuccess)
       err = hipFuncSetAttribute((const void*)k_ks_contract<512, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)contract_lds_bytes<E>(512 * kKsChunk, 512));
+    const void* compact[] = {(const void*)k_ks_compact<1024, 64, E>, (const void*)k_ks_compact<1024, 1024, E>,
+                             (const void*)k_ks_compact<512, 512, E>, (const void*)k_ks_compact<256, 256, E>};
+    for (const void* f : compact)
+      if (err == hipSuccess)
+        err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)std::max<size_t>(16 * kCompactWaveRow, kKsMaxS * sizeof(E)));
   });
   CAC_HIP(ctx, err);
   return CAC_OK;
@@ -963,12 +1004,10 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
     std::stable_sort(order.begin(), order.end());
     const size_t nchild = 2 * internal.size();
     size_t arrays = 0;
-    uint32_t max_tgt = 0;
     for (auto& nd : internal) {
       const uint32_t t = ks_target(nd.s);
       arrays += 2 * (child_bytes(nd.s, t, sizeof(E)) +
                      c64((size_t)child_pool_rows(nd.s, t) * ks_pool_stride(nd.s) * sizeof(E)));
-      max_tgt = std::max(max_tgt, t);
     }
     std::vector<Child> ch(nchild);
     std::vector<uint32_t> kout(nchild);
@@ -991,8 +1030,9 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
         x.out = cv.take<E>((size_t)t * ks_stride<E>(t));
         x.orsum = cv.take<E>(t);
         x.ormax = cv.take<E>(t);
-        x.colmap = cv.take<uint16_t>((size_t)nd.s + 8);
         x.live = cv.take<uint32_t>(t);
+        x.repcol = cv.take<uint16_t>(t);
+        x.dead = cv.take<uint32_t>(nd.s);
         x.pool_rows = child_pool_rows(nd.s, t);
         x.pool = cv.take<E>((size_t)x.pool_rows * ks_pool_stride(nd.s));
         x.s = nd.s;
@@ -1005,7 +1045,7 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
         x.bound = nd.bound;
       }
     }
-    rc = contract_level<E>(ctx, ch, d_children, d_prefix, d_kout, max_tgt, d_results, kout, s);
+    rc = contract_level<E>(ctx, ch, d_children, d_prefix, d_kout, d_results, kout, s);
     if (rc) return rc;
     // children that ran out of pool rows: again, with s pool rows each (a child
     // merges at most s - 2 times, so this cannot overflow)
@@ -1032,7 +1072,7 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
         x.pool = rv.take<E>((size_t)x.s * ks_pool_stride(x.s));
       }
       std::vector<uint32_t> rkout(no);
-      rc = contract_level<E>(ctx, rch, d_rch, d_rprefix, d_rkout, max_tgt, d_results, rkout, s);
+      rc = contract_level<E>(ctx, rch, d_rch, d_rprefix, d_rkout, d_results, rkout, s);
       if (rc) return rc;
       for (size_t k = 0; k < no; ++k) {
         if (rkout[k] == kKsOverflow) return fail(ctx, CAC_EDEVICE, "Karger-Stein row pool overflow");

@@ -17,9 +17,9 @@
 //     its place while it is live, or when the child ends, and a thread only ever
 //     reads back what it wrote itself;
 //   - a PR pass (co_mincut.h:50-63) may follow; the kernel ends by writing the
-//     column map and the list of live rows, and a separate many-workgroup kernel
-//     compacts the live rows into the child's t x t matrix with its row sums and
-//     row maxima.
+//     lists of live rows and columns and of merged-away columns, and the live
+//     rows' sums (their capacities), and a separate many-workgroup kernel compacts
+//     the live rows into the child's t x t matrix.
 // Entry type E: uint32_t when the root matrix's entries sum to less than 2^32 (no
 // entry, row sum or merged entry of the recursion can then exceed it), int64_t
 // otherwise.  The draws, the picks and the cuts are the same numbers either way.
@@ -78,8 +78,9 @@ struct KsChild {
   E* orsum;          // [tgt] row sums of out
   E* ormax;          // [tgt] row maxima of out
   E* pool;           // pool_rows merged rows of ks_pool_stride(s) entries
-  uint16_t* colmap;  // [s] column -> output index
   uint32_t* live;    // [tgt] output row -> parent row, or kLiveWork | pool row
+  uint16_t* repcol;  // [tgt] output column -> parent column that represents it
+  uint32_t* dead;    // [s - k] merged-away columns: column | representative << 16
   uint32_t s, ps, tgt, trial, nid;
   uint32_t slot, seed;  // seed: Philox key word 0 of the child's trial
   uint32_t pool_rows;

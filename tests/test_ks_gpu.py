@@ -194,3 +194,26 @@ def test_ks_entry_width_boundary(ctx, orc, n, k, deg_in, total):
     want = [orc.ks_trial(A, 9, t) for t in range(T)]
     raw, mn = ctx.ks_dense(A, 9, 0, T)
     assert raw.tolist() == want and mn == min(want)
+
+
+@pytest.mark.parametrize("block", [0, 256, 1024])
+@pytest.mark.parametrize("n,k", [(1024, 256), (1025, 256), (2048, 400), (2049, 400), (4097, 500), (8192, 700)])
+def test_ks_scaled_weights_same_picks(orc, n, k, block):
+    """All weights times 2^20: every draw falls on the same entry, so the raw cuts
+    are exactly 2^20 times as large.  The one run has 32-bit entries, the other
+    64-bit ones, with a wavefront or a whole workgroup per compacted row on
+    either side of the sizes where that changes."""
+    import cac
+
+    rng = np.random.default_rng(n)
+    A = dense(n, necklace(rng, n, k, 3 * 10**6, 2.0)) // 32
+    assert 0 < int(A.sum()) < 2**32
+    _say(f"ks scaled weights n {n} block {block}")
+    with cac.Context(0, tuning=False) as c:
+        for key in cac.TUNE_KS_COMPACT_KEYS:
+            c.tune_set(cac.TUNE_KS_COMPACT_BLOCK, key, block)
+        raw, _ = c.ks_dense(A, 3, 0, 3)
+        heavy, _ = c.ks_dense(A * 2**20, 3, 0, 3)
+    assert heavy.tolist() == [int(x) * 2**20 for x in raw]
+    if block == 0 and n <= 2049:
+        assert raw.tolist() == [orc.ks_trial(A, 3, t) for t in range(3)]
