@@ -27,6 +27,7 @@
 // Steps 2-5 run when m is large; small inputs go straight to a plain hook.
 // Any edge order is correct; the run sampling pays off when equal u are
 // adjacent (the order of the edge-list files and of the R-MAT generator).
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 
@@ -651,21 +652,112 @@ __device__ inline uint64_t keep_threshold(uint32_t i, uint64_t w) {
   return acc;
 }
 
-// Edge e is kept in copy j at level i iff lo64(Philox(i, j, e)) >= threshold;
-// kept edges are hooked into copy j's slice [j n, (j + 1) n) of the forest.
-__global__ void __launch_bounds__(kCcBlock) k_approx_hook(const cac_edge* __restrict__ edges, uint64_t m, uint32_t n,
-                                                          uint32_t copies, uint32_t level, uint32_t seed,
-                                                          uint32_t* par) {
-  for (uint64_t e = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x; e < m; e += (uint64_t)gridDim.x * kCcBlock) {
+// Order in which the approximate cut's unions hook roots: only the number of
+// trees is read, so any strict order of the ids serves, and a scrambled one (an
+// odd multiplier permutes u32) keeps the trees shallow where the id order would
+// hook a ring lattice's edges (v, v + 1) into one long path.
+__device__ inline uint32_t ap_rank(uint32_t x) { return x * 0x9E3779B1u; }
+
+// Root of x (par[r] == r) with path splitting.
+__device__ inline uint32_t ap_find(uint32_t* par, uint32_t x) {
+  uint32_t p = ld_par(par, x);
+  while (p != x) {
+    const uint32_t g = ld_par(par, p);
+    if (g != p) st_par(par, x, g);
+    x = p;
+    p = g;
+  }
+  return x;
+}
+
+// Union by ap_rank; 1 when this call hooked a root.
+__device__ inline uint32_t ap_link(uint32_t* par, uint32_t a, uint32_t b) {
+  uint32_t ra = ap_find(par, a), rb = ap_find(par, b);
+  while (ra != rb) {
+    const bool less = ap_rank(ra) < ap_rank(rb);
+    const uint32_t lo = less ? ra : rb, hi = less ? rb : ra;
+    const uint32_t old = atomicCAS(par + hi, hi, lo);
+    if (old == hi) return 1u;
+    ra = ap_find(par, old);
+    rb = ap_find(par, lo);
+  }
+  return 0u;
+}
+
+// The approximate cut's levels run kApLevels at a time (grid y), each level over
+// its own forest of copies n vertices.  Edge e is kept in copy j at level i iff
+// lo64(Philox(i, j, e)) >= threshold; kept edges are hooked into copy j's slice.
+// The components of a level are n copies - hooks.
+//
+// The edges are linked in three passes, the forest pointer-jumped in between:
+// one edge of every group of g (about one per vertex), the next three, the rest.
+// Linking them all at once is bound by contention: there are m / n times as many
+// links as vertices, all of them see roots that another XCD has hooked since
+// (its L2 is not coherent with theirs), and every such link is a chain of failing
+// CASes (Watts-Strogatz n = 32000, m = 512000, 5 copies: 1.8 ms a level).  After
+// the first two passes nearly every edge's ends have the same parent and cost
+// two loads.
+constexpr uint32_t kApLevels = 4;
+constexpr uint32_t kApSlots = 16;  // hook counters per level, 64 bytes apart
+constexpr uint32_t kApSlotWords = kApSlots * kHookStride;
+
+__global__ void __launch_bounds__(kCcBlock) k_approx_link(const cac_edge* __restrict__ edges, uint64_t m, uint32_t n,
+                                                          uint32_t copies, uint32_t level0, uint32_t seed,
+                                                          uint32_t g, uint32_t off0, uint32_t off1, uint32_t* par_all,
+                                                          uint32_t* slots) {
+  const uint32_t level = level0 + blockIdx.y;
+  uint32_t* par = par_all + (uint64_t)blockIdx.y * n * copies;
+  const uint32_t per = off1 - off0;
+  const uint64_t total = (m + g - 1) / g * per;
+  uint32_t hooks = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x; i < total; i += (uint64_t)gridDim.x * kCcBlock) {
+    const uint64_t group = i / per;  // the pass's edges of a group start at a scrambled place in it
+    const uint32_t off = off0 + (uint32_t)(i - group * per) + ((uint32_t)group * 0x9E3779B1u >> 16);
+    const uint64_t e = group * g + (off & (g - 1));
+    if (e >= m) continue;
     const cac_edge x = edges[e];
     if (x.w == 0 || x.u == x.v) continue;
-    const uint64_t q = keep_threshold(level, x.w);
+    uint64_t q = 0;
+    bool have_q = false;
     for (uint32_t j = 0; j < copies; ++j) {
+      const uint32_t a = x.u + j * n, b = x.v + j * n;
+      if (ld_par(par, a) == ld_par(par, b)) continue;  // joined already
+      if (!have_q) {
+        q = keep_threshold(level, x.w);
+        have_q = true;
+      }
       const u32x4 r = philox4x32(level, j, (uint32_t)e, (uint32_t)(e >> 32), seed, kDomApprox);
       if (lo64(r) < q) continue;
-      uf_link(par, x.u + j * n, x.v + j * n);
+      hooks += ap_link(par, a, b);
     }
   }
+  for (int d = 32; d > 0; d >>= 1) hooks += __shfl_down(hooks, d, 64);
+  const uint32_t wave = blockIdx.x * (kCcBlock / 64) + (threadIdx.x >> 6);
+  if ((threadIdx.x & 63) == 0 && hooks)
+    atomicAdd(slots + blockIdx.y * kApSlotWords + (wave % kApSlots) * kHookStride, hooks);
+}
+
+// Every vertex re-pointed at its root (grid-stride over all levels' forests; the
+// parents of a level's slice are indices into that slice).
+__global__ void __launch_bounds__(kCcBlock) k_approx_settle(uint32_t* par_all, uint32_t N) {
+  uint32_t* par = par_all + (uint64_t)blockIdx.y * N;
+  for (uint64_t i = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x; i < N; i += (uint64_t)gridDim.x * kCcBlock) {
+    const uint32_t p = ld_par_fresh(par, (uint32_t)i);
+    uint32_t r = p, up = ld_par_fresh(par, r);
+    while (up != r) {
+      r = up;
+      up = ld_par_fresh(par, r);
+    }
+    if (r != p) st_par(par, (uint32_t)i, r);
+  }
+}
+
+__global__ void __launch_bounds__(kCcBlock) k_approx_init(uint32_t* par_all, uint32_t N, uint32_t* slots) {
+  uint32_t* par = par_all + (uint64_t)blockIdx.y * N;
+  for (uint64_t i = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x; i < N; i += (uint64_t)gridDim.x * kCcBlock)
+    par[i] = (uint32_t)i;
+  if (blockIdx.x == 0)
+    for (uint32_t k = threadIdx.x; k < kApSlotWords; k += kCcBlock) slots[blockIdx.y * kApSlotWords + k] = 0;
 }
 
 }  // namespace
@@ -1149,28 +1241,44 @@ int approx_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n
                    uint32_t seed, uint32_t* first_disconnected, hipStream_t s) {
   const uint64_t N = (uint64_t)n * copies;
   if (N >= 0xFFFFFFFFull) return fail(ctx, CAC_EINVAL, "n * trials must fit in 32-bit vertex ids");
+  static_assert(kApLevels * kApSlotWords * 4 <= 4096, "the hook counters fit the context's pinned buffer");
+  // levels side by side while their forests stay small
+  const uint32_t batch = N * 4 * kApLevels <= (1ull << 30) ? kApLevels : 1u;
   void* base = nullptr;
-  int rc = scratch_reserve(ctx, carve_size(N * 4) + 512, &base);
+  int rc = scratch_reserve(ctx, carve_size(N * 4 * batch) + carve_size(kApLevels * kApSlotWords * 4) + 512, &base);
   if (rc) return rc;
   Carver cv(base);
-  uint32_t* par = cv.take<uint32_t>(N);
-  uint32_t* counter = cv.take<uint32_t>(64);
+  uint32_t* par = cv.take<uint32_t>(N * batch);
+  uint32_t* slots = cv.take<uint32_t>(kApLevels * kApSlotWords);
+  // groups of about m / n edges, a power of two
+  uint32_t g = 1;
+  while (g < 64 && (uint64_t)n * 2 * g <= m) g *= 2;
   *first_disconnected = 0;
-  for (uint32_t i = 1; i <= iters; ++i) {
-    hipLaunchKernelGGL(k_cc_init, dim3(grid_for(N, kCcBlock, 256 * 64)), dim3(kCcBlock), 0, s, par, (uint32_t)N);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, counter, 1);
+  for (uint32_t i0 = 1; i0 <= iters; i0 += batch) {
+    const uint32_t levels = std::min(batch, iters - i0 + 1);
+    const dim3 block(kCcBlock), vgrid(grid_for(N, kCcBlock, 4096), levels);
+    hipLaunchKernelGGL(k_approx_init, vgrid, block, 0, s, par, (uint32_t)N, slots);
     prof_begin(ctx, "approx_hook", s);
-    hipLaunchKernelGGL(k_approx_hook, dim3(grid_for(m, kCcBlock, 256 * 32)), dim3(kCcBlock), 0, s, d_edges, m, n,
-                       copies, i, seed, par);
+    for (uint32_t off0 = 0; off0 < g;) {
+      const uint32_t off1 = off0 == 0 ? 1 : off0 == 1 ? std::min(g, 4u) : g;
+      const dim3 egrid(grid_for((m + g - 1) / g * (off1 - off0), kCcBlock, 256 * 32), levels);
+      hipLaunchKernelGGL(k_approx_link, egrid, block, 0, s, d_edges, m, n, copies, i0, seed, g, off0, off1, par,
+                         slots);
+      if (off1 < g) hipLaunchKernelGGL(k_approx_settle, vgrid, block, 0, s, par, (uint32_t)N);
+      off0 = off1;
+    }
     prof_end(ctx, s);
-    hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(N, kCcBlock, 4096)), dim3(kCcBlock), 0, s, par, (uint32_t)N,
-                       counter);
     CAC_LAUNCH_CHECK(ctx, "approx kernels");
-    CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, counter, 4, hipMemcpyDeviceToHost, s));
+    CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, slots, levels * kApSlotWords * 4, hipMemcpyDeviceToHost, s));
     CAC_HIP(ctx, hipStreamSynchronize(s));
-    if (*(uint32_t*)ctx->pinned > copies) {
-      *first_disconnected = i;
-      break;
+    for (uint32_t l = 0; l < levels; ++l) {
+      uint64_t hooks = 0;
+      for (uint32_t k = 0; k < kApSlots; ++k)
+        hooks += ((const uint32_t*)ctx->pinned)[l * kApSlotWords + k * kHookStride];
+      if (N - hooks > copies) {
+        *first_disconnected = i0 + l;
+        return CAC_OK;
+      }
     }
   }
   return CAC_OK;
