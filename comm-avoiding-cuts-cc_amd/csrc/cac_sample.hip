@@ -26,6 +26,7 @@
 #include <mutex>
 #include <type_traits>
 #include <unordered_map>
+#include <unordered_set>
 #include <vector>
 
 #include <cstring>
@@ -47,13 +48,23 @@ constexpr int kSmpBlock = 1024;
 constexpr int kSmpWaves = kSmpBlock / 64;
 constexpr int kSmpIndex = 4096;  // LDS segment index of the weight prefix (32 KiB)
 
-// A distinct graph of a sampling launch, its flag word and its total weight.
+// A distinct graph of a sampling launch: its flag word and total weight, and for
+// trials in 32-bit arithmetic its packed form (pk null: not packed).
 struct EdgeSpan {
   const cac_edge* edges;
   uint64_t m;
   uint32_t* mixed;
   unsigned long long* total;
+  uint32_t* pk;
+  uint32_t* pre0;
+  uint32_t* tiles;  // per tile: weight sum, then the sum of the tiles before it
 };
+constexpr int kPackItems = 16;
+constexpr uint64_t kPackTile = 256 * kPackItems;
+constexpr uint64_t kPackMaxN = 65536, kPackMaxM = 1ull << 30;
+inline size_t packed_bytes(uint64_t m) {
+  return 2 * carve_size((size_t)m * 4) + carve_size((size_t)((m + kPackTile - 1) / kPackTile) * 4);
+}
 
 __global__ void k_mixed_zero(const EdgeSpan* spans, uint32_t count) {
   for (uint32_t g = blockIdx.x * 256 + threadIdx.x; g < count; g += gridDim.x * 256) {
@@ -65,26 +76,104 @@ __global__ void k_mixed_zero(const EdgeSpan* spans, uint32_t count) {
 // Grid (slices, graphs): flags graph blockIdx.y when one of its edges is a loop
 // or weighs other than its first edge (or the first weighs 0), and adds up its
 // weights, each cut to 2^31 (fewer than 2^32 edges cannot wrap the sum, and a
-// cut weight puts it past kTrialW32Total).
+// cut weight puts it past kTrialW32Total).  Packs the endpoints and sums every
+// tile's weights (loops 0; 32 bits, exact when the total allows 32-bit trials).
 __global__ void __launch_bounds__(256) k_mixed_weights(const EdgeSpan* spans) {
+  __shared__ uint64_t part[4];
+  __shared__ uint32_t tsum[4];
   const EdgeSpan sp = spans[blockIdx.y];
   if (sp.m == 0) return;
   const uint64_t w0 = sp.edges[0].w;
   bool bad = w0 == 0;
   uint64_t sum = 0;
-  for (uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x; e < sp.m; e += (uint64_t)gridDim.x * 256) {
-    const cac_edge x = sp.edges[e];
-    bad = bad || x.w != w0 || x.u == x.v;
-    sum += min((uint64_t)x.w, (uint64_t)kTrialW32Total);
+  for (uint64_t base = (uint64_t)blockIdx.x * kPackTile; base < sp.m; base += (uint64_t)gridDim.x * kPackTile) {
+    uint32_t tile = 0;
+#pragma unroll 4
+    for (int k = 0; k < kPackItems; ++k) {
+      const uint64_t e = base + (uint64_t)k * 256 + threadIdx.x;
+      if (e >= sp.m) break;
+      const cac_edge x = sp.edges[e];
+      bad = bad || x.w != w0 || x.u == x.v;
+      sum += min((uint64_t)x.w, (uint64_t)kTrialW32Total);
+      if (x.u != x.v) tile += (uint32_t)x.w;
+      if (sp.pk) sp.pk[e] = x.u | (x.v << 16);
+    }
+    if (sp.pk) {
+      tile = wave_sum<uint32_t>(tile);
+      if ((threadIdx.x & 63) == 0) tsum[threadIdx.x >> 6] = tile;
+      __syncthreads();
+      if (threadIdx.x == 0) sp.tiles[base / kPackTile] = tsum[0] + tsum[1] + tsum[2] + tsum[3];
+      __syncthreads();
+    }
   }
   if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(sp.mixed, 1u);
-  __shared__ uint64_t part[4];  // one addition per block: those to one word serialise
+  // one addition per block: those to one word are made one after another
   sum = wave_sum<uint64_t>(sum);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
   __syncthreads();
   if (threadIdx.x == 0) {
     sum = part[0] + part[1] + part[2] + part[3];
     if (sum) atomicAdd(sp.total, (unsigned long long)sum);
+  }
+}
+
+// Grid (graphs): exclusive prefix of a packed graph's tile sums.
+__global__ void __launch_bounds__(256) k_pack_scan(const EdgeSpan* spans) {
+  __shared__ uint32_t wtot[4];
+  const EdgeSpan sp = spans[blockIdx.x];
+  if (!sp.pk || *sp.mixed == 0 || *sp.total >= kTrialW32Total) return;
+  const uint64_t tiles = (sp.m + kPackTile - 1) / kPackTile;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint64_t base = 0; base < tiles; base += 256) {
+    const uint64_t i = base + threadIdx.x;
+    const uint32_t x = i < tiles ? sp.tiles[i] : 0;
+    const uint32_t inc = wave_incl_scan<uint32_t>(x);
+    if (lane == 63) wtot[wave] = inc;
+    __syncthreads();
+    uint32_t off = carry, tot = 0;
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) off += wtot[w];
+      tot += wtot[w];
+    }
+    if (i < tiles) sp.tiles[i] = off + inc - x;
+    carry += tot;
+    __syncthreads();
+  }
+}
+
+// Grid (slices, graphs): the weight prefix of every packed graph that needs one.
+__global__ void __launch_bounds__(256) k_pack_prefix(const EdgeSpan* spans) {
+  __shared__ uint32_t wtot[kPackItems][4];
+  const EdgeSpan sp = spans[blockIdx.y];
+  if (!sp.pk || sp.m == 0 || *sp.mixed == 0 || *sp.total >= kTrialW32Total) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (uint64_t base = (uint64_t)blockIdx.x * kPackTile; base < sp.m; base += (uint64_t)gridDim.x * kPackTile) {
+    uint32_t inc[kPackItems];
+#pragma unroll
+    for (int k = 0; k < kPackItems; ++k) {
+      const uint64_t e = base + (uint64_t)k * 256 + threadIdx.x;
+      uint32_t w = 0;
+      if (e < sp.m) {
+        const cac_edge x = sp.edges[e];
+        w = x.u != x.v ? (uint32_t)x.w : 0u;
+      }
+      inc[k] = wave_incl_scan<uint32_t>(w);
+      if (lane == 63) wtot[k][wave] = inc[k];
+    }
+    __syncthreads();
+    uint32_t off = sp.tiles[base / kPackTile];
+#pragma unroll
+    for (int k = 0; k < kPackItems; ++k) {
+      const uint64_t e = base + (uint64_t)k * 256 + threadIdx.x;
+      uint32_t wb = 0;
+      for (int w = 0; w < 4; ++w) {
+        if (w < wave) wb += wtot[k][w];
+      }
+      if (e < sp.m) sp.pre0[e] = off + wb + inc[k];
+      off += wtot[k][0] + wtot[k][1] + wtot[k][2] + wtot[k][3];
+    }
+    __syncthreads();
   }
 }
 
@@ -232,6 +321,283 @@ __device__ uint32_t prefix_search(const uint2* draws, uint32_t D, uint32_t need,
   return total;
 }
 
+// ---- trials in 32-bit arithmetic ------------------------------------------------
+// A trial whose graph has at most 2^16 vertices and weighs less than 2^31 works
+// on the packed graph: 4 bytes of endpoints per edge instead of 16, sums in 32
+// bits, and one u16 array in LDS that is both the labels and the union-find
+// forest (a label is the root the previous round left, so at the start of a
+// round the labels are a forest of depth one, and only entries of those roots
+// change).  The draws are the general form's: the prefix of the edges that still
+// join two super-vertices, in edge order, is the full masked prefix without its
+// repeats, so the first entry that reaches r names the same edge.
+//   - The first round's prefix is the graph's own and every trial draws from it.
+//   - A later round scans the edges that survived the round before, 16 per
+//     thread and step (four 16-byte loads in flight), and writes the survivors
+//     and their prefix compacted, in place: a step's writes end before the next
+//     step's reads begin.
+//   - Edges that all weigh the same need no prefix: draw r is survivor
+//     (r - 1) / w.
+// The unions run on LDS (a hop is tens of cycles against some hundreds for a
+// forest in L2), hooks by a 32-bit CAS on the word that holds the root's entry.
+// Against the general form: 4987 trials of Watts-Strogatz n = 32000, m = 512000
+// (one weight) 58 -> 7.5 ms; 768 planted graphs, 5 trials each (random weights)
+// 32.6 -> 6.5 ms; 58 trials of G(1000, 0.05) 0.37 -> 0.066 ms.  What bounds it
+// now is the latency of a workgroup's rounds: one 1024-thread workgroup per CU,
+// a few steps of 16384 edges per round.
+__device__ inline uint32_t l16_get(const uint16_t* par, uint32_t x) {
+  return __hip_atomic_load(par + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void l16_set(uint16_t* par, uint32_t x, uint32_t v) {
+  __hip_atomic_store(par + x, (uint16_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <bool kSplit>
+__device__ inline uint32_t l16_root(uint16_t* par, uint32_t x) {
+  uint32_t p = l16_get(par, x);
+  while (p != x) {
+    const uint32_t g = l16_get(par, p);
+    if (kSplit && g != p) l16_set(par, x, g);
+    x = p;
+    p = g;
+  }
+  return x;
+}
+// Union of the sets of a and b; true on a hook, *hooked the root that got a
+// parent.  Without path splitting (kSplit false) no other entry changes.
+template <bool kSplit>
+__device__ inline bool l16_union(uint16_t* par, uint32_t a, uint32_t b, uint32_t* hooked) {
+  uint32_t ra = l16_root<kSplit>(par, a), rb = l16_root<kSplit>(par, b);
+  while (ra != rb) {
+    const uint32_t lo = min(ra, rb), hi = max(ra, rb);
+    uint32_t* word = reinterpret_cast<uint32_t*>(par) + (hi >> 1);
+    const uint32_t sh = (hi & 1) * 16;
+    uint32_t cur = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    uint32_t old;
+    for (;;) {  // the neighbouring entry may change under the CAS
+      old = (cur >> sh) & 0xFFFFu;
+      if (old != hi) break;
+      const uint32_t prev = atomicCAS(word, cur, (cur & ~(0xFFFFu << sh)) | (lo << sh));
+      if (prev == cur) {
+        *hooked = hi;
+        return true;
+      }
+      cur = prev;
+    }
+    ra = l16_root<kSplit>(par, old);
+    rb = l16_root<kSplit>(par, lo);
+  }
+  return false;
+}
+
+__device__ inline uint32_t bsum32(uint32_t x, uint32_t* lds) {
+  x = wave_sum<uint32_t>(x);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
+  __syncthreads();
+  uint32_t t = 0;
+  for (int w = 0; w < kSmpWaves; ++w) t += lds[w];
+  __syncthreads();
+  return t;
+}
+
+// prefix_search on LDS (the same chunks, the same prefix length).
+__device__ uint32_t prefix_search16(const uint32_t* draws, uint32_t D, uint32_t need, uint16_t* par, uint32_t* lds) {
+  for (uint32_t d = threadIdx.x; d < D; d += kSmpBlock) {  // back to the round's starting forest
+    const uint32_t x = draws[d];
+    l16_set(par, x & 0xFFFFu, x & 0xFFFFu);
+    l16_set(par, x >> 16, x >> 16);
+  }
+  __syncthreads();
+  // unites the first len draws of the chunk; the sum's barriers separate it from
+  // what follows
+  auto unite = [&](uint32_t c0, uint32_t len, uint32_t* mine) {
+    bool h = false;
+    if (threadIdx.x < len) {
+      const uint32_t x = draws[c0 + threadIdx.x];
+      h = l16_union<false>(par, x & 0xFFFFu, x >> 16, mine);
+    }
+    return h;
+  };
+  uint32_t total = 0;
+  for (uint32_t c0 = 0; c0 < D; c0 += kSmpBlock) {
+    const uint32_t len = min((uint32_t)kSmpBlock, D - c0);
+    uint32_t mine = 0;
+    const bool hooked = unite(c0, len, &mine);
+    const uint32_t ch = bsum32(hooked ? 1 : 0, lds);
+    if (total + ch < need) {  // the whole chunk stays
+      total += ch;
+      continue;
+    }
+    if (hooked) l16_set(par, mine, mine);  // undo the chunk
+    __syncthreads();
+    uint32_t lo = 1, hi = len;
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      uint32_t m2 = 0;
+      const bool h2 = unite(c0, mid, &m2);
+      const uint32_t c2 = bsum32(h2 ? 1 : 0, lds);
+      if (h2) l16_set(par, m2, m2);
+      __syncthreads();
+      if (total + c2 >= need) hi = mid;
+      else lo = mid + 1;
+    }
+    uint32_t m3 = 0;
+    const bool h3 = unite(c0, lo, &m3);
+    return total + bsum32(h3 ? 1 : 0, lds);
+  }
+  return total;
+}
+
+__device__ void sample_packed(const TrialScratch& S, uint32_t idx_cap, uint32_t* idx, uint16_t* lab) {
+  typedef const __attribute__((address_space(1))) uint32_t g_u32;
+  typedef uint32_t u32x4v __attribute__((ext_vector_type(4), aligned(16)));
+  typedef const __attribute__((address_space(1))) u32x4v g_u32x4;
+  __shared__ uint32_t red[kSmpWaves];
+  __shared__ uint64_t wtot[2][64];
+  constexpr uint32_t kQ = 4, kStep = kSmpBlock * 4 * kQ;
+  const uint32_t m = (uint32_t)S.m, n = S.n, t = S.t;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wu = m > 0 && *S.mixed == 0 ? (uint32_t)S.edges[0].w : 0u;  // every edge's weight, or 0
+  uint32_t* own_list = reinterpret_cast<uint32_t*>(S.pre);
+  uint32_t* own_pre = own_list + ((m + 3u) & ~3u);
+  uint32_t* draws = reinterpret_cast<uint32_t*>(S.draws);
+  for (uint32_t v = threadIdx.x; v < (n + 1) / 2; v += kSmpBlock)
+    reinterpret_cast<uint32_t*>(lab)[v] = 2 * v | ((2 * v + 1) << 16);
+  __syncthreads();
+  const uint32_t* list = S.pk;
+  const uint32_t* pre = S.pre0;
+  uint32_t count = m, nv = n;
+  for (uint32_t round = 0; nv > t; ++round) {
+    if (round > 0) {  // the survivors of `list` into the trial's own list
+      uint32_t out = 0, wout = 0, parity = 0;
+      for (uint32_t base = 0; base < count; base += kStep, parity ^= 1) {
+        uint32_t pk[kQ][4], w[kQ][4];
+        uint64_t inc[kQ];
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; ++q) {
+          const uint32_t x0 = base + (q * kSmpBlock + threadIdx.x) * 4;
+          if (x0 + 4 <= count) {
+            const u32x4v p = *(g_u32x4*)(list + x0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) pk[q][j] = p[j];
+            if (wu == 0) {
+              const u32x4v f = *(g_u32x4*)(pre + x0);
+              const uint32_t before = x0 > 0 ? ((g_u32*)pre)[x0 - 1] : 0u;
+              w[q][0] = f[0] - before;
+#pragma unroll
+              for (int j = 1; j < 4; ++j) w[q][j] = f[j] - f[j - 1];
+            }
+          } else {
+            uint32_t last = wu == 0 && x0 > 0 && x0 - 1 < count ? ((g_u32*)pre)[x0 - 1] : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const bool in = x0 + j < count;
+              pk[q][j] = in ? ((g_u32*)list)[x0 + j] : 0u;  // (0, 0): a loop
+              const uint32_t f = in && wu == 0 ? ((g_u32*)pre)[x0 + j] : last;
+              w[q][j] = f - last;
+              last = f;
+            }
+          }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; ++q) {
+          uint64_t sum = 0;  // survivors | their weight
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const bool live = lab[pk[q][j] & 0xFFFFu] != lab[pk[q][j] >> 16];
+            if (wu != 0) w[q][j] = live ? wu : 0u;
+            else if (!live) w[q][j] = 0;
+            // a survivor of weight 0 can never be drawn: dropped with the loops
+            sum += w[q][j] ? (1ull << 32) | w[q][j] : 0ull;
+          }
+          inc[q] = wave_incl_scan<uint64_t>(sum);
+          if (lane == 63) wtot[parity][q * kSmpWaves + wave] = inc[q];
+          inc[q] -= sum;
+        }
+        __syncthreads();
+        const uint64_t sc = wave_incl_scan<uint64_t>(wtot[parity][lane]);
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; ++q) {
+          const int at = (int)(q * kSmpWaves) + wave;
+          const uint64_t off = inc[q] + (at > 0 ? readlane(sc, at - 1) : 0ull);
+          uint32_t pos = out + (uint32_t)(off >> 32), run = wout + (uint32_t)off;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (w[q][j]) {
+              run += w[q][j];
+              own_list[pos] = pk[q][j];
+              if (wu == 0) own_pre[pos] = run;
+              ++pos;
+            }
+          }
+        }
+        const uint64_t step = readlane(sc, 63);
+        out += (uint32_t)(step >> 32);
+        wout += (uint32_t)step;
+      }
+      count = out;
+      list = own_list;
+      pre = own_pre;
+      block_sync_global();  // the draws read the lists written by every wave
+    }
+    if (count == 0) break;  // only loops left: more than t components
+    const uint32_t W = wu != 0 ? wu * count : pre[count - 1];
+    if (W == 0) break;
+    uint32_t gshift = 0;
+    if (wu == 0) {  // segment index: the last prefix of every 2^gshift edges
+      while (((count + (1u << gshift) - 1) >> gshift) > idx_cap) ++gshift;
+      const uint32_t nseg = (count + (1u << gshift) - 1) >> gshift;
+      for (uint32_t k = threadIdx.x; k < nseg; k += kSmpBlock) idx[k] = pre[min(((k + 1) << gshift), count) - 1];
+      __syncthreads();
+    }
+    // draws
+    const uint32_t D = S.dpr ? S.dpr : nv;
+    for (uint32_t d = threadIdx.x; d < D; d += kSmpBlock) {
+      const u32x4 rnd = philox4x32(S.trial, round, d, 0u, S.seed, kDomSample);
+      const uint32_t r = (uint32_t)uniform1(lo64(rnd), W);
+      uint32_t e;
+      if (wu != 0) {
+        e = (r - 1) / wu;
+      } else {
+        uint32_t a = 0, b = ((count + (1u << gshift) - 1) >> gshift) - 1;
+        while (a < b) {
+          const uint32_t mid = (a + b) >> 1;
+          if (idx[mid] >= r) b = mid;
+          else a = mid + 1;
+        }
+        uint32_t lo = a << gshift, hi = min(lo + (1u << gshift), count) - 1;
+        while (lo < hi) {
+          const uint32_t mid = (lo + hi) >> 1;
+          if (((g_u32*)pre)[mid] >= r) hi = mid;
+          else lo = mid + 1;
+        }
+        e = lo;
+      }
+      const uint32_t x = ((g_u32*)list)[e];
+      draws[d] = (uint32_t)lab[x & 0xFFFFu] | ((uint32_t)lab[x >> 16] << 16);
+    }
+    __syncthreads();  // every label of the round read before the first union; a thread reads its own draws
+    uint32_t mine = 0, unused = 0;
+    for (uint32_t d = threadIdx.x; d < D; d += kSmpBlock) {
+      const uint32_t x = draws[d];
+      mine += l16_union<true>(lab, x & 0xFFFFu, x >> 16, &unused) ? 1 : 0;
+    }
+    uint32_t hooks = bsum32(mine, red);
+    if (nv - hooks <= t) {
+      block_sync_global();  // the search reads draws of other threads
+      hooks = prefix_search16(draws, D, nv - t, lab, red);
+    }
+    // canonical relabel, in place: every entry stays an ancestor of its vertex
+    for (uint32_t v = threadIdx.x; v < n; v += kSmpBlock) l16_set(lab, v, l16_root<false>(lab, l16_get(lab, v)));
+    __syncthreads();
+    nv -= hooks;
+  }
+  for (uint32_t v = threadIdx.x; v < (n + 1) / 2; v += kSmpBlock) S.lab[v] = reinterpret_cast<uint32_t*>(lab)[v];
+  if (threadIdx.x == 0) {
+    *S.nv_out = nv;
+    S.live[0] = count;
+    S.live[1] = list == own_list ? 1u : 0u;
+  }
+}
+
 // kMinWaves = 8 holds the kernel to 64 VGPRs (8 waves per SIMD), so two 16-wave
 // workgroups share a CU, at the price of a few spilled registers: for launches
 // of more workgroups than CUs.  kMinWaves = 1 leaves the registers free, for
@@ -254,6 +620,12 @@ __global__ void __launch_bounds__(kSmpBlock, kMinWaves)
   uint64_t* seg_last = smp_dyn;
   uint16_t* slab = reinterpret_cast<uint16_t*>(smp_dyn + idx_cap);
   const TrialScratch S = scratch[blockIdx.x];
+  if constexpr (kLdsLab) {
+    if (trial_packed(S)) {
+      sample_packed(S, 2 * idx_cap, reinterpret_cast<uint32_t*>(smp_dyn), slab);
+      return;
+    }
+  }
   const cac_edge* __restrict__ edges = S.edges;
   const uint64_t m = S.m;
   uint32_t gshift = 0;  // segments of 2^gshift edges, at most idx_cap of them
@@ -378,6 +750,14 @@ __global__ void __launch_bounds__(kSmpBlock, kMinWaves)
 // Dynamic LDS of k_densify_trials: the row sums of a matrix of up to kKsMaxS rows.
 constexpr size_t kDensifyLds = (size_t)kKsMaxS * 8;
 constexpr int kDensifyEdges = 4;  // edges per thread in flight
+// A launch with packed trials of at most nmax vertices: u16 labels, t row sums and
+// one row (at most 152 KiB: two 1024-thread workgroups share a CU up to half that),
+// or what an unpacked trial of the launch takes.
+constexpr size_t kDensifyLdsMax = 152 * 1024;
+inline size_t densify_lds_bytes(uint64_t nmax, uint64_t tmax) {
+  const size_t packed = ((2 * (size_t)nmax + 15) & ~size_t(15)) + 8 * (size_t)tmax;
+  return std::min(kDensifyLdsMax, std::max(packed, std::min(kDensifyLds, (size_t)tmax * 8)));
+}
 
 // The accumulation of k_densify_trials for entries of type E (row stride
 // ks_stride<E>(k)): zeroes the matrix with 16-byte stores, adds the surviving
@@ -453,6 +833,122 @@ __device__ uint64_t densify_edges(const TrialScratch& S, uint32_t k, const uint3
   return best;
 }
 
+// k_densify_trials of a packed trial: labels and row sums in LDS, and only the
+// edges that survived the trial's last scan (each that still joins two
+// super-vertices is among them), 4 bytes each and 4 of prefix, instead of the
+// whole list.  The zero fill, t^2 words, is issued first and drains behind the
+// ranking.  One super-vertex, h, holds most of a sampled graph and most surviving
+// edges touch it, so its row is summed in LDS (one atomic per edge, spread over
+// the row) and written once with its mirror column: as two matrix atomics and
+// two row-sum atomics per edge, those on h's entries contended.  h is a guess
+// from 64 edges; any choice gives the same matrix.  4987 trials of
+// Watts-Strogatz n = 32000, t = 1433: 30 ms reading the whole list, 27.7 ms with
+// the survivors alone, 11.6 ms with h's row in LDS, 3.5 TB/s of zero fill.
+// Returns the thread's part of the smallest row sum.
+__device__ uint64_t densify_packed(const TrialScratch& S, uint32_t k, unsigned char* smem, uint32_t lds_bytes,
+                                   uint32_t* wtot) {
+  typedef const __attribute__((address_space(1))) uint32_t g_u32;
+  uint32_t* mat = (uint32_t*)S.mat;
+  uint32_t* rsum = (uint32_t*)S.rsum;
+  const uint32_t n = S.n, st = ks_stride<uint32_t>(k);
+  uint16_t* lab = (uint16_t*)smem;
+  const uint32_t lab_bytes = (2 * n + 15) & ~15u;
+  const bool lds_rows = lab_bytes + 8 * k <= lds_bytes;  // else the sums take atomics in memory
+  uint32_t* row_sum = lds_rows ? (uint32_t*)(smem + lab_bytes) : rsum;
+  uint32_t* h_row = row_sum + k;  // lds_rows only
+  const uint64_t cells = (uint64_t)st * k;
+  for (uint64_t i = threadIdx.x; i < cells / 4; i += kSmpBlock) ((uint4*)mat)[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (uint32_t r = threadIdx.x; r < (lds_rows ? 2 * k : k); r += kSmpBlock) row_sum[r] = 0;
+  for (uint32_t v = threadIdx.x; v < (n + 1) / 2; v += kSmpBlock) ((uint32_t*)lab)[v] = S.lab[v];
+  __syncthreads();
+  uint16_t* rank = (uint16_t*)S.par;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint32_t base = 0; base < n; base += kSmpBlock) {
+    const uint32_t x = base + threadIdx.x;
+    const uint64_t live = __ballot(x < n && lab[x] == x);
+    if (lane == 0) wtot[wave] = (uint32_t)__popcll(live);
+    __syncthreads();
+    uint32_t off = carry, tot = 0;
+    for (int v = 0; v < kSmpWaves; ++v) {
+      if (v < wave) off += wtot[v];
+      tot += wtot[v];
+    }
+    if ((live >> lane) & 1ull) rank[x] = (uint16_t)(off + (uint32_t)__popcll(live & ((1ull << lane) - 1)));
+    carry += tot;
+    __syncthreads();
+  }
+  block_sync_global();  // ranks and zeroed rows
+  for (uint32_t x = threadIdx.x; x < n; x += kSmpBlock) lab[x] = rank[lab[x]];
+  __syncthreads();
+  const uint32_t m = (uint32_t)S.m, count = S.live[0];
+  const bool own = S.live[1] != 0;
+  const uint32_t* own_list = reinterpret_cast<const uint32_t*>(S.pre);
+  g_u32* list = (g_u32*)(own ? own_list : S.pk);
+  g_u32* pre = (g_u32*)(own ? own_list + ((m + 3u) & ~3u) : S.pre0);
+  const uint32_t wu = m > 0 && *S.mixed == 0 ? (uint32_t)S.edges[0].w : 0u;
+  if (lds_rows && wave == 0) {  // h: the most frequent endpoint of 64 edges
+    const uint32_t x = count > 0 ? list[(uint32_t)(((uint64_t)lane * count) >> 6)] : 0u;
+    const uint32_t a = lab[x & 0xFFFFu], b = lab[x >> 16];
+    uint32_t best_n = 0, best_v = 0;
+    for (int l = 0; l < 64; ++l) {
+      const uint32_t va = readlane_u32(a, l), vb = readlane_u32(b, l);
+      const uint32_t na = (uint32_t)(__popcll(__ballot(a == va)) + __popcll(__ballot(b == va)));
+      const uint32_t nb = (uint32_t)(__popcll(__ballot(a == vb)) + __popcll(__ballot(b == vb)));
+      if (va != vb && na > best_n) {
+        best_n = na;
+        best_v = va;
+      }
+      if (va != vb && nb > best_n) {
+        best_n = nb;
+        best_v = vb;
+      }
+    }
+    if (lane == 0) wtot[0] = best_v;
+  }
+  __syncthreads();
+  const uint32_t h = lds_rows ? wtot[0] : kNoSlot;
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < count; i += kSmpBlock) {
+    const uint32_t x = list[i];
+    const uint32_t a = lab[x & 0xFFFFu], b = lab[x >> 16];
+    if (a == b) continue;
+    const uint32_t w = wu != 0 ? wu : pre[i] - (i > 0 ? pre[i - 1] : 0u);
+    if (w == 0) continue;
+    if (a == h || b == h) {
+      atomicAdd(&h_row[a == h ? b : a], w);
+      continue;
+    }
+    atomicAdd(&mat[(uint64_t)a * st + b], w);
+    atomicAdd(&mat[(uint64_t)b * st + a], w);
+    atomicAdd(&row_sum[a], w);
+    atomicAdd(&row_sum[b], w);
+  }
+  if (lds_rows) {
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t r = threadIdx.x; r < k; r += kSmpBlock) {
+      const uint32_t w = h_row[r];  // h_row[h] is 0: an edge with both ends h is a loop
+      if (w == 0) continue;
+      mat[(uint64_t)h * st + r] = w;
+      mat[(uint64_t)r * st + h] = w;
+      row_sum[r] += w;
+      sum += w;
+    }
+    if (sum) atomicAdd(&row_sum[h], sum);  // no thread adds to row_sum[h] above
+    __syncthreads();
+  } else {
+    block_sync_global();
+  }
+  uint64_t best = ~0ull;
+  for (uint32_t r = threadIdx.x; r < k; r += kSmpBlock) {
+    const uint32_t acc = row_sum[r];
+    if (lds_rows) rsum[r] = acc;
+    best = acc < best ? acc : best;
+  }
+  return best;
+}
+
 // Rank the canonical labels, accumulate the surviving edges into the k x k
 // matrix (k == t unless the sampling stopped early on a disconnected graph),
 // with its row sums in LDS, and compute the trial's bound (minimum weighted
@@ -462,7 +958,7 @@ __device__ uint64_t densify_edges(const TrialScratch& S, uint32_t k, const uint3
 // rank); for callers that do not read the labels afterwards.
 template <bool kRankLabels>
 __global__ void __launch_bounds__(kSmpBlock) k_densify_trials(const TrialScratch* __restrict__ scratch, int64_t* bounds,
-                                                              int64_t* results) {
+                                                              int64_t* results, uint32_t lds_bytes) {
   __shared__ uint32_t wtot[kSmpWaves];
   __shared__ uint64_t lds[kSmpWaves + 2];
   extern __shared__ __align__(16) unsigned char densify_lds[];
@@ -476,30 +972,35 @@ __global__ void __launch_bounds__(kSmpBlock) k_densify_trials(const TrialScratch
     }
     return;
   }
-  uint32_t* rank = S.par;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < n; base += kSmpBlock) {
-    const uint32_t x = base + threadIdx.x;
-    const uint32_t live = (x < n && S.lab[x] == x) ? 1u : 0u;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t inc = wave_incl_scan<uint32_t>(live);
-    if (lane == 63) wtot[wave] = inc;
-    __syncthreads();
-    uint32_t off = carry, tot = 0;
-    for (int v = 0; v < kSmpWaves; ++v) {
-      if (v < wave) off += wtot[v];
-      tot += wtot[v];
+  uint64_t best;
+  if (kRankLabels && trial_packed(S)) {
+    best = densify_packed(S, k, densify_lds, lds_bytes, wtot);
+  } else {
+    uint32_t* rank = S.par;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < n; base += kSmpBlock) {
+      const uint32_t x = base + threadIdx.x;
+      const uint32_t live = (x < n && S.lab[x] == x) ? 1u : 0u;
+      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+      const uint32_t inc = wave_incl_scan<uint32_t>(live);
+      if (lane == 63) wtot[wave] = inc;
+      __syncthreads();
+      uint32_t off = carry, tot = 0;
+      for (int v = 0; v < kSmpWaves; ++v) {
+        if (v < wave) off += wtot[v];
+        tot += wtot[v];
+      }
+      if (live) rank[x] = off + inc - 1;
+      carry += tot;
+      __syncthreads();
     }
-    if (live) rank[x] = off + inc - 1;
-    carry += tot;
-    __syncthreads();
+    if constexpr (kRankLabels) {
+      block_sync_global();  // every rank written
+      for (uint32_t x = threadIdx.x; x < n; x += kSmpBlock) S.lab[x] = rank[S.lab[x]];
+    }
+    best = trial_w32(S) ? densify_edges<kRankLabels, uint32_t>(S, k, rank, densify_lds)
+                        : densify_edges<kRankLabels, int64_t>(S, k, rank, densify_lds);
   }
-  if constexpr (kRankLabels) {
-    block_sync_global();  // every rank written
-    for (uint32_t x = threadIdx.x; x < n; x += kSmpBlock) S.lab[x] = rank[S.lab[x]];
-  }
-  uint64_t best = trial_w32(S) ? densify_edges<kRankLabels, uint32_t>(S, k, rank, densify_lds)
-                               : densify_edges<kRankLabels, int64_t>(S, k, rank, densify_lds);
   best = wave_min<uint64_t>(best);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = best;
   __syncthreads();
@@ -592,8 +1093,11 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 // graph (one per distinct edge list) and launches the kernels that set them;
 // spans, flags and totals hold scr.size() entries.  Both are ready for any later
 // launch on s.
+// packed: the graphs' packed forms are carved from it (packed_bytes each), null:
+// none is packed.
 int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d_spans, uint32_t* d_flags,
-                       unsigned long long* d_totals, hipStream_t s) {
+                       unsigned long long* d_totals, void* packed, hipStream_t s) {
+  Carver pc(packed);
   std::unordered_map<const cac_edge*, uint32_t> index;
   std::vector<EdgeSpan> spans;
   uint64_t mmax = 0;
@@ -603,13 +1107,21 @@ int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d
     if (it == index.end()) {
       g = (uint32_t)spans.size();
       index.emplace(x.edges, g);
-      spans.push_back({x.edges, x.m, d_flags + g, d_totals + g});
+      EdgeSpan sp{x.edges, x.m, d_flags + g, d_totals + g, nullptr, nullptr, nullptr};
+      if (packed && x.n <= kPackMaxN && x.m < kPackMaxM) {
+        sp.pk = pc.take<uint32_t>(x.m);
+        sp.pre0 = pc.take<uint32_t>(x.m);
+        sp.tiles = pc.take<uint32_t>((x.m + kPackTile - 1) / kPackTile);
+      }
+      spans.push_back(sp);
       mmax = std::max(mmax, x.m);
     } else {
       g = it->second;
     }
     x.mixed = d_flags + g;
     x.total = d_totals + g;
+    x.pk = spans[g].pk;
+    x.pre0 = spans[g].pre0;
   }
   if (spans.empty()) return CAC_OK;
   const uint32_t count = (uint32_t)spans.size();
@@ -618,6 +1130,12 @@ int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d
   for (uint32_t g0 = 0; g0 < count; g0 += 65535u)  // grid y holds at most 65535 graphs
     hipLaunchKernelGGL(k_mixed_weights, dim3(grid_for(mmax, 256 * 16, 256), std::min(count - g0, 65535u)), dim3(256),
                        0, s, (const EdgeSpan*)(d_spans + g0));
+  if (packed) {
+    hipLaunchKernelGGL(k_pack_scan, dim3(count), dim3(256), 0, s, (const EdgeSpan*)d_spans);
+    for (uint32_t g0 = 0; g0 < count; g0 += 65535u)
+      hipLaunchKernelGGL(k_pack_prefix, dim3(grid_for(mmax, kPackTile, 256), std::min(count - g0, 65535u)), dim3(256),
+                         0, s, (const EdgeSpan*)(d_spans + g0));
+  }
   CAC_LAUNCH_CHECK(ctx, "weight flags");
   return CAC_OK;
 }
@@ -629,10 +1147,10 @@ int densify_attr(cac_ctx* ctx) {
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
     err = hipFuncSetAttribute((const void*)k_densify_trials<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kDensifyLds);
+                              (int)kDensifyLdsMax);
     if (err == hipSuccess)
       err = hipFuncSetAttribute((const void*)k_densify_trials<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)kDensifyLds);
+                                (int)kDensifyLdsMax);
   });
   CAC_HIP(ctx, err);
   return CAC_OK;
@@ -641,7 +1159,7 @@ int densify_attr(cac_ctx* ctx) {
 
 // Dynamic LDS a sampling workgroup may take: the CU's 160 KiB less the
 // kernel's static arrays, with room to spare.
-constexpr size_t kSmpLdsMax = 160 * 1024 - 1024;
+constexpr size_t kSmpLdsMax = 160 * 1024 - 2048;
 
 // Launch shape of k_sample_trials for trials of at most nmax vertices.
 struct SmpShape {
@@ -710,7 +1228,7 @@ int launch_sampling(cac_ctx* ctx, size_t nb, uint64_t mmax, uint64_t nmax, const
   const SmpShape sh = sampling_shape(nmax);
   const int cls = mmax < (1ull << 16) ? 0 : mmax < (1ull << 20) ? 1 : mmax < (1ull << 24) ? 2 : 3;
   const int per_cu = ctx->sample_occupancy[cls] ? ctx->sample_occupancy[cls] : 2;
-  const bool two = nb > (size_t)cus && per_cu == 2 && 2 * (sh.dyn + 1024) <= 160 * 1024;
+  const bool two = nb > (size_t)cus && per_cu == 2 && 2 * (sh.dyn + 2048) <= 160 * 1024;
   const dim3 grid((unsigned)nb), block(kSmpBlock);
   if (sh.lds_lab) {
     if (two) hipLaunchKernelGGL((k_sample_trials<8, true>), grid, block, sh.dyn, s, d_scr, sh.idx_cap);
@@ -770,9 +1288,8 @@ static uint32_t job_dpr(const cac_ctx* ctx, uint32_t n) {
 // Device bytes one sampling job needs beside the Karger-Stein levels (dpr:
 // draws per round, 0 = |V|).
 size_t job_sample_bytes(const SqrtJob& j, uint32_t dpr) {
-  return carve_size((size_t)j.n * 4) * 2 + carve_size(std::max<uint64_t>(j.m, 1) * 8) +
-         carve_size((size_t)std::max(j.n, dpr) * 8) + carve_size((size_t)j.t * j.t * 8) + carve_size((size_t)j.t * 8) +
-         256;
+  return carve_size((size_t)j.n * 4) * 2 + carve_size((j.m + 2) * 8) + carve_size((size_t)std::max(j.n, dpr) * 8) +
+         carve_size((size_t)j.t * j.t * 8) + carve_size((size_t)j.t * 8) + 512;
 }
 // Upper estimate of the Karger-Stein level arenas of one root of size t: each
 // level holds about t^2 entries in copy-on-write work rows plus the contracted
@@ -915,7 +1432,7 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
       deg[i] = cv.take<unsigned long long>((size_t)j.t + 2);  // [t] degrees, [t + 1] their minimum
       offsets[i + 1] = offsets[i] + j.m;
     }
-    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, s);
+    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, nullptr, s);
     if (rc) return rc;
     std::vector<TrialScratch> wid(scr.begin() + w0, scr.end());
     CAC_HIP(ctx, hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s));
@@ -1015,6 +1532,8 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
   return CAC_OK;
 }
 
+static bool can_pack(const SqrtJob& j) { return j.n <= kPackMaxN && j.m < kPackMaxM; }
+
 // Dense-engine jobs (t <= 8192) in chunks sized to the budget: sampling,
 // densification, then one breadth-first Karger-Stein pass per chunk, whatever
 // graphs the chunk's jobs belong to.  wide: every job runs in the wide form
@@ -1024,13 +1543,17 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
   int rc = CAC_OK;
   size_t b0 = 0;
   while (b0 < jobs.size() && rc == CAC_OK) {
-    size_t nb = 0, sample_bytes = 0, ks_bytes = 0, wide_bytes = 0;
+    size_t nb = 0, sample_bytes = 0, ks_bytes = 0, wide_bytes = 0, pack_bytes = 0;
+    std::unordered_set<const cac_edge*> graphs;  // packed once per graph of the chunk
     const size_t cap = wide ? 4096 : kMaxJobsPerChunk;
     while (b0 + nb < jobs.size() && nb < cap) {
       const SqrtJob& j = jobs[b0 + nb];
       const size_t a = job_sample_bytes(j, job_dpr(ctx, j.n)), k = job_ks_bytes(j);
       const size_t wb = wide ? wide_trial_bytes(j.m, j.n) : 0;
-      if (nb > 0 && sample_bytes + a + ks_bytes + k + wide_bytes + wb > budget) break;
+      const size_t pb = !wide && can_pack(j) && !graphs.count(j.edges) ? packed_bytes(j.m) : 0;
+      if (nb > 0 && sample_bytes + a + ks_bytes + k + wide_bytes + wb + pack_bytes + pb > budget) break;
+      if (pb) graphs.insert(j.edges);
+      pack_bytes += pb;
       sample_bytes += a;
       ks_bytes += k;
       wide_bytes += wb;
@@ -1047,7 +1570,7 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     }
     const size_t bytes = sample_bytes + carve_size(nb * sizeof(TrialScratch)) + 2 * carve_size(nb * 8) +
                          carve_size(nb * sizeof(EdgeSpan)) + carve_size(nb * 4) + carve_size(nb * 8) +
-                         carve_size(wide_bytes) + 1024;
+                         carve_size(wide_bytes) + pack_bytes + 1024;
     rc = grow_buffer(ctx, &ctx->smp_buf, &ctx->smp_bytes, bytes);
     if (rc) return rc;
     BufPin pin(ctx, kBufSmp);  // the sampled matrices are the dense roots
@@ -1074,13 +1597,15 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       x.dpr = job_dpr(ctx, j.n);
       x.lab = cv.take<uint32_t>(j.n);
       x.par = cv.take<uint32_t>(j.n);
-      x.pre = cv.take<uint64_t>(std::max<uint64_t>(j.m, 1));
+      x.pre = cv.take<uint64_t>(j.m + 2);  // a packed trial's list and prefix, each of whole 16-byte pieces
       x.draws = cv.take<uint2>(std::max(j.n, x.dpr));
       x.mat = cv.take<int64_t>((size_t)j.t * j.t);  // room for either entry type
       x.rsum = cv.take<int64_t>(j.t);
       x.nv_out = d_nv + i;
+      x.live = cv.take<uint32_t>(2);
     }
-    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, s);
+    void* packed = pack_bytes ? (void*)cv.take<unsigned char>(pack_bytes) : nullptr;
+    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, packed, s);
     if (rc) return rc;
     e = hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "job descriptors");
@@ -1093,18 +1618,27 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       prof_end(ctx, s);
     } else if (rc == CAC_OK) {
       prof_begin(ctx, "sample_trials", s);
-      uint64_t mmax_jobs = 0, nmax_jobs = 0;
-      for (size_t i = 0; i < nb; ++i) {
-        mmax_jobs = std::max<uint64_t>(mmax_jobs, jobs[b0 + i].m);
-        nmax_jobs = std::max<uint64_t>(nmax_jobs, jobs[b0 + i].n);
+      // the jobs too large for labels in LDS come first and launch apart
+      uint64_t tmax = 0, npack = 0;
+      for (size_t i = 0; i < nb && rc == CAC_OK;) {
+        const bool big = jobs[b0 + i].n > kPackMaxN;
+        const size_t i0 = i;
+        uint64_t mmax = 0, nmax = 0;
+        for (; i < nb && (jobs[b0 + i].n > kPackMaxN) == big; ++i) {
+          mmax = std::max<uint64_t>(mmax, jobs[b0 + i].m);
+          nmax = std::max<uint64_t>(nmax, jobs[b0 + i].n);
+          tmax = std::max<uint64_t>(tmax, jobs[b0 + i].t);
+        }
+        if (!big) npack = std::max(npack, nmax);
+        rc = launch_sampling(ctx, i - i0, mmax, nmax, d_scr + i0, s);
       }
-      rc = launch_sampling(ctx, nb, mmax_jobs, nmax_jobs, d_scr, s);
+      const size_t dense_lds = densify_lds_bytes(npack, tmax);
       prof_end(ctx, s);
       prof_begin(ctx, "densify_trials", s);
       if (rc == CAC_OK) rc = densify_attr(ctx);
       if (rc == CAC_OK)
-        hipLaunchKernelGGL(k_densify_trials<true>, dim3((unsigned)nb), dim3(kSmpBlock), kDensifyLds, s,
-                           (const TrialScratch*)d_scr, d_bounds, d_results);
+        hipLaunchKernelGGL(k_densify_trials<true>, dim3((unsigned)nb), dim3(kSmpBlock), dense_lds, s,
+                           (const TrialScratch*)d_scr, d_bounds, d_results, (uint32_t)dense_lds);
       prof_end(ctx, s);
       e = hipGetLastError();
       if (e != hipSuccess) rc = hip_fail(ctx, e, "sampling kernels");
@@ -1169,6 +1703,9 @@ int sqrt_cut_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int64_t* d_re
     if (below_floor)
       std::stable_sort(narrow.begin(), narrow.end(), [](const SqrtJob& a, const SqrtJob& b) { return a.n > b.n; });
   }
+  // labels fit LDS up to 2^16 vertices: the larger graphs' trials come first, so
+  // a chunk launches each kind once
+  std::stable_partition(narrow.begin(), narrow.end(), [](const SqrtJob& j) { return j.n > kPackMaxN; });
   int rc = sqrt_dense_chunks(ctx, wide, d_results, s, budget, true);
   if (rc) return rc;
   return sqrt_dense_chunks(ctx, narrow, d_results, s, budget, false);
@@ -1219,7 +1756,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   h.mat = nullptr;
   h.rsum = nullptr;
   std::vector<TrialScratch> one{h};
-  int rc = launch_mixed_flags(ctx, one, d_span, d_flag, d_total, s);
+  int rc = launch_mixed_flags(ctx, one, d_span, d_flag, d_total, nullptr, s);
   if (rc) return rc;
   h = one[0];
   h.total = nullptr;  // the merged matrix is read as int64
@@ -1236,7 +1773,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   rc = densify_attr(ctx);
   if (rc) return rc;
   hipLaunchKernelGGL(k_densify_trials<false>, dim3(1), dim3(kSmpBlock), kDensifyLds, s, (const TrialScratch*)d_scr, d_misc,
-                     d_misc + 1);
+                     d_misc + 1, (uint32_t)kDensifyLds);
   CAC_LAUNCH_CHECK(ctx, "densify trial");
   CAC_HIP(ctx, hipStreamSynchronize(s));
   out->lab = h.lab;

@@ -33,12 +33,22 @@ struct TrialScratch {
   const uint32_t* mixed;
   // [1] total edge weight of the job's graph, saturating (null: entries are 64-bit)
   const unsigned long long* total;
+  // The graph packed for trials in 32-bit arithmetic (null: not packed): endpoints
+  // u | v << 16 and the inclusive prefix of the weights with loops counted as 0
+  // (unless every edge weighs the same, with no loop).  Such a trial keeps its
+  // labels as u16 in lab, its surviving edges and their prefix in pre's 2 m
+  // words, its draws as la | lb << 16, and leaves in live[0] the number of edges
+  // of its last scan and in live[1] whether they are its own list's.
+  const uint32_t* pk;
+  const uint32_t* pre0;
+  uint32_t* live;
 };
 
 // The contracted matrix's entries add up to at most twice the graph's total
 // weight: below 2^32 the matrix and its row sums are uint32_t, else int64_t.
 constexpr unsigned long long kTrialW32Total = 1ull << 31;
 __device__ inline bool trial_w32(const TrialScratch& S) { return S.total && *S.total < kTrialW32Total; }
+__device__ inline bool trial_packed(const TrialScratch& S) { return S.pk && trial_w32(S); }
 
 // Device bytes of the per-trial state of the wide form beside TrialScratch's
 // buffers (tile totals and the round's control words).
