@@ -928,8 +928,12 @@ size_t ks_live_bytes_per_root(uint32_t n, bool w32) {
   int depth = 0;
   for (uint32_t sz = n; sz > kKsBase; sz = ks_target(sz), nodes *= 2, ++depth) {
     const uint32_t t = ks_target(sz);
-    const size_t b = 2 * nodes * (child_bytes(sz, t, esize) + sizeof(KsChild<int64_t>) + 16 +
-                                  (size_t)child_pool_rows(sz, t) * ks_pool_stride(sz) * esize);
+    // matrix, sums, live list, column list and node of a child, then its pool
+    // rows; the few spare rows beyond 1/8 are not counted: a served query's
+    // admitted bytes rest on this sum
+    const size_t b = 2 * nodes * (c64((size_t)t * t * esize) + 2 * c64((size_t)t * esize) + c64((size_t)sz * 4) +
+                                  c64((size_t)t * 4) + 104 +
+                                  (size_t)(sz - t) * ks_pool_stride(sz) * esize * 9 / 8);
     best[depth & 1] = std::max(best[depth & 1], b);
   }
   return best[0] + best[1] + 8192;
