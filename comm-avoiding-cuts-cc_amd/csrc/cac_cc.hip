@@ -13,18 +13,20 @@
 //   1. init      parent[v] = v                                    (4n bytes written)
 //   2. runs      hook the first and the last edge of every run of equal u in
 //                the edge list (the whole list is read, ~8% of it hooked on a
-//                u-sorted R-MAT list); this builds the giant component
+//                u-sorted R-MAT list); of a list in no order, the first one
+//                and a half edges a vertex: this builds the giant component
 //   3. settle    pointer-jump every vertex to its root
-//   4. mode      the most frequent root among 4096 sampled vertices: the giant
+//   4. mode      the most frequent root among 4096 sampled edges: the giant
 //   5. bitmap    bit v = (root(v) == giant root); n/8 bytes, small enough to
 //                stay resident in each XCD's L2
-//   6. hook      stream every edge; skip it when both endpoint bits are set
-//                (already connected), else union-find link.  The random
-//                lookups of almost every edge hit the L2-resident bitmap
-//                instead of the n*4-byte parent array
+//   6. hook      stream every edge; skip it when both endpoints lie in the giant
+//                (already connected), else union-find link.  A coarse map, one
+//                bit per group of vertices, sits in LDS and drops almost every
+//                edge; the rest are looked up in the bitmap, in L2
 //   7. compress  parent[v] = root(v), count roots               (8n bytes)
 //   8. (rank)    dense rank of roots by id, relabel              (scan)
-// Steps 2-5 run when m is large; small inputs go straight to a plain hook.
+// Steps 2-3 run when m is large and steps 4-5 when the list is also long for its
+// vertices; the others hook every edge whose endpoints' parents differ.
 // Any edge order is correct; the run sampling pays off when equal u are
 // adjacent (the order of the edge-list files and of the R-MAT generator).
 #include <algorithm>
@@ -46,7 +48,7 @@ constexpr int kTileEdges = 64 * kEdgesPerThread;     // edges per wavefront tile
 constexpr uint64_t kSampleMinEdges = 1ull << 18;     // below this: plain hook only
 constexpr int kModeSamples = 4096;
 constexpr int kModeTable = 8192;                     // open-addressing table, > kModeSamples
-constexpr size_t kCcTmpHead = 64;                    // u32 words: [0] component count, [1] giant root
+constexpr size_t kCcTmpHead = 64;                    // u32 words: [0] component count, [1] giant root, [2] its samples
 
 // Parent-array loads inside the union-find kernels are relaxed atomics at
 // workgroup scope: plain cached loads.  A stale parent (an older state of the
@@ -150,12 +152,49 @@ __device__ inline uint64_t ld_edge_nt(const cac_uedge* e, uint64_t i) {
 // Wave-tiled: wavefront w handles tiles w, w + W, ...; edge k * 64 + lane of a
 // tile sits in register k of that lane, so every load instruction is coalesced
 // and the neighbours of an edge (for the run test) are one lane away.
-__global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restrict__ edges, uint64_t m,
-                                                      uint32_t* par) {
+//
+// kQueue: the edges at run ends (7.5% of a u-sorted R-MAT list) are queued in LDS
+// and linked 64 at a time; linked where they are found, five lanes of a wavefront
+// wait out a chain of parent loads eight times per tile.  R-MAT 2^24 / 2^28: 1.37
+// -> 1.20 ms, the rate of the links' memory operations.  Smaller forests are the
+// other way round (2^18 / 2^22: 0.12 ms linked in place, 0.30 queued): more links
+// in flight on few vertices meet each other's roots.
+//
+// A wavefront whose first tile holds many descents of u takes the list to be in no
+// order.  Nearly every edge is then a run end, and any part of the list is as
+// good a sample as the whole: about one and a half links per vertex (the first
+// `sample_tiles` tiles) make a giant component that holds most vertices, and the
+// hook pass drops an edge inside it for far less than a link costs.  Those tiles
+// go to the first random_waves(n) wavefronts only: random links collide, the more
+// the smaller the forest (whole call with 512 / 1024 / 2048 wavefronts: n 2^18,
+// m 2^20 273 / 464 / 433 us, n 2^20, m 2^24 421 / 439 / 722 us, n 2^22, m 10M
+// 1137 / 1005 / 1532 us, n 10M, m 24M 2361 / 1661 / 1610 us; with every wavefront
+// the device holds the last took 4.2 ms).  Below 3/4 edges a vertex there is no
+// giant component to build and few links meet: all wavefronts (n 2^22, m 2.5M:
+// 457 us, with 2048 of them 512).  Any choice of tiles gives the same labels.
+inline uint32_t random_waves(uint32_t n) { return std::min(2048u, std::max(512u, n / 4096)); }
+constexpr uint32_t kQueueMinN = 1u << 22;  // queued above: the forest is past an XCD's 4 MiB L2
+
+template <bool kQueue>
+__global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restrict__ edges, uint64_t m, uint32_t* par,
+                                                      uint64_t sample_tiles, uint32_t random_waves) {
+  __shared__ uint64_t queue_lds[kCcBlock / 64][128];  // fewer than 64 left over and one step's 64
+  uint64_t* queue = queue_lds[threadIdx.x >> 6];
+  uint32_t queued = 0;  // uniform in the wavefront
   const int lane = threadIdx.x & 63;
-  const uint64_t waves = (uint64_t)gridDim.x * (kCcBlock / 64);
-  const uint64_t tiles = (m + kTileEdges - 1) / kTileEdges;
-  for (uint64_t t = (uint64_t)blockIdx.x * (kCcBlock / 64) + (threadIdx.x >> 6); t < tiles; t += waves) {
+  const uint64_t first = (uint64_t)blockIdx.x * (kCcBlock / 64) + (threadIdx.x >> 6);
+  uint64_t waves = (uint64_t)gridDim.x * (kCcBlock / 64);
+  uint64_t tiles = (m + kTileEdges - 1) / kTileEdges;
+  auto link = [&](uint32_t count) {  // the first `count` (at most 64) queued edges
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint64_t e = queue[lane];
+    const uint64_t up = (uint32_t)lane + 64 < queued ? queue[lane + 64] : 0;  // the rest moves up
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    queue[lane] = up;
+    queued -= count;
+    if ((uint32_t)lane < count) uf_link(par, (uint32_t)e, (uint32_t)(e >> 32));
+  };
+  for (uint64_t t = first; t < tiles; t += waves) {
     const uint64_t base = t * kTileEdges;
     uint32_t u[kEdgesPerThread], v[kEdgesPerThread];
 #pragma unroll
@@ -167,6 +206,19 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restric
     }
     const uint32_t before = base > 0 ? edges[base - 1].u : ~0u;
     const uint32_t after = base + kTileEdges < m ? edges[base + kTileEdges].u : ~0u;
+    if (t == first) {
+      uint32_t descents = 0;
+#pragma unroll
+      for (int k = 0; k < kEdgesPerThread; ++k) {
+        const uint32_t up = __shfl_up(u[k], 1, 64);
+        descents += (uint32_t)__popcll(__ballot(lane > 0 && u[k] < up));
+      }
+      if (sample_tiles && descents >= kTileEdges / 8) {  // no order
+        tiles = sample_tiles < tiles ? sample_tiles : tiles;
+        if (first >= random_waves || first >= tiles) return;
+        if (waves > random_waves) waves = random_waves;
+      }
+    }
 #pragma unroll
     for (int k = 0; k < kEdgesPerThread; ++k) {
       uint32_t up = __shfl_up(u[k], 1, 64);
@@ -176,9 +228,20 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restric
       if (lane == 0) up = k > 0 ? prev_last : before;
       if (lane == 63) dn = k + 1 < kEdgesPerThread ? next_first : after;
       const bool valid = base + (uint64_t)k * 64 + lane < m;
-      if (valid && u[k] != v[k] && (u[k] != up || u[k] != dn)) uf_link(par, u[k], v[k]);
+      const bool end = valid && u[k] != v[k] && (u[k] != up || u[k] != dn);
+      if constexpr (kQueue) {
+        const uint64_t mask = __ballot(end);
+        if (mask) {
+          if (end) queue[queued + (uint32_t)__popcll(mask & ((1ull << lane) - 1))] = ((uint64_t)v[k] << 32) | u[k];
+          queued += (uint32_t)__popcll(mask);
+          if (queued >= 64) link(64);
+        }
+      } else if (end) {
+        uf_link(par, u[k], v[k]);
+      }
     }
   }
+  if (kQueue && queued) link(queued);
 }
 
 // Pointer jumping over [0, n): every vertex is re-pointed at its root; returns
@@ -200,11 +263,14 @@ __device__ inline uint32_t jump_pass(uint32_t* par, uint32_t n) {
 
 __global__ void __launch_bounds__(kCcBlock) k_cc_settle(uint32_t* par, uint32_t n) { (void)jump_pass(par, n); }
 
-// Most frequent root among kModeSamples vertices spread over [0, n), each
-// sample climbing to its root (one hop on a settled forest).  Only a
-// performance choice: any root gives correct labels.
-__global__ void __launch_bounds__(1024) k_cc_mode(const uint32_t* __restrict__ par, uint32_t n,
-                                                  uint32_t* __restrict__ out_root) {
+// Most frequent root among kModeSamples vertices, each sample climbing to its
+// root (one hop on a settled forest): of edges spread over the list (their first
+// endpoints), or without a list of vertices spread over [0, n).  out[0] = the
+// root, out[1] = its samples (with a list only).  Only a performance choice: any root gives correct
+// labels.
+__global__ void __launch_bounds__(1024) k_cc_mode(const cac_uedge* __restrict__ edges, uint64_t m,
+                                                  const uint32_t* __restrict__ par, uint32_t n,
+                                                  uint32_t* __restrict__ out) {
   __shared__ uint32_t key[kModeTable], cnt[kModeTable];
   __shared__ uint64_t best_w[1024 / 64];
   for (int i = threadIdx.x; i < kModeTable; i += 1024) {
@@ -217,7 +283,8 @@ __global__ void __launch_bounds__(1024) k_cc_mode(const uint32_t* __restrict__ p
     h ^= h >> 15;
     h *= 0x85EBCA6Bu;
     h ^= h >> 13;
-    uint32_t r = (uint32_t)(((uint64_t)h * n) >> 32), up = ld_par_fresh(par, r);
+    uint32_t r = edges ? edges[__umul64hi((uint64_t)h << 32, m)].u : (uint32_t)(((uint64_t)h * n) >> 32);
+    uint32_t up = ld_par_fresh(par, r);
     while (up < r) {
       r = up;
       up = ld_par_fresh(par, r);
@@ -241,7 +308,8 @@ __global__ void __launch_bounds__(1024) k_cc_mode(const uint32_t* __restrict__ p
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 1024 / 64; ++w) best = max(best, best_w[w]);
-    out_root[0] = ~(uint32_t)best;
+    out[0] = ~(uint32_t)best;
+    if (edges) out[1] = (uint32_t)(best >> 32);
   }
 }
 
@@ -259,15 +327,11 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_bitmap(const uint32_t* __restri
   }
 }
 
-__device__ inline bool bit_of(const uint32_t* bits, uint32_t x) { return (bits[x >> 5] >> (x & 31)) & 1u; }
 
 // Thread t of the grid owns edges t, t + T, t + 2T, ... (T = total threads) so
 // each load instruction is coalesced; kEdgesPerThread loads are issued before
-// any is consumed.  With a bitmap, an edge whose two endpoints are both in the
-// giant component is dropped before any parent lookup.
-template <bool kBitmap>
-__global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restrict__ edges, uint64_t m,
-                                                      uint32_t* par, const uint32_t* __restrict__ bits) {
+// any is consumed.
+__global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restrict__ edges, uint64_t m, uint32_t* par) {
   const uint64_t T = (uint64_t)gridDim.x * kCcBlock;
   uint64_t i0 = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x;
   for (; i0 < m; i0 += T * kEdgesPerThread) {
@@ -277,26 +341,219 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restric
       uint64_t i = i0 + (uint64_t)k * T;
       e[k] = i < m ? ld_edge_nt(edges, i) : 0ull;  // empty slot = loop (0, 0)
     }
-    bool live[kEdgesPerThread];
-#pragma unroll
-    for (int k = 0; k < kEdgesPerThread; ++k) {
-      const uint32_t a = (uint32_t)e[k], b = (uint32_t)(e[k] >> 32);
-      live[k] = a != b;
-      if (kBitmap) live[k] = live[k] && !(bit_of(bits, a) && bit_of(bits, b));
-    }
     // all parent lookups of the batch are in flight before any is consumed
     uint32_t pu[kEdgesPerThread], pv[kEdgesPerThread];
 #pragma unroll
     for (int k = 0; k < kEdgesPerThread; ++k) {
-      pu[k] = live[k] ? ld_par(par, (uint32_t)e[k]) : 0u;
-      pv[k] = live[k] ? ld_par(par, (uint32_t)(e[k] >> 32)) : 0u;
+      const bool live = (uint32_t)e[k] != (uint32_t)(e[k] >> 32);
+      pu[k] = live ? ld_par(par, (uint32_t)e[k]) : 0u;
+      pv[k] = live ? ld_par(par, (uint32_t)(e[k] >> 32)) : 0u;
     }
 #pragma unroll
     for (int k = 0; k < kEdgesPerThread; ++k) {
-      if (!live[k] || pu[k] == pv[k]) continue;
+      if (pu[k] == pv[k]) continue;
       uf_link_from(par, (uint32_t)e[k], pu[k], (uint32_t)(e[k] >> 32), pv[k]);
     }
   }
+}
+
+// Coarse map of the giant component, sized for a CU's LDS.  Up to kMapBits
+// vertices it is the vertex bitmap itself.  Beyond, it is two maps of kMapBits / 2
+// bits: bit g of the first = every vertex of [g 2^shift, (g + 1) 2^shift) is in the
+// component (a group that runs past n counts as not), bit j of the second = every
+// vertex congruent to j modulo kMapBits / 2 is.  A vertex with either bit set is
+// in the component.  Two groupings of 2 G vertices certify more than one of G:
+// on an R-MAT graph of 2^20 vertices with groups of 32, 5.8% of the edges keep an
+// endpoint that neither certifies, 8.8% with one map in groups of 16.
+constexpr uint32_t kMapBits = 1u << 20;
+constexpr uint32_t kHalfBits = kMapBits / 2, kHalfWords = kHalfBits / 32;
+inline uint32_t map_shift(uint32_t n) {  // of the first map; 0: the bitmap itself
+  if (n <= kMapBits) return 0;
+  uint32_t s = 1;
+  while ((((uint64_t)n + (1ull << s) - 1) >> s) > kHalfBits) ++s;
+  return s;
+}
+inline uint32_t map_words(uint32_t n) {  // whole 16-byte pieces
+  return n > kMapBits ? 2 * kHalfWords : (uint32_t)(((uint64_t)n + 127) / 128 * 4);
+}
+
+__global__ void __launch_bounds__(kCcBlock) k_cc_coarse(const uint32_t* __restrict__ bits, uint32_t n, uint32_t shift,
+                                                        uint32_t* __restrict__ map, uint32_t words) {
+  const uint32_t w = blockIdx.x * kCcBlock + threadIdx.x;
+  if (w >= words) return;
+  const uint32_t bit_words = (uint32_t)(((uint64_t)n + 31) / 32);
+  uint32_t out = 0;
+  if (shift == 0) {
+    out = w < bit_words ? bits[w] : 0u;
+  } else if (w >= kHalfWords) {
+    out = ~0u;
+    for (uint32_t i = w - kHalfWords; i < bit_words; i += kHalfWords) {
+      const uint32_t past = i + 1 == bit_words && n % 32 ? ~0u << (n % 32) : 0u;  // no vertices there
+      out &= bits[i] | past;
+    }
+  } else if (shift < 5) {  // 2^shift words of 32 / 2^shift groups each
+    const uint32_t per = 32u >> shift, full = (1u << (1u << shift)) - 1u;
+    for (uint32_t j = 0; j < (1u << shift); ++j) {
+      const uint64_t i = ((uint64_t)w << shift) + j;
+      const uint32_t x = i < bit_words ? bits[i] : 0u;
+      for (uint32_t g = 0; g < per; ++g)
+        if (((x >> (g << shift)) & full) == full) out |= 1u << (j * per + g);
+    }
+  } else {  // 2^(shift - 5) words per group
+    for (uint32_t g = 0; g < 32; ++g) {
+      bool all = true;
+      for (uint32_t j = 0; j < (1u << (shift - 5)) && all; ++j) {
+        const uint64_t i = (((uint64_t)w * 32 + g) << (shift - 5)) + j;
+        all = i < bit_words && bits[i] == ~0u;
+      }
+      if (all) out |= 1u << g;
+    }
+  }
+  map[w] = out;
+}
+
+// One workgroup per CU streams the edge list past the coarse map in LDS.  An edge
+// with both endpoints certified is dropped; the others are queued per wavefront
+// and, 64 at a time, their uncertified endpoints are looked up in the vertex
+// bitmap, in L2; those that leave the component are queued again and linked half
+// a wavefront or more at a time, so that a wavefront does not wait out a chain of
+// parent loads for one of its lanes.  Where the component holds the first
+// endpoint of fewer than kHookShare of the sampled edges, most edges would go
+// through both queues; they compare their endpoints' parents instead, all of a
+// step's in flight.  The bound is the read of the list and the
+// latency of the lookups.  Testing both endpoints of every edge
+// against the bitmap in L2 was bound by L2 requests: R-MAT 2^24 vertices, 2^28
+// edges, 1.71 ms; the list past the map alone takes 0.34 ms (6.4 TB/s), which
+// the lookups and links raise to 0.69 ms.  16-byte loads of two edges (the list is 8-byte
+// aligned).
+constexpr int kHookBlock = 1024;
+constexpr int kHookWaves = kHookBlock / 64;
+constexpr unsigned kHookGrid = 256;  // the CUs of one MI355X
+constexpr int kHookPairs = 4;        // 16-byte loads in flight per thread
+constexpr uint32_t kHookQueue = 128;   // edges per wavefront to look up: fewer than 64 left over and one step's 64
+constexpr uint32_t kHookOutside = 96;  // edges per wavefront to link: fewer than 32 left over and a lookup's 64
+
+constexpr uint32_t kHookShare = kModeSamples / 2;
+
+__global__ void __launch_bounds__(kHookBlock) k_cc_hook_giant(const cac_uedge* __restrict__ edges, uint64_t m,
+                                                              uint32_t* par, const uint32_t* __restrict__ mode,
+                                                              const uint32_t* __restrict__ bits,
+                                                              const uint32_t* __restrict__ map, uint32_t words,
+                                                              uint32_t shift) {
+  typedef uint32_t pair_t __attribute__((ext_vector_type(4), aligned(8)));
+  extern __shared__ __align__(16) uint32_t hook_lds[];  // the map
+  __shared__ uint64_t queue_lds[kHookWaves][kHookQueue];
+  __shared__ uint64_t outside_lds[kHookWaves][kHookOutside];
+  const uint64_t T = (uint64_t)gridDim.x * kHookBlock, pairs = m / 2;
+  const uint64_t tid = (uint64_t)blockIdx.x * kHookBlock + threadIdx.x;
+  const pair_t* src = reinterpret_cast<const pair_t*>(edges);
+  if (mode[1] < kHookShare) {  // uniform in the grid
+    for (uint64_t i0 = tid; i0 < pairs; i0 += T * kHookPairs) {
+      pair_t e[kHookPairs];
+      uint32_t p[kHookPairs][4];
+#pragma unroll
+      for (int k = 0; k < kHookPairs; ++k) {
+        const uint64_t i = i0 + (uint64_t)k * T;
+        e[k] = i < pairs ? __builtin_nontemporal_load(src + i) : pair_t{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int k = 0; k < kHookPairs; ++k) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[k][j] = ld_par(par, e[k][j]);
+      }
+#pragma unroll
+      for (int k = 0; k < kHookPairs; ++k) {
+#pragma unroll
+        for (int h = 0; h < 4; h += 2)
+          if (p[k][h] != p[k][h + 1]) uf_link_from(par, e[k][h], p[k][h], e[k][h + 1], p[k][h + 1]);
+      }
+    }
+    if (m % 2 && tid == 0) uf_link(par, edges[m - 1].u, edges[m - 1].v);  // the last edge of an odd list
+    return;
+  }
+  for (uint32_t w = threadIdx.x; w < words / 4; w += kHookBlock)
+    reinterpret_cast<uint4*>(hook_lds)[w] = reinterpret_cast<const uint4*>(map)[w];
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  uint64_t* queue = queue_lds[threadIdx.x >> 6];
+  uint64_t* outside = outside_lds[threadIdx.x >> 6];
+  uint32_t queued = 0, left = 0;  // entries of each, uniform in the wavefront
+  // where there is one map, the second is the first: the same bit read twice
+  const uint32_t* second = hook_lds + (shift ? kHalfWords : 0u);
+  const uint32_t low = shift ? kHalfBits - 1 : ~0u;
+  auto sure = [&](uint32_t v) {
+    return ((hook_lds[v >> (shift + 5)] >> ((v >> shift) & 31)) | (second[(v & low) >> 5] >> (v & 31))) & 1u;
+  };
+  auto link = [&]() {  // every edge of `outside`
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t i = lane; i < left; i += 64) uf_link(par, (uint32_t)outside[i], (uint32_t)(outside[i] >> 32));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    left = 0;
+  };
+  auto look_up = [&](uint32_t count) {  // the first `count` (at most 64) queued edges
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint64_t e = (uint32_t)lane < count ? queue[lane] : 0;  // (0, 0): a loop
+    const uint64_t up = (uint32_t)lane + 64 < queued ? queue[lane + 64] : 0;  // the rest moves up
+    const uint32_t a = (uint32_t)e, b = (uint32_t)(e >> 32);
+    const uint32_t wa = sure(a) ? ~0u : bits[a >> 5], wb = sure(b) ? ~0u : bits[b >> 5];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    queue[lane] = up;
+    queued -= count;
+    const bool out = a != b && !((wa >> (a & 31)) & (wb >> (b & 31)) & 1u);
+    const uint64_t mask = __ballot(out);
+    if (mask) {
+      if (out) outside[left + (uint32_t)__popcll(mask & ((1ull << lane) - 1))] = e;
+      left += (uint32_t)__popcll(mask);
+      if (left >= 32) link();
+    }
+  };
+  // called by the whole wavefront
+  auto add = [&](bool keep, uint32_t a, uint32_t b) {
+    const uint64_t mask = __ballot(keep);
+    if (mask) {
+      if (keep) queue[queued + (uint32_t)__popcll(mask & ((1ull << lane) - 1))] = ((uint64_t)b << 32) | a;
+      queued += (uint32_t)__popcll(mask);
+      if (queued >= 64) look_up(64);
+    }
+  };
+  const uint64_t wave0 = tid - (uint64_t)lane;  // whole wavefronts step together
+  pair_t next[kHookPairs];
+#pragma unroll
+  for (int k = 0; k < kHookPairs; ++k) {
+    const uint64_t i = tid + (uint64_t)k * T;
+    next[k] = i < pairs ? __builtin_nontemporal_load(src + i) : pair_t{0, 0, 0, 0};
+  }
+  for (uint64_t i0 = wave0; i0 < pairs; i0 += T * kHookPairs) {
+    pair_t e[kHookPairs];
+#pragma unroll
+    for (int k = 0; k < kHookPairs; ++k) e[k] = next[k];
+#pragma unroll
+    for (int k = 0; k < kHookPairs; ++k) {
+      const uint64_t i = i0 + lane + T * (kHookPairs + (uint64_t)k);
+      next[k] = i < pairs ? __builtin_nontemporal_load(src + i) : pair_t{0, 0, 0, 0};
+    }
+    // the map words of all the step's edges are read before any edge is queued
+    bool keep[2 * kHookPairs];
+#pragma unroll
+    for (int k = 0; k < kHookPairs; ++k) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t a = e[k][2 * h], b = e[k][2 * h + 1];
+        keep[2 * k + h] = a != b && !(sure(a) & sure(b));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kHookPairs; ++k) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) add(keep[2 * k + h], e[k][2 * h], e[k][2 * h + 1]);
+    }
+  }
+  if (m % 2 && wave0 == 0) {  // the last edge of an odd list
+    const cac_uedge x = edges[m - 1];
+    add(lane == 0 && x.u != x.v, x.u, x.v);
+  }
+  if (queued) look_up(queued);
+  if (left) link();
 }
 
 // Final pointer jumping; counts roots (components).
@@ -762,8 +1019,10 @@ __global__ void __launch_bounds__(kCcBlock) k_approx_init(uint32_t* par_all, uin
 
 }  // namespace
 
+// The vertex bitmap, then the coarse map.
+size_t cc_fine_words(uint32_t n) { return (((size_t)n + 63) / 64 * 2 + 63) & ~size_t(63); }
 size_t cc_bitmap_words(uint64_t m, uint32_t n) {
-  return m >= kSampleMinEdges ? (((size_t)n + 63) / 64 * 2 + 63) & ~size_t(63) : 0;
+  return m >= kSampleMinEdges ? cc_fine_words(n) + ((map_words(n) + 63) & ~size_t(63)) : 0;
 }
 size_t cc_rank_tmp_words(uint32_t n) { return ((size_t)(n + 63) & ~size_t(63)) + scan_tiles(n) + 64; }
 
@@ -771,6 +1030,18 @@ size_t cc_rank_tmp_words(uint32_t n) { return ((size_t)(n + 63) & ~size_t(63)) +
 // (label_mode == RANK).
 size_t cc_tmp_words(uint64_t m, uint32_t n, int label_mode) {
   return kCcTmpHead + cc_bitmap_words(m, n) + (label_mode == CAC_LABEL_RANK ? cc_rank_tmp_words(n) : 0);
+}
+
+// The hook pass's dynamic LDS exceeds the default limit: raise it once.
+static int hook_attr(cac_ctx* ctx) {
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute((const void*)k_cc_hook_giant, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(kMapBits / 8));
+  });
+  CAC_HIP(ctx, err);
+  return CAC_OK;
 }
 
 // Launch sequence shared by cac_cc and cac_cc_dev; d_tmp holds cc_tmp_words()
@@ -785,29 +1056,51 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
   prof_end(ctx, s);
   hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, d_counter, 1);
   const bool use_sample = m >= kSampleMinEdges;
+  // Below one and a half edges a vertex the first pass links every edge of an
+  // unordered list, or most of a short sorted one, and what is left is cheaper to
+  // link than to sort out by the component (star of 2^22: 79 us against 119;
+  // blocks of 1024 in 2^18 with m = 4n 152 against 198, but R-MAT 2^18 with
+  // m = 16n 1027 against 425, uniform 2^18 with m = 4n 483 against 430).
+  const bool giant = use_sample && m >= (uint64_t)n / 2 * 3;
   if (use_sample) {
     uint32_t* d_root = d_counter + 1;
     uint64_t* d_bits = (uint64_t*)(d_counter + kCcTmpHead);
     prof_begin(ctx, "cc_runs", s);
     unsigned gr = grid_for((m + kTileEdges - 1) / kTileEdges, kCcBlock / 64, 256 * 32);
-    hipLaunchKernelGGL(k_cc_runs, dim3(gr), dim3(kCcBlock), 0, s, d_edges, m, d_lab);
+    const uint64_t sample_tiles = m < (uint64_t)n / 4 * 3 ? 0 : ((uint64_t)n * 3 / 2 + kTileEdges - 1) / kTileEdges;
+    if (n > kQueueMinN)
+      hipLaunchKernelGGL(k_cc_runs<true>, dim3(gr), dim3(kCcBlock), 0, s, d_edges, m, d_lab, sample_tiles,
+                         random_waves(n));
+    else
+      hipLaunchKernelGGL(k_cc_runs<false>, dim3(gr), dim3(kCcBlock), 0, s, d_edges, m, d_lab, sample_tiles,
+                         random_waves(n));
     prof_end(ctx, s);
     prof_begin(ctx, "cc_settle", s);
     hipLaunchKernelGGL(k_cc_settle, dim3(grid_for(n, kCcBlock, cap)), dim3(kCcBlock), 0, s, d_lab, n);
     prof_end(ctx, s);
-    prof_begin(ctx, "cc_bitmap", s);
-    hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_lab, n, d_root);
-    hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, cap)), dim3(kCcBlock), 0, s,
-                       (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
-    prof_end(ctx, s);
+    if (giant) {
+      prof_begin(ctx, "cc_bitmap", s);
+      hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, d_edges, m, (const uint32_t*)d_lab, n, d_root);
+      hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, cap)), dim3(kCcBlock), 0, s,
+                         (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
+      uint32_t* d_map = reinterpret_cast<uint32_t*>(d_bits) + cc_fine_words(n);
+      const uint32_t words = map_words(n), shift = map_shift(n);
+      hipLaunchKernelGGL(k_cc_coarse, dim3((words + kCcBlock - 1) / kCcBlock), dim3(kCcBlock), 0, s,
+                         (const uint32_t*)d_bits, n, shift, d_map, words);
+      prof_end(ctx, s);
+      prof_begin(ctx, "cc_hook", s);
+      const int rc = hook_attr(ctx);
+      if (rc) return rc;
+      const unsigned g = grid_for((m + 2 * kHookPairs - 1) / (2 * kHookPairs), kHookBlock, kHookGrid);
+      hipLaunchKernelGGL(k_cc_hook_giant, dim3(g), dim3(kHookBlock), words * 4, s, d_edges, m, d_lab,
+                         (const uint32_t*)d_root, (const uint32_t*)d_bits, (const uint32_t*)d_map, words, shift);
+      prof_end(ctx, s);
+    }
+  }
+  if (m && !giant) {
     prof_begin(ctx, "cc_hook", s);
     unsigned g = grid_for((m + kEdgesPerThread - 1) / kEdgesPerThread, kCcBlock, 256 * 32);
-    hipLaunchKernelGGL(k_cc_hook<true>, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab, (const uint32_t*)d_bits);
-    prof_end(ctx, s);
-  } else if (m) {
-    prof_begin(ctx, "cc_hook", s);
-    unsigned g = grid_for((m + kEdgesPerThread - 1) / kEdgesPerThread, kCcBlock, 256 * 32);
-    hipLaunchKernelGGL(k_cc_hook<false>, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab, (const uint32_t*)nullptr);
+    hipLaunchKernelGGL(k_cc_hook, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab);
     prof_end(ctx, s);
   }
   prof_begin(ctx, "cc_compress", s);
@@ -878,7 +1171,8 @@ int cc_csr_launch(cac_ctx* ctx, const uint32_t* d_off, const uint32_t* d_cols, u
   }
   if (lo >= n) {  // no bulk range (n within the hub prefixes): a separate sampling launch
     prof_begin(ctx, "af_mode", s);
-    hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_lab, n, d_counter + 1);
+    hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, (const cac_uedge*)nullptr, 0, (const uint32_t*)d_lab, n,
+                       d_counter + 1);
     prof_end(ctx, s);
   }
   prof_begin(ctx, "af_final", s);
@@ -917,6 +1211,8 @@ constexpr uint32_t kStaticMaxN = CAC_CC_STATIC_MAX_N;
 constexpr size_t kStaticBitsWords = (size_t)kStaticMaxN / 64 * 2;  // one u64 per 64 vertices
 constexpr size_t kStaticPreWords = (size_t)kStaticMaxN / 64;       // one u32 per bitmap word
 constexpr size_t kStaticPartWords = ((size_t)kStaticMaxN / 64 + kScanTile - 1) / kScanTile + 64;
+// The coarse map follows a graph's bitmap, where the root prefix comes later.
+static_assert(kStaticPreWords >= kMapBits / 32 + 64 && kStaticBitsWords % 64 == 0, "the coarse map fits");
 constexpr size_t kStaticWords = kCcTmpHead + kStaticBitsWords + kStaticPreWords + kStaticPartWords;
 static_assert(kStaticMaxN % 64 == 0, "whole bitmap words");
 
@@ -966,6 +1262,8 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_rank_bits(uint32_t* lab, uint32
 int cc_static_init(cac_ctx* ctx) {
   if (ctx->device < 0 || ctx->device >= kStaticMaxDevices)
     return fail(ctx, CAC_EDEVICE, "static connected-components scratch: device index beyond 63");
+  const int rc = hook_attr(ctx);
+  if (rc) return rc;
   std::lock_guard<std::mutex> lock(g_static_mu);
   if (g_static_ptr[ctx->device]) return CAC_OK;
   void* p = nullptr;
