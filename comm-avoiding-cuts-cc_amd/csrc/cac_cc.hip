@@ -601,6 +601,144 @@ __global__ void __launch_bounds__(kCcBlock) k_check_ids(const cac_uedge* e, uint
   if (b) atomicOr(bad, 1u);
 }
 
+// ---- small graphs in one workgroup ---------------------------------------------
+// At most kSmallN vertices and kSmallM edges: the id check, the unions, the
+// labels, the count and the ranks in one launch, with the forest in LDS (the
+// largest that fits beside the roots' bits).  As the general sequence a call was
+// ten launches and three copies, and the unions alone took 55 us for 3000 edges,
+// each a chain of accesses past the L2.  edges and labels may be pinned host
+// memory: a call on host arrays then copies nothing through the device.  The
+// bound is one CU's LDS atomics and the launch and its wait (about 16 us).
+// Random lists with ranks, from host arrays / device buffers, before -> now:
+// 300 vertices and 200 edges 103 / 67 -> 22 / 18 us, 3000 and 6000 135 / 89 ->
+// 31 / 25, 32000 and 32000 183 / 107 -> 79 / 61; a path of 32000 195 / 120 ->
+// 132 / 110.  out[0] = components, out[1] = 1 when an id is out of range (labels
+// are then not written).
+constexpr uint32_t kSmallN = 1u << 15;
+constexpr uint64_t kSmallM = 1u << 15;
+constexpr int kSmallBlock = 1024;
+inline size_t small_lds(uint32_t n) {  // forest, root bits and their prefix
+  const size_t words = ((size_t)n + 63) / 64;
+  return words * (64 * 4 + 8 + 4);
+}
+
+__device__ inline uint32_t sm_find(uint32_t* par, uint32_t x) {
+  uint32_t p = __hip_atomic_load(par + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  while (p != x) {
+    const uint32_t g = __hip_atomic_load(par + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (g != p) __hip_atomic_store(par + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    x = p;
+    p = g;
+  }
+  return x;
+}
+
+__global__ void __launch_bounds__(kSmallBlock) k_cc_small(const cac_uedge* edges, uint32_t m, uint32_t n,
+                                                          int label_mode, uint32_t* labels, uint32_t* out) {
+  extern __shared__ __align__(16) uint64_t small_dyn[];
+  __shared__ uint32_t bad, wtot[kSmallBlock / 64];
+  const uint32_t words = (n + 63) / 64;
+  uint64_t* roots = small_dyn;                                  // [words]
+  uint32_t* before = reinterpret_cast<uint32_t*>(roots + words);  // [words] roots in the words before
+  uint32_t* par = before + words;                               // [64 words]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) bad = 0;
+  for (uint32_t v = threadIdx.x; v < n; v += kSmallBlock) par[v] = v;
+  __syncthreads();
+  // A wavefront takes a stretch of the list and a lane four edges in a row: on a
+  // list in the order of a path a lane's edges then flatten its part, and the
+  // wavefront's parts meet in a chain of 64.  Edges taken a workgroup's width
+  // apart left chains that each step climbed (a path of 32000 edges 0.9 ms).
+  typedef uint32_t pair_t __attribute__((ext_vector_type(4), aligned(8)));
+  const pair_t* src = reinterpret_cast<const pair_t*>(edges);
+  const uint32_t stretch = (m + kSmallBlock / 64 * 256 - 1) / (kSmallBlock / 64 * 256) * 256;
+  const uint32_t end = min(m, (wave + 1) * stretch);
+  for (uint32_t i0 = wave * stretch + lane * 4; i0 < end; i0 += 256) {
+    cac_uedge e[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k += 2) {
+      const uint32_t i = i0 + k;
+      const pair_t x = i + 1 < end ? src[i / 2] : pair_t{0, 0, 0, 0};
+      e[k] = {x[0], x[1]};
+      e[k + 1] = {x[2], x[3]};
+      if (i + 1 == end) e[k] = edges[i];  // the last edge of an odd list
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (e[k].u >= n || e[k].v >= n) {
+        bad = 1;
+        continue;
+      }
+      uint32_t ra = sm_find(par, e[k].u), rb = sm_find(par, e[k].v);
+      while (ra != rb) {
+        const uint32_t lo = min(ra, rb), hi = max(ra, rb);
+        const uint32_t old = atomicCAS(par + hi, hi, lo);
+        if (old == hi) break;
+        ra = sm_find(par, old);
+        rb = sm_find(par, lo);
+      }
+    }
+  }
+  __syncthreads();
+  if (bad) {
+    if (threadIdx.x == 0) out[1] = 1;
+    return;
+  }
+  // Every vertex is pointed at its root: up to four hops a round, so the unions'
+  // chains (as long as a path given in order) shrink to a fifth or less each
+  // round.  A round stores only a vertex's own parent: a path-splitting store in
+  // flight could put an older ancestor back over a root.
+  for (bool more = true; more;) {
+    more = false;
+    for (uint32_t v = threadIdx.x; v < n; v += kSmallBlock) {
+      uint32_t p = ld_par(par, v);
+      if (p == v) continue;
+      const uint32_t from = p;
+      uint32_t up = ld_par(par, p);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        p = up;
+        up = ld_par(par, p);
+      }
+      more |= up != p;
+      if (p != from) __hip_atomic_store(par + v, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    more = __syncthreads_or(more);
+  }
+  for (uint32_t w = wave; w < words; w += kSmallBlock / 64) {
+    const uint32_t v = w * 64 + lane;
+    const uint64_t mask = __ballot(v < n && par[v] == v);
+    if (lane == 0) roots[w] = mask;
+  }
+  __syncthreads();
+  static_assert(kSmallN / 64 <= kSmallBlock, "one thread per word of root bits");
+  const uint32_t c = threadIdx.x < words ? (uint32_t)__popcll(roots[threadIdx.x]) : 0u;
+  uint32_t inc = c;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += y;
+  }
+  if (lane == 63) wtot[wave] = inc;
+  __syncthreads();
+  uint32_t off = 0, total = 0;
+  for (int w = 0; w < kSmallBlock / 64; ++w) {
+    if (w < wave) off += wtot[w];
+    total += wtot[w];
+  }
+  if (threadIdx.x < words) before[threadIdx.x] = off + inc - c;
+  __syncthreads();
+  for (uint32_t v = threadIdx.x; v < n; v += kSmallBlock) {
+    const uint32_t r = par[v];
+    labels[v] = label_mode == CAC_LABEL_RANK
+                    ? before[r >> 6] + (uint32_t)__popcll(roots[r >> 6] & ((1ull << (r & 63)) - 1))
+                    : r;
+  }
+  if (threadIdx.x == 0) {
+    out[0] = total;
+    out[1] = 0;
+  }
+}
+
 // ---- connected components on a symmetric CSR (Afforest) ---------------------
 // Sutton, Ben-Nun, Barak, "Optimizing Parallel Graph Connectivity Computation via
 // Subgraph Sampling" (IPDPS 2018): link a sample of edges, find the most frequent
@@ -1044,6 +1182,31 @@ static int hook_attr(cac_ctx* ctx) {
   return CAC_OK;
 }
 
+inline bool cc_is_small(uint64_t m, uint32_t n) { return n > 0 && n <= kSmallN && m <= kSmallM; }
+
+// One launch of the small form, waited for; the count and the id flag come back
+// through the context's pinned buffer.
+int cc_small(cac_ctx* ctx, const cac_uedge* edges, uint64_t m, uint32_t n, int label_mode, uint32_t* labels,
+             uint32_t* ncomp_out, hipStream_t s) {
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute((const void*)k_cc_small, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)small_lds(kSmallN));
+  });
+  CAC_HIP(ctx, err);
+  uint32_t* out = (uint32_t*)ctx->pinned;
+  prof_begin(ctx, "cc_small", s);
+  hipLaunchKernelGGL(k_cc_small, dim3(1), dim3(kSmallBlock), small_lds(n), s, edges, (uint32_t)m, n, label_mode,
+                     labels, out);
+  prof_end(ctx, s);
+  CAC_LAUNCH_CHECK(ctx, "cc kernel");
+  CAC_HIP(ctx, hipStreamSynchronize(s));
+  if (out[1]) return fail(ctx, CAC_EINVAL, "edge endpoint >= n");
+  *ncomp_out = out[0];
+  return CAC_OK;
+}
+
 // Launch sequence shared by cac_cc and cac_cc_dev; d_tmp holds cc_tmp_words()
 // u32 words, 256-byte aligned.  The component count lands in d_tmp[0].
 int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, int label_mode, uint32_t* d_lab,
@@ -1286,6 +1449,7 @@ int cac_cc_dev(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, i
   if (label_mode != CAC_LABEL_MIN_ID && label_mode != CAC_LABEL_RANK)
     return cac::fail(ctx, CAC_EINVAL, "label_mode must be CAC_LABEL_MIN_ID or CAC_LABEL_RANK");
   hipStream_t s = cac::pick_stream(ctx, stream);
+  if (cac::cc_is_small(m, n)) return cac::cc_small(ctx, d_edges, m, n, label_mode, d_labels, ncomp_out, s);
   size_t words = cac::cc_tmp_words(m, n, label_mode);
   void* base = nullptr;
   rc = cac::scratch_reserve(ctx, words * 4, &base);
@@ -1351,6 +1515,17 @@ int cac_cc(cac_ctx* ctx, const cac_uedge* edges, uint64_t m, uint32_t n, int lab
   if (label_mode != CAC_LABEL_MIN_ID && label_mode != CAC_LABEL_RANK)
     return cac::fail(ctx, CAC_EINVAL, "label_mode must be CAC_LABEL_MIN_ID or CAC_LABEL_RANK");
   hipStream_t s = ctx->stream;
+  if (cac::cc_is_small(m, n)) {  // at most 384 KiB of pinned staging, read and written by the kernel
+    void* stage = nullptr;
+    rc = cac::stage_reserve(ctx, m * sizeof(cac_uedge) + (size_t)n * 4, &stage);
+    if (rc) return rc;
+    cac_uedge* e = (cac_uedge*)stage;
+    uint32_t* labels = (uint32_t*)(e + m);
+    if (m) std::memcpy(e, edges, m * sizeof(cac_uedge));
+    rc = cac::cc_small(ctx, e, m, n, label_mode, labels, ncomp_out, s);
+    if (rc == CAC_OK) std::memcpy(labels_out, labels, (size_t)n * 4);
+    return rc;
+  }
   size_t e_bytes = cac::carve_size(m * sizeof(cac_uedge));
   size_t l_bytes = cac::carve_size((size_t)n * 4);
   size_t t_words = cac::cc_tmp_words(m, n, label_mode);

@@ -47,6 +47,19 @@ int scratch_reserve(cac_ctx* ctx, size_t bytes, void** base) {
   return CAC_OK;
 }
 
+int stage_reserve(cac_ctx* ctx, size_t bytes, void** base) {
+  if (bytes > ctx->stage_bytes) {
+    if (ctx->stage) CAC_HIP(ctx, hipHostFree(ctx->stage));
+    ctx->stage = nullptr;
+    ctx->stage_bytes = 0;
+    const size_t want = std::max<size_t>(2 * bytes, (size_t)1 << 16);
+    CAC_HIP(ctx, hipHostMalloc(&ctx->stage, want, hipHostMallocDefault));
+    ctx->stage_bytes = want;
+  }
+  *base = ctx->stage;
+  return CAC_OK;
+}
+
 static hipEvent_t take_event(cac_ctx* ctx) {
   if (!ctx->event_pool.empty()) {
     hipEvent_t e = ctx->event_pool.back();
@@ -189,6 +202,7 @@ int cac_ctx_destroy(cac_ctx* ctx) {
   if (ctx->lt_buf) (void)hipFree(ctx->lt_buf);
   if (ctx->serve_buf) (void)hipFree(ctx->serve_buf);
   if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return CAC_OK;

@@ -22,6 +22,10 @@ struct cac_ctx {
   size_t scratch_bytes = 0;
   // Small pinned host buffer for scalar results.
   void* pinned = nullptr;
+  // Grow-only pinned staging of small host inputs and outputs that a kernel
+  // reads and writes in place (at most 1 MiB).
+  void* stage = nullptr;
+  size_t stage_bytes = 0;
   std::string last_error;
   bool profiling = false;
   std::vector<cac_prof_rec> prof;
@@ -102,6 +106,9 @@ int scratch_reserve(cac_ctx* ctx, size_t bytes, void** base);
 // If the allocation fails, every grow-only buffer of the context that is not
 // pinned is released and the allocation is tried once more.
 int grow_buffer(cac_ctx* ctx, void** buf, size_t* cap, size_t bytes);
+
+// Pinned staging of at least `bytes` (the caller keeps it at most 1 MiB).
+int stage_reserve(cac_ctx* ctx, size_t bytes, void** base);
 
 // Ids of the context's grow-only buffers, for pinning.
 enum : int { kBufKs0 = 0, kBufKs1, kBufKsRetry, kBufSmp, kBufLt, kBufSpDense, kBufSpTmp, kBufServe, kBufSpDepth = 16 };
