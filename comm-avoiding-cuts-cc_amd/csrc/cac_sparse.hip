@@ -42,6 +42,7 @@ constexpr uint32_t kSpSort = 1024;  // LDS sort size: pivot samples, final candi
 constexpr int kSpRows = 4;          // a compaction tile is kSpRows x kSpBlock elements, row after row
 constexpr uint64_t kSpTile = (uint64_t)kSpRows * kSpBlock;  // edges per output tile
 constexpr uint32_t kSparseDenseMax = 2048;
+constexpr uint32_t kSpLdsN = 18000;  // forests in LDS up to this: 8 n bytes beside 13 KiB
 constexpr unsigned long long kSpDisconnected = ~0ull;
 
 }  // namespace
@@ -89,11 +90,14 @@ struct SpChild {
 
 // Root with path halving.  Links always point to smaller ids, so even a stale
 // view of the forest ends at a root.
+__device__ inline uint32_t sp_load(const uint32_t* par, uint32_t x) {
+  return __hip_atomic_load(par + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 __device__ inline uint32_t sp_root(uint32_t* par, uint32_t x) {
-  uint32_t p = par[x];
+  uint32_t p = sp_load(par, x);
   while (p != x) {
-    const uint32_t g = par[p];
-    if (g != p) par[x] = g;
+    const uint32_t g = sp_load(par, p);
+    if (g != p) __hip_atomic_store(par + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     x = p;
     p = g;
   }
@@ -189,25 +193,33 @@ __device__ inline void sp_tile_ranks(const bool (&keep)[kSpRows], uint32_t (&ran
   __syncthreads();  // the next tile rewrites wcnt
 }
 
-// Bitonic sort of kSpSort (key, idx) pairs in LDS, ascending by key then idx.
-__device__ inline void sp_sort(uint64_t* key, uint32_t* idx) {
+// Bitonic sort of one (key, idx) pair per thread, ascending by key then idx.
+// Partners in the same wavefront exchange by lane permutes; the ten exchanges
+// across wavefronts go through LDS (all 55 through it cost a barrier each).
+static_assert(kSpSort == kSpBlock, "one pair per thread");
+__device__ inline void sp_sort(uint64_t& key, uint32_t& idx, uint64_t* lkey, uint32_t* lidx) {
   const uint32_t i = threadIdx.x;
   for (uint32_t k = 2; k <= kSpSort; k <<= 1) {
     for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      const uint32_t p = i ^ j;
-      if (p > i) {
-        const uint64_t ka = key[i], kb = key[p];
-        const uint32_t ia = idx[i], ib = idx[p];
-        const bool greater = ka > kb || (ka == kb && ia > ib);
-        const bool up = (i & k) == 0;
-        if (greater == up) {
-          key[i] = kb;
-          key[p] = ka;
-          idx[i] = ib;
-          idx[p] = ia;
-        }
+      uint64_t ok;
+      uint32_t oi;
+      if (j >= 64) {
+        lkey[i] = key;
+        lidx[i] = idx;
+        __syncthreads();
+        ok = lkey[i ^ j];
+        oi = lidx[i ^ j];
+        __syncthreads();
+      } else {
+        ok = (uint64_t)__shfl_xor((unsigned long long)key, (int)j, 64);
+        oi = __shfl_xor(idx, (int)j, 64);
       }
-      __syncthreads();
+      const bool greater = key > ok || (key == ok && idx > oi);
+      const bool want_less = ((i & j) == 0) == ((i & k) == 0);
+      if (greater == want_less) {
+        key = ok;
+        idx = oi;
+      }
     }
   }
 }
@@ -253,36 +265,71 @@ __device__ uint64_t sp_filter(const SpChild& c, const uint32_t* src, uint64_t ns
   return base;
 }
 
+// The forests of a child: the committed one and the trial one (the identity
+// between probes), in LDS or in the child's scratch.
+template <bool kLds>
+struct SpForest {
+  uint32_t* com;
+  uint32_t* tri;
+  static __device__ void sync() {
+    if constexpr (kLds) __syncthreads();
+    else block_sync_global();
+  }
+};
+
 // Components removed by uniting, on top of the committed forest, the first p
-// candidates.  The trial forest is restored to the identity afterwards: every
-// entry a probe writes is the committed root of an endpoint of one of its
-// edges, and those are reset.
-__device__ uint32_t sp_probe(const SpChild& c, const uint32_t* list, uint64_t p, uint64_t* red) {
+// candidates.  The trial forest is restored to the identity afterwards; in
+// scratch only the entries the probe wrote: each is the committed root of an
+// endpoint of one of its edges.
+template <bool kLds>
+__device__ uint32_t sp_probe(const SpChild& c, const SpForest<kLds>& F, const uint32_t* list, uint64_t p,
+                             uint64_t* red) {
   uint64_t merged = 0;
   for (uint64_t pos = threadIdx.x; pos < p; pos += kSpBlock) {
     const cac_edge x = c.edges[sp_at(list, pos)];
-    const uint32_t a = sp_root(c.parc, x.u), b = sp_root(c.parc, x.v);
-    if (a != b && sp_union(c.part, a, b)) ++merged;
+    const uint32_t a = sp_root(F.com, x.u), b = sp_root(F.com, x.v);
+    if (a != b && sp_union(F.tri, a, b)) ++merged;
   }
-  block_sync_global();
-  for (uint64_t pos = threadIdx.x; pos < p; pos += kSpBlock) {
-    const cac_edge x = c.edges[sp_at(list, pos)];
-    const uint32_t a = sp_root(c.parc, x.u), b = sp_root(c.parc, x.v);
-    c.part[a] = a;
-    c.part[b] = b;
+  F.sync();
+  if constexpr (kLds) {
+    for (uint32_t v = threadIdx.x; v < c.n; v += kSpBlock) F.tri[v] = v;
+  } else {
+    for (uint64_t pos = threadIdx.x; pos < p; pos += kSpBlock) {
+      const cac_edge x = c.edges[sp_at(list, pos)];
+      const uint32_t a = sp_root(F.com, x.u), b = sp_root(F.com, x.v);
+      F.tri[a] = a;
+      F.tri[b] = b;
+    }
   }
   const uint64_t total = sp_sum(merged, red);
-  block_sync_global();
+  F.sync();
+  return (uint32_t)total;
+}
+
+// The same for the first p of at most one candidate per thread, whose edge joins
+// the committed roots a and b.
+template <bool kLds>
+__device__ uint32_t sp_probe_own(const SpForest<kLds>& F, uint32_t a, uint32_t b, uint64_t p, uint64_t* red) {
+  const bool mine = threadIdx.x < p && a != b;
+  const uint64_t merged = mine && sp_union(F.tri, a, b) ? 1 : 0;
+  F.sync();
+  if (mine) {
+    F.tri[a] = a;
+    F.tri[b] = b;
+  }
+  const uint64_t total = sp_sum(merged, red);
+  F.sync();
   return (uint32_t)total;
 }
 
 // Unites the first p candidates into the committed forest.
-__device__ void sp_commit(const SpChild& c, const uint32_t* list, uint64_t p) {
+template <bool kLds>
+__device__ void sp_commit(const SpChild& c, const SpForest<kLds>& F, const uint32_t* list, uint64_t p) {
   for (uint64_t pos = threadIdx.x; pos < p; pos += kSpBlock) {
     const cac_edge x = c.edges[sp_at(list, pos)];
-    sp_union(c.parc, x.u, x.v);
+    sp_union(F.com, x.u, x.v);
   }
-  block_sync_global();
+  F.sync();
 }
 
 struct KeepBelow {  // key <= tau
@@ -325,23 +372,36 @@ __global__ void __launch_bounds__(256) k_sp_keys(const SpChild* __restrict__ chi
   }
 }
 
+// One workgroup per child: chains of probes, each a union-find over the prefix it
+// tests, with a barrier between its steps.  kLds: both forests in LDS (8 n bytes;
+// two workgroups share a CU up to n = 8600).  In scratch every hop is a trip to
+// the L2 and every barrier an L1 invalidation, and the last 1024 candidates were
+// looked up again by each probe: 9924 children of about 2100 vertices and 27000
+// edges took 39.4 ms, and the whole of 48000 vertices with 16 edges each 124 of
+// 298 ms; now 4.1 ms, and 27 of 206.  The larger nodes are few (104 children of
+// 24000 vertices take 1.8 ms) and keep their forests in scratch.
+template <bool kLds>
 __global__ void __launch_bounds__(kSpBlock, 8) k_sparse_contract(const SpChild* __restrict__ children,
                                                               int64_t* __restrict__ results) {
+  extern __shared__ __align__(16) uint32_t sp_forest[];
   __shared__ uint64_t red[kSpWaves];
   __shared__ uint32_t wcnt[kSpRows * kSpWaves + 1];
   __shared__ uint64_t skey[kSpSort];
   __shared__ uint32_t sidx[kSpSort];
   const SpChild c = children[blockIdx.x];
   const uint32_t tid = threadIdx.x;
+  SpForest<kLds> F;
+  if constexpr (kLds) F = {sp_forest, sp_forest + c.n};
+  else F = {c.parc, c.part};
 
   // 1. identity forests; the race keys and their range come from k_sp_keys
   for (uint32_t v = tid; v < c.n; v += kSpBlock) {
-    c.parc[v] = v;
-    c.part[v] = v;
+    F.com[v] = v;
+    F.tri[v] = v;
   }
   uint64_t kmin = __hip_atomic_load(&c.kmm[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   uint64_t kmax = __hip_atomic_load(&c.kmm[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  block_sync_global();
+  F.sync();
 
   if (c.n > c.tgt) {  // else nothing is contracted
     // 2. narrowing: the committed forest holds the edges with key <= lo, the
@@ -353,10 +413,11 @@ __global__ void __launch_bounds__(kSpBlock, 8) k_sparse_contract(const SpChild* 
     uint32_t comps = c.n;
     uint64_t rho = 2;  // the next cut aims at rho x (unions still needed) edges
     while (ns > kSpSort && kmin < kmax) {
-      skey[tid] = c.keys[sp_at(cur, (uint64_t)tid * ns / kSpSort)];
-      sidx[tid] = tid;
+      uint64_t key = c.keys[sp_at(cur, (uint64_t)tid * ns / kSpSort)];
+      uint32_t idx = tid;
+      sp_sort(key, idx, skey, sidx);
+      skey[tid] = key;
       __syncthreads();
-      sp_sort(skey, sidx);
       const uint64_t want = (rho * (comps - c.tgt) * kSpSort + ns - 1) / ns;  // samples below the cut
       const uint32_t k = (uint32_t)max<uint64_t>(1, min<uint64_t>(want, kSpSort / 2)) - 1;
       const uint64_t tau = min(max(skey[k], kmin), kmax - 1);
@@ -364,9 +425,9 @@ __global__ void __launch_bounds__(kSpBlock, 8) k_sparse_contract(const SpChild* 
       uint32_t* nxt = nxt_i ? c.list[1] : c.list[0];
       uint64_t xmin, xmax;
       const uint64_t nx = sp_filter(c, cur, ns, KeepBelow{tau}, nxt, &xmin, &xmax, wcnt, red);
-      const uint32_t merged = sp_probe(c, nxt, nx, red);
+      const uint32_t merged = sp_probe(c, F, nxt, nx, red);
       if (comps - merged > c.tgt) {  // not enough: keep these unions, continue above tau
-        sp_commit(c, nxt, nx);
+        sp_commit(c, F, nxt, nx);
         comps -= merged;
         uint64_t rmin, rmax;
         ns = sp_filter(c, cur, ns, KeepAbove{tau}, nxt, &rmin, &rmax, wcnt, red);
@@ -382,22 +443,26 @@ __global__ void __launch_bounds__(kSpBlock, 8) k_sparse_contract(const SpChild* 
       nxt_i ^= 1;
     }
 
-    // 3. candidates in (key, index) order: sorted in LDS when few, else they all
-    //    share one key and are already in index order
-    if (ns <= kSpSort) {
+    // 3. shortest prefix of the candidates, in (key, index) order, that leaves tgt
+    //    components.  When few they are sorted, one per thread, and a probe works on
+    //    the thread's own pair of committed roots; else they all share one key and
+    //    are already in index order.
+    uint32_t own = 0, a = 0, b = 0;
+    const bool few = ns <= kSpSort;
+    if (few) {
       const bool have = tid < ns;
-      const uint32_t e = have ? sp_at(cur, tid) : 0xFFFFFFFFu;
-      skey[tid] = have ? c.keys[e] : ~0ull;
-      sidx[tid] = e;
-      __syncthreads();
-      sp_sort(skey, sidx);
-      uint32_t* dst = nxt_i ? c.list[1] : c.list[0];
-      if (have) dst[tid] = sidx[tid];
-      cur = dst;
-      block_sync_global();
+      own = have ? sp_at(cur, tid) : 0xFFFFFFFFu;
+      uint64_t key = have ? c.keys[own] : ~0ull;
+      sp_sort(key, own, skey, sidx);
+      if (have) {
+        const cac_edge x = c.edges[own];
+        a = sp_root(F.com, x.u);
+        b = sp_root(F.com, x.v);
+      }
+      F.sync();
     }
-    // shortest prefix of the candidates that leaves tgt components
-    if (comps - sp_probe(c, cur, ns, red) > c.tgt) {
+    auto probe = [&](uint64_t p) { return few ? sp_probe_own(F, a, b, p, red) : sp_probe(c, F, cur, p, red); };
+    if (comps - probe(ns) > c.tgt) {
       if (tid == 0) {
         *c.m_out = kSpDisconnected;
         atomicMin((long long*)&results[c.slot], 0ll);
@@ -407,27 +472,31 @@ __global__ void __launch_bounds__(kSpBlock, 8) k_sparse_contract(const SpChild* 
     uint64_t lo = 0, hi = ns;  // comps(lo) > tgt >= comps(hi)
     while (hi - lo > 1) {
       const uint64_t mid = lo + (hi - lo) / 2;
-      if (comps - sp_probe(c, cur, mid, red) <= c.tgt) hi = mid;
+      if (comps - probe(mid) <= c.tgt) hi = mid;
       else lo = mid;
     }
-    sp_commit(c, cur, hi);
+    if (few) {
+      if (tid < hi && a != b) sp_union(F.com, a, b);
+      F.sync();
+    } else {
+      sp_commit(c, F, cur, hi);
+    }
   }
 
-  // 4. labels: part[v] = root, parc[root] = rank of the root (minimum id) in id
+  // 4. labels: tri[v] = root, com[root] = rank of the root (minimum id) in id
   //    order, then part[v] = rank of v's root
-  for (uint32_t v = tid; v < c.n; v += kSpBlock) c.part[v] = sp_root(c.parc, v);
-  block_sync_global();
+  for (uint32_t v = tid; v < c.n; v += kSpBlock) F.tri[v] = sp_root(F.com, v);
+  F.sync();
   const uint64_t vc = ((uint64_t)c.n + kSpBlock - 1) / kSpBlock;
   const uint32_t v0 = (uint32_t)min((uint64_t)c.n, tid * vc), v1 = (uint32_t)min((uint64_t)c.n, v0 + vc);
   uint64_t cnt = 0;
-  for (uint32_t v = v0; v < v1; ++v) cnt += c.part[v] == v;
+  for (uint32_t v = v0; v < v1; ++v) cnt += F.tri[v] == v;
   uint64_t total = 0;
   uint64_t off = sp_exscan(cnt, red, &total);
   for (uint32_t v = v0; v < v1; ++v)
-    if (c.part[v] == v) c.parc[v] = (uint32_t)off++;
-  block_sync_global();
-  for (uint32_t v = tid; v < c.n; v += kSpBlock) c.part[v] = c.parc[c.part[v]];
-  block_sync_global();
+    if (F.tri[v] == v) F.com[v] = (uint32_t)off++;
+  F.sync();
+  for (uint32_t v = tid; v < c.n; v += kSpBlock) c.part[v] = F.com[F.tri[v]];
 
   // 5. the child's edges are written by k_sp_tile_count / k_sp_tile_scan /
   //    k_sp_tile_write over the whole device
@@ -510,16 +579,27 @@ __global__ void __launch_bounds__(kSpBlock) k_sp_tile_write(const SpChild* __res
 }
 
 // The contraction of nchild children (device descriptors d_children, largest
-// parent edge count mmax): keys over the whole device, then one workgroup per
-// child.
-void launch_sparse_contract(const SpChild* d_children, uint32_t nchild, uint64_t mmax, int64_t* d_results,
-                            hipStream_t s) {
+// parent edge count mmax and vertex count nmax): keys over the whole device, then
+// one workgroup per child.
+int launch_sparse_contract(cac_ctx* ctx, const SpChild* d_children, uint32_t nchild, uint64_t mmax, uint32_t nmax,
+                           int64_t* d_results, hipStream_t s) {
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute((const void*)k_sparse_contract<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(kSpLdsN * 8));
+  });
+  CAC_HIP(ctx, err);
   const uint64_t per_child = std::max<uint64_t>(1, 8192 / std::max<uint32_t>(nchild, 1));
   const unsigned gx = (unsigned)std::min<uint64_t>(std::max<uint64_t>(1, (mmax + 4095) / 4096), per_child);
   hipLaunchKernelGGL(k_sp_kmm_init, dim3(grid_for(nchild, 256, 64)), dim3(256), 0, s, d_children, nchild);
   for (uint32_t c0 = 0; c0 < nchild; c0 += 65535u)  // grid y holds at most 65535 children
     hipLaunchKernelGGL(k_sp_keys, dim3(gx, std::min(nchild - c0, 65535u)), dim3(256), 0, s, d_children + c0);
-  hipLaunchKernelGGL(k_sparse_contract, dim3(nchild), dim3(kSpBlock), 0, s, d_children, d_results);
+  if (nmax <= kSpLdsN)
+    hipLaunchKernelGGL(k_sparse_contract<true>, dim3(nchild), dim3(kSpBlock), (size_t)nmax * 8, s, d_children,
+                       d_results);
+  else
+    hipLaunchKernelGGL(k_sparse_contract<false>, dim3(nchild), dim3(kSpBlock), 0, s, d_children, d_results);
   const unsigned tiles = (unsigned)std::max<uint64_t>(1, (mmax + kSpTile - 1) / kSpTile);
   for (uint32_t c0 = 0; c0 < nchild; c0 += 65535u)
     hipLaunchKernelGGL(k_sp_tile_count, dim3(tiles, std::min(nchild - c0, 65535u)), dim3(256), 0, s, d_children + c0);
@@ -527,6 +607,7 @@ void launch_sparse_contract(const SpChild* d_children, uint32_t nchild, uint64_t
   for (uint32_t c0 = 0; c0 < nchild; c0 += 65535u)
     hipLaunchKernelGGL(k_sp_tile_write, dim3(tiles, std::min(nchild - c0, 65535u)), dim3(kSpBlock), 0, s,
                        d_children + c0);
+  return CAC_OK;
 }
 
 // Handover to the dense engine: n x n matrix and row sums from an edge list,
@@ -920,8 +1001,10 @@ struct SpRun {
       unsigned long long* d_kmm = cv.take<unsigned long long>(2 * nchild);
       std::vector<SpChild> ch(nchild);
       uint64_t mmax = 0;
+      uint32_t nmax = 0;
       for (size_t i = 0; i < count; ++i) {
         const SpNode& nd = sp[i0 + i];
+        nmax = std::max(nmax, nd.n);
         for (uint32_t k = 0; k < 2; ++k) {
           SpChild& x = ch[2 * i + k];
           x.edges = nd.edges;
@@ -946,8 +1029,9 @@ struct SpRun {
       }
       CAC_HIP(ctx, hipMemcpyAsync(d_children, ch.data(), nchild * sizeof(SpChild), hipMemcpyHostToDevice, s));
       prof_begin(ctx, "sparse_contract", s);
-      launch_sparse_contract(d_children, (uint32_t)nchild, mmax, d_results, s);
+      rc = launch_sparse_contract(ctx, d_children, (uint32_t)nchild, mmax, nmax, d_results, s);
       prof_end(ctx, s);
+      if (rc) return rc;
       CAC_LAUNCH_CHECK(ctx, "sparse contract");
       std::vector<unsigned long long> mout(nchild);
       CAC_HIP(ctx, hipMemcpyAsync(mout.data(), d_mout, nchild * 8, hipMemcpyDeviceToHost, s));
@@ -1122,7 +1206,8 @@ int cac_sparse_contract(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_
   c.tiles = cv.take<uint32_t>((mm + cac::kSpTile - 1) / cac::kSpTile);
   if (m) CAC_HIP(ctx, hipMemcpyAsync(d_in, edges, m * sizeof(cac_edge), hipMemcpyHostToDevice, s));
   CAC_HIP(ctx, hipMemcpyAsync(d_child, &c, sizeof(c), hipMemcpyHostToDevice, s));
-  cac::launch_sparse_contract(d_child, 1, m, d_res, s);
+  rc = cac::launch_sparse_contract(ctx, d_child, 1, m, n, d_res, s);
+  if (rc) return rc;
   CAC_LAUNCH_CHECK(ctx, "sparse contract");
   unsigned long long mo = 0;
   CAC_HIP(ctx, hipMemcpyAsync(&mo, d_mout, 8, hipMemcpyDeviceToHost, s));
