@@ -13,7 +13,10 @@ namespace cac {
 // raw cut goes.  w32: its entries add up to less than 2^32 and the matrix and row
 // sums are uint32_t, row stride ks_stride<uint32_t>(n) (whole 16-byte pieces);
 // else int64_t, row stride n.  Several roots may share one matrix (independent
-// trials).  Its draws are keyed by (seed, trial, node id).
+// trials).  Its draws are keyed by (seed, trial, node id).  A root of kKsBase <
+// n <= kKsListMax vertices may come as row lists in place of its matrix (mat
+// null): row r has the rp[r] & kKsListLen entries from rp[r] >> kKsListBits of
+// (cols, ws), one per column that is not 0, in any order; ws are of the entry type.
 struct KsRoot {
   const void* mat;
   const void* rsum;
@@ -22,6 +25,9 @@ struct KsRoot {
   uint32_t seed;     // Philox key word 0 of the trial
   uint32_t nid = 1;  // recursion node id of the matrix (1: the trial's root)
   bool w32 = false;
+  const uint32_t* rp = nullptr;
+  const uint16_t* cols = nullptr;
+  const void* ws = nullptr;
 };
 
 // Upper estimate of the device bytes one root holds at once in the two level

@@ -252,10 +252,12 @@ __global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf<E>* __restrict__ leav
 // cbs[nb] U | red[(kPieces + 1) B/64] U | misc[8] u32 | rep[s] u16 | wslot[s] u16,
 // rep and cap padded to 16 bytes.  With 32-bit entries that is 8 s bytes: two
 // 1024-thread workgroups of s = 8192 share a CU.
+// A parent of row lists adds row[s] U, 16-byte aligned, and rp[s] u32.
 template <typename E>
-__host__ __device__ inline size_t contract_lds_bytes(uint32_t s, int B) {
+__host__ __device__ inline size_t contract_lds_bytes(uint32_t s, int B, bool list = false) {
   const size_t e = sizeof(E), s8 = (s + 7) & ~size_t(7), nb2 = ((s + 63) / 64 + 3) & ~size_t(3);
-  return e * s8 + e * nb2 + e * (size_t)(kPieces<E> + 1) * (B / 64) + 32 + 4 * s8 + 16;
+  return e * s8 + e * nb2 + e * (size_t)(kPieces<E> + 1) * (B / 64) + 32 + 4 * s8 + 16 +
+         (list ? e * s8 + 4 * s8 + 16 : 0);
 }
 
 template <typename E>
@@ -263,9 +265,11 @@ struct KsLds {
   ks_sum_t<E>* cap;
   ks_sum_t<E>* cbs;
   ks_sum_t<E>* red;
-  uint32_t* misc;   // [0] i  [1] k  [2] rep[k]  [5] spare pool row  [6] pool rows handed out
+  uint32_t* misc;   // [0] i  [1] k  [2] rep[k]  [3], [4], [7] chains  [5] spare pool row  [6] pool rows handed out
   uint16_t* rep;    // padded entries past s hold 0xFFFF
   uint16_t* wslot;  // pool row of a merged row, or kNoRow
+  ks_sum_t<E>* row;  // row lists: a row being assembled, 0 between; in a chain row cb
+  uint32_t* rp;      // row lists: c.rp
 };
 
 template <typename E>
@@ -300,6 +304,43 @@ __device__ inline void load_row(const E* row, uint32_t qc, uint32_t s, E (&v)[kK
   }
 }
 
+// This thread's pieces of row r, whose pool row is `slot`.  A row of a parent of
+// lists is assembled in LDS, its entries written over zeros and the zeros put back
+// by the threads that read them; between two rows the block meets a barrier (one
+// wavefront's LDS accesses run in order).
+template <int B, bool kList, typename E>
+__device__ inline void fetch_row(const KsChild<E>& c, const KsLds<E>& L, uint16_t slot, uint32_t r, uint32_t qc,
+                                 uint32_t s, E (&v)[kKsChunk]) {
+  if constexpr (kList) {
+    if (slot == kNoRow) {
+      typedef ks_sum_t<E> U;
+      typedef const __attribute__((address_space(1))) E g_e;
+      typedef const __attribute__((address_space(1))) uint16_t g_u16;
+      constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
+      const uint32_t at = L.rp[r], len = at & kKsListLen;
+      g_u16* cols = (g_u16*)c.cols + (at >> kKsListBits);
+      g_e* ws = (g_e*)c.ws + (at >> kKsListBits);
+      for (uint32_t p = threadIdx.x; p < len; p += B) L.row[cols[p]] = (U)ws[p];
+      __syncthreads();
+      typedef U piece_t __attribute__((ext_vector_type(V)));
+#pragma unroll
+      for (uint32_t q = 0; q < Q; ++q) {
+        const uint32_t x = (q * B + threadIdx.x) * V;
+        const bool in = q < qc && x < s;  // the row's LDS is padded to whole pieces
+        piece_t t = {};
+        if (in) {
+          t = *(piece_t*)(L.row + x);
+          *(piece_t*)(L.row + x) = piece_t{};
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < V; ++j) v[q * V + j] = (E)t[j];
+      }
+      return;
+    }
+  }
+  load_row<B>(ks_row(c, slot, r), qc, s, v);
+}
+
 // A pool row: whole pieces, the padding past s (0 in registers) included.
 template <int B, typename E>
 __device__ inline void store_row(E* row, uint32_t qc, uint32_t s, const E (&v)[kKsChunk]) {
@@ -332,7 +373,7 @@ __device__ inline void store_row(E* row, uint32_t qc, uint32_t s, const E (&v)[k
 // barrier.  Each thread relabels only the representatives of the columns it
 // owns.  Returns the contracted weight (cap[a] + cap[b] - cap_new) / 2 in w;
 // false when the pool is exhausted.  Called by the whole block.
-template <int B, typename E>
+template <int B, bool kList, typename E>
 __device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uint32_t b, uint32_t held,
                          const E (&v)[kKsChunk], E (&u)[kKsChunk], uint32_t cached, bool u_has_other, uint32_t qc,
                          ks_sum_t<E>& w) {
@@ -348,7 +389,7 @@ __device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uin
   if (!u_has_other) {
     if (cached != kNoSlot && cached != a && cached != b)  // a merged row has a pool row
       store_row<B>(c.pool + (size_t)L.wslot[cached] * ks_pool_stride(s), qc, s, u);
-    load_row<B>(ks_row(c, other == a ? slot_a : slot_b, other), qc, s, u);
+    fetch_row<B, kList>(c, L, other == a ? slot_a : slot_b, other, qc, s, u);
   }
   U sum = 0;
 #pragma unroll
@@ -398,12 +439,299 @@ __device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uin
 // thread keeps (the picked row and the last merged row) take 16 registers and
 // the kernel fits 64 (8 waves: two 1024-thread workgroups per CU).  64-bit
 // entries take 32: at most 96 registers below 1024 threads (5 waves; at 80 the
-// kernel spills and is slower).
-template <int B, typename E>
-constexpr int kContractWaves = sizeof(E) == 4 ? 8 : B >= 1024 ? 1 : 5;
+// kernel spills and is slower).  Row lists: what their LDS leaves at about 1500
+// vertices, 6 and 4.
+template <int B, bool kList, typename E>
+constexpr int kContractWaves = sizeof(E) == 4 ? (kList ? 6 : 8) : B >= 1024 ? 1 : kList ? 4 : 5;
 
+// ---- chains ------------------------------------------------------------------
+// With a parent of row lists nearly every merge of a sparse graph joins the heavy
+// class cb and a vertex not merged before (439 picks and 1064 PR merges of a child
+// of 1505 vertices had 17 others).  Wavefront 0 follows a chain of such merges
+// alone: row cb stands in LDS, and a merge adds the vertex's list to it, where a
+// merge by the block assembles rows and meets barriers.  The class's columns keep
+// their label, cb at the chain's start, while its index `at` moves; chain_close
+// puts the row back in u and the index in rep.  One hop is a chain of LDS and list
+// loads: the 7974 children of 3987 such roots take 11.4 ms, 21.4 by the block alone
+// (16.1 ms for 6472 as matrices).
 template <int B, typename E>
-__global__ void __launch_bounds__(B, (kContractWaves<B, E>))
+__device__ void chain_open(const KsChild<E>& c, const KsLds<E>& L, uint32_t qc, const E (&u)[kKsChunk]) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
+  typedef U row_piece __attribute__((ext_vector_type(V)));
+  __syncthreads();  // every thread has read the state that led here
+#pragma unroll
+  for (uint32_t q = 0; q < Q; ++q) {
+    const uint32_t x = (q * B + threadIdx.x) * V;
+    row_piece t;
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j) t[j] = (U)u[q * V + j];
+    if (q < qc && x < c.s) *(row_piece*)(L.row + x) = t;
+  }
+  __syncthreads();
+}
+
+// After wavefront 0 has written misc[3] = at: a barrier, then u, cb, rep and wslot.
+template <int B, typename E>
+__device__ void chain_close(const KsChild<E>& c, const KsLds<E>& L, uint32_t qc, E (&u)[kKsChunk], uint32_t& cb) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
+  typedef U row_piece __attribute__((ext_vector_type(V)));
+  __syncthreads();
+  const uint32_t label = cb;
+  cb = L.misc[3];
+#pragma unroll
+  for (uint32_t q = 0; q < Q; ++q) {
+    const uint32_t x = (q * B + threadIdx.x) * V;
+    row_piece t = {};
+    if (q < qc && x < c.s) {
+      t = *(row_piece*)(L.row + x);
+      *(row_piece*)(L.row + x) = row_piece{};
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < V; ++j) u[q * V + j] = (E)t[j];
+  }
+  if (cb != label) {
+    for (uint32_t x = threadIdx.x; x < c.s; x += B)
+      if (L.rep[x] == label) L.rep[x] = (uint16_t)cb;
+    if (threadIdx.x == 0) {  // the vertices that joined had no pool rows
+      L.wslot[cb] = L.wslot[label];
+      L.wslot[label] = kNoRow;
+    }
+  }
+  __syncthreads();
+}
+
+// The first 64 entries of a row list, one per lane.
+template <typename E>
+struct ListHead {
+  uint32_t p0, p1, x;
+  ks_sum_t<E> w;
+};
+template <typename E>
+__device__ inline ListHead<E> list_head(const KsChild<E>& c, const KsLds<E>& L, uint32_t y) {
+  typedef const __attribute__((address_space(1))) E g_e;
+  typedef const __attribute__((address_space(1))) uint16_t g_u16;
+  ListHead<E> h;
+  const uint32_t at = readlane_u32(L.rp[y], 0);
+  h.p0 = at >> kKsListBits;
+  h.p1 = h.p0 + (at & kKsListLen);
+  const uint32_t p = h.p0 + (threadIdx.x & 63);
+  h.x = p < h.p1 ? ((g_u16*)c.cols)[p] : 0u;
+  h.w = p < h.p1 ? (ks_sum_t<E>)((g_e*)c.ws)[p] : 0;
+  return h;
+}
+
+// Adds vertex y's list to the chain's row (label: the class's columns, which take
+// nothing), and y to the class: returns the weight between them.  *low gets the
+// smallest column whose entry reached the bound, or kNoSlot.
+template <typename E>
+__device__ inline ks_sum_t<E> chain_add(const KsChild<E>& c, const KsLds<E>& L, uint32_t y, const ListHead<E>& h,
+                                        uint32_t label, ks_sum_t<E> bound, uint32_t* low) {
+  typedef ks_sum_t<E> U;
+  typedef const __attribute__((address_space(1))) E g_e;
+  typedef const __attribute__((address_space(1))) uint16_t g_u16;
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t m = kNoSlot, x = h.x;
+  U w = h.w;
+  for (uint32_t p = h.p0 + lane; p < h.p1; p += 64) {
+    if (p >= h.p0 + 64) {
+      x = ((g_u16*)c.cols)[p];
+      w = (U)((g_e*)c.ws)[p];
+    }
+    if (L.rep[x] != label) {  // a column once: no two lanes meet
+      const U now = L.row[x] + w;
+      L.row[x] = now;
+      if (now >= bound && x < m) m = x;
+    }
+  }
+  *low = wave_min<uint32_t>(m);
+  const U between = readlane((U)L.row[y], 0);
+  if (lane == 0) {
+    L.row[y] = 0;
+    L.rep[y] = (uint16_t)label;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  return between;
+}
+
+template <typename E>
+__device__ inline bool chain_single(const KsLds<E>& L, uint32_t y) {  // not merged before: its row is the parent's
+  return readlane_u32((uint32_t)L.rep[y], 0) == y && readlane_u32((uint32_t)L.wslot[y], 0) == kNoRow;
+}
+
+// Picks from number p on, while they join the class of cb and a single vertex.
+// Returns the first pick left to the block; W, u, cb, nv and pr1 follow.
+template <int B, typename E>
+__device__ uint32_t pick_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t p, ks_sum_t<E> bound, uint32_t qc,
+                               uint32_t nb, uint64_t& W, E (&u)[kKsChunk], uint32_t& cb, uint32_t& nv,
+                               uint32_t& pr1) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>;
+  typedef U row_piece __attribute__((ext_vector_type(V)));
+  const uint32_t s = c.s, label = cb, lane = threadIdx.x & 63;
+  chain_open<B>(c, L, qc, u);
+  if (threadIdx.x < 64) {
+    uint32_t at = cb;
+    const uint32_t span = ((s + 63) / 64 + V - 1) / V * V;  // a lane's columns of the row
+    for (; p + c.tgt < s && W != 0; ++p) {
+      const u32x4 rnd = philox4x32(c.trial, c.nid, p, 0u, c.seed, kDomKs);
+      const uint32_t i = wave_select_two_level<U>(L.cap, L.cbs, s, nb, (U)uniform1(lo64(rnd), W));
+      if (i >= s) break;
+      const U r = (U)uniform1(hi64(rnd), (uint64_t)readlane((U)L.cap[i], 0));
+      uint32_t y = i;
+      if (i == at) {  // the column of row cb whose prefix reaches r
+        U sum = 0;
+        const uint32_t x0 = lane * span, x1 = min(x0 + span, (s + V - 1) / V * V);  // padded to pieces of 0
+        for (uint32_t x = x0; x < x1; x += V) {
+          const row_piece t = *(const row_piece*)(L.row + x);
+#pragma unroll
+          for (uint32_t j = 0; j < V; ++j) sum += t[j];
+        }
+        const U inc = wave_incl_scan<U>(sum);
+        const uint64_t hit = __ballot(inc >= r);
+        if (!hit) break;
+        const int owner = __ffsll((long long)hit) - 1;
+        const U before = readlane((U)(inc - sum), owner);
+        const uint32_t x = owner * span + lane;
+        const U e = lane < span && x < s ? L.row[x] : 0;
+        const U inc2 = wave_incl_scan<U>(e);
+        const uint64_t hit2 = __ballot(lane < span && x < s && inc2 + before >= r);
+        if (!hit2) break;
+        y = owner * span + (uint32_t)(__ffsll((long long)hit2) - 1);
+      }
+      if (!chain_single(L, y)) break;
+      const ListHead<E> h = list_head(c, L, y);
+      if (i != at) {  // the column of the list whose prefix, in column order, reaches r
+        const uint32_t len = h.p1 - h.p0;
+        if (len > 64) break;
+        U below = 0;
+        for (uint32_t k = 0; k < len; ++k) {
+          const uint32_t x = readlane_u32(h.x, k);
+          const U w = readlane(h.w, k);
+          below += x < h.x ? w : 0;
+        }
+        const uint64_t hit = __ballot(lane < len && below < r && r <= below + h.w);
+        if (!hit) break;
+        const uint32_t x = readlane_u32(h.x, __ffsll((long long)hit) - 1);
+        if (readlane_u32((uint32_t)L.rep[x], 0) != label) break;
+      }
+      uint32_t low;
+      const U w = chain_add(c, L, y, h, label, bound, &low);
+      const uint32_t a = max(at, y), b = min(at, y);
+      if (lane == 0) {
+        const U ca = L.cap[a], cb0 = L.cap[b], now = ca + cb0 - 2 * w;
+        L.cbs[a / 64] -= ca;
+        L.cap[a] = 0;
+        L.cbs[b / 64] += now - cb0;
+        L.cap[b] = now;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      at = b;
+      W -= 2 * (uint64_t)w;
+      --nv;
+      if (w >= bound) ++pr1;
+    }
+    if (lane == 0) {
+      L.misc[0] = p;
+      L.misc[3] = at;
+      L.misc[4] = nv;
+      L.misc[7] = pr1;
+      ((uint32_t*)L.red)[0] = (uint32_t)W;
+      ((uint32_t*)L.red)[1] = (uint32_t)(W >> 32);
+    }
+  }
+  chain_close<B>(c, L, qc, u, cb);
+  nv = L.misc[4];
+  pr1 = L.misc[7];
+  W = ((uint64_t)((uint32_t*)L.red)[1] << 32) | ((uint32_t*)L.red)[0];
+  p = L.misc[0];
+  __syncthreads();
+  return p;
+}
+
+// Rows of the PR pass from i = cb on: while the row to check is row cb, its first
+// entry of weight >= bound leads to a single vertex, and more than two vertices are
+// left, the class takes that vertex's index.  Returns the row to check next (maybe
+// i itself), kNoSlot if none; u, cb and nv follow.
+template <int B, typename E>
+__device__ uint32_t pr_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t i, ks_sum_t<E> bound, uint32_t qc,
+                             E (&u)[kKsChunk], uint32_t& cb, uint32_t& nv) {
+  typedef ks_sum_t<E> U;
+  constexpr uint32_t V = kPiece<E>;
+  typedef U row_piece __attribute__((ext_vector_type(V)));
+  const uint32_t s = c.s, label = cb, lane = threadIdx.x & 63;
+  chain_open<B>(c, L, qc, u);
+  if (threadIdx.x < 64) {
+    uint32_t at = cb, from = 0;  // no entry before column `from` reaches the bound
+    ListHead<E> ahead;           // of vertex `guess`, the entry after the one taken
+    uint32_t guess = kNoSlot;
+    while (nv > 2) {
+      uint32_t first = kNoSlot, second = kNoSlot;
+      for (uint32_t b = from & ~(64 * V - 1); b < s && first == kNoSlot; b += 64 * V) {
+        const uint32_t x = b + lane * V;
+        const row_piece t = x < s ? *(const row_piece*)(L.row + x) : row_piece{};
+        uint32_t bits = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < V; ++k) bits |= t[k] >= bound ? 1u << k : 0u;
+        uint64_t hit = __ballot(bits != 0);
+        if (hit) {
+          const int l = __ffsll((long long)hit) - 1;
+          first = b + (uint32_t)l * V + (uint32_t)(__ffs((int)readlane_u32(bits, l)) - 1);
+          if ((int)lane == l) bits &= bits - 1;
+          hit = __ballot(bits != 0);
+          if (hit) {
+            const int l2 = __ffsll((long long)hit) - 1;
+            second = b + (uint32_t)l2 * V + (uint32_t)(__ffs((int)readlane_u32(bits, l2)) - 1);
+          }
+        }
+      }
+      bool moved = false;
+      if (first != kNoSlot) {
+        if (!chain_single(L, first)) break;
+        const ListHead<E> h = guess == first ? ahead : list_head(c, L, first);
+        guess = second;
+        if (second != kNoSlot) ahead = list_head(c, L, second);
+        uint32_t low;
+        const U w = chain_add(c, L, first, h, label, bound, &low);
+        if (lane == 0) {
+          L.cap[first] += L.cap[at] - 2 * w;
+          L.cap[at] = 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        from = min(first + 1, low);
+        at = first;
+        --nv;
+        moved = true;
+      }
+      // the next row to check: a live one, or the class itself if its index is past i
+      uint32_t next = kNoSlot;
+      for (uint32_t b = (i + 1) & ~63u; b < s && next == kNoSlot; b += 64) {
+        const uint32_t x = b + lane;
+        const uint64_t hit = __ballot(x > i && x < s && (L.rep[x] == x || x == at) && L.cap[x] >= bound);
+        if (hit) next = b + (uint32_t)(__ffsll((long long)hit) - 1);
+      }
+      i = next;
+      if (!moved || next != at) break;
+    }
+    if (lane == 0) {
+      L.misc[0] = i;
+      L.misc[3] = at;
+      L.misc[4] = nv;
+    }
+  }
+  chain_close<B>(c, L, qc, u, cb);
+  nv = L.misc[4];
+  i = L.misc[0];
+  __syncthreads();
+  return i;
+}
+
+// kList: the parents are row lists.  A sparse graph's matrix costs its n^2 entries
+// three times, written once and read about once by each child, where the lists
+// cost its edges.
+template <int B, bool kList, typename E>
+__global__ void __launch_bounds__(B, (kContractWaves<B, kList, E>))
     k_ks_contract(const KsChild<E>* __restrict__ children, uint32_t* __restrict__ k_out,
                   int64_t* __restrict__ results) {
   typedef ks_sum_t<E> U;
@@ -420,6 +748,12 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
   L.misc = (uint32_t*)(L.red + (kPieces<E> + 1) * (B / 64));
   L.rep = (uint16_t*)(((uintptr_t)(L.misc + 8) + 15) & ~uintptr_t(15));
   L.wslot = L.rep + s8;
+  if constexpr (kList) {
+    L.row = (U*)(((uintptr_t)(L.wslot + s8) + 15) & ~uintptr_t(15));
+    L.rp = (uint32_t*)(L.row + s8);
+    for (uint32_t x = threadIdx.x; x < s8; x += B) L.row[x] = 0;
+    for (uint32_t x = threadIdx.x; x < s; x += B) L.rp[x] = c.rp[x];
+  }
 
   for (uint32_t x = threadIdx.x; x < s8; x += B) {
     L.cap[x] = x < s ? (U)c.prsum[x] : 0;
@@ -453,7 +787,14 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
   // it is not loaded again
   E v[kKsChunk], u[kKsChunk];
   uint32_t cb = kNoSlot;
+  bool chain = false;  // row lists: the last pick joined cb and a single vertex
   for (uint32_t p = 0; p + c.tgt < s; ++p) {
+    if constexpr (kList) {
+      if (chain) {
+        p = pick_chain<B>(c, L, p, bound, qc, nb, W, u, cb, nv, pr1);
+        if (p + c.tgt >= s) break;
+      }
+    }
     if (W == 0) {
       status = 1;
       break;
@@ -473,7 +814,7 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
 #pragma unroll
       for (uint32_t q = 0; q < kKsChunk; ++q) v[q] = u[q];
     } else {
-      load_row<B>(ks_row(c, L.wslot[i], i), qc, s, v);
+      fetch_row<B, kList>(c, L, L.wslot[i], i, qc, s, v);
     }
     const uint32_t k =
         block_select_row<B, E>(v, qc, (U)uniform1(hi64(rnd), (uint64_t)L.cap[i]), L.red, L.misc + 1, L.rep);
@@ -483,8 +824,10 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
     }
     const uint32_t j = L.misc[2];  // rep[k], read by the selecting thread before the merge relabels
     const uint32_t a = i > j ? i : j, b = i > j ? j : i;
+    if constexpr (kList)
+      chain = (i == cb && L.wslot[j] == kNoRow) || (j == cb && L.wslot[i] == kNoRow);
     U w = 0;
-    if (!ks_merge<B, E>(c, L, a, b, i, v, u, cb, j == cb, qc, w)) {
+    if (!ks_merge<B, kList, E>(c, L, a, b, i, v, u, cb, j == cb, qc, w)) {
       status = 3;
       break;
     }
@@ -497,11 +840,19 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
   if (status == 0 && pr1 > 0 && c.bound > 0) {
     for (uint32_t i = 0; i < s && nv > 2; ++i) {
       if (L.rep[i] != i || L.cap[i] < bound) continue;
+      if constexpr (kList) {
+        // the heavy class merges into one vertex after the other, its index each
+        // time the next row to check
+        if (i == cb) {
+          i = pr_chain<B>(c, L, i, bound, qc, u, cb, nv);
+          if (i >= s || nv <= 2) break;
+        }
+      }
       if (i == cb) {
 #pragma unroll
         for (uint32_t q = 0; q < kKsChunk; ++q) v[q] = u[q];
       } else {
-        load_row<B>(ks_row(c, L.wslot[i], i), qc, s, v);
+        fetch_row<B, kList>(c, L, L.wslot[i], i, qc, s, v);
       }
       uint32_t first = kNoSlot;
 #pragma unroll
@@ -516,7 +867,7 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, E>))
       // bound, so this merge's relabelling (of class i) leaves it unchanged
       U w = 0;
       const uint32_t tgt = L.rep[first];
-      if (!ks_merge<B, E>(c, L, i, tgt, i, v, u, cb, tgt == cb, qc, w)) {
+      if (!ks_merge<B, kList, E>(c, L, i, tgt, i, v, u, cb, tgt == cb, qc, w)) {
         status = 3;
         break;
       }
@@ -607,7 +958,8 @@ __device__ inline void team_sync() {
 // (item_prefix).  The bound is the rows' HBM traffic plus the LDS passes; adding
 // every column into an accumulator by its class took s atomics per row instead
 // of s - k.  Row maxima are written for leaves only, which alone read them.
-template <int CB, int TEAM, typename E>
+// kList: the parents are row lists, a row's entries are written over zeros in LDS.
+template <int CB, int TEAM, bool kList, typename E>
 __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild<E>* __restrict__ children,
                                                    const uint32_t* __restrict__ k_out,
                                                    const uint32_t* __restrict__ item_prefix, uint32_t nchild,
@@ -645,11 +997,20 @@ __global__ void __launch_bounds__(CB) k_ks_compact(const KsChild<E>* __restrict_
   g_u32* dead = (g_u32*)c.dead;
   for (uint32_t r = r0 + team; r < r1; r += CB / TEAM) {
     const uint32_t e = c.live[r];
-    g_e* src = (g_e*)((e & kLiveWork) ? c.pool + (size_t)(e & ~kLiveWork) * ks_pool_stride(s)
-                                      : c.parent + (size_t)e * c.ps);
+    if (kList && !(e & kLiveWork)) {
+      for (uint32_t x = t; x < s; x += TEAM) row[x] = 0;
+      team_sync<TEAM>();
+      const uint32_t at = c.rp[e], len = at & kKsListLen;
+      const uint16_t* cols = c.cols + (at >> kKsListBits);
+      const E* ws = c.ws + (at >> kKsListBits);
+      for (uint32_t p = t; p < len; p += TEAM) row[cols[p]] = (AccT)ws[p];
+    } else {
+      g_e* src = (g_e*)((e & kLiveWork) ? c.pool + (size_t)(e & ~kLiveWork) * ks_pool_stride(s)
+                                        : c.parent + (size_t)e * c.ps);
 #pragma unroll 4
-    for (uint32_t x = t * V; x + V <= s; x += TEAM * V) *(piece_t*)(row + x) = *(g_piece*)(src + x);
-    for (uint32_t x = s / V * V + t; x < s; x += TEAM) row[x] = (AccT)src[x];
+      for (uint32_t x = t * V; x + V <= s; x += TEAM * V) *(piece_t*)(row + x) = *(g_piece*)(src + x);
+      for (uint32_t x = s / V * V + t; x < s; x += TEAM) row[x] = (AccT)src[x];
+    }
     team_sync<TEAM>();
 #pragma unroll 4
     for (uint32_t i = t; i < nd; i += TEAM) {
@@ -821,14 +1182,30 @@ int run_leaves(cac_ctx* ctx, const std::vector<KsLeaf<E>>& leaves, int buf, int6
 }
 
 template <int B, typename E>
-void launch_contract(const KsChild<E>* d_children, uint32_t count, uint32_t smax, uint32_t* d_kout,
+void launch_contract(const KsChild<E>* d_children, uint32_t count, uint32_t smax, bool list, uint32_t* d_kout,
                      int64_t* d_results, hipStream_t s) {
-  hipLaunchKernelGGL((k_ks_contract<B, E>), dim3(count), dim3(B), contract_lds_bytes<E>(smax, B), s, d_children,
-                     d_kout, d_results);
+  const size_t lds = contract_lds_bytes<E>(smax, B, list);
+  if (list)
+    hipLaunchKernelGGL((k_ks_contract<B, true, E>), dim3(count), dim3(B), lds, s, d_children, d_kout, d_results);
+  else
+    hipLaunchKernelGGL((k_ks_contract<B, false, E>), dim3(count), dim3(B), lds, s, d_children, d_kout, d_results);
+}
+// TEAM 0: the whole workgroup.
+template <int TEAM, typename E>
+void launch_compact(int cb, dim3 grid, size_t lds, bool list, const KsChild<E>* dc, const uint32_t* dk,
+                    const uint32_t* dp, uint32_t nc, uint32_t stride, hipStream_t s) {
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3((unsigned)cb), lds, s, dc, dk, dp, nc, stride); };
+  auto pick = [&](auto block) {
+    constexpr int CB = decltype(block)::value, T = TEAM ? TEAM : CB;
+    go(list ? k_ks_compact<CB, T, true, E> : k_ks_compact<CB, T, false, E>);
+  };
+  if (cb == 1024) pick(std::integral_constant<int, 1024>{});
+  else if (cb == 512) pick(std::integral_constant<int, 512>{});
+  else pick(std::integral_constant<int, 256>{});
 }
 
 // One level's launches for the children ch (already in d_children's order, by
-// block-size class): contraction per class; waits for the children's k_out;
+// block-size class and form of the parent): contraction per class; waits for the children's k_out;
 // then the compaction, sized by those k (a child that the PR pass collapsed
 // takes a few workgroups, not t' / rows of them), left running on the stream
 // (the next level's work follows it there).
@@ -844,7 +1221,9 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
     int B = contract_block(ctx, ch[c0].s);
     size_t c1 = c0;
     uint32_t smax = 0;
-    while (c1 < nchild && contract_block(ctx, ch[c1].s) == B) smax = std::max(smax, ch[c1++].s);
+    const bool list = ch[c0].parent == nullptr;
+    while (c1 < nchild && contract_block(ctx, ch[c1].s) == B && (ch[c1].parent == nullptr) == list)
+      smax = std::max(smax, ch[c1++].s);
     const uint32_t cnt = (uint32_t)(c1 - c0);
     group.push_back(c0);
     // Fewer children than CUs (the top levels of a small solve): the device is
@@ -855,11 +1234,11 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
     // s <= 512 has two pieces to scan and no barriers to wait at (the same
     // solve: contraction 0.82 ms with 64 threads, 0.86 with 128, 0.90 with 256).
     if (sizeof(E) == 8 && cnt < kFewChildren && B < 256) B = 256;
-    if (B == 1024) launch_contract<1024, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
-    else if (B == 512) launch_contract<512, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
-    else if (B == 256) launch_contract<256, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
-    else if (B == 128) launch_contract<128, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
-    else launch_contract<64, E>(d_children + c0, cnt, smax, d_kout + c0, d_results, s);
+    if (B == 1024) launch_contract<1024, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
+    else if (B == 512) launch_contract<512, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
+    else if (B == 256) launch_contract<256, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
+    else if (B == 128) launch_contract<128, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
+    else launch_contract<64, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
     c0 = c1;
   }
   group.push_back(nchild);
@@ -900,16 +1279,9 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
     const uint32_t* dk = d_kout + group[g];
     const uint32_t* dp = d_prefix + group[g];
     const uint32_t nc = (uint32_t)(group[g + 1] - group[g]);
-    const dim3 grid(items[g]), block((unsigned)cb);
-    if (waves) {
-      if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-      else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-      else hipLaunchKernelGGL((k_ks_compact<256, 64, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-    } else {
-      if (cb == 1024) hipLaunchKernelGGL((k_ks_compact<1024, 1024, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-      else if (cb == 512) hipLaunchKernelGGL((k_ks_compact<512, 512, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-      else hipLaunchKernelGGL((k_ks_compact<256, 256, E>), grid, block, lds, s, dc, dk, dp, nc, stride);
-    }
+    const bool list = ch[group[g]].parent == nullptr;
+    if (waves) launch_compact<64, E>(cb, dim3(items[g]), lds, list, dc, dk, dp, nc, stride, s);
+    else launch_compact<0, E>(cb, dim3(items[g]), lds, list, dc, dk, dp, nc, stride, s);
   }
   prof_end(ctx, s);
   CAC_LAUNCH_CHECK(ctx, "ks compact");
@@ -948,13 +1320,16 @@ int contract_attr(cac_ctx* ctx) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-    err = hipFuncSetAttribute((const void*)k_ks_contract<1024, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    err = hipFuncSetAttribute((const void*)k_ks_contract<1024, false, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)contract_lds_bytes<E>(kKsMaxS, 1024));
     if (err == hipSuccess)
-      err = hipFuncSetAttribute((const void*)k_ks_contract<512, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      err = hipFuncSetAttribute((const void*)k_ks_contract<512, false, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)contract_lds_bytes<E>(512 * kKsChunk, 512));
-    const void* compact[] = {(const void*)k_ks_compact<1024, 64, E>, (const void*)k_ks_compact<1024, 1024, E>,
-                             (const void*)k_ks_compact<512, 512, E>, (const void*)k_ks_compact<256, 256, E>};
+    const void* compact[] = {(const void*)k_ks_compact<1024, 64, false, E>,
+                             (const void*)k_ks_compact<1024, 1024, false, E>,
+                             (const void*)k_ks_compact<512, 512, false, E>,
+                             (const void*)k_ks_compact<256, 256, false, E>,
+                             (const void*)k_ks_compact<1024, 64, true, E>};
     for (const void* f : compact)
       if (err == hipSuccess)
         err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -978,6 +1353,9 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
     uint32_t s, trial, nid, slot;
     int64_t bound;
     uint32_t seed;
+    const uint32_t* rp = nullptr;  // row lists in place of mat
+    const uint16_t* cols = nullptr;
+    const E* ws = nullptr;
   };
   int rc = contract_attr<E>(ctx);
   if (rc) return rc;
@@ -987,7 +1365,10 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
   std::vector<Node> level;
   for (const KsRoot& r : roots) {
     if (r.n > kKsMaxS) return fail(ctx, CAC_EINVAL, "dense Karger-Stein supports at most 8192 vertices");
-    level.push_back({(const E*)r.mat, (const E*)r.rsum, nullptr, r.n, r.trial, r.nid, r.slot, r.bound, r.seed});
+    if (!r.mat && (r.n <= kKsBase || r.n > kKsListMax || !r.rp))
+      return fail(ctx, CAC_EINVAL, "dense Karger-Stein root without a matrix");
+    level.push_back({(const E*)r.mat, (const E*)r.rsum, nullptr, r.n, r.trial, r.nid, r.slot, r.bound, r.seed, r.rp,
+                     r.cols, (const E*)r.ws});
   }
   int buf = 0;  // level buffer for the children of this level; the parents are in the other one
   while (!level.empty()) {
@@ -1002,9 +1383,11 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
       if (rc) return rc;
     }
     if (internal.empty()) break;
-    // children sorted by block-size class (1024, 256, 64), two per internal node
+    // children sorted by block-size class (1024, 256, 64) and form of the parent,
+    // two per internal node
     std::vector<std::pair<int, uint32_t>> order;
-    for (uint32_t i = 0; i < internal.size(); ++i) order.push_back({-contract_block(ctx, internal[i].s), i});
+    for (uint32_t i = 0; i < internal.size(); ++i)
+      order.push_back({-2 * contract_block(ctx, internal[i].s) + (internal[i].mat ? 0 : 1), i});
     std::stable_sort(order.begin(), order.end());
     const size_t nchild = 2 * internal.size();
     size_t arrays = 0;
@@ -1047,6 +1430,9 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
         x.slot = nd.slot;
         x.seed = nd.seed;
         x.bound = nd.bound;
+        x.rp = nd.rp;
+        x.cols = nd.cols;
+        x.ws = nd.ws;
       }
     }
     rc = contract_level<E>(ctx, ch, d_children, d_prefix, d_kout, d_results, kout, s);
@@ -1088,7 +1474,7 @@ int ks_run_typed(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_resu
       if (kout[i] == kKsBad) return fail(ctx, CAC_EDEVICE, "Karger-Stein selection out of range");
       if (kout[i] == 0) continue;  // disconnected child: its 0 is already recorded
       next.push_back({ch[i].out, ch[i].orsum, ch[i].ormax, kout[i], ch[i].trial, ch[i].nid, ch[i].slot, ch[i].bound,
-                      ch[i].seed});
+                      ch[i].seed, nullptr, nullptr, nullptr});
     }
     level.swap(next);
     buf ^= 1;

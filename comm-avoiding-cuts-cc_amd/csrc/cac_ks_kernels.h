@@ -39,6 +39,8 @@ constexpr uint32_t kKsBase = 128;        // base_case_size (co_mincut.h:24)
 constexpr uint32_t kKsMaxS = 8192;       // LDS holds caps, reps and row slots for s <= this
 constexpr uint32_t kKsChunk = 8;         // row entries per thread (s <= 8 * block size), x = k * B + t
 constexpr uint32_t kKsUnit = 64;         // a pool row is padded to whole units of 64 entries
+constexpr uint32_t kKsListMax = 2048;    // a root of at most this many vertices may be given as row lists
+constexpr uint32_t kKsListBits = 12, kKsListLen = (1u << kKsListBits) - 1;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 constexpr uint16_t kNoRow = 0xFFFFu;         // LDS: the row has no pool row (pool rows per child <= s <= 8192)
 constexpr uint32_t kLiveWork = 0x80000000u;  // live[] entry: pool row of the child
@@ -85,6 +87,9 @@ struct KsChild {
   uint32_t slot, seed;  // seed: Philox key word 0 of the child's trial
   uint32_t pool_rows;
   int64_t bound;
+  const uint32_t* rp;    // a parent of row lists (parent null): see KsRoot
+  const uint16_t* cols;
+  const E* ws;
 };
 
 template <typename E>

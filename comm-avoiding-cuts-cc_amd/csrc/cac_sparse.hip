@@ -641,6 +641,174 @@ struct SpDense {
   uint16_t* eli;                 // [2m] entry index inside its band: (row - band * rows) * n + column
 };
 
+// A handed-over node goes to the dense engine as row lists, not as a matrix, when
+// its rows hold at most n / kListShare entries on average and at least kListNodes
+// nodes are handed over together.  Random graphs of 1500 vertices, 32-bit entries,
+// matrices / lists: rows of n / 60, 1024 trials 45.4 / 42.9 ms; n / 24, 48.9 / 49.5
+// (64-bit 82.1 / 81.6); n / 12, 52.8 / 54.7; 64 trials of n / 24 in 64-bit entries
+// 12.1 / 12.4.  Where a heavy class takes most merges the lists are far ahead: the
+// 11400 nodes of karger_stein on a Watts-Strogatz graph of 48000 vertices with 16
+// edges each, rows of n / 23, took 46 ms to fill and 72 to contract as matrices and
+// take 20 and 39 as lists.
+constexpr uint64_t kListShare = 20;
+constexpr size_t kListNodes = 128;
+static_assert((uint64_t)kKsListMax * kKsListMax / kListShare < (1ull << (32 - kKsListBits)) && kKsListMax <= kKsListLen + 1,
+              "entry index and row length share 32 bits");
+inline bool as_lists(uint32_t n, uint64_t m) {
+  return n > kKsBase && n <= kKsListMax && 2 * m * kListShare <= (uint64_t)n * n;
+}
+
+// The lists of a node's rows, the form of a sparse node.  One workgroup counts the
+// entries and sums of the rows in LDS, scans, and places the entries; then a
+// wavefront per row adds the entries of the same column (parallel edges: 33 entries
+// a row become 3 on Watts-Strogatz graphs) in an LDS row of its own, the next
+// row's entries already on their way.  The bound is the two reads of the edges and
+// the latency of the rows: 4052 nodes of 1505 vertices and 49000 edges take 6.1 ms
+// (7.9 as matrices, and 3.1 to bucket their entries).
+template <typename E>
+struct SpRows {
+  typedef typename std::conditional<sizeof(E) == 4, uint32_t, unsigned long long>::type A;
+  const cac_edge* edges;
+  uint64_t m;  // below 2^31
+  uint32_t n, pad;
+  E* rsum;          // [n]
+  uint32_t* rp;     // [n], cols and ws [2m]: the form of KsRoot
+  uint16_t* cols;
+  E* ws;
+  uint16_t* pcols;  // [2m] placed entries
+  E* pws;           // [2m]
+};
+constexpr uint32_t kSpRowsLds = 56u << 10;  // two workgroups per CU
+constexpr uint32_t kSpLongRow = 512;        // entries above which the workgroup takes a row
+
+template <typename E>
+__global__ void __launch_bounds__(kSpBlock, 8) k_sp_rows(const SpRows<E>* __restrict__ nodes) {
+  typedef typename SpRows<E>::A A;
+  extern __shared__ __align__(16) unsigned char sp_rows_lds[];  // kSpRowsLds
+  __shared__ uint32_t at[kKsListMax];
+  __shared__ uint32_t wtot[kSpWaves], cursor, longs, long_len;
+  __shared__ uint16_t long_row[kKsListMax * (kKsListMax / kListShare) / kSpLongRow];
+  const SpRows<E> d = nodes[blockIdx.x];
+  const uint32_t n = d.n, m = (uint32_t)d.m;
+  A* acc = (A*)sp_rows_lds;
+  for (uint32_t x = threadIdx.x; x < n; x += kSpBlock) {
+    at[x] = 0;
+    acc[x] = 0;
+  }
+  if (threadIdx.x == 0) cursor = longs = long_len = 0;
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t e = threadIdx.x; e < m; e += kSpBlock) {
+    const cac_edge x = d.edges[e];
+    atomicAdd(&at[x.u], 1u);
+    atomicAdd(&at[x.v], 1u);
+    atomicAdd(&acc[x.u], (A)x.w);
+    atomicAdd(&acc[x.v], (A)x.w);
+  }
+  __syncthreads();
+  static_assert(kKsListMax == 2 * kSpBlock, "two rows per thread");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t r0 = 2 * threadIdx.x;
+  const uint32_t c0 = r0 < n ? at[r0] : 0u, c1 = r0 + 1 < n ? at[r0 + 1] : 0u;
+  const uint32_t inc = wave_incl_scan<uint32_t>(c0 + c1);
+  if (lane == 63) wtot[wave] = inc;
+  __syncthreads();
+  uint32_t before = inc - c0 - c1;
+  for (int w = 0; w < wave; ++w) before += wtot[w];
+  if (r0 < n) at[r0] = before;
+  if (r0 + 1 < n) at[r0 + 1] = before + c0;
+  if (c0 > kSpLongRow) long_row[atomicAdd(&longs, 1u)] = (uint16_t)r0;
+  if (c1 > kSpLongRow) long_row[atomicAdd(&longs, 1u)] = (uint16_t)(r0 + 1);
+  for (uint32_t x = threadIdx.x; x < n; x += kSpBlock) d.rsum[x] = (E)acc[x];
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t e = threadIdx.x; e < m; e += kSpBlock) {
+    const cac_edge x = d.edges[e];
+    const uint32_t p = atomicAdd(&at[x.u], 1u), q = atomicAdd(&at[x.v], 1u);
+    d.pcols[p] = (uint16_t)x.v;
+    d.pws[p] = (E)x.w;
+    d.pcols[q] = (uint16_t)x.u;
+    d.pws[q] = (E)x.w;
+  }
+  const uint32_t teams = min((uint32_t)kSpWaves, kSpRowsLds / (n * (uint32_t)sizeof(A)));
+  for (uint32_t x = threadIdx.x; x < teams * n; x += kSpBlock) acc[x] = 0;
+  block_sync_global();
+  const uint64_t below = (1ull << lane) - 1;
+  for (uint32_t k = 0; k < longs; ++k) {  // the few long rows, by the workgroup
+    const uint32_t r = long_row[k], p1 = at[r], base = cursor;
+#pragma unroll 4
+    for (uint32_t p = (r ? at[r - 1] : 0u) + threadIdx.x; p < p1; p += kSpBlock)
+      atomicAdd(&acc[d.pcols[p]], (A)d.pws[p]);
+    __syncthreads();
+    for (uint32_t b = 0; b < n; b += kSpBlock) {
+      const uint32_t x = b + threadIdx.x;
+      const A v = x < n ? acc[x] : 0;
+      const uint64_t mask = __ballot(v != 0);
+      uint32_t to = 0;
+      if (lane == 0) to = base + atomicAdd(&long_len, (uint32_t)__popcll(mask));
+      to = readlane_u32(to, 0) + (uint32_t)__popcll(mask & below);
+      if (v != 0) {
+        d.cols[to] = (uint16_t)x;
+        d.ws[to] = (E)v;
+        acc[x] = 0;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      d.rp[r] = (base << kKsListBits) | long_len;
+      cursor = base + long_len;
+      long_len = 0;
+    }
+    __syncthreads();
+  }
+  if ((uint32_t)wave >= teams) return;
+  acc += (size_t)wave * n;
+  auto head = [&](uint32_t r, uint32_t& p0, uint32_t& p1, uint32_t& x, A& w) {
+    p0 = r ? at[r - 1] : 0u;  // the cursors end at the rows' ends
+    p1 = at[r];
+    if (p1 - p0 > kSpLongRow) p1 = p0;  // done
+    const uint32_t p = p0 + lane;
+    x = p < p1 ? d.pcols[p] : 0u;
+    w = p < p1 ? (A)d.pws[p] : 0;
+  };
+  uint32_t p0 = 0, p1 = 0, x = 0;
+  A w = 0;
+  if ((uint32_t)wave < n) head(wave, p0, p1, x, w);
+  for (uint32_t r = wave; r < n; r += teams) {
+    uint32_t np0 = 0, np1 = 0, nx = 0;
+    A nw = 0;
+    if (r + teams < n) head(r + teams, np0, np1, nx, nw);
+    if (p0 + lane < p1) atomicAdd(&acc[x], w);
+    for (uint32_t p = p0 + 64 + lane; p < p1; p += 64) atomicAdd(&acc[d.pcols[p]], (A)d.pws[p]);
+    // a list of more than 64 takes room for every entry
+    const A v = p0 + lane < p1 ? atomicExch(&acc[x], (A)0) : 0;  // weights are at least 1
+    uint64_t mask = __ballot(v != 0);
+    uint32_t len = (uint32_t)__popcll(mask), to = 0;
+    if (lane == 0) to = atomicAdd(&cursor, p1 - p0 > 64 ? p1 - p0 : len);
+    to = readlane_u32(to, 0);
+    if (v != 0) {
+      d.cols[to + (uint32_t)__popcll(mask & below)] = (uint16_t)x;
+      d.ws[to + (uint32_t)__popcll(mask & below)] = (E)v;
+    }
+    for (uint32_t b = p0 + 64; b < p1; b += 64) {
+      const uint32_t p = b + lane;
+      const uint32_t x2 = p < p1 ? d.pcols[p] : 0u;
+      const A v2 = p < p1 ? atomicExch(&acc[x2], (A)0) : 0;
+      mask = __ballot(v2 != 0);
+      if (v2 != 0) {
+        d.cols[to + len + (uint32_t)__popcll(mask & below)] = (uint16_t)x2;
+        d.ws[to + len + (uint32_t)__popcll(mask & below)] = (E)v2;
+      }
+      len += (uint32_t)__popcll(mask);
+    }
+    if (lane == 0 && at[r] - (r ? at[r - 1] : 0u) <= kSpLongRow) d.rp[r] = (to << kKsListBits) | len;
+    p0 = np0;
+    p1 = np1;
+    x = nx;
+    w = nw;
+  }
+}
+
 inline uint32_t band_rows(uint32_t n) { return n ? std::max(1u, std::min(n, kSpBandEntries / n)) : 1u; }
 
 // Counts (kPlace false) or places (kPlace true) the entries of one tile of a
@@ -833,6 +1001,11 @@ size_t child_tmp_bytes(const SpNode& nd) {
   return carve_size(nd.m * 8) + 2 * carve_size(nd.m * 4) + 2 * carve_size((size_t)nd.n * 4) +
          carve_size((nd.m + kSpTile - 1) / kSpTile * 4);
 }
+size_t list_bytes(const SpNode& nd) {
+  const size_t es = nd.w32 ? 4 : 8;
+  return carve_size((size_t)nd.n * es) + carve_size((size_t)nd.n * 4) + 2 * carve_size(nd.m * 4) +
+         2 * carve_size(nd.m * 2 * es) + sizeof(SpRows<int64_t>);
+}
 size_t dense_bytes(const SpNode& nd) {
   const uint32_t bands = (nd.n + band_rows(nd.n) - 1) / band_rows(nd.n);
   const size_t es = nd.w32 ? 4 : 8, st = nd.w32 ? ks_stride<uint32_t>(nd.n) : nd.n;
@@ -856,6 +1029,8 @@ int band_attr(cac_ctx* ctx) {
     if (err == hipSuccess)
       err = hipFuncSetAttribute((const void*)k_sp_band_build<E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)(kSpBandEntries * sizeof(E)));
+    if (err == hipSuccess)
+      err = hipFuncSetAttribute((const void*)k_sp_rows<E>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSpRowsLds);
   });
   CAC_HIP(ctx, err);
   return CAC_OK;
@@ -871,10 +1046,69 @@ struct SpRun {
   // Densifies nodes in batches that fit the free memory (matrices plus the
   // dense engine's level buffers) and runs the dense engine on them.
   int dense(const std::vector<SpNode>& nodes) {
-    std::vector<SpNode> kind[2];
-    for (const SpNode& nd : nodes) kind[nd.w32 ? 1 : 0].push_back(nd);
+    std::vector<SpNode> kind[4];
+    for (const SpNode& nd : nodes)
+      kind[(nd.w32 ? 1 : 0) + (nodes.size() >= kListNodes && as_lists(nd.n, nd.m) ? 2 : 0)].push_back(nd);
     int rc = dense_typed<uint32_t>(kind[1]);
-    return rc ? rc : dense_typed<int64_t>(kind[0]);
+    if (rc == CAC_OK) rc = dense_typed<int64_t>(kind[0]);
+    if (rc == CAC_OK) rc = lists_typed<uint32_t>(kind[3]);
+    if (rc == CAC_OK) rc = lists_typed<int64_t>(kind[2]);
+    return rc;
+  }
+
+  // The same for nodes that go as row lists.
+  template <typename E>
+  int lists_typed(const std::vector<SpNode>& nodes) {
+    typedef SpRows<E> Rows;
+    if (nodes.empty()) return CAC_OK;
+    int rc0 = band_attr<E>(ctx);
+    if (rc0) return rc0;
+    size_t i0 = 0;
+    while (i0 < nodes.size()) {
+      size_t avail = 0;
+      int rc = device_memory_available(ctx, &avail);
+      if (rc) return rc;
+      avail += ctx->sp_dense_bytes;
+      const size_t budget = (size_t)(0.6 * (double)avail);
+      size_t i1 = i0, bytes = 256, lists = 256;
+      while (i1 < nodes.size() && i1 - i0 < 4096) {
+        const size_t b = list_bytes(nodes[i1]) + ks_live_bytes_per_root(nodes[i1].n, sizeof(E) == 4);
+        if (i1 > i0 && bytes + b > budget) break;
+        bytes += b;
+        lists += list_bytes(nodes[i1]);
+        ++i1;
+      }
+      const size_t count = i1 - i0;
+      rc = grow_buffer(ctx, &ctx->sp_dense_buf, &ctx->sp_dense_bytes, lists);
+      if (rc) return rc;
+      BufPin pin(ctx, kBufSpDense);  // the lists are the dense roots
+      Carver cv(ctx->sp_dense_buf);
+      Rows* d_nodes = cv.take<Rows>(count);
+      std::vector<Rows> hr(count);
+      std::vector<KsRoot> roots;
+      for (size_t i = 0; i < count; ++i) {
+        const SpNode& nd = nodes[i0 + i];
+        Rows& d = hr[i];
+        d = {nd.edges, nd.m, nd.n, 0, cv.take<E>(nd.n), cv.take<uint32_t>(nd.n),
+             cv.take<uint16_t>(2 * nd.m), cv.take<E>(2 * nd.m), cv.take<uint16_t>(2 * nd.m), cv.take<E>(2 * nd.m)};
+        KsRoot r{nullptr, d.rsum, nd.n, nd.trial, nd.slot, nd.bound, nd.seed};
+        r.nid = nd.nid;
+        r.w32 = sizeof(E) == 4;
+        r.rp = d.rp;
+        r.cols = d.cols;
+        r.ws = d.ws;
+        roots.push_back(r);
+      }
+      CAC_HIP(ctx, hipMemcpyAsync(d_nodes, hr.data(), count * sizeof(Rows), hipMemcpyHostToDevice, s));
+      prof_begin(ctx, "sparse_rows", s);
+      hipLaunchKernelGGL(k_sp_rows<E>, dim3((unsigned)count), dim3(kSpBlock), kSpRowsLds, s, (const Rows*)d_nodes);
+      prof_end(ctx, s);
+      CAC_LAUNCH_CHECK(ctx, "sparse rows");
+      rc = ks_run(ctx, roots, d_results, s);
+      if (rc) return rc;
+      i0 = i1;
+    }
+    return CAC_OK;
   }
 
   template <typename E>
