@@ -34,6 +34,8 @@ struct KsRoot {
 // buffers (even depths in one, odd depths in the other, each grown to its
 // largest level: children arrays and row pools), by entry type.
 size_t ks_live_bytes_per_root(uint32_t n, bool w32);
+// Trials of t vertices whose first contractions (32-bit entries) fill the device once.
+size_t ks_wave_trials(const cac_ctx* ctx, uint32_t t);
 // Runs one trial per root (roots of different seeds share launches);
 // d_results[slot] (initialised to the root's bound) receives min(bound, leaves).
 int ks_run(cac_ctx* ctx, const std::vector<KsRoot>& roots, int64_t* d_results, hipStream_t s);

@@ -1098,7 +1098,7 @@ inline int contract_block(const cac_ctx* ctx, uint32_t s) {
   return B;
 }
 
-constexpr uint32_t kFewChildren = 256;  // the CU count of one MI355X
+constexpr uint32_t kFewChildren = 256;  // the CU count of an MI355X
 
 // Bump carving with 64-byte alignment (level buffers hold millions of small arrays).
 struct Carve64 {
@@ -1289,6 +1289,10 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
 }
 
 }  // namespace
+
+size_t ks_wave_trials(const cac_ctx* ctx, uint32_t t) {
+  return (size_t)kFewChildren * (2048 / contract_block(ctx, t)) / 2;  // 2048 threads per CU
+}
 
 size_t ks_live_bytes_per_root(uint32_t n, bool w32) {
   // children of every node at one depth with their pool rows; a depth's
