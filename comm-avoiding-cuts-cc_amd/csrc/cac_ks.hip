@@ -252,12 +252,12 @@ __global__ void __launch_bounds__(64) k_ks_sw(const KsLeaf<E>* __restrict__ leav
 // cbs[nb] U | red[(kPieces + 1) B/64] U | misc[8] u32 | rep[s] u16 | wslot[s] u16,
 // rep and cap padded to 16 bytes.  With 32-bit entries that is 8 s bytes: two
 // 1024-thread workgroups of s = 8192 share a CU.
-// A parent of row lists adds row[s] U, 16-byte aligned, and rp[s] u32.
+// A parent of row lists adds row[s] U, 16-byte aligned.
 template <typename E>
 __host__ __device__ inline size_t contract_lds_bytes(uint32_t s, int B, bool list = false) {
   const size_t e = sizeof(E), s8 = (s + 7) & ~size_t(7), nb2 = ((s + 63) / 64 + 3) & ~size_t(3);
   return e * s8 + e * nb2 + e * (size_t)(kPieces<E> + 1) * (B / 64) + 32 + 4 * s8 + 16 +
-         (list ? e * s8 + 4 * s8 + 16 : 0);
+         (list ? e * s8 + 16 : 0);
 }
 
 template <typename E>
@@ -269,7 +269,6 @@ struct KsLds {
   uint16_t* rep;    // padded entries past s hold 0xFFFF
   uint16_t* wslot;  // pool row of a merged row, or kNoRow
   ks_sum_t<E>* row;  // row lists: a row being assembled, 0 between; in a chain row cb
-  uint32_t* rp;      // row lists: c.rp
 };
 
 template <typename E>
@@ -317,7 +316,7 @@ __device__ inline void fetch_row(const KsChild<E>& c, const KsLds<E>& L, uint16_
       typedef const __attribute__((address_space(1))) E g_e;
       typedef const __attribute__((address_space(1))) uint16_t g_u16;
       constexpr uint32_t V = kPiece<E>, Q = kPieces<E>;
-      const uint32_t at = L.rp[r], len = at & kKsListLen;
+      const uint32_t at = __builtin_amdgcn_readfirstlane(c.rp[r]), len = at & kKsListLen;
       g_u16* cols = (g_u16*)c.cols + (at >> kKsListBits);
       g_e* ws = (g_e*)c.ws + (at >> kKsListBits);
       for (uint32_t p = threadIdx.x; p < len; p += B) L.row[cols[p]] = (U)ws[p];
@@ -439,10 +438,13 @@ __device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uin
 // thread keeps (the picked row and the last merged row) take 16 registers and
 // the kernel fits 64 (8 waves: two 1024-thread workgroups per CU).  64-bit
 // entries take 32: at most 96 registers below 1024 threads (5 waves; at 80 the
-// kernel spills and is slower).  Row lists: what their LDS leaves at about 1500
-// vertices, 6 and 4.
+// kernel spills and is slower).  Row lists in 32-bit entries: 64 registers from 256
+// threads up, for 8 workgroups per CU of up to 1700 vertices although a few values
+// spill (Watts-Strogatz, 32000 vertices: 34.1 ms, 38.2 with 80 registers and 6
+// workgroups), 80 below, where LDS leaves 6 waves.
 template <int B, bool kList, typename E>
-constexpr int kContractWaves = sizeof(E) == 4 ? (kList ? 6 : 8) : B >= 1024 ? 1 : kList ? 4 : 5;
+constexpr int kContractWaves =
+    sizeof(E) == 4 ? (kList && B < 256 ? 6 : 8) : B >= 1024 ? 1 : kList ? 4 : 5;
 
 // ---- chains ------------------------------------------------------------------
 // With a parent of row lists nearly every merge of a sparse graph joins the heavy
@@ -452,7 +454,7 @@ constexpr int kContractWaves = sizeof(E) == 4 ? (kList ? 6 : 8) : B >= 1024 ? 1 
 // merge by the block assembles rows and meets barriers.  The class's columns keep
 // their label, cb at the chain's start, while its index `at` moves; chain_close
 // puts the row back in u and the index in rep.  One hop is a chain of LDS and list
-// loads: the 7974 children of 3987 such roots take 11.4 ms, 21.4 by the block alone
+// loads: the 7974 children of 3987 such roots take 10.5 ms, 21.4 by the block alone
 // (16.1 ms for 6472 as matrices).
 template <int B, typename E>
 __device__ void chain_open(const KsChild<E>& c, const KsLds<E>& L, uint32_t qc, const E (&u)[kKsChunk]) {
@@ -513,7 +515,7 @@ __device__ inline ListHead<E> list_head(const KsChild<E>& c, const KsLds<E>& L, 
   typedef const __attribute__((address_space(1))) E g_e;
   typedef const __attribute__((address_space(1))) uint16_t g_u16;
   ListHead<E> h;
-  const uint32_t at = readlane_u32(L.rp[y], 0);
+  const uint32_t at = __builtin_amdgcn_readfirstlane(c.rp[__builtin_amdgcn_readfirstlane(y)]);
   h.p0 = at >> kKsListBits;
   h.p1 = h.p0 + (at & kKsListLen);
   const uint32_t p = h.p0 + (threadIdx.x & 63);
@@ -750,9 +752,7 @@ __global__ void __launch_bounds__(B, (kContractWaves<B, kList, E>))
   L.wslot = L.rep + s8;
   if constexpr (kList) {
     L.row = (U*)(((uintptr_t)(L.wslot + s8) + 15) & ~uintptr_t(15));
-    L.rp = (uint32_t*)(L.row + s8);
     for (uint32_t x = threadIdx.x; x < s8; x += B) L.row[x] = 0;
-    for (uint32_t x = threadIdx.x; x < s; x += B) L.rp[x] = c.rp[x];
   }
 
   for (uint32_t x = threadIdx.x; x < s8; x += B) {

@@ -833,6 +833,119 @@ __device__ uint64_t densify_edges(const TrialScratch& S, uint32_t k, const uint3
   return best;
 }
 
+// The contracted graph of a packed trial as row lists: most edges touch h and are
+// summed in its row in LDS; the edges between others are counted (in at), placed
+// row by row, and the entries of a row's columns added up by a wavefront in an LDS
+// row of its own, where the labels were.  False, with at and h_row 0 again, when
+// the lists exceed their room.  4987 trials of Watts-Strogatz n = 32000, t = 1433:
+// 11.6 ms as matrices, 5.5 as lists, and the contractions 25.6 and 18.7 ms.
+__device__ bool trial_lists(const TrialScratch& S, uint32_t k, const uint16_t* lab, uint32_t lab_bytes, uint32_t* at,
+                            uint32_t* h_row, const __attribute__((address_space(1))) uint32_t* list,
+                            const __attribute__((address_space(1))) uint32_t* pre, uint32_t count, uint32_t wu,
+                            uint32_t h, uint32_t* wtot, uint64_t* best_out) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const TrialLists T(S.mat, k, kListShare);
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < count; i += kSmpBlock) {
+    const uint32_t x = list[i];
+    const uint32_t a = lab[x & 0xFFFFu], b = lab[x >> 16];
+    if (a == b) continue;
+    const uint32_t w = wu != 0 ? wu : pre[i] - (i > 0 ? pre[i - 1] : 0u);
+    if (w == 0) continue;
+    if (a == h || b == h) {
+      atomicAdd(&h_row[a == h ? b : a], w);
+    } else {
+      atomicAdd(&at[a], 1u);
+      atomicAdd(&at[b], 1u);
+    }
+  }
+  __syncthreads();
+  static_assert(kKsListMax <= 2 * kSmpBlock, "two rows per thread");
+  const uint32_t r0 = 2 * threadIdx.x;
+  const uint32_t c0 = r0 < k ? at[r0] : 0u, c1 = r0 + 1 < k ? at[r0 + 1] : 0u;
+  const uint32_t inc = wave_incl_scan<uint32_t>(c0 + c1);
+  if (lane == 63) wtot[wave] = inc;
+  __syncthreads();
+  uint32_t before = inc - c0 - c1, total = 0;
+  for (int w = 0; w < kSmpWaves; ++w) {
+    if (w < wave) before += wtot[w];
+    total += wtot[w];
+  }
+  __syncthreads();
+  if (total + 2 * k > T.cap) {
+    for (uint32_t r = threadIdx.x; r < k; r += kSmpBlock) at[r] = h_row[r] = 0;
+    return false;
+  }
+  if (r0 < k) at[r0] = before;
+  if (r0 + 1 < k) at[r0 + 1] = before + c0;
+  if (threadIdx.x == 0) wtot[0] = 0;  // entries handed out
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < count; i += kSmpBlock) {
+    const uint32_t x = list[i];
+    const uint32_t a = lab[x & 0xFFFFu], b = lab[x >> 16];
+    if (a == b || a == h || b == h) continue;
+    const uint32_t w = wu != 0 ? wu : pre[i] - (i > 0 ? pre[i - 1] : 0u);
+    if (w == 0) continue;
+    const uint32_t p = atomicAdd(&at[a], 1u), q = atomicAdd(&at[b], 1u);
+    T.pcols[p] = (uint16_t)b;
+    T.pws[p] = w;
+    T.pcols[q] = (uint16_t)a;
+    T.pws[q] = w;
+  }
+  block_sync_global();
+  const uint32_t teams = min((uint32_t)kSmpWaves, lab_bytes / (4 * k));  // at least one: n >= 2 k
+  uint32_t* acc = (uint32_t*)lab;
+  for (uint32_t x = threadIdx.x; x < teams * k; x += kSmpBlock) acc[x] = 0;
+  __syncthreads();
+  uint64_t best = ~0ull;
+  uint32_t* rsum = (uint32_t*)S.rsum;
+  if ((uint32_t)wave < teams) {
+    acc += (size_t)wave * k;
+    const uint64_t below = (1ull << lane) - 1;
+    for (uint32_t r = wave; r < k; r += teams) {
+      const uint32_t p0 = r ? at[r - 1] : 0u, p1 = at[r];  // the cursors end at the rows' ends
+      for (uint32_t p = p0 + lane; p < p1; p += 64) atomicAdd(&acc[T.pcols[p]], T.pws[p]);
+      uint32_t to = 0, len = 0, sum = 0;
+      if (lane == 0) to = atomicAdd(&wtot[0], r == h ? k : p1 - p0 + 1);
+      to = readlane_u32(to, 0);
+      // row h: its LDS row; another: its own entries, then the one of column h
+      const uint32_t e0 = r == h ? 0u : p0, e1 = r == h ? k : p1 + 1;
+      for (uint32_t e = e0; e < e1; e += 64) {
+        const uint32_t p = e + lane;
+        uint32_t x = 0, v = 0;
+        if (r == h) {
+          x = p;
+          v = p < k ? h_row[p] : 0u;  // h_row[h] is 0
+        } else if (p < p1) {
+          x = T.pcols[p];
+          v = atomicExch(&acc[x], 0u);  // weights are at least 1
+        } else if (p == p1) {
+          x = h;
+          v = h_row[r];
+        }
+        const uint64_t mask = __ballot(v != 0);
+        if (v != 0) {
+          const uint32_t d = to + len + (uint32_t)__popcll(mask & below);
+          T.cols[d] = (uint16_t)x;
+          T.ws[d] = v;
+        }
+        len += (uint32_t)__popcll(mask);
+        sum += v;
+      }
+      sum = wave_sum<uint32_t>(sum);
+      if (lane == 0) {
+        T.rp[r] = (to << kKsListBits) | len;
+        rsum[r] = sum;
+      }
+      best = sum < best ? sum : best;
+    }
+  }
+  if (threadIdx.x == 0) S.live[1] = 2;
+  *best_out = best;
+  return true;
+}
+
 // k_densify_trials of a packed trial: labels and row sums in LDS, and only the
 // edges that survived the trial's last scan (each that still joins two
 // super-vertices is among them), 4 bytes each and 4 of prefix, instead of the
@@ -857,7 +970,11 @@ __device__ uint64_t densify_packed(const TrialScratch& S, uint32_t k, unsigned c
   uint32_t* row_sum = lds_rows ? (uint32_t*)(smem + lab_bytes) : rsum;
   uint32_t* h_row = row_sum + k;  // lds_rows only
   const uint64_t cells = (uint64_t)st * k;
-  for (uint64_t i = threadIdx.x; i < cells / 4; i += kSmpBlock) ((uint4*)mat)[i] = make_uint4(0u, 0u, 0u, 0u);
+  auto zero_mat = [&]() {
+    for (uint64_t i = threadIdx.x; i < cells / 4; i += kSmpBlock) ((uint4*)mat)[i] = make_uint4(0u, 0u, 0u, 0u);
+  };
+  const bool may_list = lds_rows && k > kKsBase && k <= kKsListMax && n >= 2 * k;
+  if (!may_list) zero_mat();
   for (uint32_t r = threadIdx.x; r < (lds_rows ? 2 * k : k); r += kSmpBlock) row_sum[r] = 0;
   for (uint32_t v = threadIdx.x; v < (n + 1) / 2; v += kSmpBlock) ((uint32_t*)lab)[v] = S.lab[v];
   __syncthreads();
@@ -904,10 +1021,25 @@ __device__ uint64_t densify_packed(const TrialScratch& S, uint32_t k, unsigned c
         best_v = vb;
       }
     }
-    if (lane == 0) wtot[0] = best_v;
+    const uint64_t others = __ballot(a != b && a != best_v && b != best_v);
+    if (lane == 0) {
+      wtot[0] = best_v;
+      wtot[1] = (uint32_t)__popcll(others);
+    }
   }
   __syncthreads();
   const uint32_t h = lds_rows ? wtot[0] : kNoSlot;
+  if (may_list) {
+    // edges between others, by the sample; the lists hold them twice and h's row
+    // and column
+    const uint64_t guess = (uint64_t)count * wtot[1] / 64;
+    uint64_t best;
+    if (2 * (guess + k) <= (uint64_t)k * k / kListShare * 3 / 2 &&
+        trial_lists(S, k, lab, lab_bytes, row_sum, h_row, list, pre, count, wu, h, wtot, &best))
+      return best;
+    zero_mat();
+    block_sync_global();
+  }
 #pragma unroll 4
   for (uint32_t i = threadIdx.x; i < count; i += kSmpBlock) {
     const uint32_t x = list[i];
@@ -1662,7 +1794,9 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     std::vector<uint32_t> nvs(nb);
     std::vector<int64_t> hb(nb);
     std::vector<unsigned long long> totals(nb);
+    std::vector<uint32_t> live(2 * nb, 0u);
     if (rc == CAC_OK) {
+      if (pack_bytes) (void)hipMemcpyAsync(live.data(), d_live, 8 * nb, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(nvs.data(), d_nv, nb * 4, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(hb.data(), d_bounds, nb * 8, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s);
@@ -1672,9 +1806,18 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     if (rc == CAC_OK) {
       std::vector<KsRoot> roots;
       for (size_t i = 0; i < nb; ++i)
-        if (nvs[i] >= 2 && nvs[i] <= scr[i].t)
-          roots.push_back({scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed, 1,
-                           totals[scr[i].total - d_totals] < kTrialW32Total});
+        if (nvs[i] >= 2 && nvs[i] <= scr[i].t) {
+          KsRoot r{scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed, 1,
+                   totals[scr[i].total - d_totals] < kTrialW32Total};
+          if (scr[i].pk && r.w32 && live[2 * i + 1] == 2) {
+            const TrialLists T(scr[i].mat, r.n, kListShare);
+            r.mat = nullptr;
+            r.rp = T.rp;
+            r.cols = T.cols;
+            r.ws = T.ws;
+          }
+          roots.push_back(r);
+        }
       rc = ks_run(ctx, roots, d_results, s);
     }
     (void)hipStreamSynchronize(s);

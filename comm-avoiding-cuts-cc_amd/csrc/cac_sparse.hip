@@ -650,7 +650,6 @@ struct SpDense {
 // 11400 nodes of karger_stein on a Watts-Strogatz graph of 48000 vertices with 16
 // edges each, rows of n / 23, took 46 ms to fill and 72 to contract as matrices and
 // take 20 and 39 as lists.
-constexpr uint64_t kListShare = 20;
 constexpr size_t kListNodes = 128;
 static_assert((uint64_t)kKsListMax * kKsListMax / kListShare < (1ull << (32 - kKsListBits)) && kKsListMax <= kKsListLen + 1,
               "entry index and row length share 32 bits");

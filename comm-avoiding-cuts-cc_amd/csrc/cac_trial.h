@@ -41,7 +41,22 @@ struct TrialScratch {
   // of its last scan and in live[1] whether they are its own list's.
   const uint32_t* pk;
   const uint32_t* pre0;
-  uint32_t* live;
+  uint32_t* live;  // live[1] = 2 when the contracted graph is left as row lists (TrialLists) in mat's place
+};
+
+// Row lists of a packed trial's contracted graph (the form of KsRoot) in the t^2
+// words of its matrix; cap entries, and as many placed ones before they are merged.
+struct TrialLists {
+  uint32_t cap;
+  uint32_t *rp, *ws, *pws;
+  uint16_t *cols, *pcols;
+  __host__ __device__ TrialLists(void* mat, uint32_t k, uint32_t share) : cap(k * k / share) {
+    rp = (uint32_t*)mat;
+    ws = rp + k;
+    pws = ws + cap;
+    cols = (uint16_t*)(pws + cap);
+    pcols = cols + cap;
+  }
 };
 
 // The contracted matrix's entries add up to at most twice the graph's total
