@@ -438,13 +438,13 @@ __device__ bool ks_merge(const KsChild<E>& c, const KsLds<E>& L, uint32_t a, uin
 // thread keeps (the picked row and the last merged row) take 16 registers and
 // the kernel fits 64 (8 waves: two 1024-thread workgroups per CU).  64-bit
 // entries take 32: at most 96 registers below 1024 threads (5 waves; at 80 the
-// kernel spills and is slower).  Row lists in 32-bit entries: 64 registers from 256
-// threads up, for 8 workgroups per CU of up to 1700 vertices although a few values
+// kernel spills and is slower).  Row lists in 32-bit entries: 64 registers at 256
+// threads, for 8 workgroups per CU of up to 1700 vertices although a few values
 // spill (Watts-Strogatz, 32000 vertices: 34.1 ms, 38.2 with 80 registers and 6
-// workgroups), 80 below, where LDS leaves 6 waves.
+// workgroups), 80 otherwise, where LDS leaves 6 waves.
 template <int B, bool kList, typename E>
 constexpr int kContractWaves =
-    sizeof(E) == 4 ? (kList && B < 256 ? 6 : 8) : B >= 1024 ? 1 : kList ? 4 : 5;
+    sizeof(E) == 4 ? (kList && B != 256 ? 6 : 8) : B >= 1024 ? 1 : kList ? 4 : 5;
 
 // ---- chains ------------------------------------------------------------------
 // With a parent of row lists nearly every merge of a sparse graph joins the heavy
@@ -1329,6 +1329,12 @@ int contract_attr(cac_ctx* ctx) {
     if (err == hipSuccess)
       err = hipFuncSetAttribute((const void*)k_ks_contract<512, false, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)contract_lds_bytes<E>(512 * kKsChunk, 512));
+    if (err == hipSuccess)
+      err = hipFuncSetAttribute((const void*)k_ks_contract<512, true, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)contract_lds_bytes<E>(kKsListMax, 512, true));
+    if (err == hipSuccess)
+      err = hipFuncSetAttribute((const void*)k_ks_contract<1024, true, E>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)contract_lds_bytes<E>(kKsListMax, 1024, true));
     const void* compact[] = {(const void*)k_ks_compact<1024, 64, false, E>,
                              (const void*)k_ks_compact<1024, 1024, false, E>,
                              (const void*)k_ks_compact<512, 512, false, E>,

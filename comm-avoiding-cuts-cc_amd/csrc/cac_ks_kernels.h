@@ -39,7 +39,8 @@ constexpr uint32_t kKsBase = 128;        // base_case_size (co_mincut.h:24)
 constexpr uint32_t kKsMaxS = 8192;       // LDS holds caps, reps and row slots for s <= this
 constexpr uint32_t kKsChunk = 8;         // row entries per thread (s <= 8 * block size), x = k * B + t
 constexpr uint32_t kKsUnit = 64;         // a pool row is padded to whole units of 64 entries
-constexpr uint32_t kKsListMax = 2048;    // a root of at most this many vertices may be given as row lists
+constexpr uint32_t kKsListMax = 4096;    // a root of at most this many vertices may be given as row lists
+constexpr uint32_t kListBuildMax = 2048;  // lists built by one workgroup: two rows per thread
 constexpr uint64_t kListShare = 20;      // a root goes as row lists at n / kListShare entries a row or fewer
 constexpr uint32_t kKsListBits = 12, kKsListLen = (1u << kKsListBits) - 1;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;

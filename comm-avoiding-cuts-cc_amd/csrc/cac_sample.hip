@@ -860,7 +860,7 @@ __device__ bool trial_lists(const TrialScratch& S, uint32_t k, const uint16_t* l
     }
   }
   __syncthreads();
-  static_assert(kKsListMax <= 2 * kSmpBlock, "two rows per thread");
+  static_assert(kListBuildMax <= 2 * kSmpBlock, "two rows per thread");
   const uint32_t r0 = 2 * threadIdx.x;
   const uint32_t c0 = r0 < k ? at[r0] : 0u, c1 = r0 + 1 < k ? at[r0 + 1] : 0u;
   const uint32_t inc = wave_incl_scan<uint32_t>(c0 + c1);
@@ -973,7 +973,7 @@ __device__ uint64_t densify_packed(const TrialScratch& S, uint32_t k, unsigned c
   auto zero_mat = [&]() {
     for (uint64_t i = threadIdx.x; i < cells / 4; i += kSmpBlock) ((uint4*)mat)[i] = make_uint4(0u, 0u, 0u, 0u);
   };
-  const bool may_list = lds_rows && k > kKsBase && k <= kKsListMax && n >= 2 * k;
+  const bool may_list = lds_rows && k > kKsBase && k <= kListBuildMax && n >= 2 * k;
   if (!may_list) zero_mat();
   for (uint32_t r = threadIdx.x; r < (lds_rows ? 2 * k : k); r += kSmpBlock) row_sum[r] = 0;
   for (uint32_t v = threadIdx.x; v < (n + 1) / 2; v += kSmpBlock) ((uint32_t*)lab)[v] = S.lab[v];
@@ -1079,6 +1079,53 @@ __device__ uint64_t densify_packed(const TrialScratch& S, uint32_t k, unsigned c
     best = acc < best ? acc : best;
   }
   return best;
+}
+
+__host__ __device__ inline bool rows_from_matrix(uint32_t k) { return k > kKsBase && k <= kKsListMax; }
+
+__global__ void k_zero_live(uint32_t* live, uint32_t count) {
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) live[i] = 0;
+}
+
+// Row lists of the trials that are not packed, from their 32-bit matrices, a
+// wavefront per row: one read of the matrix, its rows' second reads from cache.  A
+// contraction with the lists follows the heavy vertex's merges in one wavefront at
+// 1.3 us each; by the block with rows of the matrix they take 2.5 us, and a served
+// group of a few large graphs is as long as one child's merges.
+__global__ void __launch_bounds__(256) k_trial_rows(const TrialScratch* __restrict__ scratch) {
+  const TrialScratch S = scratch[blockIdx.y];
+  const uint32_t k = *S.nv_out;
+  if (k > S.t || !rows_from_matrix(k) || !trial_w32(S) || trial_packed(S)) return;
+  const uint32_t st = ks_stride<uint32_t>(k);
+  const uint32_t* mat = (const uint32_t*)S.mat;
+  const TrialLists T((uint32_t*)S.mat + (size_t)st * k, k, kListShare);
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint32_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < k; r += gridDim.x * 4) {
+    const uint32_t* row = mat + (size_t)r * st;
+    uint32_t len = 0;
+#pragma unroll 4
+    for (uint32_t x = lane; x < k; x += 64) len += row[x] != 0;
+    len = wave_sum<uint32_t>(len);
+    uint32_t to = 0;
+    if (lane == 0) {
+      to = atomicAdd(&S.live[0], len);
+      if (to + len > T.cap) S.live[1] = 3;
+      else T.rp[r] = (to << kKsListBits) | len;
+    }
+    to = readlane_u32(to, 0);
+    if (to + len > T.cap) return;  // too dense for lists
+    for (uint32_t b = 0; b < k; b += 64) {
+      const uint32_t x = b + lane;
+      const uint32_t v = x < k ? row[x] : 0u;
+      const uint64_t mask = __ballot(v != 0);
+      if (v != 0) {
+        const uint32_t d = to + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+        T.cols[d] = (uint16_t)x;
+        T.ws[d] = v;
+      }
+      to += (uint32_t)__popcll(mask);
+    }
+  }
 }
 
 // Rank the canonical labels, accumulate the surviving edges into the k x k
@@ -1757,6 +1804,10 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     if (rc) return rc;
     e = hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "job descriptors");
+    bool from_matrix = false;  // some trial's lists may come from its matrix
+    for (size_t i = 0; i < nb; ++i) from_matrix = from_matrix || (!scr[i].pk && scr[i].t > kKsBase);
+    if (rc == CAC_OK && from_matrix)
+      hipLaunchKernelGGL(k_zero_live, dim3(grid_for(2 * nb, 256, 64)), dim3(256), 0, s, d_live, (uint32_t)(2 * nb));
     if (rc == CAC_OK && wide) {
       prof_begin(ctx, "wide_sample", s);
       rc = wide_sample(ctx, scr, d_scr, wide_work, s);
@@ -1791,12 +1842,18 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       e = hipGetLastError();
       if (e != hipSuccess) rc = hip_fail(ctx, e, "sampling kernels");
     }
+    if (rc == CAC_OK && from_matrix) {
+      prof_begin(ctx, "trial_rows", s);
+      hipLaunchKernelGGL(k_trial_rows, dim3(std::max(4u, (unsigned)(4096 / nb)), (unsigned)nb), dim3(256), 0, s,
+                         (const TrialScratch*)d_scr);
+      prof_end(ctx, s);
+    }
     std::vector<uint32_t> nvs(nb);
     std::vector<int64_t> hb(nb);
     std::vector<unsigned long long> totals(nb);
     std::vector<uint32_t> live(2 * nb, 0u);
     if (rc == CAC_OK) {
-      if (pack_bytes) (void)hipMemcpyAsync(live.data(), d_live, 8 * nb, hipMemcpyDeviceToHost, s);
+      if (pack_bytes || from_matrix) (void)hipMemcpyAsync(live.data(), d_live, 8 * nb, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(nvs.data(), d_nv, nb * 4, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(hb.data(), d_bounds, nb * 8, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s);
@@ -1809,8 +1866,11 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
         if (nvs[i] >= 2 && nvs[i] <= scr[i].t) {
           KsRoot r{scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed, 1,
                    totals[scr[i].total - d_totals] < kTrialW32Total};
-          if (scr[i].pk && r.w32 && live[2 * i + 1] == 2) {
-            const TrialLists T(scr[i].mat, r.n, kListShare);
+          const bool in_place = scr[i].pk && live[2 * i + 1] == 2;
+          const bool behind = !scr[i].pk && from_matrix && rows_from_matrix(r.n) && live[2 * i + 1] == 0;
+          if (r.w32 && (in_place || behind)) {
+            const size_t at = behind ? (size_t)ks_stride<uint32_t>(r.n) * r.n : 0;
+            const TrialLists T((uint32_t*)scr[i].mat + at, r.n, kListShare);
             r.mat = nullptr;
             r.rp = T.rp;
             r.cols = T.cols;

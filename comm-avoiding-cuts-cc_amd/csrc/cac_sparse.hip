@@ -651,10 +651,10 @@ struct SpDense {
 // edges each, rows of n / 23, took 46 ms to fill and 72 to contract as matrices and
 // take 20 and 39 as lists.
 constexpr size_t kListNodes = 128;
-static_assert((uint64_t)kKsListMax * kKsListMax / kListShare < (1ull << (32 - kKsListBits)) && kKsListMax <= kKsListLen + 1,
+static_assert((uint64_t)kListBuildMax * kListBuildMax / kListShare < (1ull << (32 - kKsListBits)) && kListBuildMax <= kKsListLen + 1,
               "entry index and row length share 32 bits");
 inline bool as_lists(uint32_t n, uint64_t m) {
-  return n > kKsBase && n <= kKsListMax && 2 * m * kListShare <= (uint64_t)n * n;
+  return n > kKsBase && n <= kListBuildMax && 2 * m * kListShare <= (uint64_t)n * n;
 }
 
 // The lists of a node's rows, the form of a sparse node.  One workgroup counts the
@@ -684,9 +684,9 @@ template <typename E>
 __global__ void __launch_bounds__(kSpBlock, 8) k_sp_rows(const SpRows<E>* __restrict__ nodes) {
   typedef typename SpRows<E>::A A;
   extern __shared__ __align__(16) unsigned char sp_rows_lds[];  // kSpRowsLds
-  __shared__ uint32_t at[kKsListMax];
+  __shared__ uint32_t at[kListBuildMax];
   __shared__ uint32_t wtot[kSpWaves], cursor, longs, long_len;
-  __shared__ uint16_t long_row[kKsListMax * (kKsListMax / kListShare) / kSpLongRow];
+  __shared__ uint16_t long_row[kListBuildMax * (kListBuildMax / kListShare) / kSpLongRow];
   const SpRows<E> d = nodes[blockIdx.x];
   const uint32_t n = d.n, m = (uint32_t)d.m;
   A* acc = (A*)sp_rows_lds;
@@ -705,7 +705,7 @@ __global__ void __launch_bounds__(kSpBlock, 8) k_sp_rows(const SpRows<E>* __rest
     atomicAdd(&acc[x.v], (A)x.w);
   }
   __syncthreads();
-  static_assert(kKsListMax == 2 * kSpBlock, "two rows per thread");
+  static_assert(kListBuildMax == 2 * kSpBlock, "two rows per thread");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t r0 = 2 * threadIdx.x;
   const uint32_t c0 = r0 < n ? at[r0] : 0u, c1 = r0 + 1 < n ? at[r0 + 1] : 0u;

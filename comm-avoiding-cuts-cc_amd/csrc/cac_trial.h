@@ -43,6 +43,8 @@ struct TrialScratch {
   const uint32_t* pre0;
   uint32_t* live;  // live[1] = 2 when the contracted graph is left as row lists (TrialLists) in mat's place
 };
+// Of a trial that is not packed, once k_trial_rows has run: live[1] = 0 when its
+// 32-bit matrix is followed by its row lists (live[0] entries), else 3.
 
 // Row lists of a packed trial's contracted graph (the form of KsRoot) in the t^2
 // words of its matrix; cap entries, and as many placed ones before they are merged.

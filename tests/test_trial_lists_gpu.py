@@ -2,7 +2,8 @@
 super-vertices, at least twice as many vertices, most surviving edges at one
 super-vertex), and the matrix form on either side of those limits and where the
 lists exceed their room: raw cuts equal the oracle's.  Ring lattices with random
-chords and two communities with a weak link between them."""
+chords and two communities with a weak link between them.  Above 2^16 vertices and
+in the wide form the lists come from the matrix, up to 4096 super-vertices."""
 import numpy as np
 import pytest
 
@@ -35,4 +36,17 @@ def test_trial_lists(ctx, orc, n, d, t, kind, weights):
     raw = ctx.sqrt_cut_trials(e, n, t, 7, 2, 4)
     want = [orc.sqrt_trial(n, e, t, 7, 2 + i, 0) for i in range(4)]
     print(f"trial lists {kind} {weights} n {n} m {len(e)} t {t}: cuts {sorted(set(want))}", flush=True)
+    assert raw.tolist() == want
+
+
+@pytest.mark.parametrize("n,d,t", [(65537, 3, 128), (65537, 3, 129), (70001, 3, 2049), (70001, 4, 4096),
+                                   (70001, 4, 4097), (150000, 7, 1100), (70001, 1, 1000)])
+@pytest.mark.parametrize("kind", ["ring", "two"])
+@pytest.mark.parametrize("scale", [1, 2**20])
+def test_lists_from_matrix(ctx, orc, n, d, t, kind, scale):
+    e = _graph(np.random.default_rng(n + t), kind, n, d, "mixed")
+    e[:, 2] *= np.uint64(scale)  # 2^20: a total of 2^31 or more keeps 64-bit matrices
+    raw = ctx.sqrt_cut_trials(e, n, t, 7, 2, 2)
+    want = [orc.sqrt_trial(n, e, t, 7, 2 + i, 0) for i in range(2)]
+    print(f"lists from matrix {kind} {scale} n {n} m {len(e)} t {t}: cuts {sorted(set(want))}", flush=True)
     assert raw.tolist() == want
