@@ -652,14 +652,16 @@ __device__ uint32_t pick_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t 
   return p;
 }
 
-// Rows of the PR pass from i = cb on: while the row to check is row cb, its first
-// entry of weight >= bound leads to a single vertex, and more than two vertices are
-// left, the class takes that vertex's index.  Returns the row to check next (maybe
-// i itself), kNoSlot if none; u, cb and nv follow.
+// Rows of the PR pass from i = cb on, while more than two vertices are left: row cb
+// whose first entry of weight >= bound leads to a single vertex (the class takes its
+// index), and single vertices whose first such entry leads to the class.  Returns
+// the row left to the block, kNoSlot if none; u, cb and nv follow.
 template <int B, typename E>
 __device__ uint32_t pr_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t i, ks_sum_t<E> bound, uint32_t qc,
                              E (&u)[kKsChunk], uint32_t& cb, uint32_t& nv) {
   typedef ks_sum_t<E> U;
+  typedef const __attribute__((address_space(1))) E g_e;
+  typedef const __attribute__((address_space(1))) uint16_t g_u16;
   constexpr uint32_t V = kPiece<E>;
   typedef U row_piece __attribute__((ext_vector_type(V)));
   const uint32_t s = c.s, label = cb, lane = threadIdx.x & 63;
@@ -669,43 +671,65 @@ __device__ uint32_t pr_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t i,
     ListHead<E> ahead;           // of vertex `guess`, the entry after the one taken
     uint32_t guess = kNoSlot;
     while (nv > 2) {
-      uint32_t first = kNoSlot, second = kNoSlot;
-      for (uint32_t b = from & ~(64 * V - 1); b < s && first == kNoSlot; b += 64 * V) {
-        const uint32_t x = b + lane * V;
-        const row_piece t = x < s ? *(const row_piece*)(L.row + x) : row_piece{};
-        uint32_t bits = 0;
+      uint32_t first = kNoSlot, second = kNoSlot, low = kNoSlot;
+      if (i == at) {
+        for (uint32_t b = from & ~(64 * V - 1); b < s && first == kNoSlot; b += 64 * V) {
+          const uint32_t x = b + lane * V;
+          const row_piece t = x < s ? *(const row_piece*)(L.row + x) : row_piece{};
+          uint32_t bits = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < V; ++k) bits |= t[k] >= bound ? 1u << k : 0u;
-        uint64_t hit = __ballot(bits != 0);
-        if (hit) {
-          const int l = __ffsll((long long)hit) - 1;
-          first = b + (uint32_t)l * V + (uint32_t)(__ffs((int)readlane_u32(bits, l)) - 1);
-          if ((int)lane == l) bits &= bits - 1;
-          hit = __ballot(bits != 0);
+          for (uint32_t k = 0; k < V; ++k) bits |= t[k] >= bound ? 1u << k : 0u;
+          uint64_t hit = __ballot(bits != 0);
           if (hit) {
-            const int l2 = __ffsll((long long)hit) - 1;
-            second = b + (uint32_t)l2 * V + (uint32_t)(__ffs((int)readlane_u32(bits, l2)) - 1);
+            const int l = __ffsll((long long)hit) - 1;
+            first = b + (uint32_t)l * V + (uint32_t)(__ffs((int)readlane_u32(bits, l)) - 1);
+            if ((int)lane == l) bits &= bits - 1;
+            hit = __ballot(bits != 0);
+            if (hit) {
+              const int l2 = __ffsll((long long)hit) - 1;
+              second = b + (uint32_t)l2 * V + (uint32_t)(__ffs((int)readlane_u32(bits, l2)) - 1);
+            }
           }
         }
-      }
-      bool moved = false;
-      if (first != kNoSlot) {
-        if (!chain_single(L, first)) break;
-        const ListHead<E> h = guess == first ? ahead : list_head(c, L, first);
-        guess = second;
-        if (second != kNoSlot) ahead = list_head(c, L, second);
-        uint32_t low;
-        const U w = chain_add(c, L, first, h, label, bound, &low);
-        if (lane == 0) {
-          L.cap[first] += L.cap[at] - 2 * w;
-          L.cap[at] = 0;
+        if (first != kNoSlot) {
+          if (!chain_single(L, first)) break;
+          const ListHead<E> h = guess == first ? ahead : list_head(c, L, first);
+          guess = second;
+          if (second != kNoSlot) ahead = list_head(c, L, second);
+          const U w = chain_add(c, L, first, h, label, bound, &low);
+          if (lane == 0) {
+            L.cap[first] += L.cap[at] - 2 * w;
+            L.cap[at] = 0;
+          }
+          from = min(first + 1, low);
+          at = first;
+          --nv;
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        from = min(first + 1, low);
-        at = first;
-        --nv;
-        moved = true;
+      } else {
+        if (!chain_single(L, i)) break;
+        const ListHead<E> h = guess == i ? ahead : list_head(c, L, i);
+        uint32_t x = h.x;
+        U w = h.w;
+        for (uint32_t p = h.p0 + lane; p < h.p1; p += 64) {
+          if (p >= h.p0 + 64) {
+            x = ((g_u16*)c.cols)[p];
+            w = (U)((g_e*)c.ws)[p];
+          }
+          if (w >= bound && x < first) first = x;
+        }
+        first = wave_min<uint32_t>(first);
+        if (first != kNoSlot) {
+          if (readlane_u32((uint32_t)L.rep[first], 0) != label) break;
+          const U between = chain_add(c, L, i, h, label, bound, &low);
+          if (lane == 0) {
+            L.cap[at] += L.cap[i] - 2 * between;
+            L.cap[i] = 0;
+          }
+          from = min(from, low);
+          --nv;
+        }
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       // the next row to check: a live one, or the class itself if its index is past i
       uint32_t next = kNoSlot;
       for (uint32_t b = (i + 1) & ~63u; b < s && next == kNoSlot; b += 64) {
@@ -714,7 +738,11 @@ __device__ uint32_t pr_chain(const KsChild<E>& c, const KsLds<E>& L, uint32_t i,
         if (hit) next = b + (uint32_t)(__ffsll((long long)hit) - 1);
       }
       i = next;
-      if (!moved || next != at) break;
+      if (next == kNoSlot) break;
+      if (next != at && next != guess) {
+        guess = next;
+        ahead = list_head(c, L, next);
+      }
     }
     if (lane == 0) {
       L.misc[0] = i;
