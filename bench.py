@@ -257,7 +257,8 @@ def bench_c3(ctx, cac, trials: int, cpu_budget_s: float = 0.0):
                               f"graph, {per_trial:.1f} s on one core (cut {ref_cut}); x{trials} trials = "
                               f"{per_trial * trials:.0f} s per solve"}
     d_adj.free()
-    bytes_per_trial = 22.88e9  # sum over recursion children of 8 (s^2 + t'^2) + 8 * 128^2 per leaf
+    # sum over recursion children of 4 (s^2 + t'^2) + 4 * 128^2 per leaf: the total weight is below 2^32
+    bytes_per_trial = 11.44e9
     return {"workload": f"dense Karger-Stein, complete graph n={n}, weights U[1,42], {trials} trials, seed 0",
             "seconds_per_solve": dt, "trials_per_s": trials / dt, "cut": int(cut), "min_degree": deg_min,
             "raw_cuts_equal_bound": bool(np.all(raw == deg_min)),

@@ -100,7 +100,8 @@ int cac_memcpy_d2d(cac_ctx* ctx, void* dst, const void* src, size_t bytes, void*
 /* CAC_TUNE_KS_COMPACT_BLOCK: threads per workgroup of the dense Karger-Stein
  * compaction for children of t' vertices, keyed by class: key 512 holds
  * t' <= 512, keys 1024, 2048, 4096 and 8192 hold t' in (key/2, key].  value 0
- * restores the built-in 512; otherwise 256, 512 or 1024, CAC_EINVAL else.
+ * restores the built-in rule (256, and 512 where a parent row is above 16 KiB);
+ * otherwise 256, 512 or 1024, CAC_EINVAL else.
  * Results never depend on it. */
 #define CAC_TUNE_KS_COMPACT_BLOCK 4
 int cac_tune_set(cac_ctx* ctx, int knob, uint32_t key, int32_t value);
