@@ -9,13 +9,16 @@
 // target_number_of_vertices_for_contraction (co_mincut.cpp:18-20).
 //
 // Per level of the recursion tree:
-//   1. k_ks_contract<B>: one workgroup per child (B = 64, 256 or 1024 threads by
-//      size) draws s - t' picks, merges rows into pool rows, runs the PR pass and
-//      writes the lists of live rows, live columns and merged-away columns;
+//   1. k_ks_contract<B>: one workgroup per child (B = 64 to 1024 threads by size)
+//      draws s - t' picks, merges rows into pool rows, runs the PR pass and writes
+//      the lists of live rows, live columns and merged-away columns.  The parent is
+//      a matrix, or at the root the lists of its rows;
 //   2. k_ks_compact: teams of threads each fold a live row's merged-away columns
 //      into their representatives in LDS and write the child's row;
 //   3. children of at most 128 vertices are leaves: k_ks_cert settles most of them
-//      from row sums and maxima; k_ks_sw runs Stoer-Wagner on the rest.
+//      from row sums and maxima; k_ks_sw runs the phases of Stoer and Wagner with
+//      the contractions of Nagamochi and Ibaraki on the rest.
+// Entries are 32-bit where a root's total weight is below 2^32, else 64-bit.
 // Device memory for a level comes from two grow-only buffers of the context used
 // alternately (the parents live in one, the children in the other).
 #include <algorithm>

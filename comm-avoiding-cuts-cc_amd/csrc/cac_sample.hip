@@ -17,9 +17,12 @@
 //      counting its successful hooks;
 //   4. canonical relabel: every vertex takes the smallest original id of its
 //      super-vertex (hooks always attach the larger root under the smaller).
+// Graphs of at most 2^16 vertices and total weight below 2^31 are packed, and their
+// trials run in 32 bits with labels and forest in LDS (sample_packed).
 // Densification then ranks the canonical labels and accumulates the weights of
-// the surviving edges into a t x t int64 matrix (the merge of parallel edges),
-// which feeds one dense Karger-Stein trial per sqrt-cut trial.
+// the surviving edges into a t x t matrix, 32- or 64-bit (the merge of parallel
+// edges), or where they are few into the lists of its rows, which feeds one dense
+// Karger-Stein trial per sqrt-cut trial.
 #include <algorithm>
 #include <cmath>
 #include <functional>

@@ -17,7 +17,8 @@
 // is the node's edges in their order, relabelled by the rank of each
 // component's minimum id, loops dropped and parallel edges kept.  A node with
 // n <= 2048, or with m >= n^2/32 and n <= 8192, is densified (band by band in
-// LDS: every matrix entry written once) and continues in the dense engine under
+// LDS: every matrix entry written once), or turned into the lists of its rows where
+// many nodes with short rows come together, and continues in the dense engine under
 // its own node id.  Every node uses the trial's bound,
 // the minimum weighted degree of the input.
 #include <algorithm>
