@@ -1272,7 +1272,7 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 
 
 // Points scr[i].mixed and scr[i].total at a flag word and a total weight of its
-// graph (one per distinct edge list) and launches the kernels that set them;
+// graph (one per distinct graph) and launches the kernels that set them;
 // spans, flags and totals hold scr.size() entries.  Both are ready for any later
 // launch on s.
 // packed: the graphs' packed forms are carved from it (packed_bytes each), null:
@@ -1280,15 +1280,16 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d_spans, uint32_t* d_flags,
                        unsigned long long* d_totals, void* packed, hipStream_t s) {
   Carver pc(packed);
-  std::unordered_map<const cac_edge*, uint32_t> index;
+  std::unordered_map<GraphKey, uint32_t, GraphHash> index;
   std::vector<EdgeSpan> spans;
   uint64_t mmax = 0;
   for (TrialScratch& x : scr) {
-    auto it = index.find(x.edges);
+    const GraphKey key{x.edges, x.m, x.n};
+    auto it = index.find(key);
     uint32_t g = 0;
     if (it == index.end()) {
       g = (uint32_t)spans.size();
-      index.emplace(x.edges, g);
+      index.emplace(key, g);
       EdgeSpan sp{x.edges, x.m, d_flags + g, d_totals + g, nullptr, nullptr, nullptr};
       if (packed && x.n <= kPackMaxN && x.m < kPackMaxM) {
         sp.pk = pc.take<uint32_t>(x.m);
@@ -1727,13 +1728,13 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
   size_t b0 = 0;
   while (b0 < jobs.size() && rc == CAC_OK) {
     size_t nb = 0, sample_bytes = 0, ks_bytes = 0, wide_bytes = 0, pack_bytes = 0;
-    std::unordered_set<const cac_edge*> graphs;  // packed once per graph of the chunk
+    std::unordered_set<GraphKey, GraphHash> graphs;  // packed once per graph of the chunk
     const size_t cap = wide ? 4096 : kMaxJobsPerChunk;
     while (b0 + nb < jobs.size() && nb < cap) {
       const SqrtJob& j = jobs[b0 + nb];
       const size_t a = job_sample_bytes(j, job_dpr(ctx, j.n)), k = job_ks_bytes(j);
       const size_t wb = wide ? wide_trial_bytes(j.m, j.n) : 0;
-      const size_t pb = !wide && can_pack(j) && !graphs.count(j.edges) ? packed_bytes(j.m) : 0;
+      const size_t pb = !wide && can_pack(j) && !graphs.count({j.edges, j.m, j.n}) ? packed_bytes(j.m) : 0;
       // The packed lists live in the half of the Karger-Stein estimate (8 bytes an
       // entry) that a packed graph's 4-byte entries leave free, and count only
       // where they take more.  Counted in full, a served group, whose budget is
@@ -1742,7 +1743,7 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       const size_t saved = (ks_bytes + k) / 2;
       const size_t over = pack_bytes + pb > saved ? pack_bytes + pb - saved : 0;
       if (nb > 0 && sample_bytes + a + ks_bytes + k + wide_bytes + wb + over > budget) break;
-      if (pb) graphs.insert(j.edges);
+      if (pb) graphs.insert({j.edges, j.m, j.n});
       pack_bytes += pb;
       sample_bytes += a;
       ks_bytes += k;

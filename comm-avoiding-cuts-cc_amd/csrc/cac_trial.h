@@ -67,6 +67,23 @@ constexpr unsigned long long kTrialW32Total = 1ull << 31;
 __device__ inline bool trial_w32(const TrialScratch& S) { return S.total && *S.total < kTrialW32Total; }
 __device__ inline bool trial_packed(const TrialScratch& S) { return S.pk && trial_w32(S); }
 
+// What makes two jobs' graphs one: the jobs of a batch may take different parts of
+// one edge list from the same place (prefixes of it), and a graph's flag, total
+// and packed form belong to all of its m edges; n decides whether it is packed.
+struct GraphKey {
+  const cac_edge* edges;
+  uint64_t m;
+  uint32_t n;
+  bool operator==(const GraphKey& o) const { return edges == o.edges && m == o.m && n == o.n; }
+};
+struct GraphHash {
+  size_t operator()(const GraphKey& k) const {
+    uint64_t h = (uint64_t)(uintptr_t)k.edges;
+    for (const uint64_t x : {k.m, (uint64_t)k.n}) h = (h ^ (h >> 29)) * 0x9E3779B97F4A7C15ull + x;
+    return (size_t)(h ^ (h >> 32));
+  }
+};
+
 // Device bytes of the per-trial state of the wide form beside TrialScratch's
 // buffers (tile totals and the round's control words).
 size_t wide_trial_bytes(uint64_t m, uint32_t n);
