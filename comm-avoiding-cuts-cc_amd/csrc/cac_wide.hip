@@ -726,7 +726,7 @@ WideLayout wide_layout(const std::vector<TrialScratch>& h, void* work) {
   L.d_st = cv.take<WideState>(h.size());
   L.d_gs = cv.take<WideGraph>(h.size());
   L.st.assign(h.size(), WideState{});
-  std::unordered_map<const cac_edge*, uint32_t> index;
+  std::unordered_map<GraphKey, uint32_t, GraphHash> index;
   for (size_t i = 0; i < h.size(); ++i) {
     WideState& w = L.st[i];
     const uint64_t tiles = tiles_of(std::max<uint64_t>(h[i].m, h[i].n)) + 1;
@@ -734,14 +734,15 @@ WideLayout wide_layout(const std::vector<TrialScratch>& h, void* work) {
     w.tcnt = cv.take<uint32_t>(tiles);
     w.list[0] = cv.take<uint32_t>(std::max<uint64_t>(h[i].m, 1));
     w.list[1] = cv.take<uint32_t>(std::max<uint64_t>(h[i].m, 1));
-    auto it = index.find(h[i].edges);
+    const GraphKey key{h[i].edges, h[i].m, h[i].n};
+    auto it = index.find(key);
     if (it == index.end()) {
       WideGraph g{};
       g.edges = h[i].edges;
       g.m = h[i].m;
       g.pre0 = cv.take<uint64_t>(std::max<uint64_t>(h[i].m, 1));
       g.tsum0 = cv.take<uint64_t>(tiles_of(h[i].m) + 1);
-      it = index.emplace(h[i].edges, (uint32_t)L.gs.size()).first;
+      it = index.emplace(key, (uint32_t)L.gs.size()).first;
       L.gs.push_back(g);
     }
     w.g = it->second;

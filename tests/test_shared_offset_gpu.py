@@ -65,3 +65,13 @@ def test_one_list_as_two_vertex_counts(ctx, orc, order):
     n = 400
     e = _ring(np.random.default_rng(3), n, 900)
     _check(ctx, orc, e, _orders((len(e), n), (len(e), 70001))[order], trials=1)
+
+
+@pytest.mark.parametrize("order", [0, 1])
+def test_prefixes_in_the_wide_form(orc, order):
+    """Every trial sampled by grid-wide kernels: a round-0 prefix per graph."""
+    n = 701
+    e = _ring(np.random.default_rng(4), n, 5 * n)
+    with cac.Context(0) as c:
+        c.tune_set(cac.TUNE_WIDE_SAMPLING, 0, 1)
+        _check(c, orc, e, _orders((n + 137, n), (3 * n, n), (len(e), n))[order])
