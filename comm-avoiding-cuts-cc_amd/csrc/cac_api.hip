@@ -82,8 +82,9 @@ struct EmitEdge {
   }
 };
 
-// Uploads a host edge list and validates it; *total = sum of weights.
-int upload_edges(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, cac_edge** d_out, hipStream_t s) {
+// Uploads a host edge list and validates it; *total (may be null) = sum of weights.
+int upload_edges(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, cac_edge** d_out, uint64_t* total,
+                 hipStream_t s) {
   cac_edge* d = nullptr;
   CAC_HIP(ctx, hipMalloc((void**)&d, std::max<uint64_t>(m, 1) * sizeof(cac_edge) + 256));
   if (m) {
@@ -117,7 +118,34 @@ int upload_edges(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, ca
     return fail(ctx, CAC_ERANGE, "edge weights too large for int64 cut accumulation");
   }
   *d_out = d;
+  if (total) *total = ((uint64_t)hi << 32) + lo;  // below 2^61
   return CAC_OK;
+}
+
+// cac_mincut_dev on edges that weigh `total` (kTotalUnknown: not summed).
+int mincut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, double p, uint32_t seed, uint64_t total,
+               int64_t* cut, uint32_t* trials, hipStream_t s) {
+  if (!(p >= 0.0 && p < 1.0)) return fail(ctx, CAC_EINVAL, "success probability must be in [0, 1)");
+  const uint32_t t = sqrt_intermediate_size(n, m);
+  const uint32_t T = std::max<uint32_t>(1, sqrt_trials_host(n, m, p));
+  std::vector<uint32_t> ids(T);
+  for (uint32_t i = 0; i < T; ++i) ids[i] = i;
+  int64_t* d_res = nullptr;
+  CAC_HIP(ctx, hipMalloc((void**)&d_res, 8 * (size_t)T));
+  int rc = sqrt_cut_run(ctx, d_edges, m, n, t, seed, ids, total, d_res, s);
+  if (rc == CAC_OK) {
+    std::vector<int64_t> res(T);
+    hipError_t e = hipMemcpyAsync(res.data(), d_res, 8 * (size_t)T, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) rc = hip_fail(ctx, e, "mincut results");
+    else {
+      *cut = *std::min_element(res.begin(), res.end());
+      if (trials) *trials = T;
+    }
+  }
+  (void)hipStreamSynchronize(s);
+  (void)hipFree(d_res);
+  return rc;
 }
 
 }  // namespace
@@ -143,28 +171,7 @@ int cac_mincut_dev(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n
   int rc = cac::bind(ctx);
   if (rc) return rc;
   if (!d_edges || !cut || m == 0 || n < 2) return cac::fail(ctx, CAC_EINVAL, "need n >= 2 and at least one edge");
-  if (!(p >= 0.0 && p < 1.0)) return cac::fail(ctx, CAC_EINVAL, "success probability must be in [0, 1)");
-  hipStream_t s = cac::pick_stream(ctx, stream);
-  const uint32_t t = cac::sqrt_intermediate_size(n, m);
-  const uint32_t T = std::max<uint32_t>(1, cac::sqrt_trials_host(n, m, p));
-  std::vector<uint32_t> ids(T);
-  for (uint32_t i = 0; i < T; ++i) ids[i] = i;
-  int64_t* d_res = nullptr;
-  CAC_HIP(ctx, hipMalloc((void**)&d_res, 8 * (size_t)T));
-  rc = cac::sqrt_cut_run(ctx, d_edges, m, n, t, seed, ids, d_res, s);
-  if (rc == CAC_OK) {
-    std::vector<int64_t> res(T);
-    hipError_t e = hipMemcpyAsync(res.data(), d_res, 8 * (size_t)T, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = cac::hip_fail(ctx, e, "mincut results");
-    else {
-      *cut = *std::min_element(res.begin(), res.end());
-      if (trials) *trials = T;
-    }
-  }
-  (void)hipStreamSynchronize(s);
-  (void)hipFree(d_res);
-  return rc;
+  return cac::mincut_run(ctx, d_edges, m, n, p, seed, cac::kTotalUnknown, cut, trials, cac::pick_stream(ctx, stream));
 }
 
 int cac_sqrt_cut_trials(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, uint32_t t, uint32_t seed,
@@ -176,14 +183,15 @@ int cac_sqrt_cut_trials(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_
   if (t > n) t = n;
   hipStream_t s = ctx->stream;
   cac_edge* d = nullptr;
-  rc = cac::upload_edges(ctx, edges, m, n, &d, s);
+  uint64_t total = 0;
+  rc = cac::upload_edges(ctx, edges, m, n, &d, &total, s);
   if (rc) return rc;
   std::vector<uint32_t> ids(ntrials);
   for (uint32_t i = 0; i < ntrials; ++i) ids[i] = first_trial + i;
   int64_t* d_res = nullptr;
   hipError_t e = hipMalloc((void**)&d_res, 8 * (size_t)ntrials);
   if (e != hipSuccess) rc = cac::hip_fail(ctx, e, "results");
-  if (rc == CAC_OK) rc = cac::sqrt_cut_run(ctx, d, m, n, t, seed, ids, d_res, s);
+  if (rc == CAC_OK) rc = cac::sqrt_cut_run(ctx, d, m, n, t, seed, ids, total, d_res, s);
   if (rc == CAC_OK) {
     e = hipMemcpyAsync(raw_cuts, d_res, 8 * (size_t)ntrials, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -201,9 +209,10 @@ int cac_mincut(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, doub
   if (rc) return rc;
   if (!edges || !cut || m == 0 || n < 2) return cac::fail(ctx, CAC_EINVAL, "need n >= 2 and at least one edge");
   cac_edge* d = nullptr;
-  rc = cac::upload_edges(ctx, edges, m, n, &d, ctx->stream);
+  uint64_t total = 0;
+  rc = cac::upload_edges(ctx, edges, m, n, &d, &total, ctx->stream);
   if (rc) return rc;
-  rc = cac_mincut_dev(ctx, d, m, n, p, seed, cut, trials, ctx->stream);
+  rc = cac::mincut_run(ctx, d, m, n, p, seed, total, cut, trials, ctx->stream);
   (void)hipFree(d);
   return rc;
 }
@@ -218,7 +227,7 @@ int cac_sample_contract(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_
   if (t > n) t = n;
   hipStream_t s = ctx->stream;
   cac_edge* d_e = nullptr;
-  rc = cac::upload_edges(ctx, edges, m, n, &d_e, s);
+  rc = cac::upload_edges(ctx, edges, m, n, &d_e, nullptr, s);
   if (rc) return rc;
   cac::SampleOut so;
   rc = cac::sample_contract_one(ctx, d_e, m, n, t, seed, trial, &so, s);
@@ -295,7 +304,7 @@ int cac_approx_cut(cac_ctx* ctx, const cac_edge* edges, uint64_t m, uint32_t n, 
   const uint32_t iters = (uint32_t)std::ceil(std::log((double)total));
   const uint32_t T = cac_approx_trials(p);
   cac_edge* d = nullptr;
-  rc = cac::upload_edges(ctx, edges, m, n, &d, s);
+  rc = cac::upload_edges(ctx, edges, m, n, &d, nullptr, s);
   if (rc) return rc;
   uint32_t first = 0;
   rc = cac::approx_cut_run(ctx, d, m, n, T, iters, seed, &first, s);

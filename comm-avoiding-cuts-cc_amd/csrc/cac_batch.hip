@@ -160,6 +160,42 @@ bool planted_hard_graph(uint32_t g, uint32_t seed, uint32_t n, uint32_t k, uint3
   return true;
 }
 
+// cac_mincut_batch_dev on graphs that weigh totals[g] (empty: not summed).
+int batch_run(cac_ctx* ctx, const cac_edge* d_edges, const cac_graph_desc* descs, uint32_t count, double p,
+              uint32_t seed, const std::vector<uint64_t>& totals, int64_t* cuts, uint32_t* trials_out, hipStream_t s) {
+  if (!d_edges || !descs || !cuts || count == 0) return fail(ctx, CAC_EINVAL, "null pointer or empty batch");
+  if (!(p >= 0.0 && p < 1.0)) return fail(ctx, CAC_EINVAL, "success probability must be in [0, 1)");
+  std::vector<SqrtJob> jobs;
+  std::vector<uint64_t> first_slot(count + 1);
+  for (uint32_t g = 0; g < count; ++g) {
+    const cac_graph_desc& d = descs[g];
+    if (d.n < 2 || d.m == 0) return fail(ctx, CAC_EINVAL, "every graph needs n >= 2 and at least one edge");
+    const uint32_t t = sqrt_intermediate_size(d.n, d.m);
+    const uint32_t T = d.trials ? d.trials : std::max<uint32_t>(1, sqrt_trials_host(d.n, d.m, p));
+    first_slot[g] = jobs.size();
+    if (jobs.size() + T > 0xFFFFFFFFull) return fail(ctx, CAC_EINVAL, "too many trials in one batch");
+    for (uint32_t i = 0; i < T; ++i)
+      jobs.push_back({d_edges + d.edge_offset, d.m, d.n, t, i, (uint32_t)jobs.size(), seed,
+                      totals.empty() ? kTotalUnknown : totals[g]});
+    if (trials_out) trials_out[g] = T;
+  }
+  first_slot[count] = jobs.size();
+  int64_t* d_res = nullptr;
+  CAC_HIP(ctx, hipMalloc((void**)&d_res, 8 * jobs.size()));
+  int rc = sqrt_cut_batch(ctx, jobs, d_res, s, 0, true);
+  if (rc == CAC_OK) {
+    std::vector<int64_t> res(jobs.size());
+    hipError_t e = hipMemcpyAsync(res.data(), d_res, 8 * res.size(), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) rc = hip_fail(ctx, e, "batch results");
+    for (uint32_t g = 0; g < count && rc == CAC_OK; ++g)
+      cuts[g] = *std::min_element(res.begin() + first_slot[g], res.begin() + first_slot[g + 1]);
+  }
+  (void)hipStreamSynchronize(s);
+  (void)hipFree(d_res);
+  return rc;
+}
+
 }  // namespace
 }  // namespace cac
 
@@ -278,37 +314,7 @@ int cac_mincut_batch_dev(cac_ctx* ctx, const cac_edge* d_edges, const cac_graph_
                          uint32_t seed, int64_t* cuts, uint32_t* trials_out, void* stream) {
   int rc = cac::bind(ctx);
   if (rc) return rc;
-  if (!d_edges || !descs || !cuts || count == 0) return cac::fail(ctx, CAC_EINVAL, "null pointer or empty batch");
-  if (!(p >= 0.0 && p < 1.0)) return cac::fail(ctx, CAC_EINVAL, "success probability must be in [0, 1)");
-  std::vector<cac::SqrtJob> jobs;
-  std::vector<uint64_t> first_slot(count + 1);
-  for (uint32_t g = 0; g < count; ++g) {
-    const cac_graph_desc& d = descs[g];
-    if (d.n < 2 || d.m == 0) return cac::fail(ctx, CAC_EINVAL, "every graph needs n >= 2 and at least one edge");
-    const uint32_t t = cac::sqrt_intermediate_size(d.n, d.m);
-    const uint32_t T = d.trials ? d.trials : std::max<uint32_t>(1, cac::sqrt_trials_host(d.n, d.m, p));
-    first_slot[g] = jobs.size();
-    if (jobs.size() + T > 0xFFFFFFFFull) return cac::fail(ctx, CAC_EINVAL, "too many trials in one batch");
-    for (uint32_t i = 0; i < T; ++i)
-      jobs.push_back({d_edges + d.edge_offset, d.m, d.n, t, i, (uint32_t)jobs.size(), seed});
-    if (trials_out) trials_out[g] = T;
-  }
-  first_slot[count] = jobs.size();
-  hipStream_t s = cac::pick_stream(ctx, stream);
-  int64_t* d_res = nullptr;
-  CAC_HIP(ctx, hipMalloc((void**)&d_res, 8 * jobs.size()));
-  rc = cac::sqrt_cut_batch(ctx, jobs, d_res, s, 0, true);
-  if (rc == CAC_OK) {
-    std::vector<int64_t> res(jobs.size());
-    hipError_t e = hipMemcpyAsync(res.data(), d_res, 8 * res.size(), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = cac::hip_fail(ctx, e, "batch results");
-    for (uint32_t g = 0; g < count && rc == CAC_OK; ++g)
-      cuts[g] = *std::min_element(res.begin() + first_slot[g], res.begin() + first_slot[g + 1]);
-  }
-  (void)hipStreamSynchronize(s);
-  (void)hipFree(d_res);
-  return rc;
+  return cac::batch_run(ctx, d_edges, descs, count, p, seed, {}, cuts, trials_out, cac::pick_stream(ctx, stream));
 }
 
 int cac_mincut_batch(cac_ctx* ctx, const cac_edge* edges, const cac_graph_desc* descs, uint32_t count, double p,
@@ -317,11 +323,12 @@ int cac_mincut_batch(cac_ctx* ctx, const cac_edge* edges, const cac_graph_desc* 
   if (rc) return rc;
   if (!edges || !descs || count == 0) return cac::fail(ctx, CAC_EINVAL, "null pointer or empty batch");
   uint64_t total = 0;
+  std::vector<uint64_t> wsums(count);
   for (uint32_t g = 0; g < count; ++g) {
     const cac_graph_desc& d = descs[g];
     if (d.edge_offset > UINT64_MAX - d.m) return cac::fail(ctx, CAC_EINVAL, "edge range overflows");
     total = std::max(total, d.edge_offset + d.m);
-    uint64_t wsum = 0;
+    uint64_t& wsum = wsums[g];
     for (uint64_t i = 0; i < d.m; ++i) {
       const cac_edge& x = edges[d.edge_offset + i];
       if (x.u >= d.n || x.v >= d.n) return cac::fail(ctx, CAC_EINVAL, "edge endpoint >= its graph's n");
@@ -335,7 +342,7 @@ int cac_mincut_batch(cac_ctx* ctx, const cac_edge* edges, const cac_graph_desc* 
   CAC_HIP(ctx, hipMalloc((void**)&d, std::max<uint64_t>(total, 1) * sizeof(cac_edge)));
   hipError_t e = hipMemcpyAsync(d, edges, total * sizeof(cac_edge), hipMemcpyHostToDevice, s);
   if (e != hipSuccess) rc = cac::hip_fail(ctx, e, "batch upload");
-  if (rc == CAC_OK) rc = cac_mincut_batch_dev(ctx, d, descs, count, p, seed, cuts, trials_out, s);
+  if (rc == CAC_OK) rc = cac::batch_run(ctx, d, descs, count, p, seed, wsums, cuts, trials_out, s);
   (void)hipStreamSynchronize(s);
   (void)hipFree(d);
   return rc;

@@ -48,10 +48,12 @@ uint32_t sqrt_trials_host(uint32_t n, uint64_t m, double p);
 // One sqrt-cut job: trial 'trial' of the graph (edges, m, n) shrunk to t
 // super-vertices with the draws of Philox key `seed`, raw cut to
 // d_results[slot].  Jobs of different graphs and seeds share launches.
+constexpr uint64_t kTotalUnknown = ~0ull;
 struct SqrtJob {
   const cac_edge* edges;
   uint64_t m;
   uint32_t n, t, trial, slot, seed;
+  uint64_t total = kTotalUnknown;  // the graph's total edge weight, where the caller has summed it
 };
 constexpr size_t kMaxJobsPerChunk = 8192;
 // Jobs of any mix of graphs, in chunks of shared launches whose estimated
@@ -66,9 +68,19 @@ size_t job_sample_bytes(const SqrtJob& j, uint32_t dpr = 0);
 // Draws per round of the high-concurrency sampling rule for n0 vertices.
 uint32_t hc_draws_host(uint32_t n0);
 size_t job_ks_bytes(const SqrtJob& j);
+// A chunk of jobs [first, first + jobs) that share launches: the bytes of its
+// sampling scratch, of the wide form's buffers and of its packed graphs.
+struct SqrtChunk {
+  size_t jobs = 0, sample = 0, wide = 0, pack = 0;
+  bool packed = true;  // false: no graph of the chunk is packed
+};
+// The chunk that starts at `first`: as many jobs as fit the budget, at least one.
+// rule: the sampling rule (CAC_SAMPLE_*); wide: the jobs run in the wide form.
+SqrtChunk sqrt_chunk(const std::vector<SqrtJob>& jobs, size_t first, size_t budget, bool wide, int rule);
 // Sqrt-cut trials on a device edge list: raw cut of trial_ids[i] to d_results[i].
+// total: the graph's total weight, or kTotalUnknown.
 int sqrt_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t t, uint32_t seed,
-                 const std::vector<uint32_t>& trial_ids, int64_t* d_results, hipStream_t s);
+                 const std::vector<uint32_t>& trial_ids, uint64_t total, int64_t* d_results, hipStream_t s);
 // Sparse Karger-Stein trials on a checked device edge list (u < v, 1 <= w < 2^40):
 // raw cut of trial_ids[i] to d_results[i], which must already hold the bound.
 int ks_sparse_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t seed,

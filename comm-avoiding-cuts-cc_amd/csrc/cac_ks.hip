@@ -1338,7 +1338,8 @@ size_t ks_live_bytes_per_root(uint32_t n, bool w32) {
     // matrix, sums, live list, column list and node of a child, then its pool
     // rows; the few spare rows beyond 1/8 are not counted: a served query's
     // admitted bytes rest on this sum
-    const size_t b = 2 * nodes * (c64((size_t)t * t * esize) + 2 * c64((size_t)t * esize) + c64((size_t)sz * 4) +
+    const size_t stride = w32 ? ks_stride<uint32_t>(t) : t;
+    const size_t b = 2 * nodes * (c64(stride * t * esize) + 2 * c64((size_t)t * esize) + c64((size_t)sz * 4) +
                                   c64((size_t)t * 4) + 104 +
                                   (size_t)(sz - t) * ks_pool_stride(sz) * esize * 9 / 8);
     best[depth & 1] = std::max(best[depth & 1], b);

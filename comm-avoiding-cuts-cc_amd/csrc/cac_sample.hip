@@ -1271,27 +1271,45 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 }
 
 
+inline GraphKey graph_key(const SqrtJob& j) { return {j.edges, j.m, j.n}; }
+
+// Whether a job's graph is packed: not when it is known to be too heavy for trials
+// in 32 bits.
+inline bool can_pack(const SqrtJob& j) {
+  return j.n <= kPackMaxN && j.m < kPackMaxM && (j.total == kTotalUnknown || j.total < kTrialW32Total);
+}
+
 // Points scr[i].mixed and scr[i].total at a flag word and a total weight of its
 // graph (one per distinct graph) and launches the kernels that set them;
 // spans, flags and totals hold scr.size() entries.  Both are ready for any later
 // launch on s.
-// packed: the graphs' packed forms are carved from it (packed_bytes each), null:
-// none is packed.
-int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, EdgeSpan* d_spans, uint32_t* d_flags,
-                       unsigned long long* d_totals, void* packed, hipStream_t s) {
+// packed: the packed forms of the graphs of jobs (one per entry of scr) that can be
+// are carved from it (packed_bytes each), null: none is packed.
+int launch_mixed_flags(cac_ctx* ctx, std::vector<TrialScratch>& scr, const SqrtJob* jobs, EdgeSpan* d_spans,
+                       uint32_t* d_flags, unsigned long long* d_totals, void* packed, hipStream_t s) {
   Carver pc(packed);
   std::unordered_map<GraphKey, uint32_t, GraphHash> index;
+  GraphKey last{};
   std::vector<EdgeSpan> spans;
   uint64_t mmax = 0;
-  for (TrialScratch& x : scr) {
+  for (size_t i = 0; i < scr.size(); ++i) {
+    TrialScratch& x = scr[i];
     const GraphKey key{x.edges, x.m, x.n};
+    if (i > 0 && key == last) {  // a graph's trials come together
+      x.mixed = scr[i - 1].mixed;
+      x.total = scr[i - 1].total;
+      x.pk = scr[i - 1].pk;
+      x.pre0 = scr[i - 1].pre0;
+      continue;
+    }
+    last = key;
     auto it = index.find(key);
     uint32_t g = 0;
     if (it == index.end()) {
       g = (uint32_t)spans.size();
       index.emplace(key, g);
       EdgeSpan sp{x.edges, x.m, d_flags + g, d_totals + g, nullptr, nullptr, nullptr};
-      if (packed && x.n <= kPackMaxN && x.m < kPackMaxM) {
+      if (packed && can_pack(jobs[i])) {
         sp.pk = pc.take<uint32_t>(x.m);
         sp.pre0 = pc.take<uint32_t>(x.m);
         sp.tiles = pc.take<uint32_t>((x.m + kPackTile - 1) / kPackTile);
@@ -1463,10 +1481,9 @@ uint32_t hc_draws_host(uint32_t n0) {
   return (uint32_t)std::pow((float)n0, 1 + epsilon / 2);
 }
 
-// Draws per round of a job under the context's sampling rule (0: |V|).
-static uint32_t job_dpr(const cac_ctx* ctx, uint32_t n) {
-  return ctx->sample_rule == CAC_SAMPLE_HC ? hc_draws_host(n) : 0u;
-}
+// Draws per round of a job under a sampling rule (0: |V|).
+static uint32_t rule_dpr(int rule, uint32_t n) { return rule == CAC_SAMPLE_HC ? hc_draws_host(n) : 0u; }
+static uint32_t job_dpr(const cac_ctx* ctx, uint32_t n) { return rule_dpr(ctx->sample_rule, n); }
 
 // Device bytes one sampling job needs beside the Karger-Stein levels (dpr:
 // draws per round, 0 = |V|).
@@ -1616,7 +1633,7 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
       deg[i] = cv.take<unsigned long long>((size_t)j.t + 2);  // [t] degrees, [t + 1] their minimum
       offsets[i + 1] = offsets[i] + j.m;
     }
-    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, nullptr, s);
+    rc = launch_mixed_flags(ctx, scr, nullptr, d_spans, d_flags, d_totals, nullptr, s);
     if (rc) return rc;
     std::vector<TrialScratch> wid(scr.begin() + w0, scr.end());
     CAC_HIP(ctx, hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s));
@@ -1716,7 +1733,66 @@ static int sqrt_large_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs_in, i
   return CAC_OK;
 }
 
-static bool can_pack(const SqrtJob& j) { return j.n <= kPackMaxN && j.m < kPackMaxM; }
+// Bytes of a trial's matrix and row sums: 4-byte entries in whole rows for a trial
+// known to be packed (its row lists take less), else room for either entry type, or
+// for a 32-bit matrix with its lists behind.
+static size_t mat_bytes(const SqrtJob& j, bool packed) {
+  return packed ? (size_t)j.t * ks_stride<uint32_t>(j.t) * 4 : (size_t)j.t * j.t * 8;
+}
+static size_t rsum_bytes(const SqrtJob& j, bool packed) { return (size_t)j.t * (packed ? 4 : 8); }
+
+// The estimate of a job that sizes a chunk, and that a served group's budget is made
+// of, counts 8-byte entries.  What 4-byte entries leave free of it, in graphs known
+// to weigh little enough, holds the packed lists, and they count only beyond that.
+// Counted in full, a served group lost its last trials to a second chunk: 25
+// queries of n 1000-18000 took 9.0 ms instead of 7.1.  A graph of unknown weight
+// leaves nothing free.  A first job that does not fit with its graph packed runs
+// unpacked.
+SqrtChunk sqrt_chunk(const std::vector<SqrtJob>& jobs, size_t first, size_t budget, bool wide, int rule) {
+  SqrtChunk c;
+  std::unordered_set<GraphKey, GraphHash> graphs;  // packed once per graph of the chunk
+  const size_t cap = wide ? 4096 : kMaxJobsPerChunk;
+  size_t estimate = 0, free_bytes = 0;
+  // the bytes of one job; a graph's trials come together and share them (adding the
+  // levels up again for each of 4987 trials took 0.4 ms of a 33 ms solve)
+  const SqrtJob* like = nullptr;
+  size_t a = 0, k = 0, wb = 0, spare_ks = 0, spare_mat = 0;
+  while (first + c.jobs < jobs.size() && c.jobs < cap) {
+    const SqrtJob& j = jobs[first + c.jobs];
+    const bool pack = !wide && c.packed && can_pack(j);
+    const bool same = like && graph_key(*like) == graph_key(j) && like->t == j.t;
+    if (!same) {
+      const bool light = j.total < kTrialW32Total;
+      a = job_sample_bytes(j, rule_dpr(rule, j.n));
+      k = job_ks_bytes(j);
+      wb = wide ? wide_trial_bytes(j.m, j.n) : 0;
+      spare_ks = light ? k - ks_live_bytes_per_root(j.t, true) : 0;
+      spare_mat = light && pack ? carve_size(mat_bytes(j, false)) + carve_size(rsum_bytes(j, false)) -
+                                      carve_size(mat_bytes(j, true)) - carve_size(rsum_bytes(j, true))
+                                : 0;
+    }
+    const size_t pb = pack && !same && !graphs.count(graph_key(j)) ? packed_bytes(j.m) : 0;
+    const size_t spare = free_bytes + spare_ks + spare_mat;
+    const size_t over = c.pack + pb > spare ? c.pack + pb - spare : 0;
+    if (estimate + a + k + wb + over > budget) {
+      if (c.jobs > 0) break;
+      if (pb) {
+        c.packed = false;
+        like = nullptr;
+        continue;
+      }
+    }
+    if (pb) graphs.insert(graph_key(j));
+    like = &j;
+    c.pack += pb;
+    c.sample += a - spare_mat;
+    c.wide += wb;
+    estimate += a + k + wb;
+    free_bytes = spare;
+    ++c.jobs;
+  }
+  return c;
+}
 
 // Dense-engine jobs (t <= 8192) in chunks sized to the budget: sampling,
 // densification, then one breadth-first Karger-Stein pass per chunk, whatever
@@ -1727,29 +1803,9 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
   int rc = CAC_OK;
   size_t b0 = 0;
   while (b0 < jobs.size() && rc == CAC_OK) {
-    size_t nb = 0, sample_bytes = 0, ks_bytes = 0, wide_bytes = 0, pack_bytes = 0;
-    std::unordered_set<GraphKey, GraphHash> graphs;  // packed once per graph of the chunk
-    const size_t cap = wide ? 4096 : kMaxJobsPerChunk;
-    while (b0 + nb < jobs.size() && nb < cap) {
-      const SqrtJob& j = jobs[b0 + nb];
-      const size_t a = job_sample_bytes(j, job_dpr(ctx, j.n)), k = job_ks_bytes(j);
-      const size_t wb = wide ? wide_trial_bytes(j.m, j.n) : 0;
-      const size_t pb = !wide && can_pack(j) && !graphs.count({j.edges, j.m, j.n}) ? packed_bytes(j.m) : 0;
-      // The packed lists live in the half of the Karger-Stein estimate (8 bytes an
-      // entry) that a packed graph's 4-byte entries leave free, and count only
-      // where they take more.  Counted in full, a served group, whose budget is
-      // its admitted estimate, lost its last trials to a second chunk: 25 queries
-      // of n 1000-18000 took 9.0 ms instead of 7.1.
-      const size_t saved = (ks_bytes + k) / 2;
-      const size_t over = pack_bytes + pb > saved ? pack_bytes + pb - saved : 0;
-      if (nb > 0 && sample_bytes + a + ks_bytes + k + wide_bytes + wb + over > budget) break;
-      if (pb) graphs.insert({j.edges, j.m, j.n});
-      pack_bytes += pb;
-      sample_bytes += a;
-      ks_bytes += k;
-      wide_bytes += wb;
-      ++nb;
-    }
+    const SqrtChunk chunk = sqrt_chunk(jobs, b0, budget, wide, ctx->sample_rule);
+    size_t nb = chunk.jobs, wide_bytes = chunk.wide;
+    const size_t sample_bytes = chunk.sample, pack_bytes = chunk.pack;
     // whole waves of sampling workgroups, and where there are that many of the
     // first contractions (two children a trial): a last partial wave would leave
     // most of the GPU idle while it runs (Watts-Strogatz, 32000 vertices with 16
@@ -1798,13 +1854,14 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       x.par = cv.take<uint32_t>(j.n);
       x.pre = cv.take<uint64_t>(j.m + 2);  // a packed trial's list and prefix, each of whole 16-byte pieces
       x.draws = cv.take<uint2>(std::max(j.n, x.dpr));
-      x.mat = cv.take<int64_t>((size_t)j.t * j.t);  // room for either entry type
-      x.rsum = cv.take<int64_t>(j.t);
+      const bool light = !wide && chunk.packed && j.total < kTrialW32Total && can_pack(j);
+      x.mat = cv.take<unsigned char>(mat_bytes(j, light));
+      x.rsum = cv.take<unsigned char>(rsum_bytes(j, light));
       x.nv_out = d_nv + i;
       x.live = d_live + 2 * i;
     }
     void* packed = pack_bytes ? (void*)cv.take<unsigned char>(pack_bytes) : nullptr;
-    rc = launch_mixed_flags(ctx, scr, d_spans, d_flags, d_totals, packed, s);
+    rc = launch_mixed_flags(ctx, scr, jobs.data() + b0, d_spans, d_flags, d_totals, packed, s);
     if (rc) return rc;
     e = hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "job descriptors");
@@ -1936,9 +1993,9 @@ int sqrt_cut_batch(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int64_t* d_re
 
 // Trials trial_ids of one graph; raw cut of trial_ids[i] to d_results[i].
 int sqrt_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t t, uint32_t seed,
-                 const std::vector<uint32_t>& trial_ids, int64_t* d_results, hipStream_t s) {
+                 const std::vector<uint32_t>& trial_ids, uint64_t total, int64_t* d_results, hipStream_t s) {
   std::vector<SqrtJob> jobs(trial_ids.size());
-  for (size_t i = 0; i < trial_ids.size(); ++i) jobs[i] = {d_edges, m, n, t, trial_ids[i], (uint32_t)i, seed};
+  for (size_t i = 0; i < trial_ids.size(); ++i) jobs[i] = {d_edges, m, n, t, trial_ids[i], (uint32_t)i, seed, total};
   return sqrt_cut_batch(ctx, jobs, d_results, s);
 }
 
@@ -1979,7 +2036,7 @@ int sample_contract_one(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint3
   h.mat = nullptr;
   h.rsum = nullptr;
   std::vector<TrialScratch> one{h};
-  int rc = launch_mixed_flags(ctx, one, d_span, d_flag, d_total, nullptr, s);
+  int rc = launch_mixed_flags(ctx, one, nullptr, d_span, d_flag, d_total, nullptr, s);
   if (rc) return rc;
   h = one[0];
   h.total = nullptr;  // the merged matrix is read as int64

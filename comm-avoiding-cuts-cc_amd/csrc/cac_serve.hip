@@ -61,13 +61,14 @@ struct Pending {
   size_t scratch;           // device scratch of its work (for a min cut: its trials' chunk)
   uint64_t work;            // a min cut's trials x edges (its share of a group), 0 for CC
   const cac_edge* d_edges;  // a registered graph's device edges (checked once), or null
+  uint64_t total;           // and their total weight
 };
 
 // A graph registered with the server: its edges stay in device memory, checked
 // once, and queries name it instead of bringing their edges.
 struct Resident {
   cac_edge* d_edges;
-  uint64_t m;
+  uint64_t m, total;  // edges and their total weight
   uint32_t n;
   size_t bytes;
   uint32_t users;  // queries submitted and not yet finished
@@ -343,7 +344,8 @@ void run_mincut_group(cac_ctx* ctx, std::vector<Pending>& grp, std::vector<cac_q
     res[i].t = t;
     res[i].trials = T;
     const cac_edge* qe = grp[i].d_edges ? grp[i].d_edges : d_e + eoff[i];
-    for (uint32_t k = 0; k < T; ++k) jobs.push_back({qe, q.m, q.n, t, k, (uint32_t)jobs.size(), q.seed});
+    const uint64_t total = grp[i].d_edges ? grp[i].total : chk[3 * i + 1];
+    for (uint32_t k = 0; k < T; ++k) jobs.push_back({qe, q.m, q.n, t, k, (uint32_t)jobs.size(), q.seed, total});
   }
   first[grp.size()] = jobs.size();
   if (rc == CAC_OK && !jobs.empty()) {
@@ -510,6 +512,7 @@ int cac_server_submit(cac_server* S, const cac_query* q, uint64_t* id_out) {
   cac::Pending p;
   p.q = *q;
   p.d_edges = nullptr;
+  p.total = 0;
   std::lock_guard<std::mutex> lk(S->mu);
   int v = CAC_OK;
   if (q->graph) {  // a registered graph: its size and device edges come from the registration
@@ -521,6 +524,7 @@ int cac_server_submit(cac_server* S, const cac_query* q, uint64_t* id_out) {
       p.q.m = it->second.m;
       p.q.edges = nullptr;
       p.d_edges = it->second.d_edges;
+      p.total = it->second.total;
     }
   }
   if (v == CAC_OK) v = cac::validate(p.q, p.d_edges != nullptr);
@@ -586,7 +590,7 @@ int cac_server_register_graph(cac_server* S, const cac_edge* edges, uint64_t m, 
   }
   std::lock_guard<std::mutex> lk(S->mu);
   const uint64_t g = S->next_graph++;
-  S->graphs[g] = cac::Resident{(cac_edge*)d, m, n, bytes, 0u, false};
+  S->graphs[g] = cac::Resident{(cac_edge*)d, m, h[1], n, bytes, 0u, false};
   S->resident += bytes;
   *graph_out = g;
   return CAC_OK;
