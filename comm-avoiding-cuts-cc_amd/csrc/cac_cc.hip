@@ -1157,17 +1157,21 @@ __global__ void __launch_bounds__(kCcBlock) k_approx_init(uint32_t* par_all, uin
 
 }  // namespace
 
-// The vertex bitmap, then the coarse map.
-size_t cc_fine_words(uint32_t n) { return (((size_t)n + 63) / 64 * 2 + 63) & ~size_t(63); }
+// The vertex bitmap, and the coarse map that follows it unless the caller gives the
+// map a place.
 size_t cc_bitmap_words(uint64_t m, uint32_t n) {
-  return m >= kSampleMinEdges ? cc_fine_words(n) + ((map_words(n) + 63) & ~size_t(63)) : 0;
+  return m >= kSampleMinEdges ? (((size_t)n + 63) / 64 * 2 + 63) & ~size_t(63) : 0;
+}
+size_t cc_map_words(uint64_t m, uint32_t n) {
+  return m >= kSampleMinEdges ? (map_words(n) + 63) & ~size_t(63) : 0;
 }
 size_t cc_rank_tmp_words(uint32_t n) { return ((size_t)(n + 63) & ~size_t(63)) + scan_tiles(n) + 64; }
 
-// Device scratch of cc_launch, in u32 words: head, bitmap (large m), rank tables
-// (label_mode == RANK).
-size_t cc_tmp_words(uint64_t m, uint32_t n, int label_mode) {
-  return kCcTmpHead + cc_bitmap_words(m, n) + (label_mode == CAC_LABEL_RANK ? cc_rank_tmp_words(n) : 0);
+// Device scratch of cc_launch, in u32 words: head, bitmap and coarse map (large m),
+// rank tables (label_mode == RANK).  own_map false: without the map.
+size_t cc_tmp_words(uint64_t m, uint32_t n, int label_mode, bool own_map) {
+  return kCcTmpHead + cc_bitmap_words(m, n) + (own_map ? cc_map_words(m, n) : 0) +
+         (label_mode == CAC_LABEL_RANK ? cc_rank_tmp_words(n) : 0);
 }
 
 // The hook pass's dynamic LDS exceeds the default limit: raise it once.
@@ -1208,11 +1212,13 @@ int cc_small(cac_ctx* ctx, const cac_uedge* edges, uint64_t m, uint32_t n, int l
 }
 
 // Launch sequence shared by cac_cc and cac_cc_dev; d_tmp holds cc_tmp_words()
-// u32 words, 256-byte aligned.  The component count lands in d_tmp[0].
+// u32 words, 256-byte aligned.  The component count lands in d_tmp[0].  d_map:
+// cc_map_words() words, 16-byte aligned, for the coarse map, or null: it is in d_tmp.
 int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, int label_mode, uint32_t* d_lab,
-              uint32_t* d_tmp, hipStream_t s) {
+              uint32_t* d_tmp, uint32_t* d_map, hipStream_t s) {
   uint32_t* d_counter = d_tmp;
-  uint32_t* d_rank_tmp = d_tmp + kCcTmpHead + cc_bitmap_words(m, n);
+  uint32_t* d_rank_tmp = d_tmp + kCcTmpHead + cc_bitmap_words(m, n) + (d_map ? 0 : cc_map_words(m, n));
+  if (!d_map) d_map = d_tmp + kCcTmpHead + cc_bitmap_words(m, n);
   const unsigned cap = 256 * 64;
   prof_begin(ctx, "cc_init", s);
   hipLaunchKernelGGL(k_cc_init, dim3(grid_for(n, kCcBlock, cap)), dim3(kCcBlock), 0, s, d_lab, n);
@@ -1246,7 +1252,6 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
       hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, d_edges, m, (const uint32_t*)d_lab, n, d_root);
       hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, cap)), dim3(kCcBlock), 0, s,
                          (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
-      uint32_t* d_map = reinterpret_cast<uint32_t*>(d_bits) + cc_fine_words(n);
       const uint32_t words = map_words(n), shift = map_shift(n);
       hipLaunchKernelGGL(k_cc_coarse, dim3((words + kCcBlock - 1) / kCcBlock), dim3(kCcBlock), 0, s,
                          (const uint32_t*)d_bits, n, shift, d_map, words);
@@ -1450,12 +1455,12 @@ int cac_cc_dev(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, i
     return cac::fail(ctx, CAC_EINVAL, "label_mode must be CAC_LABEL_MIN_ID or CAC_LABEL_RANK");
   hipStream_t s = cac::pick_stream(ctx, stream);
   if (cac::cc_is_small(m, n)) return cac::cc_small(ctx, d_edges, m, n, label_mode, d_labels, ncomp_out, s);
-  size_t words = cac::cc_tmp_words(m, n, label_mode);
+  size_t words = cac::cc_tmp_words(m, n, label_mode, true);
   void* base = nullptr;
   rc = cac::scratch_reserve(ctx, words * 4, &base);
   if (rc) return rc;
   uint32_t* counter = (uint32_t*)base;
-  rc = cac::cc_launch(ctx, d_edges, m, n, label_mode, d_labels, counter, s);
+  rc = cac::cc_launch(ctx, d_edges, m, n, label_mode, d_labels, counter, nullptr, s);
   if (rc) return rc;
   CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, counter, 4, hipMemcpyDeviceToHost, s));
   CAC_HIP(ctx, hipStreamSynchronize(s));
@@ -1480,7 +1485,7 @@ int cac_cc_static_dev(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32
   // per-kernel timing would create events: off for this call
   const bool prof = ctx->profiling;
   ctx->profiling = false;
-  rc = cac::cc_launch(ctx, d_edges, m, n, CAC_LABEL_MIN_ID, d_labels, tmp, s);
+  rc = cac::cc_launch(ctx, d_edges, m, n, CAC_LABEL_MIN_ID, d_labels, tmp, nullptr, s);
   if (rc == CAC_OK && label_mode == CAC_LABEL_RANK && n) {
     uint64_t* bits = reinterpret_cast<uint64_t*>(tmp + cac::kCcTmpHead);
     uint32_t* pre = tmp + cac::kCcTmpHead + cac::kStaticBitsWords;
@@ -1528,7 +1533,7 @@ int cac_cc(cac_ctx* ctx, const cac_uedge* edges, uint64_t m, uint32_t n, int lab
   }
   size_t e_bytes = cac::carve_size(m * sizeof(cac_uedge));
   size_t l_bytes = cac::carve_size((size_t)n * 4);
-  size_t t_words = cac::cc_tmp_words(m, n, label_mode);
+  size_t t_words = cac::cc_tmp_words(m, n, label_mode, true);
   void* base = nullptr;
   rc = cac::scratch_reserve(ctx, e_bytes + l_bytes + cac::carve_size(t_words * 4) + 256, &base);
   if (rc) return rc;
@@ -1546,7 +1551,7 @@ int cac_cc(cac_ctx* ctx, const cac_uedge* edges, uint64_t m, uint32_t n, int lab
   CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, tmp, 4, hipMemcpyDeviceToHost, s));
   CAC_HIP(ctx, hipStreamSynchronize(s));
   if (*(uint32_t*)ctx->pinned) return cac::fail(ctx, CAC_EINVAL, "edge endpoint >= n");
-  rc = cac::cc_launch(ctx, d_e, m, n, label_mode, d_l, tmp, s);
+  rc = cac::cc_launch(ctx, d_e, m, n, label_mode, d_l, tmp, nullptr, s);
   if (rc) return rc;
   CAC_HIP(ctx, hipMemcpyAsync(ctx->pinned, tmp, 4, hipMemcpyDeviceToHost, s));
   if (n) CAC_HIP(ctx, hipMemcpyAsync(labels_out, d_l, (size_t)n * 4, hipMemcpyDeviceToHost, s));

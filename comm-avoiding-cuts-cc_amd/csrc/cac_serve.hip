@@ -39,9 +39,10 @@
 
 namespace cac {
 
-size_t cc_tmp_words(uint64_t m, uint32_t n, int label_mode);
+size_t cc_tmp_words(uint64_t m, uint32_t n, int label_mode, bool own_map);
+size_t cc_map_words(uint64_t m, uint32_t n);
 int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, int label_mode, uint32_t* d_lab,
-              uint32_t* d_tmp, hipStream_t s);
+              uint32_t* d_tmp, uint32_t* d_map, hipStream_t s);
 
 namespace {
 
@@ -96,7 +97,8 @@ void mincut_plan(uint32_t n, uint64_t m, double p, uint32_t trials, uint32_t* t,
 void footprint(const cac_query& q, bool resident, size_t* upload, size_t* scratch) {
   *upload = resident ? 0 : carve_size(q.m * sizeof(cac_edge));
   if (q.kind == CAC_QUERY_CC) {
-    *scratch = carve_size(q.m * sizeof(cac_uedge)) + carve_size((size_t)q.n * 4) + cc_tmp_words(q.m, q.n, 0) * 4 + 4096;
+    *scratch = carve_size(q.m * sizeof(cac_uedge)) + carve_size((size_t)q.n * 4) +
+               cc_tmp_words(q.m, q.n, CAC_LABEL_MIN_ID, false) * 4 + 4096;
     return;
   }
   uint32_t t, T;
@@ -228,7 +230,7 @@ void run_cc_group(cac_ctx* ctx, std::vector<Pending>& grp, std::vector<cac_query
     N += grp[i].q.n;
     M += grp[i].q.m;
   }
-  const size_t tw = cc_tmp_words(M, (uint32_t)N, CAC_LABEL_MIN_ID);
+  const size_t tw = cc_tmp_words(M, (uint32_t)N, CAC_LABEL_MIN_ID, false);
   // the worker's grow-only buffer: no allocation (and no device-wide wait
   // of a free) per group once it has grown
   int rc = grow_buffer(ctx, &ctx->serve_buf, &ctx->serve_bytes,
@@ -258,7 +260,11 @@ void run_cc_group(cac_ctx* ctx, std::vector<Pending>& grp, std::vector<cac_query
                          (uint32_t)voff[i], d_e + eoff[i], d_bad + i);
     }
     if (e != hipSuccess) rc = hip_fail(ctx, e, "serve cc upload");
-    if (rc == CAC_OK) rc = cc_launch(ctx, d_e, M, (uint32_t)N, CAC_LABEL_MIN_ID, d_l, d_t, s);
+    // The coarse map (at most 128 KiB, from 2^18 edges on) takes the uploaded edges'
+    // place, which nothing reads any more: in room of its own it would count in the
+    // footprint, and a query that a server's budget just fits would be refused.
+    uint32_t* d_map = (uint32_t*)d_in;
+    if (rc == CAC_OK) rc = cc_launch(ctx, d_e, M, (uint32_t)N, CAC_LABEL_MIN_ID, d_l, d_t, d_map, s);
     if (rc == CAC_OK) {
       e = hipMemcpyAsync(lab.data(), d_l, N * 4, hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipMemcpyAsync(bad.data(), d_bad, grp.size() * 4, hipMemcpyDeviceToHost, s);

@@ -38,3 +38,21 @@ def test_budget_of_exactly_the_admitted_bytes(orc, wmax, alone):
             e3 = np.stack([e["u"], e["v"], e["w"]], axis=1).astype(np.uint64)
             want = min(orc.sqrt_trial(n, e3, int(r["t"]), sd, i) for i in range(T))
             assert r["cut"] == want, (n, wmax, r["cut"], want)
+
+
+@pytest.mark.parametrize("n,d", [(3000, 4.0), (150001, 4.0), (400000, 1.4), (1050000, 3.2)])
+def test_cc_query_fits_its_edges_labels_and_bitmap(orc, n, d):
+    """A components query takes its upload, its endpoints, its labels and, from 2^18
+    edges, a bit per vertex; the coarse map of the giant component takes no more."""
+    e = cac.gen_gnp(n, d, 3, 1, wmax=9)
+    m = len(e)
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    bitmap = up((n + 63) // 64 * 8) if m >= 1 << 18 else 0
+    need = up(16 * m) + up(8 * m) + up(4 * n) + 256 + bitmap + 4096
+    lab = np.zeros(n, dtype=np.uint32)
+    with cac.Server(0, workers=1, hbm_budget=need, max_batch=4) as srv:
+        res = srv.replay([cac.Server.query(cac.QUERY_CC, e, n, labels=lab)], np.zeros(1))
+        assert res[0]["status"] == 0
+        assert srv.stats()[0] == need
+    want, nc = orc.cc(np.stack([e["u"], e["v"]], 1).astype(np.uint32), n)
+    assert res[0]["ncomp"] == nc and np.array_equal(lab, want)
