@@ -1720,10 +1720,18 @@ int approx_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n
   const uint64_t N = (uint64_t)n * copies;
   if (N >= 0xFFFFFFFFull) return fail(ctx, CAC_EINVAL, "n * trials must fit in 32-bit vertex ids");
   static_assert(kApLevels * kApSlotWords * 4 <= 4096, "the hook counters fit the context's pinned buffer");
-  // levels side by side while their forests stay small
-  const uint32_t batch = N * 4 * kApLevels <= (1ull << 30) ? kApLevels : 1u;
+  // levels side by side while their forests stay small and there is room for them
+  uint32_t batch = N * 4 * kApLevels <= (1ull << 30) ? kApLevels : 1u;
   void* base = nullptr;
-  int rc = scratch_reserve(ctx, carve_size(N * 4 * batch) + carve_size(kApLevels * kApSlotWords * 4) + 512, &base);
+  auto reserve = [&] {
+    return scratch_reserve(ctx, carve_size(N * 4 * batch) + carve_size(kApLevels * kApSlotWords * 4) + 512, &base);
+  };
+  int rc = reserve();
+  if (rc == CAC_ENOMEM && batch > 1) {
+    (void)hipGetLastError();
+    batch = 1;
+    rc = reserve();
+  }
   if (rc) return rc;
   Carver cv(base);
   uint32_t* par = cv.take<uint32_t>(N * batch);
