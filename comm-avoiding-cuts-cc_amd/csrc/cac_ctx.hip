@@ -292,7 +292,7 @@ int cac_memcpy_d2d(cac_ctx* ctx, void* dst, const void* src, size_t bytes, void*
 // the edge-count class bound), a value 0 (built-in: 2), 1 or 2;
 // CAC_TUNE_WIDE_SAMPLING key 0, a value 0 (built-in: 2^20 edges) to 63 (never);
 // CAC_TUNE_KS_COMPACT_BLOCK keys 512, 1024, 2048, 4096, 8192 (child-size class
-// upper bounds), a value 0 (built-in: 512), 256, 512 or 1024.
+// upper bounds), a value 0 (built-in: by the length of a parent row), 256, 512 or 1024.
 static int tune_slot(int knob, uint32_t key) {
   if (knob == CAC_TUNE_KS_CONTRACT_BLOCK) {
     switch (key) {
