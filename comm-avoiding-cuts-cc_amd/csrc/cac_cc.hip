@@ -358,7 +358,8 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restric
 }
 
 // Coarse map of the giant component, sized for a CU's LDS.  Up to kMapBits
-// vertices it is the vertex bitmap itself.  Beyond, it is two maps of kMapBits / 2
+// vertices it is the vertex bitmap itself (a copy of it was one launch more: R-MAT
+// 2^16 / 2^21 169 -> 166 us without).  Beyond, it is two maps of kMapBits / 2
 // bits: bit g of the first = every vertex of [g 2^shift, (g + 1) 2^shift) is in the
 // component (a group that runs past n counts as not), bit j of the second = every
 // vertex congruent to j modulo kMapBits / 2 is.  A vertex with either bit set is
@@ -383,9 +384,7 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_coarse(const uint32_t* __restri
   if (w >= words) return;
   const uint32_t bit_words = (uint32_t)(((uint64_t)n + 31) / 32);
   uint32_t out = 0;
-  if (shift == 0) {
-    out = w < bit_words ? bits[w] : 0u;
-  } else if (w >= kHalfWords) {
+  if (w >= kHalfWords) {
     out = ~0u;
     for (uint32_t i = w - kHalfWords; i < bit_words; i += kHalfWords) {
       const uint32_t past = i + 1 == bit_words && n % 32 ? ~0u << (n % 32) : 0u;  // no vertices there
@@ -1163,7 +1162,7 @@ size_t cc_bitmap_words(uint64_t m, uint32_t n) {
   return m >= kSampleMinEdges ? (((size_t)n + 63) / 64 * 2 + 63) & ~size_t(63) : 0;
 }
 size_t cc_map_words(uint64_t m, uint32_t n) {
-  return m >= kSampleMinEdges ? (map_words(n) + 63) & ~size_t(63) : 0;
+  return m >= kSampleMinEdges && n > kMapBits ? (map_words(n) + 63) & ~size_t(63) : 0;
 }
 size_t cc_rank_tmp_words(uint32_t n) { return ((size_t)(n + 63) & ~size_t(63)) + scan_tiles(n) + 64; }
 
@@ -1253,8 +1252,10 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
       hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, cap)), dim3(kCcBlock), 0, s,
                          (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
       const uint32_t words = map_words(n), shift = map_shift(n);
-      hipLaunchKernelGGL(k_cc_coarse, dim3((words + kCcBlock - 1) / kCcBlock), dim3(kCcBlock), 0, s,
-                         (const uint32_t*)d_bits, n, shift, d_map, words);
+      if (shift == 0) d_map = reinterpret_cast<uint32_t*>(d_bits);  // the bitmap itself
+      else
+        hipLaunchKernelGGL(k_cc_coarse, dim3((words + kCcBlock - 1) / kCcBlock), dim3(kCcBlock), 0, s,
+                           (const uint32_t*)d_bits, n, shift, d_map, words);
       prof_end(ctx, s);
       prof_begin(ctx, "cc_hook", s);
       const int rc = hook_attr(ctx);
