@@ -26,7 +26,8 @@
 //   7. compress  parent[v] = root(v), count roots               (8n bytes)
 //   8. (rank)    dense rank of roots by id, relabel              (scan)
 // Steps 2-3 run when m is large and steps 4-5 when the list is also long for its
-// vertices; the others hook every edge whose endpoints' parents differ.
+// vertices; the others hook every edge whose endpoints' parents differ, those of
+// many vertices in no order past the bitmap.
 // Any edge order is correct; the run sampling pays off when equal u are
 // adjacent (the order of the edge-list files and of the R-MAT generator).
 #include <algorithm>
@@ -48,7 +49,8 @@ constexpr int kTileEdges = 64 * kEdgesPerThread;     // edges per wavefront tile
 constexpr uint64_t kSampleMinEdges = 1ull << 18;     // below this: plain hook only
 constexpr int kModeSamples = 4096;
 constexpr int kModeTable = 8192;                     // open-addressing table, > kModeSamples
-constexpr size_t kCcTmpHead = 64;                    // u32 words: [0] component count, [1] giant root, [2] its samples
+// u32 words: [0] component count, [1] giant root, [2] its samples, [3] 1: list in no order
+constexpr size_t kCcTmpHead = 64;
 
 // Parent-array loads inside the union-find kernels are relaxed atomics at
 // workgroup scope: plain cached loads.  A stale parent (an older state of the
@@ -177,7 +179,8 @@ constexpr uint32_t kQueueMinN = 1u << 22;  // queued above: the forest is past a
 
 template <bool kQueue>
 __global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restrict__ edges, uint64_t m, uint32_t* par,
-                                                      uint64_t sample_tiles, uint32_t random_waves) {
+                                                      uint64_t sample_tiles, uint32_t random_waves,
+                                                      uint32_t* unordered) {
   __shared__ uint64_t queue_lds[kCcBlock / 64][128];  // fewer than 64 left over and one step's 64
   uint64_t* queue = queue_lds[threadIdx.x >> 6];
   uint32_t queued = 0;  // uniform in the wavefront
@@ -213,10 +216,13 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_runs(const cac_uedge* __restric
         const uint32_t up = __shfl_up(u[k], 1, 64);
         descents += (uint32_t)__popcll(__ballot(lane > 0 && u[k] < up));
       }
-      if (sample_tiles && descents >= kTileEdges / 8) {  // no order
-        tiles = sample_tiles < tiles ? sample_tiles : tiles;
-        if (first >= random_waves || first >= tiles) return;
-        if (waves > random_waves) waves = random_waves;
+      if (descents >= kTileEdges / 8) {  // no order
+        if (first < 64 && lane == 0) __hip_atomic_store(unordered, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sample_tiles) {
+          tiles = sample_tiles < tiles ? sample_tiles : tiles;
+          if (first >= random_waves || first >= tiles) return;
+          if (waves > random_waves) waves = random_waves;
+        }
       }
     }
 #pragma unroll
@@ -266,13 +272,19 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_settle(uint32_t* par, uint32_t 
 // Most frequent root among kModeSamples vertices, each sample climbing to its
 // root (one hop on a settled forest): of edges spread over the list (their first
 // endpoints), or without a list of vertices spread over [0, n).  out[0] = the
-// root, out[1] = its samples (with a list only).  Only a performance choice: any root gives correct
-// labels.
+// root, out[1] = its samples (with a list only).  Only a performance choice: any root
+// gives correct labels.  unordered (may be null): where it holds 0, out[0] = kNoRoot.
+constexpr uint32_t kNoRoot = ~0u;
+
 __global__ void __launch_bounds__(1024) k_cc_mode(const cac_uedge* __restrict__ edges, uint64_t m,
                                                   const uint32_t* __restrict__ par, uint32_t n,
-                                                  uint32_t* __restrict__ out) {
+                                                  const uint32_t* __restrict__ unordered, uint32_t* __restrict__ out) {
   __shared__ uint32_t key[kModeTable], cnt[kModeTable];
   __shared__ uint64_t best_w[1024 / 64];
+  if (unordered && *unordered == 0) {
+    if (threadIdx.x == 0) out[0] = kNoRoot;
+    return;
+  }
   for (int i = threadIdx.x; i < kModeTable; i += 1024) {
     key[i] = ~0u;
     cnt[i] = 0;
@@ -313,10 +325,12 @@ __global__ void __launch_bounds__(1024) k_cc_mode(const cac_uedge* __restrict__ 
   }
 }
 
-// bits[v / 64] bit (v % 64) = (par[v] == root); one ballot per 64 vertices.
+// bits[v / 64] bit (v % 64) = (par[v] == root); one ballot per 64 vertices.  Nothing
+// for kNoRoot.
 __global__ void __launch_bounds__(kCcBlock) k_cc_bitmap(const uint32_t* __restrict__ par, uint32_t n,
                                                         const uint32_t* __restrict__ root, uint64_t* __restrict__ bits) {
   const uint32_t R = root[0];
+  if (R == kNoRoot) return;
   const int lane = threadIdx.x & 63;
   const uint64_t waves = (uint64_t)gridDim.x * (kCcBlock / 64);
   for (uint64_t w = (uint64_t)blockIdx.x * (kCcBlock / 64) + (threadIdx.x >> 6); w * 64 < n; w += waves) {
@@ -327,11 +341,17 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_bitmap(const uint32_t* __restri
   }
 }
 
+__device__ inline bool bit_of(const uint32_t* bits, uint32_t x) { return (bits[x >> 5] >> (x & 31)) & 1u; }
 
 // Thread t of the grid owns edges t, t + T, t + 2T, ... (T = total threads) so
 // each load instruction is coalesced; kEdgesPerThread loads are issued before
-// any is consumed.
-__global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restrict__ edges, uint64_t m, uint32_t* par) {
+// any is consumed.  kBits: unless *root is kNoRoot, an edge with both ends in the
+// giant component is dropped before its parents are read, two lines each.
+template <bool kBits>
+__global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restrict__ edges, uint64_t m, uint32_t* par,
+                                                      const uint32_t* __restrict__ root,
+                                                      const uint32_t* __restrict__ bits) {
+  const bool use_bits = kBits && *root != kNoRoot;
   const uint64_t T = (uint64_t)gridDim.x * kCcBlock;
   uint64_t i0 = (uint64_t)blockIdx.x * kCcBlock + threadIdx.x;
   for (; i0 < m; i0 += T * kEdgesPerThread) {
@@ -342,16 +362,21 @@ __global__ void __launch_bounds__(kCcBlock) k_cc_hook(const cac_uedge* __restric
       e[k] = i < m ? ld_edge_nt(edges, i) : 0ull;  // empty slot = loop (0, 0)
     }
     // all parent lookups of the batch are in flight before any is consumed
+    bool live[kEdgesPerThread];
+#pragma unroll
+    for (int k = 0; k < kEdgesPerThread; ++k) {
+      const uint32_t a = (uint32_t)e[k], b = (uint32_t)(e[k] >> 32);
+      live[k] = a != b && !(use_bits && bit_of(bits, a) && bit_of(bits, b));
+    }
     uint32_t pu[kEdgesPerThread], pv[kEdgesPerThread];
 #pragma unroll
     for (int k = 0; k < kEdgesPerThread; ++k) {
-      const bool live = (uint32_t)e[k] != (uint32_t)(e[k] >> 32);
-      pu[k] = live ? ld_par(par, (uint32_t)e[k]) : 0u;
-      pv[k] = live ? ld_par(par, (uint32_t)(e[k] >> 32)) : 0u;
+      pu[k] = live[k] ? ld_par(par, (uint32_t)e[k]) : 0u;
+      pv[k] = live[k] ? ld_par(par, (uint32_t)(e[k] >> 32)) : 0u;
     }
 #pragma unroll
     for (int k = 0; k < kEdgesPerThread; ++k) {
-      if (pu[k] == pv[k]) continue;
+      if (!live[k] || pu[k] == pv[k]) continue;
       uf_link_from(par, (uint32_t)e[k], pu[k], (uint32_t)(e[k] >> 32), pv[k]);
     }
   }
@@ -1222,7 +1247,7 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
   prof_begin(ctx, "cc_init", s);
   hipLaunchKernelGGL(k_cc_init, dim3(grid_for(n, kCcBlock, cap)), dim3(kCcBlock), 0, s, d_lab, n);
   prof_end(ctx, s);
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, d_counter, 1);
+  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, d_counter, 4);
   const bool use_sample = m >= kSampleMinEdges;
   // Below one and a half edges a vertex the first pass links every edge of an
   // unordered list, or most of a short sorted one, and what is left is cheaper to
@@ -1230,6 +1255,11 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
   // blocks of 1024 in 2^18 with m = 4n 152 against 198, but R-MAT 2^18 with
   // m = 16n 1027 against 425, uniform 2^18 with m = 4n 483 against 430).
   const bool giant = use_sample && m >= (uint64_t)n / 2 * 3;
+  // There a list in no order whose parents are past an XCD's L2 makes the
+  // plain hook read two random parents an edge; it drops the giant
+  // component's edges by the bitmap (n 2^24, m 10.5M: 371 us plain, 188 with the
+  // bitmap and its making).
+  const bool bitmap = use_sample && !giant && n > kQueueMinN;
   if (use_sample) {
     uint32_t* d_root = d_counter + 1;
     uint64_t* d_bits = (uint64_t*)(d_counter + kCcTmpHead);
@@ -1238,25 +1268,28 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
     const uint64_t sample_tiles = m < (uint64_t)n / 4 * 3 ? 0 : ((uint64_t)n * 3 / 2 + kTileEdges - 1) / kTileEdges;
     if (n > kQueueMinN)
       hipLaunchKernelGGL(k_cc_runs<true>, dim3(gr), dim3(kCcBlock), 0, s, d_edges, m, d_lab, sample_tiles,
-                         random_waves(n));
+                         random_waves(n), d_counter + 3);
     else
       hipLaunchKernelGGL(k_cc_runs<false>, dim3(gr), dim3(kCcBlock), 0, s, d_edges, m, d_lab, sample_tiles,
-                         random_waves(n));
+                         random_waves(n), d_counter + 3);
     prof_end(ctx, s);
     prof_begin(ctx, "cc_settle", s);
     hipLaunchKernelGGL(k_cc_settle, dim3(grid_for(n, kCcBlock, cap)), dim3(kCcBlock), 0, s, d_lab, n);
     prof_end(ctx, s);
-    if (giant) {
+    const uint32_t words = map_words(n), shift = map_shift(n);
+    if (giant || bitmap) {
       prof_begin(ctx, "cc_bitmap", s);
-      hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, d_edges, m, (const uint32_t*)d_lab, n, d_root);
-      hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, cap)), dim3(kCcBlock), 0, s,
-                         (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
-      const uint32_t words = map_words(n), shift = map_shift(n);
+      hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, d_edges, m, (const uint32_t*)d_lab, n,
+                         giant ? (const uint32_t*)nullptr : d_counter + 3, d_root);
+      hipLaunchKernelGGL(k_cc_bitmap, dim3(grid_for(((uint64_t)n + 63) / 64, kCcBlock / 64, giant ? cap : 2048)),
+                         dim3(kCcBlock), 0, s, (const uint32_t*)d_lab, n, (const uint32_t*)d_root, d_bits);
       if (shift == 0) d_map = reinterpret_cast<uint32_t*>(d_bits);  // the bitmap itself
-      else
+      else if (giant)
         hipLaunchKernelGGL(k_cc_coarse, dim3((words + kCcBlock - 1) / kCcBlock), dim3(kCcBlock), 0, s,
                            (const uint32_t*)d_bits, n, shift, d_map, words);
       prof_end(ctx, s);
+    }
+    if (giant) {
       prof_begin(ctx, "cc_hook", s);
       const int rc = hook_attr(ctx);
       if (rc) return rc;
@@ -1269,7 +1302,12 @@ int cc_launch(cac_ctx* ctx, const cac_uedge* d_edges, uint64_t m, uint32_t n, in
   if (m && !giant) {
     prof_begin(ctx, "cc_hook", s);
     unsigned g = grid_for((m + kEdgesPerThread - 1) / kEdgesPerThread, kCcBlock, 256 * 32);
-    hipLaunchKernelGGL(k_cc_hook, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab);
+    if (bitmap)
+      hipLaunchKernelGGL(k_cc_hook<true>, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab,
+                         (const uint32_t*)(d_counter + 1), (const uint32_t*)(d_counter + kCcTmpHead));
+    else
+      hipLaunchKernelGGL(k_cc_hook<false>, dim3(g), dim3(kCcBlock), 0, s, d_edges, m, d_lab, (const uint32_t*)nullptr,
+                         (const uint32_t*)nullptr);
     prof_end(ctx, s);
   }
   prof_begin(ctx, "cc_compress", s);
@@ -1341,7 +1379,7 @@ int cc_csr_launch(cac_ctx* ctx, const uint32_t* d_off, const uint32_t* d_cols, u
   if (lo >= n) {  // no bulk range (n within the hub prefixes): a separate sampling launch
     prof_begin(ctx, "af_mode", s);
     hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(1024), 0, s, (const cac_uedge*)nullptr, 0, (const uint32_t*)d_lab, n,
-                       d_counter + 1);
+                       (const uint32_t*)nullptr, d_counter + 1);
     prof_end(ctx, s);
   }
   prof_begin(ctx, "af_final", s);
