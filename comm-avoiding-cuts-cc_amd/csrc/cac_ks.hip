@@ -1249,7 +1249,7 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
   std::vector<size_t> group;  // first child of each block-size class, then nchild
   size_t c0 = 0;
   while (c0 < nchild) {
-    int B = contract_block(ctx, ch[c0].s);
+    const int B = contract_block(ctx, ch[c0].s);
     size_t c1 = c0;
     uint32_t smax = 0;
     const bool list = ch[c0].parent == nullptr;
@@ -1257,14 +1257,11 @@ int contract_level(cac_ctx* ctx, const std::vector<KsChild<E>>& ch, KsChild<E>* 
       smax = std::max(smax, ch[c1++].s);
     const uint32_t cnt = (uint32_t)(c1 - c0);
     group.push_back(c0);
-    // Fewer children than CUs (the top levels of a small solve): the device is
-    // idle but for these workgroups, and with 64-bit entries a wider block
-    // shortens each pick's row scans (ER(1000, 0.05) square_root: contraction
-    // 1.5 -> 1.33 ms per solve).  With many children the narrow block keeps
-    // occupancy up, and with 32-bit entries the one wavefront of a child of
-    // s <= 512 has two pieces to scan and no barriers to wait at (the same
-    // solve: contraction 0.82 ms with 64 threads, 0.86 with 128, 0.90 with 256).
-    if (sizeof(E) == 8 && cnt < kFewChildren && B < 256) B = 256;
+    // The narrow block also where children are fewer than CUs: its wavefronts have
+    // several pieces of a row to scan and fewer barriers to wait at (square_root of
+    // G(1000, 0.05): contraction 0.82 ms with 64 threads, 0.86 with 128, 0.90 with
+    // 256; of G(1000, 0.02) with weights to 2^30, 64-bit entries: the solve 1.37
+    // ms with 64, 1.38 with 128, 1.42 with 256).
     if (B == 1024) launch_contract<1024, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
     else if (B == 512) launch_contract<512, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
     else if (B == 256) launch_contract<256, E>(d_children + c0, cnt, smax, list, d_kout + c0, d_results, s);
