@@ -91,15 +91,22 @@ __global__ void __launch_bounds__(256) k_mixed_weights(const EdgeSpan* spans) {
   uint64_t sum = 0;
   for (uint64_t base = (uint64_t)blockIdx.x * kPackTile; base < sp.m; base += (uint64_t)gridDim.x * kPackTile) {
     uint32_t tile = 0;
-#pragma unroll 4
-    for (int k = 0; k < kPackItems; ++k) {
-      const uint64_t e = base + (uint64_t)k * 256 + threadIdx.x;
-      if (e >= sp.m) break;
-      const cac_edge x = sp.edges[e];
-      bad = bad || x.w != w0 || x.u == x.v;
-      sum += min((uint64_t)x.w, (uint64_t)kTrialW32Total);
-      if (x.u != x.v) tile += (uint32_t)x.w;
-      if (sp.pk) sp.pk[e] = x.u | (x.v << 16);
+    for (int k0 = 0; k0 < kPackItems; k0 += kPackItems / 2) {
+      cac_edge x[kPackItems / 2];  // in flight together: a graph of a few tiles waits for each step
+#pragma unroll
+      for (int k = 0; k < kPackItems / 2; ++k) {
+        const uint64_t e = base + (uint64_t)(k0 + k) * 256 + threadIdx.x;
+        x[k] = e < sp.m ? sp.edges[e] : cac_edge{0, 1, w0};  // changes no flag; its weight is not counted
+      }
+#pragma unroll
+      for (int k = 0; k < kPackItems / 2; ++k) {
+        const uint64_t e = base + (uint64_t)(k0 + k) * 256 + threadIdx.x;
+        bad = bad || x[k].w != w0 || x[k].u == x[k].v;
+        if (e >= sp.m) continue;
+        sum += min((uint64_t)x[k].w, (uint64_t)kTrialW32Total);
+        if (x[k].u != x[k].v) tile += (uint32_t)x[k].w;
+        if (sp.pk) sp.pk[e] = x[k].u | (x[k].v << 16);
+      }
     }
     if (sp.pk) {
       tile = wave_sum<uint32_t>(tile);
@@ -1273,11 +1280,10 @@ __global__ void k_lt_set(int64_t* p, const unsigned long long* v) {
 
 inline GraphKey graph_key(const SqrtJob& j) { return {j.edges, j.m, j.n}; }
 
-// Whether a job's graph is packed: not when it is known to be too heavy for trials
-// in 32 bits.
-inline bool can_pack(const SqrtJob& j) {
-  return j.n <= kPackMaxN && j.m < kPackMaxM && (j.total == kTotalUnknown || j.total < kTrialW32Total);
-}
+// Whether a job's trials may run in 32 bits: not those of a graph known to be too heavy.
+inline bool may_w32(const SqrtJob& j) { return j.total == kTotalUnknown || j.total < kTrialW32Total; }
+// Whether a job's graph is packed.
+inline bool can_pack(const SqrtJob& j) { return j.n <= kPackMaxN && j.m < kPackMaxM && may_w32(j); }
 
 // Points scr[i].mixed and scr[i].total at a flag word and a total weight of its
 // graph (one per distinct graph) and launches the kernels that set them;
@@ -1865,8 +1871,9 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     if (rc) return rc;
     e = hipMemcpyAsync(d_scr, scr.data(), nb * sizeof(TrialScratch), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "job descriptors");
-    bool from_matrix = false;  // some trial's lists may come from its matrix
-    for (size_t i = 0; i < nb; ++i) from_matrix = from_matrix || (!scr[i].pk && scr[i].t > kKsBase);
+    bool from_matrix = false;  // some trial's lists may come from its matrix, if that has 4-byte entries
+    for (size_t i = 0; i < nb; ++i)
+      from_matrix = from_matrix || (!scr[i].pk && scr[i].t > kKsBase && may_w32(jobs[b0 + i]));
     if (rc == CAC_OK && from_matrix)
       hipLaunchKernelGGL(k_zero_live, dim3(grid_for(2 * nb, 256, 64)), dim3(256), 0, s, d_live, (uint32_t)(2 * nb));
     if (rc == CAC_OK && wide) {
