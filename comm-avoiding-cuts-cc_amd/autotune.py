@@ -109,9 +109,9 @@ def tune(device: int = 0, reps: int = 3, log=print):
     return table, timings
 
 
-# (class key, graph, trials): one graph per edge-count class and enough trials
-# to fill the device several times over.
-SAMPLE_CLASSES = ((16, ("er", 2000, 20.0), 4096), (20, ("ws", 32000, 16), 2048), (24, ("er", 100000, 100.0), 512))
+# (class key, graph, trials): one graph per edge-count class, of vertices whose labels
+# leave LDS for two workgroups, and enough trials to fill the device several times over.
+SAMPLE_CLASSES = ((16, ("er", 2000, 20.0), 4096), (20, ("er", 8000, 60.0), 2048), (24, ("er", 100000, 100.0), 512))
 
 
 def _sample_graph(spec):
