@@ -26,11 +26,21 @@ __global__ void __launch_bounds__(256) k_check_edges(const cac_edge* e, uint64_t
   __shared__ unsigned long long part[4];
   uint32_t b = 0;
   unsigned long long s = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (uint64_t)gridDim.x * blockDim.x) {
-    const cac_edge x = e[i];
-    if (x.u >= n || x.v >= n) b = 1;
-    if (x.w >= (1ull << 40)) b |= 2;  // single weights this large would risk int64 sums
-    else s += x.w;
+  constexpr int kPer = 8;  // edges of a thread in flight: a short list is one step
+  for (uint64_t base = (uint64_t)blockIdx.x * 256 * kPer; base < m; base += (uint64_t)gridDim.x * 256 * kPer) {
+    cac_edge x[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const uint64_t i = base + (uint64_t)k * 256 + threadIdx.x;
+      x[k] = i < m ? e[i] : cac_edge{0, 0, 0};
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const bool in = base + (uint64_t)k * 256 + threadIdx.x < m;
+      if (in && (x[k].u >= n || x[k].v >= n)) b |= 1;
+      if (x[k].w >= (1ull << 40)) b |= 2;  // single weights this large would risk int64 sums
+      else s += x[k].w;
+    }
   }
   if (b) atomicOr(bad, b);
   s = wave_sum<uint64_t>(s);

@@ -1920,11 +1920,13 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
     std::vector<int64_t> hb(nb);
     std::vector<unsigned long long> totals(nb);
     std::vector<uint32_t> live(2 * nb, 0u);
+    bool summed = true;  // every graph's total came with its jobs
+    for (size_t i = 0; i < nb; ++i) summed = summed && jobs[b0 + i].total != kTotalUnknown;
     if (rc == CAC_OK) {
       if (pack_bytes || from_matrix) (void)hipMemcpyAsync(live.data(), d_live, 8 * nb, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(nvs.data(), d_nv, nb * 4, hipMemcpyDeviceToHost, s);
       (void)hipMemcpyAsync(hb.data(), d_bounds, nb * 8, hipMemcpyDeviceToHost, s);
-      (void)hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s);
+      if (!summed) (void)hipMemcpyAsync(totals.data(), d_totals, nb * 8, hipMemcpyDeviceToHost, s);
       e = hipStreamSynchronize(s);
       if (e != hipSuccess) rc = hip_fail(ctx, e, "sampling kernels");
     }
@@ -1932,8 +1934,9 @@ static int sqrt_dense_chunks(cac_ctx* ctx, const std::vector<SqrtJob>& jobs, int
       std::vector<KsRoot> roots;
       for (size_t i = 0; i < nb; ++i)
         if (nvs[i] >= 2 && nvs[i] <= scr[i].t) {
+          const uint64_t total = summed ? jobs[b0 + i].total : totals[scr[i].total - d_totals];
           KsRoot r{scr[i].mat, scr[i].rsum, nvs[i], scr[i].trial, scr[i].slot, hb[i], scr[i].seed, 1,
-                   totals[scr[i].total - d_totals] < kTrialW32Total};
+                   total < kTrialW32Total};
           const bool in_place = scr[i].pk && live[2 * i + 1] == 2;
           const bool behind = !scr[i].pk && from_matrix && rows_from_matrix(r.n) && live[2 * i + 1] == 0;
           if (r.w32 && (in_place || behind)) {
