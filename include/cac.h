@@ -296,7 +296,8 @@ int cac_mincut_dev(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n
  * Many independent graphs in one call.  The reference solves one graph per MPI
  * job (src/SquareRootCut.cpp:15-25, src/executables/square_root.cpp); there is
  * no batch interface to replace.  Graph g's edges are
- * d_edges[edge_offset .. edge_offset + m) with ids local to the graph (< n).
+ * d_edges[edge_offset .. edge_offset + m) with ids local to the graph (< n);
+ * the ranges of graphs may overlap (prefixes of one list, say).
  * Graph g runs square-root-cut trials 0 .. T_g - 1 exactly as cac_mincut would
  * on that graph alone (t = cac_intermediate_size(n, m)), so every cut equals the
  * one-graph result with the same T_g:
