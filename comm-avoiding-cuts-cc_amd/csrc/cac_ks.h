@@ -77,6 +77,7 @@ struct SqrtChunk {
 // The chunk that starts at `first`: as many jobs as fit the budget, at least one.
 // rule: the sampling rule (CAC_SAMPLE_*); wide: the jobs run in the wide form.
 SqrtChunk sqrt_chunk(const std::vector<SqrtJob>& jobs, size_t first, size_t budget, bool wide, int rule);
+size_t even_share(size_t all, size_t most, size_t budget);
 // Sqrt-cut trials on a device edge list: raw cut of trial_ids[i] to d_results[i].
 // total: the graph's total weight, or kTotalUnknown.
 int sqrt_cut_run(cac_ctx* ctx, const cac_edge* d_edges, uint64_t m, uint32_t n, uint32_t t, uint32_t seed,
